@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "device_utils.h"
+#include "host_staging.h"
 #include "kernels.h"
 
 using namespace mummu;
@@ -74,9 +75,7 @@ struct mummu_moe {
     mummu_moe_config cfg{};
     std::vector<Layer> layers;
     hipStream_t stream = nullptr;
-    // pinned host staging for the host-pointer entry points: [input | output | flags]; small calls go through
-    // it with asynchronous copies and one synchronisation
-    uint8_t *pin = nullptr;
+    bool staging = false;   // this handle holds the pool of pinned slabs open
     std::mutex mu;
     mutable std::string err;
 
@@ -326,7 +325,7 @@ int reset_flags(mummu_moe *h) {
     return MUMMU_OK;
 }
 
-int flags_to_status(mummu_moe *h, const int32_t *f);
+int flags_to_status(mummu_moe *h, const int32_t *f, int n_experts);
 
 constexpr unsigned long long kFallbacksBeforeGivingUp = 64;
 
@@ -346,90 +345,60 @@ int check_flags(mummu_moe *h, hipStream_t s) {
         if (fb - h->fallbacks_seen >= kFallbacksBeforeGivingUp) h->router_exchange = 0;
         h->fallbacks_seen = fb;
     }
-    return flags_to_status(h, f);
+    return flags_to_status(h, f, h->cfg.num_experts);
 }
 
-int flags_to_status(mummu_moe *h, const int32_t *f) {
+// (n_experts: the row length of the logits the call routed)
+int flags_to_status(mummu_moe *h, const int32_t *f, int n_experts) {
     if (f[FLAG_NONFINITE] == 0 && f[FLAG_BAD_ID] == 0) return MUMMU_OK;
     int rc = reset_flags(h);
     if (rc != MUMMU_OK) return rc;
     if (f[FLAG_NONFINITE]) {
-        const int E = h->cfg.num_experts;
         char buf[160];
-        snprintf(buf, sizeof(buf), "router logit for token %d expert %d is not finite", f[FLAG_NONFINITE_INDEX] / E,
-                 f[FLAG_NONFINITE_INDEX] % E);
+        snprintf(buf, sizeof(buf), "router logit for token %d expert %d is not finite", f[FLAG_NONFINITE_INDEX] / n_experts,
+                 f[FLAG_NONFINITE_INDEX] % n_experts);
         return fail(h, MUMMU_ERR_NONFINITE, buf);
     }
     return fail(h, MUMMU_ERR_RANGE, "a routed expert id is out of range");
 }
 
-// Host-pointer calls of up to kPinIO bytes each way: the input is staged through pinned memory (the
-// copy is then truly asynchronous), and the output and the error flags come back with one
-// synchronisation instead of one per copy.  Larger calls copy straight from / to the caller's memory.
-constexpr size_t kPinIO = 256 * 1024;
-
-// The routing of n*k pairs back to the caller (ids, weights; logits too when asked for) under one
-// synchronisation, with the error flags.
-int download_routing(mummu_moe *h, int32_t *ids, float *weights, size_t pairs, float *logits, size_t n_logits, hipStream_t s);
-
-// (pin_offset: where in the input half this upload is staged - a call with two inputs gives each its own place)
-int upload_rows(mummu_moe *h, float *dev, const float *host, size_t bytes, hipStream_t s, size_t pin_offset = 0) {
-    if (h->pin && pin_offset + bytes <= kPinIO) {
-        memcpy(h->pin + pin_offset, host, bytes);
-        HIPCHK(h, hipMemcpyAsync(dev, h->pin + pin_offset, bytes, hipMemcpyHostToDevice, s));
-    } else {
-        HIPCHK(h, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
-    }
+// The host-pointer entry points move their rows through pinned memory (HostStaging); without any to be had they copy
+// straight from / to the caller's memory.
+int upload_rows(mummu_moe *h, HostStaging &io, void *dev, const void *host, size_t bytes, hipStream_t s) {
+    if (io.valid()) HIPCHK(h, io.upload(dev, host, bytes, s));
+    else HIPCHK(h, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
     return MUMMU_OK;
 }
 
-// Wait for the stream, report what the device flagged, hand the result rows to the caller.
-int download_rows(mummu_moe *h, float *host, const float *dev, size_t bytes, hipStream_t s, bool with_flags) {
-    if (h->pin && bytes <= kPinIO) {
-        int32_t *pf = (int32_t *)(h->pin + 2 * kPinIO);
-        if (with_flags) HIPCHK(h, hipMemcpyAsync(pf, h->flags, sizeof(int32_t) * kFlagWords, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipMemcpyAsync(h->pin + kPinIO, dev, bytes, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipStreamSynchronize(s));
-        if (with_flags) {
-            const int rc = flags_to_status(h, pf);
-            if (rc) return rc;
-        }
-        memcpy(host, h->pin + kPinIO, bytes);
-        return MUMMU_OK;
+// Wait for the stream, report what the device flagged, hand the result arrays to the caller.
+int download(mummu_moe *h, HostStaging &io, const HostStaging::Piece *pieces, int n, bool with_flags, int n_experts, hipStream_t s) {
+    int status = MUMMU_OK;
+    if (io.valid()) {
+        HIPCHK(h, io.download(pieces, n, with_flags ? h->flags : nullptr, sizeof(int32_t) * kFlagWords, s,
+                              [&](const void *f) { return flags_to_status(h, (const int32_t *)f, n_experts); }, &status));
+        return status;
     }
+    HIPCHK(h, hipStreamSynchronize(s));
     if (with_flags) {
-        const int rc = check_flags(h, s);
-        if (rc) return rc;
-    } else {
-        HIPCHK(h, hipStreamSynchronize(s));
+        int32_t f[kFlagWords];
+        HIPCHK(h, hipMemcpy(f, h->flags, sizeof(f), hipMemcpyDeviceToHost));
+        if ((status = flags_to_status(h, f, n_experts))) return status;
     }
-    HIPCHK(h, hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
+    for (int i = 0; i < n; i++) HIPCHK(h, hipMemcpy(pieces[i].host, pieces[i].dev, pieces[i].bytes, hipMemcpyDeviceToHost));
     return MUMMU_OK;
 }
 
-int download_routing(mummu_moe *h, int32_t *ids, float *weights, size_t pairs, float *logits, size_t n_logits, hipStream_t s) {
-    const size_t ib = sizeof(int32_t) * pairs, wb = sizeof(float) * pairs, lb = logits ? sizeof(float) * n_logits : 0;
-    if (h->pin && ib + wb + lb <= kPinIO) {
-        uint8_t *p = h->pin + kPinIO;
-        int32_t *pf = (int32_t *)(h->pin + 2 * kPinIO);
-        HIPCHK(h, hipMemcpyAsync(pf, h->flags, sizeof(int32_t) * kFlagWords, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipMemcpyAsync(p, h->ids, ib, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipMemcpyAsync(p + ib, h->weights, wb, hipMemcpyDeviceToHost, s));
-        if (lb) HIPCHK(h, hipMemcpyAsync(p + ib + wb, h->logits, lb, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipStreamSynchronize(s));
-        const int rc = flags_to_status(h, pf);
-        if (rc) return rc;
-        memcpy(ids, p, ib);
-        memcpy(weights, p + ib, wb);
-        if (lb) memcpy(logits, p + ib + wb, lb);
-        return MUMMU_OK;
-    }
-    const int rc = check_flags(h, s);
-    if (rc) return rc;
-    HIPCHK(h, hipMemcpy(ids, h->ids, ib, hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(weights, h->weights, wb, hipMemcpyDeviceToHost));
-    if (lb) HIPCHK(h, hipMemcpy(logits, h->logits, lb, hipMemcpyDeviceToHost));
-    return MUMMU_OK;
+int download_rows(mummu_moe *h, HostStaging &io, void *host, const void *dev, size_t bytes, hipStream_t s, bool with_flags) {
+    const HostStaging::Piece p{host, dev, bytes};
+    return download(h, io, &p, 1, with_flags, h->cfg.num_experts, s);
+}
+
+// The routing of n*k pairs (ids, weights; logits too when asked for).
+int download_routing(mummu_moe *h, HostStaging &io, int32_t *ids, float *weights, size_t pairs, float *logits, size_t n_logits,
+                     int n_experts, hipStream_t s) {
+    const HostStaging::Piece p[3] = {{ids, h->ids, sizeof(int32_t) * pairs}, {weights, h->weights, sizeof(float) * pairs},
+                                     {logits, h->logits, sizeof(float) * n_logits}};
+    return download(h, io, p, logits ? 3 : 2, true, n_experts, s);
 }
 
 // Per-kernel timing: binds a pair of pooled events to the one kernel the enclosed launcher
@@ -1065,10 +1034,8 @@ int mummu_moe_create(const mummu_moe_config *cfg, mummu_moe **out) {
     };
     if (hipSetDevice(0) != hipSuccess) return bail(fail(h, MUMMU_ERR_DEVICE, "hipSetDevice(0) failed"));
     if (hipStreamCreate(&h->stream) != hipSuccess) return bail(fail(h, MUMMU_ERR_DEVICE, "hipStreamCreate failed"));
-    if (hipHostMalloc((void **)&h->pin, 2 * kPinIO + 64, hipHostMallocDefault) != hipSuccess) {
-        h->pin = nullptr;  // not fatal: the calls then copy straight from the caller's memory
-        (void)hipGetLastError();
-    }
+    HostStaging::retain();
+    h->staging = true;
     if (hipEventCreate(&h->t0) != hipSuccess || hipEventCreate(&h->t1) != hipSuccess)
         return bail(fail(h, MUMMU_ERR_DEVICE, "hipEventCreate failed"));
     if (hipMalloc(&h->flags, sizeof(int32_t) * kFlagWords) != hipSuccess) return bail(fail(h, MUMMU_ERR_DEVICE, "hipMalloc(flags) failed"));
@@ -1123,8 +1090,8 @@ void mummu_moe_destroy(mummu_moe *h) {
     for (auto e : h->event_pool) (void)hipEventDestroy(e);
     if (h->t0) (void)hipEventDestroy(h->t0);
     if (h->t1) (void)hipEventDestroy(h->t1);
-    if (h->pin) (void)hipHostFree(h->pin);
     if (h->stream) (void)hipStreamDestroy(h->stream);
+    if (h->staging) HostStaging::release();
     delete h;
 }
 
@@ -1287,9 +1254,10 @@ int mummu_moe_forward(mummu_moe *h, int layer, const float *x, int64_t n, int to
     if (!x || !out) return fail(h, MUMMU_ERR_ARG, "null buffer");
     if ((rc = ensure_ws(h, n, n * top_k, 0))) return rc;
     const size_t bytes = sizeof(float) * (size_t)n * (size_t)h->cfg.hidden_size;
-    if ((rc = upload_rows(h, h->xin, x, bytes, h->stream))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, x, bytes, h->stream))) return rc;
     if ((rc = forward_impl(h, layer, h->xin, n, top_k, norm, nullptr, h->xout, h->stream))) return rc;
-    return download_rows(h, out, h->xout, bytes, h->stream, true);
+    return download_rows(h, io, out, h->xout, bytes, h->stream, true);
 }
 
 int mummu_moe_forward_typed(mummu_moe *h, int layer, const void *x, int x_type, int64_t n, int top_k, int norm, void *out) {
@@ -1311,7 +1279,8 @@ int mummu_moe_forward_typed(mummu_moe *h, int layer, const void *x, int x_type, 
     const dim3 grid((unsigned)((count + 255) / 256)), block(256);
     // the 16-bit rows land in the output buffer (not yet needed), are widened into the input buffer, and after the
     // block has run the f32 result is narrowed into the input buffer (no longer needed) and read back from there
-    if ((rc = upload_rows(h, h->xout, (const float *)x, bytes16, s))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xout, x, bytes16, s))) return rc;
     if (x_type == MUMMU_F16) launch_kernel(widen_rows_kernel<T_F16>, grid, block, 0, s, (const uint16_t *)h->xout, count, h->xin);
     else launch_kernel(widen_rows_kernel<T_BF16>, grid, block, 0, s, (const uint16_t *)h->xout, count, h->xin);
     HIPCHK(h, hipGetLastError());
@@ -1319,7 +1288,7 @@ int mummu_moe_forward_typed(mummu_moe *h, int layer, const void *x, int x_type, 
     if (x_type == MUMMU_F16) launch_kernel(narrow_rows_kernel<T_F16>, grid, block, 0, s, (const float *)h->xout, count, (uint16_t *)h->xin);
     else launch_kernel(narrow_rows_kernel<T_BF16>, grid, block, 0, s, (const float *)h->xout, count, (uint16_t *)h->xin);
     HIPCHK(h, hipGetLastError());
-    return download_rows(h, (float *)out, h->xin, bytes16, s, true);
+    return download_rows(h, io, out, h->xin, bytes16, s, true);
 }
 
 int mummu_moe_route(mummu_moe *h, int layer, const float *x, int64_t n, int top_k, int norm, int32_t *ids, float *weights,
@@ -1337,11 +1306,12 @@ int mummu_moe_route(mummu_moe *h, int layer, const float *x, int64_t n, int top_
     const Layer &L = h->layers[layer];
     const int E = h->cfg.num_experts, H = h->cfg.hidden_size;
     hipStream_t s = h->stream;
-    HIPCHK(h, hipMemcpyAsync(h->xin, x, sizeof(float) * (size_t)n * H, hipMemcpyHostToDevice, s));
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, x, sizeof(float) * (size_t)n * (size_t)H, s))) return rc;
     LAUNCH(h, K_ROUTER_LOGITS, s, launch_router_logits(h->xin, L.router, L.router_type, h->logits, (int)n, H, E, QAct(), s));
     LAUNCH(h, K_ROUTE_TOPK, s,
            launch_route_topk(h->logits, (int)n, E, top_k, h->cfg.router_flavour, norm, h->ids, h->weights, nullptr, h->flags, s));
-    return download_routing(h, ids, weights, (size_t)(n * top_k), logits, (size_t)n * (size_t)E, s);
+    return download_routing(h, io, ids, weights, (size_t)(n * top_k), logits, (size_t)n * (size_t)E, E, s);
 }
 
 int mummu_route_logits(mummu_moe *h, const float *logits, int64_t n, int n_experts, int top_k, int flavour, int norm,
@@ -1360,21 +1330,10 @@ int mummu_route_logits(mummu_moe *h, const float *logits, int64_t n, int n_exper
     int rc = ensure_ws(h, n, n * top_k, n_experts);
     if (rc) return rc;
     hipStream_t s = h->stream;
-    HIPCHK(h, hipMemcpyAsync(h->logits, logits, sizeof(float) * (size_t)n * n_experts, hipMemcpyHostToDevice, s));
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->logits, logits, sizeof(float) * (size_t)n * (size_t)n_experts, s))) return rc;
     LAUNCH(h, K_ROUTE_TOPK, s, launch_route_topk(h->logits, (int)n, n_experts, top_k, flavour, norm, h->ids, h->weights, nullptr, h->flags, s));
-    HIPCHK(h, hipStreamSynchronize(s));
-    int32_t f[4];
-    HIPCHK(h, hipMemcpy(f, h->flags, sizeof(f), hipMemcpyDeviceToHost));
-    if (f[FLAG_NONFINITE]) {
-        if ((rc = reset_flags(h))) return rc;
-        char buf[160];
-        snprintf(buf, sizeof(buf), "router logit for token %d expert %d is not finite", f[FLAG_NONFINITE_INDEX] / n_experts,
-                 f[FLAG_NONFINITE_INDEX] % n_experts);
-        return fail(h, MUMMU_ERR_NONFINITE, buf);
-    }
-    HIPCHK(h, hipMemcpy(ids, h->ids, sizeof(int32_t) * (size_t)(n * top_k), hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(weights, h->weights, sizeof(float) * (size_t)(n * top_k), hipMemcpyDeviceToHost));
-    return MUMMU_OK;
+    return download_routing(h, io, ids, weights, (size_t)(n * top_k), nullptr, 0, n_experts, s);
 }
 
 int mummu_moe_apply_routing(mummu_moe *h, int layer, const int32_t *ids, const float *weights, const float *xs, int64_t n,
@@ -1395,9 +1354,10 @@ int mummu_moe_apply_routing(mummu_moe *h, int layer, const int32_t *ids, const f
     if ((rc = ensure_ws(h, n, n * top_k, 0))) return rc;
     hipStream_t s = h->stream;
     const size_t bytes = sizeof(float) * (size_t)n * (size_t)h->cfg.hidden_size;
-    HIPCHK(h, hipMemcpyAsync(h->xin, xs, bytes, hipMemcpyHostToDevice, s));
-    HIPCHK(h, hipMemcpyAsync(h->ids, ids, sizeof(int32_t) * (size_t)(n * top_k), hipMemcpyHostToDevice, s));
-    HIPCHK(h, hipMemcpyAsync(h->weights, weights, sizeof(float) * (size_t)(n * top_k), hipMemcpyHostToDevice, s));
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, xs, bytes, s))) return rc;
+    if ((rc = upload_rows(h, io, h->ids, ids, sizeof(int32_t) * (size_t)(n * top_k), s))) return rc;
+    if ((rc = upload_rows(h, io, h->weights, weights, sizeof(float) * (size_t)(n * top_k), s))) return rc;
     Layer &L = h->layers[layer];
     // hit counters, nn/moe.rs:1562-1564 (the routing came from the host, so count here)
     {
@@ -1409,7 +1369,7 @@ int mummu_moe_apply_routing(mummu_moe *h, int layer, const int32_t *ids, const f
         HIPCHK(h, hipMemcpy(L.hits, cur.data(), sizeof(unsigned long long) * cur.size(), hipMemcpyHostToDevice));
     }
     if ((rc = run_experts(h, L, h->xin, false, n, top_k, nullptr, h->xout, s))) return rc;
-    return download_rows(h, out, h->xout, bytes, s, true);
+    return download_rows(h, io, out, h->xout, bytes, s, true);
 }
 
 int mummu_moe_routed(mummu_moe *h, int layer, const float *router_logits, const float *xs, int64_t n, int top_k, float *out) {
@@ -1428,8 +1388,9 @@ int mummu_moe_routed(mummu_moe *h, int layer, const float *router_logits, const 
     const int E = h->cfg.num_experts, H = h->cfg.hidden_size;
     hipStream_t s = h->stream;
     const size_t lbytes = sizeof(float) * (size_t)n * (size_t)E, xbytes = sizeof(float) * (size_t)n * (size_t)H;
-    if ((rc = upload_rows(h, h->logits, router_logits, lbytes, s, 0))) return rc;
-    if ((rc = upload_rows(h, h->xin, xs, xbytes, s, lbytes <= kPinIO ? (lbytes + 63) / 64 * 64 : kPinIO))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->logits, router_logits, lbytes, s))) return rc;
+    if ((rc = upload_rows(h, io, h->xin, xs, xbytes, s))) return rc;
     const ExpertBanks b = banks_of(h, L);
     if (n <= 8 && n < batched_from(h, L) && is_quant_type(L.gate_type) && H % 64 == 0 && gate_up_routes_inline(b, top_k) &&
         down_combine_supported(b, top_k)) {
@@ -1444,12 +1405,12 @@ int mummu_moe_routed(mummu_moe *h, int layer, const float *router_logits, const 
         LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(h->xin, (int)n, H, h->xq, s));
         LAUNCH(h, K_GATE_UP, s, launch_gate_up_routed(b, h->xq, route, (int)n, top_k, h->actq, h->flags, s));
         LAUNCH(h, K_DOWN_COMBINE, s, launch_down_combine(b, h->actq, h->ids, h->weights, (int)n, top_k, nullptr, h->xout, s));
-        return download_rows(h, out, h->xout, xbytes, s, true);
+        return download_rows(h, io, out, h->xout, xbytes, s, true);
     }
     LAUNCH(h, K_ROUTE_TOPK, s,
            launch_route_topk(h->logits, (int)n, E, top_k, MUMMU_ROUTER_QWEN4EXP, 1, h->ids, h->weights, L.hits, h->flags, s));
     if ((rc = run_experts(h, L, h->xin, false, n, top_k, nullptr, h->xout, s))) return rc;
-    return download_rows(h, out, h->xout, xbytes, s, true);
+    return download_rows(h, io, out, h->xout, xbytes, s, true);
 }
 
 int mummu_expert_run(mummu_moe *h, int layer, int expert, const float *x, int64_t rows, int hidden, float *out) {
@@ -1468,12 +1429,13 @@ int mummu_expert_run(mummu_moe *h, int layer, int expert, const float *x, int64_
     if ((rc = ensure_ws(h, rows, rows, 0))) return rc;
     hipStream_t s = h->stream;
     const size_t bytes = sizeof(float) * (size_t)rows * (size_t)hidden;
-    if ((rc = upload_rows(h, h->xin, x, bytes, s))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, x, bytes, s))) return rc;
     ExpertBanks b = banks_of(h, h->layers[layer]);
     if (is_quant_type(b.gate_type)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(h->xin, (int)rows, hidden, h->xq, s));
     LAUNCH(h, K_GATE_UP, s, launch_gate_up(b, h->xin, h->xq, nullptr, (int)rows, 1, expert, h->act, h->actq, h->flags, s));
     LAUNCH(h, K_DOWN, s, launch_down(b, h->act, h->actq, nullptr, (int)rows, 1, expert, h->y, s));
-    return download_rows(h, out, h->y, bytes, s, false);
+    return download_rows(h, io, out, h->y, bytes, s, false);
 }
 
 int mummu_expert_gate_energy(mummu_moe *h, int layer, int expert, const float *x, int64_t rows, int hidden, float *energy) {
@@ -1492,7 +1454,8 @@ int mummu_expert_gate_energy(mummu_moe *h, int layer, int expert, const float *x
     if (hidden > 8192) return fail(h, MUMMU_ERR_SHAPE, "gate_energy: hidden above 8192 is not supported");
     if ((rc = ensure_ws(h, rows, rows, 0))) return rc;
     hipStream_t s = h->stream;
-    if ((rc = upload_rows(h, h->xin, x, sizeof(float) * (size_t)rows * (size_t)hidden, s))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, x, sizeof(float) * (size_t)rows * (size_t)hidden, s))) return rc;
     const Layer &L = h->layers[layer];
     const int I = h->cfg.expert_intermediate_size;
     const size_t n = (size_t)I * (size_t)hidden;
@@ -1537,9 +1500,10 @@ int mummu_moe_stack_forward(mummu_moe *h, const float *x, int64_t n, int top_k, 
     if (!x || !out) return fail(h, MUMMU_ERR_ARG, "null buffer");
     if ((rc = ensure_ws(h, n, n * top_k, 0))) return rc;
     const size_t bytes = sizeof(float) * (size_t)n * (size_t)h->cfg.hidden_size;
-    if ((rc = upload_rows(h, h->xin, x, bytes, h->stream))) return rc;
+    HostStaging io;
+    if ((rc = upload_rows(h, io, h->xin, x, bytes, h->stream))) return rc;
     if ((rc = stack_impl(h, h->xin, n, top_k, norm, h->xout, h->stream, ids))) return rc;
-    return download_rows(h, out, h->xout, bytes, h->stream, true);
+    return download_rows(h, io, out, h->xout, bytes, h->stream, true);
 }
 
 int mummu_dequantize(int type, const void *bytes, size_t nbytes, float *out) {

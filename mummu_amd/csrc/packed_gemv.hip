@@ -18,6 +18,7 @@
 // reference runs a short prefill row by row through the same op (nn/packed_gemv.rs:138-150); a row's
 // sums are the same whatever shares the launch.
 #include "device_utils.h"
+#include "host_staging.h"
 #include "kernels.h"
 
 #include <mutex>
@@ -208,6 +209,7 @@ static int packed_create(const uint32_t *words, const float *scales, int k, int 
         return pfail(nullptr, MUMMU_ERR_DEVICE, "no HIP device");
     }
     auto *w = new mummu_packed_weight();
+    HostStaging::retain();
     w->k = k;
     w->n = n;
     w->bits = value_bits;
@@ -272,6 +274,7 @@ void mummu_packed_weight_destroy(mummu_packed_weight *w) {
     (void)hipFree(w->x);
     (void)hipFree(w->y);
     (void)hipFree(w->partial);
+    HostStaging::release();
     delete w;
 }
 
@@ -287,12 +290,20 @@ int mummu_q4s_gemv(mummu_packed_weight *w, const float *x, int64_t m, int k, flo
     if (m < 0 || m > kMaxRows) return pfail(w, MUMMU_ERR_TOKENS, std::to_string(m) + " rows: the packed GEMV takes 0 to 64 rows a call");
     if (m == 0) return MUMMU_OK;
     if (!x || !y) return pfail(w, MUMMU_ERR_ARG, "null buffer");
-    hipError_t e = hipMemcpyAsync(w->x, x, sizeof(float) * (size_t)m * (size_t)k, hipMemcpyHostToDevice, w->stream);
+    HostStaging io;
+    const size_t xb = sizeof(float) * (size_t)m * (size_t)k, yb = sizeof(float) * (size_t)m * (size_t)w->n;
+    hipError_t e = io.valid() ? io.upload(w->x, x, xb, w->stream) : hipMemcpyAsync(w->x, x, xb, hipMemcpyHostToDevice, w->stream);
     if (e != hipSuccess) return pfail(w, MUMMU_ERR_DEVICE, std::string("packed gemv upload: ") + hipGetErrorString(e));
     const int rc = enqueue(w, w->x, (int)m, w->y, w->stream);
     if (rc) return rc;
-    e = hipMemcpyAsync(y, w->y, sizeof(float) * (size_t)m * (size_t)w->n, hipMemcpyDeviceToHost, w->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(w->stream);
+    if (io.valid()) {
+        const HostStaging::Piece out{y, w->y, yb};
+        int status = 0;
+        e = io.download(&out, 1, nullptr, 0, w->stream, [](const void *) { return 0; }, &status);
+    } else {
+        e = hipMemcpyAsync(y, w->y, yb, hipMemcpyDeviceToHost, w->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(w->stream);
+    }
     if (e != hipSuccess) return pfail(w, MUMMU_ERR_DEVICE, std::string("packed gemv: ") + hipGetErrorString(e));
     return MUMMU_OK;
 }
