@@ -35,6 +35,19 @@ constexpr int kDispatchThreads = 1024;
 constexpr int kDispatchWaves = kDispatchThreads / 64;
 constexpr int kDispatchMaxExperts = 512;
 
+// Expert e's n tiles over its `rows` sorted rows from `begin`: whole units of rows dealt evenly, the first tiles one more.
+__device__ inline void write_tiles(int32_t *__restrict__ tiles, int at, int n, int e, int begin, int rows, int unit) {
+    if (n == 0) return;
+    const int units = (rows + unit - 1) / unit, each = units / n, more = units - each * n;
+    for (int i = 0, r = 0; i < n; i++) {
+        const int take = (each + (i < more ? 1 : 0)) * unit;
+        tiles[3 * (at + i)] = e;
+        tiles[3 * (at + i) + 1] = begin + r;
+        tiles[3 * (at + i) + 2] = rows - r < take ? rows - r : take;
+        r += take;
+    }
+}
+
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_count_kernel(const int32_t *__restrict__ ids, int n_assign,
                                                                           int n_experts, int32_t *__restrict__ rank_out,
                                                                           int32_t *__restrict__ counts,
@@ -81,7 +94,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_count_kernel(const 
 // of L2 - instead of waiting for a launch of one workgroup to do it once (a third launch costs 4-5 us, the repeated
 // scan a fraction of that even at 64k tokens); workgroup 0 also writes offsets, the tile list and the hit counters.
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
-    const int32_t *__restrict__ ids, int n_assign, int n_experts, int n_chunks, int tile_rows,
+    const int32_t *__restrict__ ids, int n_assign, int n_experts, int n_chunks, int tile_rows, int unit,
     const int32_t *__restrict__ rank_in, const int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
     int32_t *__restrict__ sorted, int32_t *__restrict__ inv, int32_t *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     unsigned long long *__restrict__ hits) {
@@ -126,12 +139,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
             offsets[e] = begin;
             if (e == n_experts - 1) offsets[n_experts] = begin + total;
             if (tiles != nullptr) {
-                int nt = base_t + incl_t - my_tiles;
-                for (int r = 0; r < total; r += tile_rows, nt++) {
-                    tiles[3 * nt] = e;
-                    tiles[3 * nt + 1] = begin + r;
-                    tiles[3 * nt + 2] = (total - r) < tile_rows ? (total - r) : tile_rows;
-                }
+                write_tiles(tiles, base_t + incl_t - my_tiles, my_tiles, e, begin, total, unit);
                 if (e == n_experts - 1) *n_tiles = base_t + incl_t;
             }
         }
@@ -154,7 +162,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
 constexpr int kFusedChunks = 1;
 
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
-    const int32_t *__restrict__ ids, int n_assign, int n_experts, int tile_rows, int32_t *__restrict__ offsets,
+    const int32_t *__restrict__ ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *__restrict__ offsets,
     int32_t *__restrict__ sorted, int32_t *__restrict__ inv, int32_t *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     unsigned long long *__restrict__ hits, int32_t *__restrict__ flags) {
     __shared__ int s_wave[kDispatchWaves][kDispatchMaxExperts];   // per-wave counts of the current chunk
@@ -241,12 +249,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
         s_off[e] = begin;
         if (e == n_experts - 1) offsets[n_experts] = begin + total;
         if (tiles != nullptr) {
-            int nt = base_t + incl_t - my_tiles;
-            for (int r = 0; r < total; r += tile_rows, nt++) {
-                tiles[3 * nt] = e;
-                tiles[3 * nt + 1] = begin + r;
-                tiles[3 * nt + 2] = (total - r) < tile_rows ? (total - r) : tile_rows;
-            }
+            write_tiles(tiles, base_t + incl_t - my_tiles, my_tiles, e, begin, total, unit);
             if (e == n_experts - 1) *n_tiles = base_t + incl_t;
         }
     }
@@ -287,14 +290,14 @@ size_t dispatch_scratch_ints(int n_assign, int n_experts) {
     return (size_t)n_assign + chunks * (size_t)n_experts;
 }
 
-hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int32_t *offsets,
+hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *offsets,
                            int32_t *sorted, int32_t *inv, int32_t *tiles, int32_t *n_tiles, int32_t *scratch,
                            unsigned long long *hits, int32_t *flags, hipStream_t s) {
     if (n_assign <= 0) return hipSuccess;
-    if (n_experts > kDispatchMaxExperts || tile_rows < 1) return hipErrorInvalidValue;
+    if (n_experts > kDispatchMaxExperts || tile_rows < 1 || unit < 1 || tile_rows % unit != 0) return hipErrorInvalidValue;
     const int chunks = (n_assign + kDispatchThreads - 1) / kDispatchThreads;
     if (chunks <= kFusedChunks) {
-        launch_kernel(dispatch_fused_kernel, dim3(1), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, tile_rows, offsets,
+        launch_kernel(dispatch_fused_kernel, dim3(1), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, tile_rows, unit, offsets,
                       sorted, inv, tiles, n_tiles, hits, flags);
         return hipGetLastError();
     }
@@ -307,7 +310,7 @@ hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int 
     g_launch_timing.start = nullptr;
     g_launch_timing.stop = timing.stop;
     launch_kernel(dispatch_scan_place_kernel, dim3(chunks), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, chunks,
-                  tile_rows, (const int32_t *)rank, (const int32_t *)counts, offsets, sorted, inv, tiles, n_tiles, hits);
+                  tile_rows, unit, (const int32_t *)rank, (const int32_t *)counts, offsets, sorted, inv, tiles, n_tiles, hits);
     g_launch_timing = timing;
     return hipGetLastError();
 }

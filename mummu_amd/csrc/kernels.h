@@ -170,7 +170,9 @@ hipError_t launch_gate_energy(const float *w, const float *x, int rows, int hidd
 // triples.  scratch: dispatch_scratch_ints(A, E) ints.  hits (optional): per-expert row counters to
 // add this batch to.
 size_t dispatch_scratch_ints(int n_assign, int n_experts);
-hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int32_t *offsets,
+// unit: an expert's tiles, as few as tile_rows allows, share its rows evenly in multiples of this many (tile_rows: all
+// but the last are full).
+hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *offsets,
                            int32_t *sorted, int32_t *inv, int32_t *tiles, int32_t *n_tiles, int32_t *scratch,
                            unsigned long long *hits, int32_t *flags, hipStream_t s);
 
@@ -212,5 +214,15 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
 hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float *act32, QAct64 actq, HAct acth, int n_assign,
                             const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows, float *y, hipStream_t s,
                             bool q8_half = false);
+
+// gemm_wide.hip -----------------------------------------------------------------------
+// The F16 / BF16 grouped GEMM on tiles of up to kWideRows rows (a work list made with that tile size), for many rows per
+// expert; same operands as the form above.
+constexpr int kWideRows = 320, kWideUnit = 64;
+bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign);   // can and should
+hipError_t launch_wide_gate_up(const ExpertBanks &b, const _Float16 *x16, const int32_t *sorted, int k_slots, const int32_t *tiles,
+                               const int32_t *n_tiles, int max_tiles, _Float16 *act16, hipStream_t s);
+hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, const int32_t *n_tiles, int max_tiles,
+                            float *y, hipStream_t s);
 
 }  // namespace mummu

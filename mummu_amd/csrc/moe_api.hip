@@ -517,6 +517,8 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         const bool q8h = h->gemm_q8_f16 && grouped_gemm_q8_f16(b);
         int tile_rows = hf_down ? grouped_gemm_tile_rows_q4k_f16(na, b.n_experts) : grouped_gemm_tile_rows(b, na, b.n_experts, q8h);
         if (hf_down && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
+        const bool wide = wide_gemm_takes(b, (int)n, na);
+        if (wide) tile_rows = kWideRows;
         // (the launches' grids cover the most tiles this batch can have, not the most the workspace holds)
         const int tiles_bound = std::min(h->max_tiles, b.n_experts + (na + tile_rows - 1) / tile_rows + 1);
         // (f16 / bf16 banks: x as halfs in the same buffer)
@@ -528,8 +530,15 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         else if (half_banks) LAUNCH(h, K_QUANTIZE, s, launch_convert_rows_f16(x, (int)n, b.hidden, xh.hi, s));
         else if (grouped_gemm_quantized(b)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows64(x, (int)n, b.hidden, xq64, s));
         LAUNCH(h, K_DISPATCH, s,
-               launch_dispatch(h->ids, na, b.n_experts, tile_rows, h->offsets, h->sorted, h->inv, h->tiles, h->n_tiles, h->disp_scratch,
-                               count_hits ? L.hits : nullptr, h->flags, s));
+               launch_dispatch(h->ids, na, b.n_experts, tile_rows, wide ? kWideUnit : tile_rows, h->offsets, h->sorted, h->inv, h->tiles,
+                               h->n_tiles, h->disp_scratch, count_hits ? L.hits : nullptr, h->flags, s));
+        if (wide) {
+            LAUNCH(h, K_GEMM_GATE_UP, s,
+                   launch_wide_gate_up(b, xh.hi, h->sorted, k, h->tiles, h->n_tiles, tiles_bound, (_Float16 *)h->act16, s));
+            LAUNCH(h, K_GEMM_DOWN, s, launch_wide_down(b, (const _Float16 *)h->act16, h->tiles, h->n_tiles, tiles_bound, h->y, s));
+            LAUNCH(h, K_COMBINE, s, launch_combine(h->y, h->ids, h->weights, h->inv, (int)n, k, b.hidden, residual, out, s));
+            return MUMMU_OK;
+        }
         LAUNCH(h, K_GEMM_GATE_UP, s,
                launch_gemm_gate_up(b, x, xq64, xh, h->sorted, k, h->tiles, h->n_tiles, tiles_bound, tile_rows, h->act16, h->act, actq64,
                                    acth, s, q8h));
