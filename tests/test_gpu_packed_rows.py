@@ -1,0 +1,38 @@
+"""The packed GEMV at the edges of its tiles: every count of rows where another form takes over, K around the 32 of a stage
+and short of its slices, column counts that fill no group, and operands that are not 16-byte aligned - against the oracle,
+and each row bit for bit as when it comes alone."""
+import numpy as np
+import pytest
+
+from mummu_amd import moe as M
+from oracle import binding as orc
+from tests.packed_helpers import pack_words, quantize_block32
+
+pytestmark = pytest.mark.gpu
+
+
+class At:
+    def __init__(self, buf, offset):
+        self.buf, self.ptr = buf, buf.ptr + offset
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("k,n", [(31, 32), (32, 288), (33, 256), (444, 544), (1028, 1312), (2050, 96)])
+def test_rows_and_edges(k, n, bits):
+    g = np.random.default_rng(k + n + bits)
+    codes, scales = quantize_block32(g.uniform(-1, 1, (k, n)).astype(np.float32), bits)
+    words = pack_words(codes, bits)
+    x = g.uniform(-1, 1, (64, k)).astype(np.float32)
+    want = orc.q4s_gemv(words, scales, k, n, bits, x)
+    peak = np.abs(want).max()
+    # the words and x 4 bytes into their buffers
+    wd = M.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.uint32), words.ravel()]))
+    xd = M.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+    sd, yd = M.DeviceBuffer.from_array(scales), M.DeviceBuffer(4 * 64 * n)
+    with M.PackedWeight(words, scales, k, n, bits) as w, M.PackedWeight.wrap_device(At(wd, 4), sd, k, n, bits) as odd:
+        alone = np.concatenate([w.gemv(x[i]).reshape(1, n) for i in range(64)])
+        assert np.abs(alone - want).max() <= 1e-5 * peak
+        for m in (2, 4, 5, 8, 9, 16, 17, 32, 33, 64):
+            assert np.array_equal(w.gemv(x[:m]).view(np.uint32), alone[:m].view(np.uint32)), m
+            odd.gemv_device(At(xd, 4), m, yd)
+            assert np.array_equal(yd.download(np.float32, (64, n))[:m].view(np.uint32), alone[:m].view(np.uint32)), m
