@@ -63,6 +63,32 @@ __device__ inline half2v biased_pair(uint32_t t, bool upper) {
     return h;
 }
 
+// Codes at bits 0-3 and 16-19 (4-7 and 20-23 with HIGH) of t as halfs: the code itself, as a subnormal, is code * 2^-24
+// (16 code * 2^-24), which one packed product turns into code * mul.
+template <bool HIGH>
+__device__ inline half2v code_pair(uint32_t t, half2v mul) {
+    const uint32_t u = t & (HIGH ? 0x00F000F0u : 0x000F000Fu);
+    half2v h;
+    __builtin_memcpy(&h, &u, 4);
+    return h * mul;
+}
+// Eight Q4_K codes (the low or high nibbles of two words, in the element order of HAct) times their sub-block's scale, over
+// 2^14 (exact: up to 63 * 15 in units of 2^-14): two masks, a shift and four products a word.
+template <bool HIGH>
+__device__ inline half8 q4k_operand(uint32_t w0, uint32_t w1, half2v mul) {
+    const half2v f[4] = {code_pair<HIGH>(w0, mul), code_pair<HIGH>(w0 >> 8, mul), code_pair<HIGH>(w1, mul), code_pair<HIGH>(w1 >> 8, mul)};
+    half8 o;
+    __builtin_memcpy(&o, f, 16);
+    return o;
+}
+// ... with mul for a sub-block scale sc: sc * 2^10 for the low nibbles, sc * 2^6 for the high ones.
+template <bool HIGH>
+__device__ inline half2v q4k_mul(uint32_t sc) {
+    const _Float16 m = (_Float16)__fmul_rn((float)sc, HIGH ? 64.0f : 1024.0f);
+    return half2v{m, m};
+}
+constexpr float kQ4kUnit = 16384.0f;
+
 // Eight Q8_0 codes (two words of int8) times the block scale d as two halfs each, hi = rn(d * code) and
 // lo = d * code - hi (exact: a 19-bit product, subnormal halfs included, which the vector and the matrix units
 // both keep): a code b becomes the half 1024 + (b ^ 0x80) = b + 1152 by a byte permute, minus 1152 is exact.
@@ -1074,19 +1100,13 @@ __global__ __launch_bounds__(256 * WM, GATE_UP ? 2 : 3) void grouped_gemm_q4k_f1
     const float16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     // one 64-element step: st = which step of the super-block, buf = which tile holds its activations
     auto multiply = [&](int st, int buf, const u32x4 (&rw)[NB]) {
-        half2v ml2[NB], al2[NB], mh2[NB], ah2[NB];
+        half2v ml2[NB], mh2[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             // sub-blocks 2 st (the low nibbles) and 2 st + 1 (the high nibbles)
             const uint32_t sw = sc4[b][st >> 1] >> (16 * (st & 1));
-            const float sc_lo = (float)(sw & 0xFFu), sc_hi = (float)((sw >> 8) & 0xFFu);
-            // low nibbles: (1024 + q) * sc - 1024 sc; high nibbles, left in place: (1024 + 16 q) * (sc / 16) - 64 sc
-            const _Float16 ml = (_Float16)sc_lo, al = (_Float16)__fmul_rn(-1024.0f, sc_lo);
-            const _Float16 mh = (_Float16)__fmul_rn(0.0625f, sc_hi), ah = (_Float16)__fmul_rn(-64.0f, sc_hi);
-            ml2[b] = half2v{ml, ml};
-            al2[b] = half2v{al, al};
-            mh2[b] = half2v{mh, mh};
-            ah2[b] = half2v{ah, ah};
+            ml2[b] = q4k_mul<false>(sw & 0xFFu);
+            mh2[b] = q4k_mul<true>((sw >> 8) & 0xFFu);
         }
         const uint8_t *tile = s_raw + (size_t)buf * L::kBuf + (size_t)(row0 + (lane & 31)) * kRow + 32 * g;
         // the A operands of instruction group kk + 1 are read from the tile before group kk is issued
@@ -1108,14 +1128,7 @@ __global__ __launch_bounds__(256 * WM, GATE_UP ? 2 : 3) void grouped_gemm_q4k_f1
 #pragma unroll
             for (int b = 0; b < NB; b++) {
                 const uint32_t w_a = (kk & 1) ? rw[b][2] : rw[b][0], w_b = (kk & 1) ? rw[b][3] : rw[b][1];
-                const uint32_t mask = kk < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
-                const half2v mul = kk < 2 ? ml2[b] : mh2[b], add = kk < 2 ? al2[b] : ah2[b];
-                half2v f[4];
-                f[0] = __builtin_elementwise_fma(biased_pair(w_a & mask, false), mul, add);
-                f[1] = __builtin_elementwise_fma(biased_pair(w_a & mask, true), mul, add);
-                f[2] = __builtin_elementwise_fma(biased_pair(w_b & mask, false), mul, add);
-                f[3] = __builtin_elementwise_fma(biased_pair(w_b & mask, true), mul, add);
-                __builtin_memcpy(&bfrag[b], f, 16);
+                bfrag[b] = kk < 2 ? q4k_operand<false>(w_a, w_b, ml2[b]) : q4k_operand<true>(w_a, w_b, mh2[b]);
             }
             // (the hi products of every block first, then the lo products: instructions that accumulate into the same
             // registers are NB * MW apart)
@@ -1136,7 +1149,7 @@ __global__ __launch_bounds__(256 * WM, GATE_UP ? 2 : 3) void grouped_gemm_q4k_f1
     auto fold = [&](int part, int sum_buf) {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-            const float d = half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu));
+            const float d = __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu)));
             const float ndmin = -half_bits_to_float((uint16_t)(dd[b] >> 16));
             // the block offsets m as halfs (exact), in the order of the block sums
             _Float16 mh[NSUM];
@@ -1382,19 +1395,14 @@ __global__ __launch_bounds__(512, 4) void grouped_gemm_q4k_f16_m16_kernel(
 
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     auto multiply = [&](int hs, int buf, const u32x4 (&rw)[NB], bool first) {
-        half2v ml2[NB], al2[NB], mh2[NB], ah2[NB];
+        half2v ml2[NB], mh2[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             // this lane's bytes belong to sub-blocks 4 hs + 2 (kg / 2) (low nibbles) and the one after (high nibbles)
             // (hs is a constant at every call: picked with a conditional, an index would send the array to LDS)
             const uint32_t sw = (hs ? sc4[b][1] : sc4[b][0]) >> (16 * (kg >> 1));
-            const float sc_lo = (float)(sw & 0xFFu), sc_hi = (float)((sw >> 8) & 0xFFu);
-            const _Float16 ml = (_Float16)sc_lo, al = (_Float16)__fmul_rn(-1024.0f, sc_lo);
-            const _Float16 mh = (_Float16)__fmul_rn(0.0625f, sc_hi), ah = (_Float16)__fmul_rn(-64.0f, sc_hi);
-            ml2[b] = half2v{ml, ml};
-            al2[b] = half2v{al, al};
-            mh2[b] = half2v{mh, mh};
-            ah2[b] = half2v{ah, ah};
+            ml2[b] = q4k_mul<false>(sw & 0xFFu);
+            mh2[b] = q4k_mul<true>((sw >> 8) & 0xFFu);
         }
         const uint8_t *tile_p = s_raw + (size_t)buf * kBuf + (size_t)(lane & 15) * kRow + 128 * (kg >> 1) + 32 * (kg & 1);
         half8 a_hi[2], a_lo[2];
@@ -1411,14 +1419,7 @@ __global__ __launch_bounds__(512, 4) void grouped_gemm_q4k_f16_m16_kernel(
 #pragma unroll
             for (int b = 0; b < NB; b++) {
                 const uint32_t w_a = (q & 1) ? rw[b][2] : rw[b][0], w_b = (q & 1) ? rw[b][3] : rw[b][1];
-                const uint32_t mask = q < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
-                const half2v mul = q < 2 ? ml2[b] : mh2[b], add = q < 2 ? al2[b] : ah2[b];
-                half2v f[4];
-                f[0] = __builtin_elementwise_fma(biased_pair(w_a & mask, false), mul, add);
-                f[1] = __builtin_elementwise_fma(biased_pair(w_a & mask, true), mul, add);
-                f[2] = __builtin_elementwise_fma(biased_pair(w_b & mask, false), mul, add);
-                f[3] = __builtin_elementwise_fma(biased_pair(w_b & mask, true), mul, add);
-                __builtin_memcpy(&bfrag[b], f, 16);
+                bfrag[b] = q < 2 ? q4k_operand<false>(w_a, w_b, ml2[b]) : q4k_operand<true>(w_a, w_b, mh2[b]);
             }
 #pragma unroll
             for (int b = 0; b < NB; b++)
@@ -1437,7 +1438,7 @@ __global__ __launch_bounds__(512, 4) void grouped_gemm_q4k_f16_m16_kernel(
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-            const float d = half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu));
+            const float d = __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu)));
             const float ndmin = -half_bits_to_float((uint16_t)(dd[b] >> 16));
             // K index 4 kg + i of the fold: sub-block (4 kg + i) % 8 with ROW, else 4 hs + i (its K groups 2, 3 meet zeros)
             // (with one scale per row the word depends on the lane: blended with a mask - a conditional between the two

@@ -109,6 +109,7 @@ __device__ inline void quantize_store64(float4 v, bool active, const QAct64 &q, 
 // 128 elements; a producer that sees whole rows (quantize_rows_h) writes the same scale into all of a
 // row's entries, one that sees 128 columns at a time (the gate/up epilogue) a scale per entry.
 //   hi, lo : f16 [rows][D]      scale : f32 [rows][D/128]      ssum : f32 [rows][D/32], sum of x / scale
+// Elements of a run of four lie in the order 0, 2, 1, 3: as masking a word of packed codes yields them in pairs.
 struct HAct {
     _Float16 *hi = nullptr;
     _Float16 *lo = nullptr;
@@ -157,8 +158,9 @@ __device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_
     sum = __fadd_rn(sum, dpp_move<0x141>(sum));
     if (active) {
         uint2 hw, lw;
-        __builtin_memcpy(&hw, hi, 8);
-        __builtin_memcpy(&lw, lo, 8);
+        const _Float16 ho[4] = {hi[0], hi[2], hi[1], hi[3]}, oo[4] = {lo[0], lo[2], lo[1], lo[3]};
+        __builtin_memcpy(&hw, ho, 8);
+        __builtin_memcpy(&lw, oo, 8);
         *(uint2 *)(q.hi + row * (size_t)d + elem0) = hw;
         *(uint2 *)(q.lo + row * (size_t)d + elem0) = lw;
         if ((elem0 & 31) == 0) q.ssum[row * (size_t)(d / 32) + (elem0 >> 5)] = sum;
