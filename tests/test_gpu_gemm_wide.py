@@ -35,3 +35,27 @@ def test_every_tile_edge_matches_the_f64_reference(dtype):
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, ot), ids, w, x)
     assert orc.rel_err(got, want, mag).max() <= 4e-3
     assert (np.linalg.norm(got - want, axis=1) <= 2e-3 * np.linalg.norm(want, axis=1)).all()
+
+
+def test_gates_far_beyond_the_exponential_keep_silu_finite():
+    # Rows that are a power of two times one pattern: gates from -1000 to 1000, e^-x past the largest f32 among them.
+    H, I, E, n = 256, 128, 224, 72 * 224
+    row = lambda v: np.float16(v).view(np.uint16)
+    gate = np.zeros((E, I, H), np.uint16)
+    gate[:, :, 0] = row(np.linspace(-1000, 1000, I))
+    up = np.full((E, I, H), row(0), np.uint16)
+    up[:, :, 1] = row(1.0)
+    down = np.zeros((E, H, I), np.uint16)
+    down[:, np.arange(I), np.arange(I)] = row(1.0)
+    x = np.zeros((n, H), np.float32)
+    x[:, 0], x[:, 1] = np.where(np.arange(n) % 2, 1.0, 0.125), 1.0
+    ids = (np.arange(n, dtype=np.int32) % E)[:, None]
+    w = np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.uint16), M.F16, gate, M.F16, up, M.F16, down, M.F16)
+        got = m.apply_routing(0, ids, w, x)[:, :I]
+    g = x[:, :1].astype(np.float64) * gate[0, :, 0].view(np.float16).astype(np.float64)
+    want = g / (1.0 + np.exp(np.minimum(-g, 700.0)))
+    assert np.isfinite(got).all()
+    # (silu carries an f32 rounding or three and is stored as a half: half an ulp, 2^-11; below 2^-14 half of its last bit)
+    assert (np.abs(got - want) <= np.abs(want) * 2.0 ** -10.9 + 2.0 ** -24).all()
