@@ -103,6 +103,20 @@ __device__ inline uint32_t upper_halves(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
+// One row times one column over k0 <= k < k1, term by term: for sums that came out as NaN.  The split of an infinite x*scale
+// has inf - inf in its second part, where the products themselves are infinite and their sum may well be.
+template <int BITS>
+__device__ inline float plain_sum(const PackedArgs &p, int row, size_t col, int k0, int k1) {
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int k = k0; k < k1; k++) {
+        const uint32_t w = p.words[(size_t)k * (size_t)p.n_words + col * BITS / 32] << (32 - BITS - (int)(col % (32 / BITS)) * BITS);
+        const float xs = __fmul_rn(p.x[(size_t)row * (size_t)p.k_len + (size_t)k], p.scales[(size_t)k * (size_t)p.n_blocks + col / 32]);
+        sum = __fadd_rn(sum, __fmul_rn((float)((int32_t)w >> (32 - BITS)), xs));
+    }
+    return sum;
+}
+
 template <int BITS, int R, int RT>
 struct PackedMap {
     static constexpr int WORDS = kPgGroup * BITS / 32;  // words of a pair's columns at one k
@@ -136,6 +150,11 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
     const int k0 = (int)((int64_t)slice * p.stages / n_slices) * KS, k_end = (int)((int64_t)(slice + 1) * p.stages / n_slices) * KS;
     const int k1 = k_end < p.k_len ? k_end : p.k_len;
     const int most = (p.stages + n_slices - 1) / n_slices;
+    auto k_bound = [&](int part) {   // where the workgroups of K part `part` begin
+        const int k = (int)((int64_t)part * kPgSlices * p.stages / n_slices) * KS;
+        return k < p.k_len ? k : p.k_len;
+    };
+    const int part_k0 = k_bound(kpart), part_k1 = k_bound(kpart + 1);
 
     // A stage in LDS.  Row rho of its 32 is k = 8 (rho % 4) + rho / 4: lane group g reads its k = 8 g + i at rho = 4 i + g.
     // Words of row rho change places with those at ^ turn(rho): the four groups' reads then meet all banks.
@@ -350,6 +369,7 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
 #pragma unroll
                 for (int s = 0; s < kPgSlices; s++) sum = __fadd_rn(sum, s_sum[(s * R + r) * kSumRow + place]);
                 if (BITS == 4) sum = __fmul_rn(sum, 16.0f);
+                if (sum != sum) sum = plain_sum<BITS>(p, row0 + R * t + r, col, part_k0, part_k1);
                 float *dst = p.out + ((size_t)kpart * (size_t)p.m + (size_t)(row0 + R * t + r)) * out_n + col;
                 if (last_adds) __hip_atomic_store(dst, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // past this XCD's L2
                 else *dst = sum;

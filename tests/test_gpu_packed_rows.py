@@ -36,3 +36,23 @@ def test_rows_and_edges(k, n, bits):
             assert np.array_equal(w.gemv(x[:m]).view(np.uint32), alone[:m].view(np.uint32)), m
             odd.gemv_device(At(xd, 4), m, yd)
             assert np.array_equal(yd.download(np.float32, (64, n))[:m].view(np.uint32), alone[:m].view(np.uint32)), m
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_infinite_rows_give_infinite_sums(bits):
+    # an infinity times a code is an infinity of the code's sign, times 0 it is NaN; the rows beside it stay as they are
+    k, n, m = 700, 288, 9
+    g = np.random.default_rng(bits)
+    codes, scales = quantize_block32(g.uniform(-1, 1, (k, n)).astype(np.float32), bits)
+    words = pack_words(codes, bits)
+    x = g.uniform(-1, 1, (m, k)).astype(np.float32)
+    bad = x.copy()
+    bad[1, 3], bad[4, 699], bad[6, 350], bad[8, 40], bad[8, 690] = np.inf, -np.inf, np.nan, 3.0e38, np.inf
+    with M.PackedWeight(words, scales, k, n, bits) as w:
+        got, plain = w.gemv(bad), w.gemv(x)
+    want = orc.q4s_gemv(words, scales, k, n, bits, bad)
+    for r in (1, 4, 6, 8):
+        assert not np.isfinite(want[r]).any()
+        assert np.array_equal(got[r], want[r], equal_nan=True), r
+    ok = [r for r in range(m) if r not in (1, 4, 6, 8)]
+    assert np.array_equal(got[ok].view(np.uint32), plain[ok].view(np.uint32))
