@@ -178,7 +178,7 @@ hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int 
 
 // One expert serving rows 0..n-1 in order: sorted[i] = i and the tile list of expert 0 (tiles: 3 ints
 // per tile, at least ceil(n / tile_rows) tiles).
-hipError_t launch_identity_tiles(int n, int tile_rows, int32_t *sorted, int32_t *tiles, int32_t *n_tiles, hipStream_t s);
+hipError_t launch_identity_tiles(int n, int tile_rows, int expert, int32_t *sorted, int32_t *tiles, int32_t *n_tiles, hipStream_t s);
 
 // gemm.hip ----------------------------------------------------------------------------
 // Grouped GEMMs over the dispatch-sorted assignments on the matrix cores (hidden and inter

@@ -562,6 +562,44 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
     return MUMMU_OK;
 }
 
+// Rows from which one expert alone takes the grouped GEMM pair of the f16 units: the per-row kernels decode every weight again
+// for each few rows, a GEMM of one expert has few workgroups and the latency of its loop over K.  Host call, OLMoE Q4_K, the
+// former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323.  Only banks that are Q4_K
+// throughout: their GEMM holds rows as pairs of halfs (1.0e-7 off the 64-bit result, the per-row kernels 2.8e-5), the int8
+// GEMM of the other types a scale per 64 elements, where the per-row kernels have one per 16.
+constexpr int kOneExpertGemm = 64;
+
+// Its tiles: the smallest whose launch is at most one workgroup per CU (512 rows of OLMoE, tiles of 16 / 32 / 64 rows: 323 / 330 /
+// 337 us, 1024 rows: 865 / 598 / 585).
+int one_expert_tile_rows(const ExpertBanks &b, int rows) {
+    const int slabs = (b.inter + 127) / 128;
+    for (int t = 16; t < 64; t *= 2)
+        if ((rows + t - 1) / t * slabs <= 256) return t;
+    return 64;
+}
+
+// One expert's SwiGLU on `rows` rows (at most the workspace's tokens), in order, into out.
+int run_one_expert(mummu_moe *h, const Layer &L, int expert, const float *x, int rows, float *out, hipStream_t s) {
+    const ExpertBanks b = banks_of(h, L);
+    const HalfPlan hp = half_plan(h, b, rows, 1);
+    if (hp.hf_down && rows >= kOneExpertGemm) {
+        const int tile_rows = one_expert_tile_rows(b, rows), tiles = (rows + tile_rows - 1) / tile_rows;
+        const HAct acth{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum};
+        LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows_h(x, rows, b.hidden, hp.xh, s));
+        LAUNCH(h, K_DISPATCH, s, launch_identity_tiles(rows, tile_rows, expert, h->sorted, h->tiles, h->n_tiles, s));
+        LAUNCH(h, K_GEMM_GATE_UP, s,
+               launch_gemm_gate_up(b, nullptr, QAct64(), hp.xh, h->sorted, 1, h->tiles, h->n_tiles, tiles, tile_rows, nullptr, nullptr, QAct64(),
+                                   acth, s));
+        LAUNCH(h, K_GEMM_DOWN, s,
+               launch_gemm_down(b, nullptr, nullptr, QAct64(), acth, rows, h->tiles, h->n_tiles, tiles, tile_rows, out, s));
+        return MUMMU_OK;
+    }
+    if (is_quant_type(b.gate_type)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(x, rows, b.hidden, h->xq, s));
+    LAUNCH(h, K_GATE_UP, s, launch_gate_up(b, x, h->xq, nullptr, rows, 1, expert, h->act, h->actq, h->flags, s));
+    LAUNCH(h, K_DOWN, s, launch_down(b, h->act, h->actq, nullptr, rows, 1, expert, out, s));
+    return MUMMU_OK;
+}
+
 // The three-launch decode form (router logits + quantization, gate/up with the routing inside,
 // down + combine): nothing but the first launch reads the float activations.
 bool decode_three_launches(const mummu_moe *h, const Layer &L, int64_t n, int k) {
@@ -857,7 +895,7 @@ int forward_impl(mummu_moe *h, int layer, const float *x, int64_t n, int k, int 
         const int tile_rows = grouped_gemm_tile_rows(b, (int)n, 1);
         const QAct64 xq64{h->xq.hi, h->xq.lo, h->xq.scale, (float *)h->xq.sum};
         const QAct64 actq64{h->sh_actq.hi, h->sh_actq.lo, h->sh_actq.scale, (float *)h->sh_actq.sum};
-        LAUNCH(h, K_SHARED, s, launch_identity_tiles((int)n, tile_rows, h->sh_sorted, h->sh_tiles, h->sh_ntiles, s));
+        LAUNCH(h, K_SHARED, s, launch_identity_tiles((int)n, tile_rows, 0, h->sh_sorted, h->sh_tiles, h->sh_ntiles, s));
         // (the routed path may have left the 16-bit activations in the decode layout, or not made them)
         // (Q4_K on the f16 units as in the routed path; the routed products are done with their output buffer)
         const bool small32 = (size_t)n * (size_t)(b.hidden > b.inter ? b.hidden : b.inter) * 2 < (1ull << 32);
@@ -1443,10 +1481,7 @@ int mummu_expert_run(mummu_moe *h, int layer, int expert, const float *x, int64_
     const size_t bytes = sizeof(float) * (size_t)rows * (size_t)hidden;
     HostStaging io;
     if ((rc = upload_rows(h, io, h->xin, x, bytes, s))) return rc;
-    ExpertBanks b = banks_of(h, h->layers[layer]);
-    if (is_quant_type(b.gate_type)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(h->xin, (int)rows, hidden, h->xq, s));
-    LAUNCH(h, K_GATE_UP, s, launch_gate_up(b, h->xin, h->xq, nullptr, (int)rows, 1, expert, h->act, h->actq, h->flags, s));
-    LAUNCH(h, K_DOWN, s, launch_down(b, h->act, h->actq, nullptr, (int)rows, 1, expert, h->y, s));
+    if ((rc = run_one_expert(h, h->layers[layer], expert, h->xin, (int)rows, h->y, s))) return rc;
     return download_rows(h, io, out, h->y, bytes, s, false);
 }
 
@@ -1648,11 +1683,7 @@ int mummu_expert_run_device(mummu_moe *h, int layer, int expert, const float *x_
     if (rows == 0) return MUMMU_OK;
     hipStream_t s = (hipStream_t)stream;
     if ((rc = flush_pending(h))) return rc;
-    ExpertBanks b = banks_of(h, h->layers[layer]);
-    if (is_quant_type(b.gate_type)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(x_dev, (int)rows, hidden, h->xq, s));
-    LAUNCH(h, K_GATE_UP, s, launch_gate_up(b, x_dev, h->xq, nullptr, (int)rows, 1, expert, h->act, h->actq, h->flags, s));
-    LAUNCH(h, K_DOWN, s, launch_down(b, h->act, h->actq, nullptr, (int)rows, 1, expert, out_dev, s));
-    return MUMMU_OK;
+    return run_one_expert(h, h->layers[layer], expert, x_dev, (int)rows, out_dev, s);
 }
 
 int mummu_moe_stack_forward_device(mummu_moe *h, const float *x_dev, int64_t n, int top_k, int norm, float *out_dev, void *stream) {

@@ -104,3 +104,21 @@ def test_rows_of_zeros_and_tiny_and_huge_rows(monkeypatch):
     keep = np.ones(n, dtype=bool)
     keep[20] = False   # (|x|^2-sized products of a 1e20 row overflow f32 in the reference arithmetic as well)
     assert err[keep].max() <= 3e-5, f"max relative error {err[keep].max():.3e}"
+
+
+# one expert alone: 8 slabs, so 16-row tiles to 512 rows, 32-row tiles to 1024, then 64; the last tile full and with a row
+@pytest.mark.parametrize("rows", [64, 65, 511, 512, 513, 1024, 1025])
+def test_one_expert_with_many_rows(rows):
+    H, I, E, e = 256, 1024, 3, 2
+    gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (21, 22))
+    down = synth.random_bank_fast(M.Q4_K, [I, H, E], 23)
+    x = normal((rows, H), rows)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=rows) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q4_K, up, M.Q4_K, down, M.Q4_K)
+        got = m.expert_run(0, e, x)
+        xd, yd = M.DeviceBuffer.from_array(x), M.DeviceBuffer(4 * rows * H)
+        m.expert_run_device(0, e, xd, rows, yd)
+        assert np.array_equal(yd.download(np.float32, (rows, H)).view(np.uint32), got.view(np.uint32))
+    banks = orc.LayerBanks(H, I, E, gate, up, down, orc.Q4_K, orc.Q4_K, orc.Q4_K)
+    want, mag = orc.moe_ref_f64(banks, np.full((rows, 1), e, np.uint32), np.ones((rows, 1), np.float32), x)
+    assert orc.rel_err(got, want, mag).max() <= 3e-5
