@@ -1599,7 +1599,10 @@ bool grouped_gemm_supported(const ExpertBanks &b) {
 // expected tiles within 1 % of the 32-row form's: 64 experts x 8 slabs of 16-row tiles are exactly the 512
 // workgroups the chip holds at once, and the first second tiles start a second round - 72 / 80 tokens: 104 / 114 us
 // per layer with 16-row tiles, 105 / 106-112 us with 32-row tiles).
-int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts) {
+// With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
+// products together: OLMoE Q4_K with Q6_K downs, 32 / 64 rows: 150 tokens 154 / 206 us, 230: 181 / 208, 260: 225 / 214; the
+// 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013.
+int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts, bool int8_down) {
     const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
     const double sigma = __builtin_sqrt(avg > 1.0 ? avg : 1.0);
     auto expected_tiles = [&](double rows) {
@@ -1613,7 +1616,7 @@ int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts) {
     };
     const double e16 = expected_tiles(16.0), e32 = expected_tiles(32.0), e64 = expected_tiles(64.0);
     if (0.99 * e16 < e32 && 0.99 * 0.55 * e16 < e64) return 16;
-    return 0.55 * e32 < e64 ? 32 : 64;
+    return (int8_down ? 0.69 : 0.55) * e32 < e64 ? 32 : 64;
 }
 
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half) {
