@@ -1765,6 +1765,10 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
         return launch_gemm_f16<true, T_Q8_0>(b.gate, b.up, xh.hi, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden,
                                              b.inter, (_Float16 *)act16, nullptr, s);
     }
+    if (xh.hi != nullptr && xh.lo != nullptr && b.gate_type == T_Q8_0) {
+        if (!q8_gemm_takes(b) || acth.hi == nullptr || tile_rows != 32) return hipErrorInvalidValue;
+        return launch_q8_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, s);
+    }
     if (xh.hi != nullptr && xh.lo != nullptr) {
         if (!grouped_gemm_q4k_f16(b)) return hipErrorInvalidValue;
         const bool out_h = acth.hi != nullptr;
@@ -1809,6 +1813,10 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
         if (!grouped_gemm_q8_f16(b) || acth.hi != nullptr) return hipErrorInvalidValue;
         return launch_gemm_f16<false, T_Q8_0>(b.down, nullptr, (const _Float16 *)act16, nullptr, 1, tiles, n_tiles, max_tiles,
                                               tile_rows, b.inter, b.hidden, nullptr, y, s);
+    }
+    if (acth.hi != nullptr && b.down_type == T_Q8_0) {
+        if (!q8_gemm_takes(b) || tile_rows != 32) return hipErrorInvalidValue;
+        return launch_q8_down(b, acth, tiles, n_tiles, max_tiles, y, s);
     }
     if (acth.hi != nullptr) {
         if (!grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;

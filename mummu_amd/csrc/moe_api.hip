@@ -93,6 +93,7 @@ struct mummu_moe {
     // batches at least this large take dispatch + grouped GEMM (measured crossovers on the OLMoE shape:
     // the 16-bit float decode kernels lose from 7 tokens on, the f32 ones from 10, the integer ones from 19)
     int gemm_min_f16 = 7, gemm_min_quant = 19, gemm_min_f32 = 10;
+    int gemm_min_q8 = 13;    // Q8_0 banks on the f16 units (10 / 12 / 14 tokens: 137 / 137 / 138 against 121 / 140 / 155 us)
     int gemm_min_q4k = 18;   // Q4_K banks on the f16 units (17 tokens: 88.8 us either way; 18: 89.1 against 92.6 us)
     int gemm_q4k_f16 = 1;        // Q4_K banks of the batched path on the f16 units (0: the int8 form)
     int gemm_q8_f16 = 0;         // 1: Q8_0 banks of the batched path through the f16 kernel (x and activations as halfs)
@@ -468,6 +469,9 @@ int check_topk(mummu_moe *h, int top_k, int n_experts) {
     return MUMMU_OK;
 }
 
+// Q8_0 banks go through gemm_q8.hip (MUMMU_GEMM_Q8_F16=1 asks for halfs alone instead).
+bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_takes(b) && !(h->gemm_q8_f16 && grouped_gemm_q8_f16(b)); }
+
 // experts of an already-made routing: gate/up -> down -> combine.  x_quantized says h->xq
 // already holds the 16-bit form of x (the fused router produced it).
 // Smallest batch of this layer that takes the batched path (INT_MAX: never).
@@ -476,23 +480,35 @@ int batched_from(const mummu_moe *h, const Layer &L) {
     if (!grouped_gemm_supported(b)) return 0x7fffffff;
     if (b.gate_type == T_F32) return h->gemm_min_f32;
     if (h->gemm_q4k_f16 && grouped_gemm_q4k_f16_down(b)) return h->gemm_min_q4k;
+    if (q8_half_pairs(h, b)) return h->gemm_min_q8;
     return grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
 }
 
-// Q4_K banks on the f16 units (batched path): whether gate/up (hf) and down (hf_down) take that form for this batch,
+// Q4_K and Q8_0 banks on the f16 units (batched path): whether gate/up (hf) and down (hf_down) take that form for this batch,
 // and where x goes as pairs of halfs: the (not yet written) buffer of the down product's output.
 struct HalfPlan {
-    bool hf = false, hf_down = false;
+    bool hf = false, hf_down = false, q8 = false;
     HAct xh;
 };
 
-HalfPlan half_plan(const mummu_moe *h, const ExpertBanks &b, int64_t n, int k) {
+// Where the 32-row tiles of gemm_q8.hip are ahead of the int8 form's 64-row ones, by the rows of an expert (OLMoE layers, here /
+// int8): up to 33, where next to none needs a second tile (150 tokens: 153 / 204 us, 260: 198 / 219), and from where many need a
+// second tile of 64 (400 tokens = 50 rows: 283 / 332, 700: 382 / 401, 1500: 671 / 673).  In between one tile of 64 holds
+// an expert (300 tokens: 243 / 228), and beyond 190 rows the weights are read too often (2048 tokens: 876 / 865).
+bool q8_gemm_should(size_t n_assign, int n_experts) {
+    const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
+    return avg <= 33.0 || (avg + 2.2 * __builtin_sqrt(avg) >= 64.0 && avg <= 190.0);
+}
+
+// (one_expert: all n rows go to the same one)
+HalfPlan half_plan(const mummu_moe *h, const ExpertBanks &b, int64_t n, int k, bool one_expert = false) {
     HalfPlan p;
     const size_t na = (size_t)(n * k);
     // (its kernels address the activation planes with 32-bit byte offsets)
     const bool small32 = na * (size_t)(b.hidden > b.inter ? b.hidden : b.inter) * 2 < (1ull << 32);
-    p.hf = h->gemm_q4k_f16 && small32 && grouped_gemm_q4k_f16(b);
-    p.hf_down = p.hf && grouped_gemm_q4k_f16_down(b);
+    p.q8 = small32 && q8_half_pairs(h, b) && (one_expert || q8_gemm_should(na, b.n_experts));
+    p.hf = p.q8 || (h->gemm_q4k_f16 && small32 && grouped_gemm_q4k_f16(b));
+    p.hf_down = p.q8 || (p.hf && grouped_gemm_q4k_f16_down(b));
     // x as pairs of halfs borrows h->y (the down product's output, written only after the gate/up launch has read x) and
     // the scale / sum arrays of the 16-bit form (unused on this path): run_experts keeps the order quantize -> gate/up ->
     // down on one stream, and nothing else may hold h->y across the gate/up launch
@@ -519,6 +535,7 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         // (gate/up alone on the f16 units: the int8 down product takes a tile of 16 rows like one of 32)
         if (hf && !hf_down) tile_rows = grouped_gemm_tile_rows_q4k_f16(na, b.n_experts, true);
         if (hf_down && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
+        if (hp.q8) tile_rows = 32;
         const bool wide = wide_gemm_takes(b, (int)n, na);
         if (wide) tile_rows = kWideRows;
         // (the launches' grids cover the most tiles this batch can have, not the most the workspace holds)
@@ -563,12 +580,12 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
 
 // Rows from which one expert alone takes the grouped GEMM pair of the f16 units: the per-row kernels decode every weight again
 // for each few rows, a GEMM of one expert has few workgroups and the latency of its loop over K.  Host call, OLMoE Q4_K, the
-// former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323.  Only banks that are Q4_K
-// throughout: their GEMM holds rows as pairs of halfs (1.0e-7 off the 64-bit result, the per-row kernels 2.8e-5), the int8
+// former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323;
+// Q8_0 64: 121 / 106, 128: 223 / 143, 512: 789 / 353.  Only banks that are Q4_K or Q8_0 throughout: their GEMM holds rows as pairs of halfs (1.0e-7 off the 64-bit result, the per-row kernels 2.8e-5), the int8
 // GEMM of the other types a scale per 64 elements, where the per-row kernels have one per 16.
 constexpr int kOneExpertGemm = 64;
 
-// Its tiles: the smallest whose launch is at most one workgroup per CU (512 rows of OLMoE, tiles of 16 / 32 / 64 rows: 323 / 330 /
+// The Q4_K form's tiles: the smallest whose launch is at most one workgroup per CU (512 rows of OLMoE, tiles of 16 / 32 / 64 rows: 323 / 330 /
 // 337 us, 1024 rows: 865 / 598 / 585).
 int one_expert_tile_rows(const ExpertBanks &b, int rows) {
     const int slabs = (b.inter + 127) / 128;
@@ -580,9 +597,9 @@ int one_expert_tile_rows(const ExpertBanks &b, int rows) {
 // One expert's SwiGLU on `rows` rows (at most the workspace's tokens), in order, into out.
 int run_one_expert(mummu_moe *h, const Layer &L, int expert, const float *x, int rows, float *out, hipStream_t s) {
     const ExpertBanks b = banks_of(h, L);
-    const HalfPlan hp = half_plan(h, b, rows, 1);
+    const HalfPlan hp = half_plan(h, b, rows, 1, true);
     if (hp.hf_down && rows >= kOneExpertGemm) {
-        const int tile_rows = one_expert_tile_rows(b, rows), tiles = (rows + tile_rows - 1) / tile_rows;
+        const int tile_rows = hp.q8 ? 32 : one_expert_tile_rows(b, rows), tiles = (rows + tile_rows - 1) / tile_rows;
         const HAct acth{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum};
         LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows_h(x, rows, b.hidden, hp.xh, s));
         LAUNCH(h, K_DISPATCH, s, launch_identity_tiles(rows, tile_rows, expert, h->sorted, h->tiles, h->n_tiles, s));
@@ -1073,7 +1090,7 @@ int mummu_moe_create(const mummu_moe_config *cfg, mummu_moe **out) {
     // MUMMU_GEMM_MIN_TOKENS: smallest batch that takes dispatch + grouped GEMM instead of the decode kernels
     if (const char *e = getenv("MUMMU_GEMM_MIN_TOKENS")) {
         const int v = atoi(e);
-        if (v >= 1) h->gemm_min_f16 = h->gemm_min_quant = h->gemm_min_f32 = h->gemm_min_q4k = v;
+        if (v >= 1) h->gemm_min_f16 = h->gemm_min_quant = h->gemm_min_f32 = h->gemm_min_q4k = h->gemm_min_q8 = v;
     }
     h->layers.resize((size_t)cfg->num_layers);
     auto bail = [&](int rc) {
