@@ -38,6 +38,9 @@ __global__ __launch_bounds__(256) void stage_copy_kernel(StageRanges r) {
         const size_t tail = r.bytes[i] & 15;
         if (blockIdx.x == 0 && threadIdx.x < tail) dst[(n16 << 4) + threadIdx.x] = src[(n16 << 4) + threadIdx.x];
         if (r.done) {
+            // (each wave's own stores have arrived before the workgroup meets: a barrier alone, and the release of the one thread
+            // behind it, wait for no other wave's)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             if (threadIdx.x == 0)
                 __hip_atomic_store(r.done + r.row[i] * kStageWgs + (int)blockIdx.x, r.mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
