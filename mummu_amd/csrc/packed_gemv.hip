@@ -24,9 +24,10 @@
 // Two waves take 256 columns (whole 128-byte lines of words: with half lines the requests are the limit, 34 against 29 us
 // on [8192, 20480]) and a slice of K, the words, scales and x straight from memory into LDS, a stage of 32 k ahead.  A word
 // holds 8 (or 4) columns at one k, so reading it for eight k gives a lane the B operands of as many columns without a
-// transposition.  Four such pairs are a workgroup and meet in LDS in ascending order, the workgroups of a column group through
-// partial sums, added in ascending order by the one that comes last, or, if they are many, by a second kernel.  Which slice
-// a k belongs to and the order of every sum depend on the weight alone: a row's bits are the same whatever shares the launch.
+// transposition.  Four such pairs are a workgroup and meet in LDS in ascending order, the workgroups of a column group (and of
+// the same rows) through partial sums, added in ascending order by the one that comes last, or, if they are many, by a second
+// kernel.  Which slice a k belongs to and the order of every sum depend on the weight alone: a row's bits are the same whatever
+// shares the launch.
 //
 // [5120, 17408] Q4S, 1 / 4 / 16 / 64 rows: 17.6 / 29.1 / 86 / 327 -> 17.5 / 17.8 / 26.9 / 88 us; Q8S 25.8 / 38.0 / 108 / 407 ->
 // 22.9 / 24.4 / 37 / 102; [2048, 4096] Q4S 9.4 / 17.6 / 18.3 / 36.5 -> 8.0 / 8.7 / 11.0 / 16.4.  Now the vector ALUs bound it
@@ -67,8 +68,8 @@ struct PackedArgs {
     int wg_x, grid_k;        // column groups of kPgGroup, workgroups along K
     bool words16, x16;       // the words, the rows of x are 16-byte aligned
     float *out;              // y, or [grid_k][m][n] partial sums
-    float *y;                // not null: the last workgroup of a column group adds the partial sums into it
-    unsigned *arrived;       // ... counted here, [wg_x], 0 between launches
+    float *y;                // not null: the last workgroup of a row and column group adds the partial sums into it
+    unsigned *arrived;       // ... counted here, [row group][wg_x], 0 between launches
 };
 
 __device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -380,13 +381,15 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     unsigned *s_last = (unsigned *)s_lds;
-    if (tid == 0) *s_last = atomicInc(p.arrived + wg, (unsigned)p.grid_k - 1);
+    // (one counter per row group, blockIdx.y, too: it stands for the sums of these rows alone, and they alone are added)
+    if (tid == 0) *s_last = atomicInc(p.arrived + (size_t)blockIdx.y * (size_t)p.wg_x + wg, (unsigned)p.grid_k - 1);
     __syncthreads();
     if (*s_last != (unsigned)p.grid_k - 1) return;
+    const int own = (rows < RT * R ? rows : RT * R) * kPgGroup;
     // ascending parts, 16 loads out before the first add (a missing part adds +0.0, which changes nothing)
     auto add = [&](auto items, auto parts) {
         constexpr int ITEMS = decltype(items)::value, PARTS = decltype(parts)::value;
-        for (int i0 = tid; i0 < p.m * kPgGroup; i0 += 512 * ITEMS) {
+        for (int i0 = tid; i0 < own; i0 += 512 * ITEMS) {
             float sum[ITEMS];
             size_t at[ITEMS];
             bool in[ITEMS];
@@ -394,8 +397,8 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
             for (int j = 0; j < ITEMS; j++) {
                 const int i = i0 + 512 * j, c = wg * kPgGroup + i % kPgGroup;
                 sum[j] = 0.0f;
-                in[j] = i < p.m * kPgGroup && c < p.n_blocks * 32;
-                at[j] = (size_t)(in[j] ? i / kPgGroup : 0) * out_n + (size_t)(in[j] ? c : 0);
+                in[j] = i < own && c < p.n_blocks * 32;
+                at[j] = (size_t)(row0 + (in[j] ? i / kPgGroup : 0)) * out_n + (size_t)(in[j] ? c : 0);
             }
             for (int s0 = 0; s0 < p.grid_k; s0 += PARTS) {
                 float v[ITEMS][PARTS];
@@ -464,7 +467,7 @@ struct mummu_packed_weight {
     uint32_t *words = nullptr;  // device [K][n_words]
     float *scales = nullptr;    // device [K][N/32]
     float *x = nullptr, *y = nullptr, *partial = nullptr;  // staging for the host-pointer call and the K partials
-    unsigned *arrived = nullptr;  // per column group: workgroups that have left their partial sums
+    unsigned *arrived = nullptr;  // per row and column group: workgroups that have left their partial sums
     int k = 0, n = 0, bits = 4, wg_x = 1, grid_k = 1, stages = 1;
     bool owns_weight = true;  // false: words and scales are the caller's device buffers
     hipStream_t stream = nullptr;
@@ -475,9 +478,10 @@ struct mummu_packed_weight {
 namespace {
 
 constexpr int kMaxRows = 64;  // nn/packed_gemv.rs:138: row by row up to 64 rows
-// Rows times workgroups along K up to which the last workgroup of a column group adds the partial sums: a second launch costs
+// Rows times workgroups along K up to which the last workgroup of a row and column group adds the partial sums: a second launch costs
 // 3 us, reading them past the L2 0.05 us a row and workgroup.
 constexpr int kLastAdds = 64;
+constexpr int kRowGroups = kMaxRows / 16;   // most row groups of a launch: it takes 16 rows or more each, or has one
 thread_local std::string g_packed_error;
 
 int pfail(mummu_packed_weight *w, int code, const std::string &msg) {
@@ -548,8 +552,8 @@ static int packed_create(const uint32_t *words, const float *scales, int k, int 
     if (e == hipSuccess) e = hipMalloc(&w->x, sizeof(float) * (size_t)kMaxRows * (size_t)k);
     if (e == hipSuccess) e = hipMalloc(&w->y, sizeof(float) * (size_t)kMaxRows * (size_t)n);
     if (e == hipSuccess) e = hipMalloc(&w->partial, sizeof(float) * (size_t)w->grid_k * (size_t)kMaxRows * (size_t)n);
-    if (e == hipSuccess) e = hipMalloc(&w->arrived, sizeof(unsigned) * (size_t)w->wg_x);
-    if (e == hipSuccess) e = hipMemset(w->arrived, 0, sizeof(unsigned) * (size_t)w->wg_x);
+    if (e == hipSuccess) e = hipMalloc(&w->arrived, sizeof(unsigned) * (size_t)kRowGroups * (size_t)w->wg_x);
+    if (e == hipSuccess) e = hipMemset(w->arrived, 0, sizeof(unsigned) * (size_t)kRowGroups * (size_t)w->wg_x);
     if (e == hipSuccess) e = hipStreamCreate(&w->stream);
     if (e == hipSuccess && !on_device) e = hipMemcpy(w->words, words, wb, hipMemcpyHostToDevice);
     if (e == hipSuccess && !on_device) e = hipMemcpy(w->scales, scales, sb, hipMemcpyHostToDevice);
