@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "slab_pool.h"
+
 namespace mummu {
 
 // One call's way between the caller's pageable memory and the GPU: a slab of pinned memory cut into slots, filled (or
@@ -18,13 +20,12 @@ namespace mummu {
 // What has arrived is marked by the kernel in words that the calling thread watches: an event per slot cost 25 us a slot, the wait
 // for the stream's end 4 (expert_run of 96 / 192 / 512 / 1024 Q4_K rows: 135 / 175 / 317 / 596 -> 106 / 155 / 310 / 549 us).
 //
-// A slab belongs to one call at a time.  Slabs come from a pool of the process: at most kMaxIdle wait there between calls
-// (a call that finds none allocates one), and the last handle to go frees them.
+// A slab (8.4 MB) belongs to one call at a time.  Slabs come from a pool of the process, which keeps as many as calls have run
+// side by side, at most one per handle (slab_pool.h).
 class HostStaging {
 public:
     static constexpr size_t kSlot = 512 * 1024;
     static constexpr int kSlots = 8;       // each way
-    static constexpr int kMaxIdle = 4;
 
     HostStaging();                         // takes a slab; valid() is false if pinned memory cannot be had
     ~HostStaging();                        // hands it back (every transfer has to have been waited for, or is waited for here)
@@ -54,13 +55,12 @@ public:
         return finish_download(s);
     }
 
-    static void retain();    // a handle was made / is gone: the pool's slabs are freed with the last one
+    static void retain();    // a handle was made / is gone: the pool holds a slab per handle at most
     static void release();
 
 private:
     struct Slab;
-    struct Pool;
-    static Pool &pool();
+    static SlabPool<Slab> &pool();
     const void *early_host() const;
     hipError_t begin_download(const Piece *pieces, int n, const void *early, size_t early_bytes, hipStream_t s);
     hipError_t finish_download(hipStream_t s);

@@ -2,8 +2,6 @@
 #include "host_staging.h"
 
 #include <cstring>
-#include <mutex>
-#include <vector>
 
 #include "device_utils.h"
 
@@ -99,60 +97,20 @@ struct HostStaging::Slab {
     }
 };
 
-struct HostStaging::Pool {
-    std::mutex mu;
-    std::vector<Slab *> idle;
-    int handles = 0;
-};
-
-HostStaging::Pool &HostStaging::pool() {
-    static Pool *p = new Pool();  // (never destroyed: handles may outlive static objects)
+SlabPool<HostStaging::Slab> &HostStaging::pool() {
+    static auto *p = new SlabPool<Slab>();  // (never destroyed: handles may outlive static objects)
     return *p;
 }
 
-void HostStaging::retain() {
-    {
-        Pool &p = pool();
-        std::lock_guard<std::mutex> lock(p.mu);
-        if (p.handles++ > 0 || !p.idle.empty()) return;
-    }
-    HostStaging first;  // the first handle's creation pays for the slab, not its first call
-}
+void HostStaging::retain() { pool().retain(); }
+void HostStaging::release() { pool().release(); }
 
-void HostStaging::release() {
-    std::vector<Slab *> gone;
-    {
-        Pool &p = pool();
-        std::lock_guard<std::mutex> lock(p.mu);
-        if (--p.handles == 0) gone.swap(p.idle);
-    }
-    for (Slab *s : gone) s->free();
-}
-
-HostStaging::HostStaging() {
-    {
-        Pool &p = pool();
-        std::lock_guard<std::mutex> lock(p.mu);
-        if (!p.idle.empty()) {
-            slab_ = p.idle.back();
-            p.idle.pop_back();
-        }
-    }
-    if (!slab_) slab_ = Slab::make();
-}
+HostStaging::HostStaging() { slab_ = pool().take(); }
 
 HostStaging::~HostStaging() {
     if (!slab_) return;
     if (in_flight_) (void)hipStreamSynchronize(pending_);  // (a call that failed half way)
-    {
-        Pool &p = pool();
-        std::lock_guard<std::mutex> lock(p.mu);
-        if (p.handles > 0 && (int)p.idle.size() < kMaxIdle) {
-            p.idle.push_back(slab_);
-            slab_ = nullptr;
-        }
-    }
-    if (slab_) slab_->free();
+    pool().give(slab_);
 }
 
 hipError_t HostStaging::upload(void *dev, const void *host, size_t bytes, hipStream_t s) {
