@@ -99,23 +99,10 @@ __device__ inline float nibble(uint32_t w) {
 template <int B>
 __device__ inline float byte_code(uint32_t w) { return (float)(int8_t)(w >> (8 * B)); }
 
-// bf16 pair: the upper halves of two floats.
-__device__ inline uint32_t upper_halves(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
-// One row times one column over k0 <= k < k1, term by term: for sums that came out as NaN.  The split of an infinite x*scale
-// has inf - inf in its second part, where the products themselves are infinite and their sum may well be.
-template <int BITS>
-__device__ inline float plain_sum(const PackedArgs &p, int row, size_t col, int k0, int k1) {
-    float sum = 0.0f;
-#pragma unroll 1
-    for (int k = k0; k < k1; k++) {
-        const uint32_t w = p.words[(size_t)k * (size_t)p.n_words + col * BITS / 32] << (32 - BITS - (int)(col % (32 / BITS)) * BITS);
-        const float xs = __fmul_rn(p.x[(size_t)row * (size_t)p.k_len + (size_t)k], p.scales[(size_t)k * (size_t)p.n_blocks + col / 32]);
-        sum = __fadd_rn(sum, __fmul_rn((float)((int32_t)w >> (32 - BITS)), xs));
-    }
-    return sum;
+// bf16 pair: the upper halves of two floats (with kNoHalves: two zeros).
+constexpr uint32_t kUpperHalves = 0x07060302u, kNoHalves = 0x0C0C0C0Cu;
+__device__ inline uint32_t upper_halves(float lo, float hi, uint32_t pick = kUpperHalves) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), pick);
 }
 
 template <int BITS, int R, int RT>
@@ -126,22 +113,21 @@ struct PackedMap {
     static constexpr int LANE_WORDS = BITS == 8 && R == 4 ? 2 : 1;
     // bytes of a stage: words [kPgStage][WORDS], scales [kPgStage][8], x [RT * R][kPgStage]
     static constexpr int S_AT = kPgStage * WORDS * 4, X_AT = S_AT + kPgStage * 32, STAGE = X_AT + RT * R * kPgStage * 4;
+    // ... of the slices' sums, rows a little longer than the columns; behind them a word per wave
+    static constexpr int SUM_ROW = kPgGroup + 4, SUMS = kPgSlices * R * SUM_ROW * 4, RING = kPgSlices * 2 * STAGE;
+    static constexpr int LDS = RING > SUMS + 32 ? RING : SUMS + 32;
 };
 
-// RT row tiles of R rows.
+// RT row tiles of R rows of workgroup `lin`'s columns and part of K, into p.out; true if a sum of this lane came out as NaN.
+// lower: kUpperHalves; kNoHalves: x*scale is its first part alone, and only sums that are NaN in p.out are written.
 template <int BITS, int R, int RT>
-__global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4)) void packed_gemv_kernel(PackedArgs p) {
+__device__ inline bool packed_tile(const PackedArgs &p, uint8_t *s_lds, int tid, int lin, uint32_t lower) {
     using Map = PackedMap<BITS, R, RT>;
     constexpr int WORDS = Map::WORDS, GROUPS = Map::GROUPS, SETS = Map::SETS, LW = Map::LANE_WORDS;
     constexpr int PIECES = WORDS / 4, KS = kPgStage;
     constexpr int S_AT = Map::S_AT, X_AT = Map::X_AT, STAGE = Map::STAGE;
-    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // [kPgSlices][2][STAGE]; then the slices' sums
-    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    const int lane = tid & 63, wave = uniform(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
-    // workgroups of an XCD (equal ids modulo 8) take neighbouring column groups: they share the lines of the scales
-    const int total = p.wg_x * p.grid_k, per_xcd = (total + 7) >> 3;
-    const int lin = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || lin >= total) return;
     const int kpart = lin / p.wg_x, wg = lin - kpart * p.wg_x;
     const int row0 = (int)blockIdx.y * (RT * R), rows = p.m - row0;
     const int half = wave & 1, slice = kpart * kPgSlices + (wave >> 1);
@@ -151,11 +137,6 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
     const int k0 = (int)((int64_t)slice * p.stages / n_slices) * KS, k_end = (int)((int64_t)(slice + 1) * p.stages / n_slices) * KS;
     const int k1 = k_end < p.k_len ? k_end : p.k_len;
     const int most = (p.stages + n_slices - 1) / n_slices;
-    auto k_bound = [&](int part) {   // where the workgroups of K part `part` begin
-        const int k = (int)((int64_t)part * kPgSlices * p.stages / n_slices) * KS;
-        return k < p.k_len ? k : p.k_len;
-    };
-    const int part_k0 = k_bound(kpart), part_k1 = k_bound(kpart + 1);
 
     // A stage in LDS.  Row rho of its 32 is k = 8 (rho % 4) + rho / 4: lane group g reads its k = 8 g + i at rho = 4 i + g.
     // Words of row rho change places with those at ^ turn(rho): the four groups' reads then meet all banks.
@@ -213,7 +194,7 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
             }
             return;
         }
-        const int last = p.k_len - 1 - kb;   // (rows past the end of K repeat the last: x counts as 0 there)
+        const int last = p.k_len - 1 - kb;   // (rows past the end of K repeat the last: x and scales count as 0 there)
         auto k_in = [&](int k) { return (uint32_t)(k < last ? k : last); };
         for (int i = 0; i < 4 * W16; i++) {
             const int d = 64 * (half * 4 * W16 + i) + lane, rho = d / WORDS;
@@ -249,9 +230,12 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
     for (int i = 0, kb = k0; i < most; i++, kb += KS) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         uint8_t *st = s_lds + (size_t)(wave >> 1) * (2 * STAGE) + (size_t)(i & 1) * STAGE;
-        if (kb < k1 && kb + KS > k1)   // past the end of K
+        if (kb < k1 && kb + KS > k1) {   // past the end of K
             for (int d = half * 64 * X4 + lane; d < (half + 1) * 64 * X4; d += 64)
                 if (kb + x_k(d) >= k1) *(float *)(st + X_AT + 4 * d) = 0.0f;
+            for (int d = half * 64 * S4 + lane; d < (half + 1) * 64 * S4; d += 64)
+                if (kb + k_of(d >> 3) >= k1) *(float *)(st + S_AT + 4 * d) = 0.0f;
+        }
         // the stage is there for both waves of the pair, and everybody has read the one before it
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (kb + KS < k1) stage(~i & 1, kb + KS);
@@ -284,7 +268,7 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
                     for (int part = 0; part < 3; part++) {
                         u32x4 v;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) v[i] = upper_halves(r[2 * i], r[2 * i + 1]);
+                        for (int i = 0; i < 4; i++) v[i] = upper_halves(r[2 * i], r[2 * i + 1], part > 0 ? lower : kUpperHalves);
                         __builtin_memcpy(&a[t][part], &v, 16);
                         if (part < 2)
 #pragma unroll
@@ -342,7 +326,7 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
 
     // The slices' sums, [kPgSlices][R][kSumRow]: a wave's columns as its accumulators hold them (lane n of operand c of pass b
     // at (b SETS + c) 16 + n), the row a little longer than the columns, so that its four lane groups write side by side.
-    constexpr int kSumRow = kPgGroup + 4;
+    constexpr int kSumRow = Map::SUM_ROW;
     float *s_sum = (float *)s_lds;
     const size_t out_n = (size_t)p.n_blocks * 32;
     const bool last_adds = p.y != nullptr;
@@ -350,6 +334,7 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
     const int in_block = BITS == 8 ? (R == 4 ? 4 * ((pn & 3) + 4 * (pc >> 2)) + (pc & 3) : 4 * (pn & 7) + (R == 16 ? 2 * (pn >> 3) : 0) + pc)
                                    : 8 * (pn & 3) + (R == 4 ? pc : (R == 8 ? ((pn >> 2) & 1) + 2 * pc : (pn >> 2) + 4 * pc));
     const size_t col = (size_t)wg * kPgGroup + (size_t)(place / kPgCols * kPgCols + 32 * (pb * (4 / GROUPS) + pn / R) + in_block);
+    bool nan = false;
 #pragma unroll
     for (int t = 0; t < RT; t++) {
         __syncthreads();
@@ -364,32 +349,41 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
                         s_sum[((wave >> 1) * R + 4 * g % R + e) * kSumRow + half * kPgCols + (b * SETS + c) * 16 + n] = acc[t][b][c][e];
         }
         __syncthreads();
-        if (col < out_n)
-            for (int r = tid / kPgGroup; r < R && R * t + r < rows; r += 512 / kPgGroup) {
-                float sum = 0.0f;
+        constexpr int EACH = R * kPgGroup / 512;   // (all reads out before the first sum is stored: 34.6 -> 33.6 us, [4096, 8192] Q8S, 32 rows)
+        float sum[EACH];
 #pragma unroll
-                for (int s = 0; s < kPgSlices; s++) sum = __fadd_rn(sum, s_sum[(s * R + r) * kSumRow + place]);
-                if (BITS == 4) sum = __fmul_rn(sum, 16.0f);
-                if (sum != sum) sum = plain_sum<BITS>(p, row0 + R * t + r, col, part_k0, part_k1);
-                float *dst = p.out + ((size_t)kpart * (size_t)p.m + (size_t)(row0 + R * t + r)) * out_n + col;
-                if (last_adds) __hip_atomic_store(dst, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // past this XCD's L2
-                else *dst = sum;
+        for (int i = 0; i < EACH; i++) {
+            sum[i] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < kPgSlices; s++) sum[i] = __fadd_rn(sum[i], s_sum[(s * R + tid / kPgGroup + 512 / kPgGroup * i) * kSumRow + place]);
+            if (BITS == 4) sum[i] = __fmul_rn(sum[i], 16.0f);
+        }
+#pragma unroll
+        for (int i = 0; i < EACH; i++) {
+            const int r = R * t + tid / kPgGroup + 512 / kPgGroup * i;
+            if (r >= rows || col >= out_n) continue;
+            float *dst = p.out + ((size_t)kpart * (size_t)p.m + (size_t)(row0 + r)) * out_n + col;
+            if (lower == kNoHalves) {
+                const float was = __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (this lane's own store)
+                if (was == was) continue;
             }
+            nan |= sum[i] != sum[i];
+            if (last_adds) __hip_atomic_store(dst, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // past this XCD's L2
+            else *dst = sum[i];
+        }
     }
-    if (!last_adds) return;
-    // the sums of this workgroup are in memory before it counts; the counter returns to 0 with the last
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    unsigned *s_last = (unsigned *)s_lds;
-    // (one counter per row group, blockIdx.y, too: it stands for the sums of these rows alone, and they alone are added)
-    if (tid == 0) *s_last = atomicInc(p.arrived + (size_t)blockIdx.y * (size_t)p.wg_x + wg, (unsigned)p.grid_k - 1);
-    __syncthreads();
-    if (*s_last != (unsigned)p.grid_k - 1) return;
-    const int own = (rows < RT * R ? rows : RT * R) * kPgGroup;
+    return nan;
+}
+
+// The partial sums of one row and column group into p.y, by the workgroup that has left the last of them.
+template <int ROWS>
+__device__ inline void add_parts(const PackedArgs &p, int wg, int row0) {
+    const size_t out_n = (size_t)p.n_blocks * 32;
+    const int own = (p.m - row0 < ROWS ? p.m - row0 : ROWS) * kPgGroup;
     // ascending parts, 16 loads out before the first add (a missing part adds +0.0, which changes nothing)
     auto add = [&](auto items, auto parts) {
         constexpr int ITEMS = decltype(items)::value, PARTS = decltype(parts)::value;
-        for (int i0 = tid; i0 < own; i0 += 512 * ITEMS) {
+        for (int i0 = (int)threadIdx.x; i0 < own; i0 += 512 * ITEMS) {
             float sum[ITEMS];
             size_t at[ITEMS];
             bool in[ITEMS];
@@ -425,10 +419,48 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
 }
 
 template <int BITS, int R, int RT>
+__global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4)) void packed_gemv_kernel(PackedArgs p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // [kPgSlices][2][STAGE]; then the slices' sums, and a word per wave
+    // workgroups of an XCD (equal ids modulo 8) take neighbouring column groups: they share the lines of the scales
+    const int total = p.wg_x * p.grid_k, per_xcd = (total + 7) >> 3;
+    const int lin = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || lin >= total) return;
+    int *s_nan = (int *)(s_lds + PackedMap<BITS, R, RT>::SUMS);
+    // An infinite x*scale has inf - inf in its second part, where the products themselves are infinite and their sum may well be.
+    // A workgroup that finds a sum to be NaN forms its sums again of first parts alone: they hold the infinities, beside which the rest
+    // does not count; what was a number stays.  (One such row among 4: [5120, 17408] Q4S 20 -> 30 us, Q8S 26 -> 37, [2048, 50304] Q4S
+    // 25 -> 39.  Term by term, each row and column by a lane, it made 184, 201 and 275 of them.)
+    for (uint32_t lower = kUpperHalves;; lower = kNoHalves) {
+        // (nothing derived from these is kept in registers for the second time: the kernel's one argument, read again, and its ids)
+        int tid = threadIdx.x, id = lin;
+        const __attribute__((address_space(4))) PackedArgs *args = (const __attribute__((address_space(4))) PackedArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+v"(tid), "+s"(id), "+s"(args), "+s"(lower));
+        const PackedArgs q = *(const PackedArgs *)args;
+        const int nan = __ballot(packed_tile<BITS, R, RT>(q, s_lds, tid, id, lower)) != 0;
+        if ((threadIdx.x & 63) == 0) s_nan[threadIdx.x >> 6] = nan;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (no wait for the stores of the sums)
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < 2 * kPgSlices; w++) any |= s_nan[w];
+        if (uniform(any) == 0 || lower == kNoHalves) break;
+        __syncthreads();
+    }
+    if (p.y == nullptr) return;
+    // the sums of this workgroup are in memory before it counts; the counter returns to 0 with the last
+    const int wg = lin % p.wg_x;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned *s_last = (unsigned *)s_lds;
+    // (one counter per row group, blockIdx.y, too: it stands for the sums of these rows alone, and they alone are added)
+    if (threadIdx.x == 0) *s_last = atomicInc(p.arrived + (size_t)blockIdx.y * (size_t)p.wg_x + wg, (unsigned)p.grid_k - 1);
+    __syncthreads();
+    if (*s_last == (unsigned)p.grid_k - 1) add_parts<RT * R>(p, wg, (int)blockIdx.y * (RT * R));
+}
+
+template <int BITS, int R, int RT>
 void launch_packed(const PackedArgs &p, hipStream_t s) {
-    const size_t ring = (size_t)kPgSlices * 2 * PackedMap<BITS, R, RT>::STAGE, sums = (size_t)kPgSlices * R * (kPgGroup + 4) * 4;
     const dim3 grid((unsigned)(p.wg_x * p.grid_k + 7) / 8 * 8, (unsigned)(p.m + RT * R - 1) / (RT * R));
-    launch_kernel(packed_gemv_kernel<BITS, R, RT>, grid, dim3(512), ring > sums ? ring : sums, s, p);
+    launch_kernel(packed_gemv_kernel<BITS, R, RT>, grid, dim3(512), (size_t)PackedMap<BITS, R, RT>::LDS, s, p);
 }
 
 template <int BITS>

@@ -73,3 +73,51 @@ def test_infinite_rows_give_infinite_sums(bits):
         assert np.array_equal(got[r], want[r], equal_nan=True), r
     ok = [r for r in range(m) if r not in (1, 4, 6, 8)]
     assert np.array_equal(got[ok].view(np.uint32), plain[ok].view(np.uint32))
+
+
+@pytest.mark.parametrize("m", [1, 4, 8, 16, 32])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_infinities_in_every_form_and_in_the_last_scale(bits, m):
+    # (no code 0 beside an infinity: every sum is one; K ends inside a stage, so the infinite scale is that of its padding too)
+    k, n = 1037, 288
+    g = np.random.default_rng(bits + m)
+    codes, scales = quantize_block32(g.uniform(-1, 1, (k, n)).astype(np.float32), bits)
+    bad = m // 2
+    x = g.uniform(0.5, 1, (m, k)).astype(np.float32)
+    x[bad, 5] = np.inf
+    codes[5][codes[5] == 0] = 1
+    codes[k - 1] = np.where(codes[5] < 0, -1, 1)
+    with M.PackedWeight(pack_words(codes, bits), scales, k, n, bits) as w:
+        got = w.gemv(x)
+    assert np.array_equal(got[bad], np.where(codes[5] < 0, -np.inf, np.inf).astype(np.float32))
+    assert np.isfinite(np.delete(got, bad, 0)).all()
+    scales[k - 1, 2] = np.inf
+    with M.PackedWeight(pack_words(codes, bits), scales, k, n, bits) as w:
+        got = w.gemv(x)
+    want = np.where(codes[k - 1, 64:96] < 0, -np.inf, np.inf).astype(np.float32)
+    assert np.array_equal(got[:, 64:96], np.broadcast_to(want, (m, 32)))
+    assert np.isfinite(np.delete(np.delete(got, bad, 0), np.s_[64:96], 1)).all()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_an_infinite_row_costs_a_second_pass_and_no_more(bits):
+    # twice the loop, and the launch: under three times a call without one (a row and column redone term by term: over twenty)
+    k, n, m = 5120, 4096, 4
+    g = np.random.default_rng(bits)
+    wd = M.DeviceBuffer.from_array(g.integers(0, 1 << 32, (k, n * bits // 32), dtype=np.uint32))
+    sd = M.DeviceBuffer.from_array(g.uniform(0.001, 0.01, (k, n // 32)).astype(np.float32))
+    x = g.standard_normal((m, k)).astype(np.float32)
+    bad = x.copy()
+    bad[1, 7] = np.inf
+    yd = M.DeviceBuffer(4 * m * n)
+    with M.SparseMoe(M.SparseMoeConfig(64, 64, 2, 1), max_tokens=1) as clock, M.PackedWeight.wrap_device(wd, sd, k, n, bits) as w:
+        def best(rows):
+            xd, times = M.DeviceBuffer.from_array(rows), []
+            for _ in range(8):
+                clock.timer_start()
+                for _ in range(20):
+                    w.gemv_device(xd, m, yd, clock.stream)
+                times.append(clock.timer_stop())
+            return min(times)
+        plain, infinite = best(x), best(bad)
+    assert infinite <= 3.0 * plain, (infinite, plain)
