@@ -64,14 +64,15 @@ __device__ inline half8 weight_operand(u32x4 v) {
 // what rounding it lost, so that the exponential is good to an ulp or two for every x; about twelve instructions where
 // det_silu has sixty, which were a fifth of a gate/up tile's time.  The exponent stops at +-87, where e^-x and its
 // reciprocal are both normal numbers: beyond it inf - inf and inf * 0 would give NaN.  Above 87 the quotient is x as it is, below
-// -87 it stays under 2e-38 |x|, which no gate of half operands makes large enough to leave the half's zero.
+// -87 it stays under 2e-38 |x|, which no gate of half operands makes large enough to leave the half's zero.  A gate of -inf
+// (a row with an element beyond the halfs) is NaN as in det_silu and the reference: -inf * 0.
 __device__ inline float fast_silu(float x) {
     const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
     const float y = __fmul_rn(c, -1.44269504f);
     const float lost = __builtin_fmaf(c, -1.44269504f, -y);
     float t = __builtin_amdgcn_exp2f(y);
     t = __builtin_fmaf(t, __fmul_rn(lost, 0.693147181f), t);
-    return __fmul_rn(x, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, t)));
+    return x == -__builtin_inff() ? __builtin_nanf("") : __fmul_rn(x, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, t)));
 }
 
 struct WideArgs {

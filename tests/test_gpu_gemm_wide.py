@@ -59,3 +59,22 @@ def test_gates_far_beyond_the_exponential_keep_silu_finite():
     assert np.isfinite(got).all()
     # (silu carries an f32 rounding or three and is stored as a half: half an ulp, 2^-11; below 2^-14 half of its last bit)
     assert (np.abs(got - want) <= np.abs(want) * 2.0 ** -10.9 + 2.0 ** -24).all()
+
+
+def test_infinite_gates_come_out_as_in_the_narrow_kernel():
+    # x beyond the halfs is an infinity to both kernels: a gate of -inf is NaN (-inf * 0), one of +inf an infinity
+    H, I, E, n = 256, 128, 224, 72 * 224
+    one, minus = np.float16(1.0).view(np.uint16), np.float16(-1.0).view(np.uint16)
+    gate, up, down = (np.full(s, one, np.uint16) for s in ((E, I, H), (E, I, H), (E, H, I)))
+    gate[1::2] = minus   # every second expert
+    x = np.full((n, H), 0.01, np.float32)
+    x[5:7, 0] = 1e6
+    ids = (np.arange(n, dtype=np.int32) % E)[:, None]   # rows 5 and 6: experts 5 and 6
+    w = np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.uint16), M.F16, gate, M.F16, up, M.F16, down, M.F16)
+        wide, narrow = m.apply_routing(0, ids, w, x), m.apply_routing(0, ids[:64], w[:64], x[:64])
+    for got in (wide, narrow):
+        assert np.isnan(got[5]).all()
+        assert np.array_equal(got[6], np.full(H, np.inf, np.float32))
+        assert np.isfinite(np.delete(got, (5, 6), 0)).all()
