@@ -197,26 +197,30 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * s = max|x| over the block / 32512.  Every integer sum is exact; what is lost is |x - s*q| <= s/2 per element, so
  *     |y - y_exact| <= sum over blocks of (max|x| of the block / 65024) * (sum of |w| over the block).
  * Measured as the reference measures it (error relative to the root-sum-square of the terms, experts.rs:1264-1271)
- * that is 1e-4 (Q4_K) / 6e-5 (Q8_0) on the decode path and 6e-4 / 9e-5 on the batched path for the benchmark shapes,
+ * that is 1e-4 (Q4_K) / 6e-5 (Q8_0) on the decode path and 6e-4 (Q4_K) on the batched path for the benchmark shapes,
  * against the 2e-3 bar.  The bound is absolute per block, not relative per element: an element 2^10 below its
  * block's maximum keeps 5 bits.  This shows in one corner: a token whose SwiGLU hidden row is all but zero except
  * for one or two elements (every gate pre-activation far below zero) has outputs orders of magnitude below the
  * batch's, and relative to THAT magnitude single elements come out up to 4e-3 off (2e-8 of the batch's typical
  * output).  F32 / F16 / BF16 banks do not take this path (f32 or f16 products).
- * One exception on the batched path: Q4_K gate/up (and down) banks.  A Q4_K weight is d * (sc * q) - dmin * m
+ * Two exceptions on the batched path.  Q4_K gate/up (and down) banks: a Q4_K weight is d * (sc * q) - dmin * m
  * with sc * q < 1024 an exact half, so their grouped GEMM runs on the f16 matrix units against activations held
  * as PAIRS of halfs, x = 2^e * (hi + lo), hi = f16(x / 2^e), lo = f16(x / 2^e - hi), 2^e one power of two per row
- * (per 128 elements between the two products): 22 significant bits per element, every element of a row down to
- * 2^-24 of the row's largest.  That form measures 2e-6 by the reference's measure and has no such corner; it is
- * also the faster one.  (A row that holds an infinity comes out NaN in that form, where f32 products give an infinity.)  The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
+ * (per 128 elements between the two products): 22 significant bits per element down to 2^-13 of the row's largest, an
+ * absolute error of at most 2^-34 of that largest one below.  That form measures 2e-6 by the reference's measure and has no
+ * such corner; it is also the faster one.  (A row that holds an infinity comes out NaN in that form, where f32 products give an
+ * infinity.)  Q8_0 banks (gate, up and down, hidden and inter multiples of 128) are held against the same pairs where that form is
+ * the faster one, by the rows an expert has; 2.5e-7 off the 64-bit result where the integer form is by 4.5e-5.  Its one corner: a row
+ * whose large elements fill blocks of 64 of their own AND meet weights of 0 keeps less of its small ones than the integer form
+ * (elements 2^-20 of the row's largest 2^-13 of themselves, 2^-26 2^-7).  mummu_expert_run takes these forms from 64 rows on.
+ * The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
  * integer form above; MUMMU_GEMM_TILE_ROWS=16, 32 or 64 fixes the rows per tile of these kernels (by default the
  * library picks the form with the smallest expected cost for the batch: same results, different speed).
- * Q8_0 banks have an optional second form on the batched path, MUMMU_GEMM_Q8_F16=1 (read by mummu_moe_create):
+ * Q8_0 banks have an optional further form on the batched path, MUMMU_GEMM_Q8_F16=1 (read by mummu_moe_create):
  * the grouped GEMM of the F16 banks with every weight d * code held exactly as two halfs, x and the activations
  * between the two products rounded to halfs as for F16 / BF16 banks (values beyond 65504 overflow there).  It is
- * 1.1 to 1.5 times faster and measures 1.3e-3 to 1.6e-3 by the reference's measure where the integer form measures
- * 2e-4, which is why it is not the default; a layer with a block whose |d| * 128 is no finite half keeps the
- * integer form. */
+ * 1.1 to 1.5 times faster than the integer form and measures 1.3e-3 to 1.6e-3 by the reference's measure where that measures
+ * 2e-4, which is why it is not the default; a layer with a block whose |d| * 128 is no finite half does not take it. */
 
 /* ---- device-pointer entry points (no host copies, no synchronisation) ------------------
  * stream is a hipStream_t (NULL = the null stream).  Safe to capture into a HIP graph:

@@ -8,6 +8,11 @@
 // stage (128 elements) come in one piece, 64 neighbouring dwords a load, straight into LDS, two stages ahead: 141 us (OLMoE layer, 19
 // to 100 tokens; 150: 204 -> 153, 512: 350 -> 294), 2.5e-7 off the 64-bit result where the int8 form is by 4.5e-5.
 //
+// x has one scale for its whole row (HAct): an element is off by at most 2^-34 of the row's largest, where the int8 form's is off
+// by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of their own and
+// meet weights of 0: a block 2^20 (2^26) above the rest 1.0e-4 (6.4e-3) off the 64-bit result, the int8 form 4.6e-5.  A single element
+// 2^20 above it, its weights 0: 5.0e-5, the int8 form, which loses its 63 neighbours, 2.4e-1; weights as they come: 3.3e-7 and 3.1e-5.
+//
 // A workgroup has 256 weight rows (128 of gate and 128 of up), a wave 32 of them, which it loads for itself; the activation tile is
 // shared.  Lane (column c, K group g) reads 16 of a block's 32 codes, so element 16 g + 8 kk + i of the block is the K index
 // 8 g + i of its product kk, and the A operands are read from the tile to match.

@@ -583,7 +583,8 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
 // former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323; Q8_0 64: 121 / 106,
 // 128: 223 / 143, 512: 789 / 353.  Only banks that are Q4_K or Q8_0 throughout: their GEMM holds rows as pairs of halfs (1.0e-7
 // and 2.5e-7 off the 64-bit result, the per-row kernels 2.8e-5 and 3.3e-5), the int8 GEMM of the other types a scale per 64
-// elements, where the per-row kernels have one per 16.
+// elements, where the per-row kernels have one per 16.  (One scale per row there, one per 16 elements in the per-row kernels: a row
+// whose large elements fill blocks of 16 and meet weights of 0 keeps more of its small ones in the latter, see gemm_q8.hip.)
 constexpr int kOneExpertGemm = 64;
 
 // The Q4_K form's tiles: the smallest whose launch is at most one workgroup per CU (512 rows of OLMoE, tiles of 16 / 32 / 64 rows: 323 / 330 /

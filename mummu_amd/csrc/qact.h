@@ -101,10 +101,10 @@ __device__ inline void quantize_store64(float4 v, bool active, const QAct64 &q, 
     }
 }
 
-// Activations for the products of Q4_K banks on the f16 matrix units: every element as a pair of
+// Activations for the products of Q4_K and Q8_0 banks on the f16 matrix units: every element as a pair of
 // halfs, x = scale * (hi + lo) with hi = f16(x / scale), lo = f16(x / scale - hi), and a power-of-two
 // scale chosen so that the largest |x / scale| it covers lies in [2^9, 2^10): 22 significant bits per
-// element (elements more than 2^24 below that largest one keep an absolute error of 2^-25 of it), and
+// element down to 2^-13 of that largest one, an absolute error of at most 2^-34 of it below, and
 // sums of 32 scaled elements stay below 2^15, inside a half's range.  The scale array has one entry per
 // 128 elements; a producer that sees whole rows (quantize_rows_h) writes the same scale into all of a
 // row's entries, one that sees 128 columns at a time (the gate/up epilogue) a scale per entry.

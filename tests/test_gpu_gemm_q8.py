@@ -34,3 +34,56 @@ def test_tile_edges_match_the_f64_reference(H, I):
     for rows, y in alone.items():
         want, mag = orc.moe_ref_f64(banks, np.full((rows, 1), E - 1, np.uint32), np.ones((rows, 1), np.float32), x[:rows])
         assert orc.rel_err(y, want, mag).max() <= 3e-5
+
+
+def outlier_case(wide_block):
+    # Rows with one element (or one block of 64) standing out by 2^20; the weights that meet it are 0, so that what comes out is
+    # made of the small ones.
+    H, I, E, n = 512, 256, 4, 130
+    banks = [np.frombuffer(synth.random_bank_fast(M.Q8_0, ne, s), np.uint8).copy() for s, ne in ((1, [H, I, E]), (2, [H, I, E]), (3, [I, H, E]))]
+    x = np.random.default_rng(9).standard_normal((n, H)).astype(np.float32)
+    blocks = [b.reshape(-1, H // 32, 34) for b in banks[:2]]
+    if wide_block:
+        x[:, :64] *= np.float32(2.0 ** 20)
+        for b in blocks:
+            b[:, :2, 2:] = 0
+    else:
+        x[:, 7] = np.float32(2.0 ** 20) * np.sign(x[:, 7])
+        for b in blocks:
+            b[:, 0, 2 + 7] = 0
+    return H, I, E, n, banks, x
+
+
+@pytest.mark.parametrize("factor", [1.0, 2000.0, 2.0 ** 20])
+def test_rows_with_one_element_standing_out_keep_their_small_elements(factor):
+    H, I, E, n = 512, 256, 4, 130
+    gate, up = (synth.random_bank_fast(M.Q8_0, [H, I, E], seed) for seed in (1, 2))
+    down = synth.random_bank_fast(M.Q8_0, [I, H, E], 3)
+    x = np.random.default_rng(9).standard_normal((n, H)).astype(np.float32)
+    x[:, 7] *= np.float32(factor)
+    x[::3, 500] *= np.float32(-factor)
+    ids, w = (np.arange(n, dtype=np.int32) % E)[:, None], np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got, alone = m.apply_routing(0, ids, w, x), m.expert_run(0, 1, x)
+    banks = orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0)
+    want, mag = orc.moe_ref_f64(banks, ids, w, x)
+    assert orc.rel_err(got, want, mag).max() <= 3e-5
+    want, mag = orc.moe_ref_f64(banks, np.ones((n, 1), np.uint32), w, x)
+    assert orc.rel_err(alone, want, mag).max() <= 3e-5
+
+
+@pytest.mark.parametrize("wide_block", [False, True])
+def test_the_limit_of_one_scale_per_row(wide_block):
+    # An element is off by at most 2^-34 of its row's largest (2^20 times up to 4.5 here), at random: at most 2^-11.8 of an element of
+    # 1, by root mean square a quarter of that (rows' largest are half of it, errors are uniform), in gate and up alike, whose product
+    # carries both: 2^-12 of the result in norm.
+    H, I, E, n, (gate, up, down), x = outlier_case(wide_block)
+    ids, w = (np.arange(n, dtype=np.int32) % E)[:, None], np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got, alone = m.apply_routing(0, ids, w, x), m.expert_run(0, 1, x)
+    banks = orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0)
+    for y, e in ((got, ids), (alone, np.ones((n, 1)))):
+        want, _ = orc.moe_ref_f64(banks, e.astype(np.uint32), w, x)
+        assert np.linalg.norm(y - want) <= 2.0 ** -12 * np.linalg.norm(want)
