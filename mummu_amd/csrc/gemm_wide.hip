@@ -243,8 +243,11 @@ bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign) {
           (size_t)n_assign * (size_t)b.inter * 2 < (1ull << 32)))
         return false;
     // Up to 64 rows per expert either kernel streams the weights once, and the smaller workgroups of grouped_gemm_f16_kernel,
-    // several to a CU, do it better (OLMoE layers, 64 rows: 180 us there, 186 us here; 80 rows: 211 / 195; 125: 278 / 224).
-    // One workgroup fills a CU here, so a launch needs about as many of them as there are CUs.
+    // several to a CU, do it better (OLMoE layers, 64 rows: 207 us there, 237 us here; 72: 256 / 245, 80: 260 / 249, 128: 325 / 276; 512
+    // experts of 2560 x 640, 64: 1852 / 1907, 72: 2195 / 2018; 128 of 2048 x 768, 64: 366 / 354, 72: 427 / 381; 16 of 4096 x 1792, 64: 411 /
+    // 402, 72: 428 / 417, 128: 568 / 490).
+    // One workgroup fills a CU here, so the line also asks for about as many of them as there are CUs.  The one smaller launch that
+    // was measured on both sides is ahead all the same (8 experts of 4096 x 1536, 96 workgroups, 72 rows 311 / 275, 256: 491 / 484).
     const size_t tiles = (size_t)n_assign / kWideRows > (size_t)b.n_experts ? (size_t)n_assign / kWideRows : (size_t)b.n_experts;
     const size_t out_dim = (size_t)(b.inter * 2 < b.hidden ? b.inter * 2 : b.hidden);
     return (size_t)n_assign >= 72 * (size_t)b.n_experts && tiles * (out_dim / kWCols) >= 224;

@@ -93,7 +93,12 @@ struct mummu_moe {
     // batches at least this large take dispatch + grouped GEMM (measured crossovers on the OLMoE shape:
     // the 16-bit float decode kernels lose from 7 tokens on, the f32 ones from 10, the integer ones from 19)
     int gemm_min_f16 = 7, gemm_min_quant = 19, gemm_min_f32 = 10;
-    int gemm_min_q8 = 13;    // Q8_0 banks on the f16 units (10 / 12 / 14 tokens: 137 / 137 / 138 against 121 / 140 / 155 us)
+    // Q8_0 banks on the f16 units: us of the batched against the decode kernels at 10 / 12 / 13 / 14 / 18 tokens, 64 experts (2048 x
+    // 1024, top-8) 121 / 125 / 127 / 127 / 132 against 109 / 129 / 138 / 145 / 175, 16 (4096 x 1792, top-2) 112 / 113 / 114 / 114 / 120
+    // against 126 / 143 / 163 / 173 / 222, 512 (2560 x 640, top-10) 174 / 219 / 223 / 230 / 285 against 206 / 245 / 264 / 277 / 352.  The
+    // line is late for the last and early for 128 experts (2048 x 768, top-8: 119 / 133 / 137 / 141 / 171 against 97 / 116 / 127 / 136 /
+    // 162, alike from 19), where the batched kernels' results are a hundred times nearer the 64-bit ones.
+    int gemm_min_q8 = 13;
     int gemm_min_q4k = 18;   // Q4_K banks on the f16 units (17 tokens: 88.8 us either way; 18: 89.1 against 92.6 us)
     int gemm_q4k_f16 = 1;        // Q4_K banks of the batched path on the f16 units (0: the int8 form)
     int gemm_q8_f16 = 0;         // 1: Q8_0 banks of the batched path through the f16 kernel (x and activations as halfs)
@@ -491,13 +496,22 @@ struct HalfPlan {
     HAct xh;
 };
 
-// Where the 32-row tiles of gemm_q8.hip are ahead of the int8 form's 64-row ones, by the rows of an expert (OLMoE layers, here /
-// int8): up to 33, where next to none needs a second tile (150 tokens: 153 / 204 us, 260: 198 / 219), and from where many need a
-// second tile of 64 (400 tokens = 50 rows: 283 / 332, 700: 382 / 401, 1500: 671 / 673).  In between one tile of 64 holds
-// an expert (300 tokens: 243 / 228), and beyond 190 rows the weights are read too often (2048 tokens: 876 / 865).
-bool q8_gemm_should(size_t n_assign, int n_experts) {
-    const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
-    return avg <= 33.0 || (avg + 2.2 * __builtin_sqrt(avg) >= 64.0 && avg <= 190.0);
+// Which Q8_0 batches take the 32-row tiles of gemm_q8.hip and which the int8 form's 64-row ones, by the rows of an expert.  Layers of
+// 64 / 128 / 512 experts (hidden x inter 2048 x 1024, 2048 x 768, 2560 x 640) and 16 (4096 x 1792), us here / int8:
+//   up to 33 rows next to none needs a second tile: 16 rows 142 / 179, 216 / 271, 917 / 990, 236 / 315; 33: 224 / 217, 331 / 363, 1386 /
+//   1400, 324 / 364.
+//   While a tile of 64 holds every expert the int8 form reads the weights once: 40 rows 237 / 228, 372 / 374, 1595 / 1477, 364 / 428;
+//   42: 237 / 228, 378 / 384.
+//   Beyond, some need a second one.  In a launch of a few rounds of workgroups that is another round for all: 44 rows 238 / 311, 381 /
+//   383, 381 / 448; 64: 289 / 347, 473 / 530, 496 / 562; 80: 334 / 387, 564 / 622, 517 / 577.  In one of many rounds it costs what it
+//   weighs, and the two are nearly alike from where half the experts do: 512 experts, 52 rows 1889 / 1778, 64: 2277 / 2254, 80: 2743 / 2746.
+//   From 90 rows on the weights are read more often here: 96 rows 392 / 376, 636 / 632, 607 / 602; 128: 495 / 495, 785 / 775, 759 / 858;
+//   160: 575 / 556, 973 / 937, 937 / 923.  Up to 190 the pairs of halfs, a hundred times nearer the 64-bit result, are kept for these few
+//   per cent; at 256 rows it is 6 (871 / 823, 1394 / 1299, 1307 / 1245).
+bool q8_gemm_should(const ExpertBanks &b, size_t n_assign) {
+    const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
+    const size_t workgroups = (size_t)b.n_experts * (size_t)(b.inter / 128);   // of a gate/up launch with a tile per expert
+    return avg <= 33.0 || (avg + (workgroups <= 1024 ? 3.2 : 2.2) * __builtin_sqrt(avg) >= 64.0 && avg <= 190.0);
 }
 
 // (one_expert: all n rows go to the same one)
@@ -506,7 +520,7 @@ HalfPlan half_plan(const mummu_moe *h, const ExpertBanks &b, int64_t n, int k, b
     const size_t na = (size_t)(n * k);
     // (its kernels address the activation planes with 32-bit byte offsets)
     const bool small32 = na * (size_t)(b.hidden > b.inter ? b.hidden : b.inter) * 2 < (1ull << 32);
-    p.q8 = small32 && q8_half_pairs(h, b) && (one_expert || q8_gemm_should(na, b.n_experts));
+    p.q8 = small32 && q8_half_pairs(h, b) && (one_expert || q8_gemm_should(b, na));
     p.hf = p.q8 || (h->gemm_q4k_f16 && small32 && grouped_gemm_q4k_f16(b));
     p.hf_down = p.q8 || (p.hf && grouped_gemm_q4k_f16_down(b));
     // x as pairs of halfs borrows h->y (the down product's output, written only after the gate/up launch has read x) and
@@ -581,7 +595,9 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
 // Rows from which one expert alone takes the grouped GEMM pair of the f16 units: the per-row kernels decode every weight again
 // for each few rows, a GEMM of one expert has few workgroups and the latency of its loop over K.  Host call, OLMoE Q4_K, the
 // former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323; Q8_0 64: 121 / 106,
-// 128: 223 / 143, 512: 789 / 353.  Only banks that are Q4_K or Q8_0 throughout: their GEMM holds rows as pairs of halfs (1.0e-7
+// 128: 223 / 143, 512: 789 / 353.  On the device alone the lines cross at 53 rows there, and for 2048 x 768 / 2560 x 768 / 4096 x 1792 at
+// 58 / 34 / 24 (Q4_K) and 46, 51 / 40 / 22 (Q8_0): 64 rows 36 / 32, 31 / 30, 52 / 32, 113 / 51 us (Q4_K), 65 / 49, 54 / 45, 76 / 52,
+// 220 / 84 (Q8_0).  Only banks that are Q4_K or Q8_0 throughout: their GEMM holds rows as pairs of halfs (1.0e-7
 // and 2.5e-7 off the 64-bit result, the per-row kernels 2.8e-5 and 3.3e-5), the int8 GEMM of the other types a scale per 64
 // elements, where the per-row kernels have one per 16.  (One scale per row there, one per 16 elements in the per-row kernels: a row
 // whose large elements fill blocks of 16 and meet weights of 0 keeps more of its small ones in the latter, see gemm_q8.hip.)
