@@ -169,6 +169,27 @@ __device__ inline float det_silu(float x) {
     return __fdiv_rn(x, den);
 }
 
+// ---- values that are the same in every lane, and loads from global memory straight into LDS ----
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline const uint8_t *uniform(const uint8_t *p) {
+    const uint64_t v = (uint64_t)p;
+    return (const uint8_t *)((uint64_t)(uint32_t)uniform((int)v) | (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32);
+}
+
+// Where a __shared__ object lies, as the loads below take it.
+__device__ inline uint32_t lds_offset(const void *shared) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)shared;
+}
+
+// 16 or 4 bytes a lane from base + off into LDS at lds + 16 (4) * lane, lds and base the same in every lane.  In flight until the
+// wave has waited for vmcnt; the caller sees to that and to the barrier behind it.
+__device__ inline void load_to_lds16(uint32_t lds, const uint8_t *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
+}
+__device__ inline void load_to_lds4(uint32_t lds, const uint8_t *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
+}
+
 // Butterfly sum over aligned groups of `width` lanes (width a power of two <= 64).
 __device__ inline float group_sum(float v, int width) {
     for (int off = width >> 1; off >= 1; off >>= 1) v = __fadd_rn(v, __shfl_xor(v, off, kWave));

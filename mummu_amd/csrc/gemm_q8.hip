@@ -39,19 +39,6 @@ constexpr int kLdsBytes = kRing * kStageW + 2 * kStageA;
 constexpr int kRowC = 128 + 4;               // f32 row of the gate/up epilogue
 static_assert(32 * kRowW % 256 == 0 && 2 * kRows * kRowC * 4 <= kLdsBytes, "whole loads; the epilogue fits the stages");
 
-__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline const uint8_t *uniform(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    return (const uint8_t *)((uint64_t)(uint32_t)uniform((int)v) | (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32);
-}
-// 16 or 4 bytes a lane from base + off into LDS at lds + 16 (4) * lane.
-__device__ inline void load_to_lds16(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
-}
-__device__ inline void load_to_lds4(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
-}
-
 // Eight codes as halfs, in the element order of HAct: a byte b ^ 0x80 under 0x64 is the half 1024 + 128 + b.
 __device__ inline half8 q8_codes(uint32_t w0, uint32_t w1) {
     const half2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
@@ -86,8 +73,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     const int e = uniform(tiles[3 * tile]), p0 = uniform(tiles[3 * tile + 1]), rows = uniform(tiles[3 * tile + 2]);
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 31, g = lane >> 5;
     const uint32_t row_bytes = (uint32_t)(in_dim / kStep) * kRowW;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)s_lds;
-    const uint32_t lds_as = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)(uint8_t *)s_as;
+    const uint32_t lds0 = lds_offset(s_lds);
+    const uint32_t lds_as = lds_offset(s_as);
     const int n_steps = in_dim / kStep;
 
     // this wave's weight rows: first .. first + 31 of gate (waves 0-3), up (4-7) or down

@@ -30,17 +30,6 @@ constexpr int kWCols = 256;                      // weight rows of a tile
 constexpr int kWATile = kWideRows * kWK * 2;     // bytes of a stage: activation rows, then weight rows
 constexpr int kWStage = kWATile + kWCols * kWK * 2;
 
-__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline const uint8_t *uniform(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    return (const uint8_t *)((uint64_t)(uint32_t)uniform((int)v) | (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32);
-}
-
-// 16 bytes a lane from base + off into LDS at lds + 16 * lane.
-__device__ inline void load_to_lds(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(base) : "memory");
-}
-
 // Every load this wave has asked for has landed, every LDS read it has asked for is in its registers; then everybody's.
 __device__ inline void settle() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -95,9 +84,9 @@ struct Loader {
     __device__ void stage(uint32_t at, int step, int wave) const {
         const uint8_t *ab = a_base + (size_t)step * (kWK * 2), *bb = b_base + (size_t)step * (kWK * 2);
 #pragma unroll
-        for (int i = 0; i < MW; i++) load_to_lds(at + (uint32_t)(8 * MW * wave + 8 * i) * (kWK * 2), ab, a_off[i]);
+        for (int i = 0; i < MW; i++) load_to_lds16(at + (uint32_t)(8 * MW * wave + 8 * i) * (kWK * 2), ab, a_off[i]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) load_to_lds(at + kWATile + (uint32_t)(32 * wave + 8 * i) * (kWK * 2), bb, b_off[i]);
+        for (int i = 0; i < 4; i++) load_to_lds16(at + kWATile + (uint32_t)(32 * wave + 8 * i) * (kWK * 2), bb, b_off[i]);
     }
 };
 
@@ -107,7 +96,7 @@ __device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3, g = lane >> 5, lr = lane & 31;
     const uint32_t row_bytes = (uint32_t)p.in_dim * 2u;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)s_lds;
+    const uint32_t lds0 = lds_offset(s_lds);
     const int n_steps = p.in_dim / kWK;
 
     Loader<MW> l;

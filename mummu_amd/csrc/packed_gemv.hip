@@ -72,20 +72,6 @@ struct PackedArgs {
     unsigned *arrived;       // ... counted here, [row group][wg_x], 0 between launches
 };
 
-__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline const uint8_t *uniform(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    return (const uint8_t *)((uint64_t)(uint32_t)uniform((int)v) | (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32);
-}
-
-// 16 or 4 bytes a lane from base + off into LDS at lds + 16 (4) * lane.
-__device__ inline void load_to_lds16(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
-}
-__device__ inline void load_to_lds4(uint32_t lds, const uint8_t *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
-}
-
 // The four-bit code in the low half of byte `b` of w, over 16 (the sums are multiplied by 16 at the end).
 template <int B>
 __device__ inline float nibble(uint32_t w) {
@@ -147,7 +133,7 @@ __device__ inline bool packed_tile(const PackedArgs &p, uint8_t *s_lds, int tid,
     auto x_row = [&](int row) { return row < rows ? row : rows - 1; };
     auto x_k = [&](int d) { return ((d % KS / 4) ^ x_turn(d / KS)) * 4 + (d & 3); };   // k of dword d
     const uint32_t row_bytes = (uint32_t)p.n_words * 4u, srow_bytes = (uint32_t)p.n_blocks * 4u;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)s_lds + (uint32_t)(wave >> 1) * (2 * STAGE);
+    const uint32_t lds0 = lds_offset(s_lds) + (uint32_t)(wave >> 1) * (2 * STAGE);
     auto block = [&](int b) { return block0 + b < p.n_blocks ? block0 + b : p.n_blocks - 1; };   // (columns past the last block repeat it)
     // byte offset in a k row of the word at place w of row rho
     auto word_off = [&](int rho, int w) {
