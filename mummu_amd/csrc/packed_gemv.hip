@@ -24,15 +24,15 @@
 // Two waves take 256 columns (whole 128-byte lines of words: with half lines the requests are the limit, 34 against 29 us
 // on [8192, 20480]) and a slice of K, the words, scales and x straight from memory into LDS, a stage of 32 k ahead.  A word
 // holds 8 (or 4) columns at one k, so reading it for eight k gives a lane the B operands of as many columns without a
-// transposition.  Four such pairs are a workgroup and meet in LDS in ascending order, the workgroups of a column group (and of
-// the same rows) through partial sums, added in ascending order by the one that comes last, or, if they are many, by a second
-// kernel.  Which slice a k belongs to and the order of every sum depend on the weight alone: a row's bits are the same whatever
+// transposition.  Four such pairs are a workgroup and meet in LDS in ascending order, the workgroups of a column group through
+// partial sums, added in ascending order by the one that comes last, or, if they or the rows are many, by a second kernel.  Which slice a k belongs to and the order of every sum depend on the weight alone: a row's bits are the same whatever
 // shares the launch.
 //
 // [5120, 17408] Q4S, 1 / 4 / 16 / 64 rows: 17.6 / 29.1 / 86 / 327 -> 17.5 / 17.8 / 26.9 / 88 us; Q8S 25.8 / 38.0 / 108 / 407 ->
-// 22.9 / 24.4 / 37 / 102; [2048, 4096] Q4S 9.4 / 17.6 / 18.3 / 36.5 -> 8.0 / 8.7 / 11.0 / 16.4.  Now the vector ALUs bound it
-// (700 clocks of decoding and splitting per 32 x 128 weights at up to 4 rows, 1220 at 16), below 10 MB the chain of launch, first
-// load and meeting of the partial sums (6 us).
+// 22.9 / 24.4 / 37 / 102; [2048, 4096] Q4S 9.4 / 17.6 / 18.3 / 36.5 -> 7.8 / 8.2 / 10.9 / 16.5.  Nearest to
+// a bound now are the vector ALUs (700 clocks of decoding and splitting per 32 x 128 weights at up to 4 rows, 1220 at 16; a launch of 4
+// rows, 18.9 us or some 42 k clocks in a trace, has 17.8 k clocks of them and 8.2 k of the matrix units on each SIMD), below 10 MB the
+// chain of launch, first load and meeting of the partial sums (6 us).
 #include "device_utils.h"
 #include "host_staging.h"
 #include "kernels.h"
@@ -58,6 +58,7 @@ constexpr int kPgSlices = 4;      // K slices of a workgroup, each a pair of wav
 constexpr int kPgCols = 128;      // columns of a wave: four scale blocks
 constexpr int kPgGroup = 2 * kPgCols;   // columns of a pair, and of the workgroup
 constexpr int kPgStage = 32;      // K elements of a stage
+constexpr int kLastRows = 8;      // up to which the last workgroup of a column group may add the partial sums: one row group
 
 struct PackedArgs {
     const uint32_t *words;   // [k_len][n_words]
@@ -68,8 +69,8 @@ struct PackedArgs {
     int wg_x, grid_k;        // column groups of kPgGroup, workgroups along K
     bool words16, x16;       // the words, the rows of x are 16-byte aligned
     float *out;              // y, or [grid_k][m][n] partial sums
-    float *y;                // not null: the last workgroup of a row and column group adds the partial sums into it
-    unsigned *arrived;       // ... counted here, [row group][wg_x], 0 between launches
+    float *y;                // not null (one row group only): the last workgroup of a column group adds the partial sums into it
+    unsigned *arrived;       // ... counted here, [wg_x], 0 between launches
 };
 
 // The four-bit code in the low half of byte `b` of w, over 16 (the sums are multiplied by 16 at the end).
@@ -315,7 +316,7 @@ __device__ inline bool packed_tile(const PackedArgs &p, uint8_t *s_lds, int tid,
     constexpr int kSumRow = Map::SUM_ROW;
     float *s_sum = (float *)s_lds;
     const size_t out_n = (size_t)p.n_blocks * 32;
-    const bool last_adds = p.y != nullptr;
+    const bool last_adds = R <= kLastRows && p.y != nullptr;
     const int place = tid % kPgGroup, pn = place & 15, pc = (place >> 4) % SETS, pb = place % kPgCols / (16 * SETS);
     const int in_block = BITS == 8 ? (R == 4 ? 4 * ((pn & 3) + 4 * (pc >> 2)) + (pc & 3) : 4 * (pn & 7) + (R == 16 ? 2 * (pn >> 3) : 0) + pc)
                                    : 8 * (pn & 3) + (R == 4 ? pc : (R == 8 ? ((pn >> 2) & 1) + 2 * pc : (pn >> 2) + 4 * pc));
@@ -361,15 +362,13 @@ __device__ inline bool packed_tile(const PackedArgs &p, uint8_t *s_lds, int tid,
     return nan;
 }
 
-// The partial sums of one row and column group into p.y, by the workgroup that has left the last of them.
-template <int ROWS>
-__device__ inline void add_parts(const PackedArgs &p, int wg, int row0) {
+// The partial sums of a column group into p.y, by the workgroup that has left the last of them.
+__device__ inline void add_parts(const PackedArgs &p, int wg) {
     const size_t out_n = (size_t)p.n_blocks * 32;
-    const int own = (p.m - row0 < ROWS ? p.m - row0 : ROWS) * kPgGroup;
     // ascending parts, 16 loads out before the first add (a missing part adds +0.0, which changes nothing)
     auto add = [&](auto items, auto parts) {
         constexpr int ITEMS = decltype(items)::value, PARTS = decltype(parts)::value;
-        for (int i0 = (int)threadIdx.x; i0 < own; i0 += 512 * ITEMS) {
+        for (int i0 = (int)threadIdx.x; i0 < p.m * kPgGroup; i0 += 512 * ITEMS) {
             float sum[ITEMS];
             size_t at[ITEMS];
             bool in[ITEMS];
@@ -377,8 +376,8 @@ __device__ inline void add_parts(const PackedArgs &p, int wg, int row0) {
             for (int j = 0; j < ITEMS; j++) {
                 const int i = i0 + 512 * j, c = wg * kPgGroup + i % kPgGroup;
                 sum[j] = 0.0f;
-                in[j] = i < own && c < p.n_blocks * 32;
-                at[j] = (size_t)(row0 + (in[j] ? i / kPgGroup : 0)) * out_n + (size_t)(in[j] ? c : 0);
+                in[j] = i < p.m * kPgGroup && c < p.n_blocks * 32;
+                at[j] = (size_t)(in[j] ? i / kPgGroup : 0) * out_n + (size_t)(in[j] ? c : 0);
             }
             for (int s0 = 0; s0 < p.grid_k; s0 += PARTS) {
                 float v[ITEMS][PARTS];
@@ -431,16 +430,17 @@ __global__ __launch_bounds__(512, (PackedMap<BITS, R, RT>::STAGE > 10240 ? 2 : 4
         if (uniform(any) == 0 || lower == kNoHalves) break;
         __syncthreads();
     }
-    if (p.y == nullptr) return;
-    // the sums of this workgroup are in memory before it counts; the counter returns to 0 with the last
-    const int wg = lin % p.wg_x;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    unsigned *s_last = (unsigned *)s_lds;
-    // (one counter per row group, blockIdx.y, too: it stands for the sums of these rows alone, and they alone are added)
-    if (threadIdx.x == 0) *s_last = atomicInc(p.arrived + (size_t)blockIdx.y * (size_t)p.wg_x + wg, (unsigned)p.grid_k - 1);
-    __syncthreads();
-    if (*s_last == (unsigned)p.grid_k - 1) add_parts<RT * R>(p, wg, (int)blockIdx.y * (RT * R));
+    if constexpr (R <= kLastRows) {   // (the counter and the sums are those of all rows: forms with one row group)
+        if (p.y == nullptr) return;
+        // the sums of this workgroup are in memory before it counts; the counter returns to 0 with the last
+        const int wg = lin % p.wg_x;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        unsigned *s_last = (unsigned *)s_lds;
+        if (threadIdx.x == 0) *s_last = atomicInc(p.arrived + wg, (unsigned)p.grid_k - 1);
+        __syncthreads();
+        if (*s_last == (unsigned)p.grid_k - 1) add_parts(p, wg);
+    }
 }
 
 template <int BITS, int R, int RT>
@@ -485,7 +485,7 @@ struct mummu_packed_weight {
     uint32_t *words = nullptr;  // device [K][n_words]
     float *scales = nullptr;    // device [K][N/32]
     float *x = nullptr, *y = nullptr, *partial = nullptr;  // staging for the host-pointer call and the K partials
-    unsigned *arrived = nullptr;  // per row and column group: workgroups that have left their partial sums
+    unsigned *arrived = nullptr;  // per column group: workgroups that have left their partial sums
     int k = 0, n = 0, bits = 4, wg_x = 1, grid_k = 1, stages = 1;
     bool owns_weight = true;  // false: words and scales are the caller's device buffers
     hipStream_t stream = nullptr;
@@ -496,10 +496,6 @@ struct mummu_packed_weight {
 namespace {
 
 constexpr int kMaxRows = 64;  // nn/packed_gemv.rs:138: row by row up to 64 rows
-// Rows times workgroups along K up to which the last workgroup of a row and column group adds the partial sums: a second launch costs
-// 3 us, reading them past the L2 0.05 us a row and workgroup.
-constexpr int kLastAdds = 64;
-constexpr int kRowGroups = kMaxRows / 16;   // most row groups of a launch: it takes 16 rows or more each, or has one
 thread_local std::string g_packed_error;
 
 int pfail(mummu_packed_weight *w, int code, const std::string &msg) {
@@ -508,9 +504,23 @@ int pfail(mummu_packed_weight *w, int code, const std::string &msg) {
     return code;
 }
 
+// Whether the last workgroup of a column group adds the partial sums or a second launch does, for 0.3 to 0.8 us.  What the last one
+// costs grows with the rows, the parts and the workgroups that end together with it; from 64 column groups on, two workgroups to a CU,
+// they end one after the other (us, last workgroup / second launch, Q4S):
+//   parts x column groups   3 x 16     6 x 7      6 x 16     8 x 7      8 x 16     12 x 4     16 x 4     16 x 16     16 x 32     7 x 68
+//   1 row                   7.3/7.8    7.2/7.8    7.8/7.9    7.3/7.8    8.2/7.7    7.5/8.1    7.7/8.1    10.2/8.3    11.3/11.0   19.8/20.0
+//   4 rows                  7.6/8.1    7.8/8.2    8.4/8.2    8.0/8.2    8.8/8.1    8.9/8.5    9.1/8.5    11.5/8.7    12.3/11.5   19.7/20.3
+//   8 rows                  8.6/9.2    9.5/9.3    9.9/9.3    9.5/9.2    10.3/9.1   11.7/9.5   11.9/9.5   14.3/9.8    16.2/13.7   23.2/23.8
+// (16 rows, several row groups: 2 x 16 10.9/10.8, 8 x 16 13.4/10.9, 16 x 16 20.0/11.7; 32 parts lose at any number of rows)
+bool last_workgroup_adds(const mummu_packed_weight *w, int m) {
+    const int parts = w->grid_k, workgroups = parts * w->wg_x;
+    if (m > kLastRows) return false;
+    return w->wg_x >= 64 || (m * parts <= 32 && (parts <= 6 || workgroups <= 64 || (workgroups > 256 && parts <= 16)));
+}
+
 int enqueue(mummu_packed_weight *w, const float *x_dev, int m, float *y_dev, hipStream_t s) {
     const size_t out_n = (size_t)m * (size_t)w->n;
-    const bool parts = w->grid_k > 1, last_adds = parts && m * w->grid_k <= kLastAdds;
+    const bool parts = w->grid_k > 1, last_adds = parts && last_workgroup_adds(w, m);
     const PackedArgs p{w->words, w->scales, x_dev, m, w->k, w->n * w->bits / 32, w->n / 32, w->stages, w->wg_x, w->grid_k,
                        ((uintptr_t)w->words & 15) == 0, ((uintptr_t)x_dev & 15) == 0 && w->k % 4 == 0, parts ? w->partial : y_dev, last_adds ? y_dev : nullptr, w->arrived};
     if (w->bits == 4) launch_packed_rows<4>(p, s);
@@ -570,8 +580,8 @@ static int packed_create(const uint32_t *words, const float *scales, int k, int 
     if (e == hipSuccess) e = hipMalloc(&w->x, sizeof(float) * (size_t)kMaxRows * (size_t)k);
     if (e == hipSuccess) e = hipMalloc(&w->y, sizeof(float) * (size_t)kMaxRows * (size_t)n);
     if (e == hipSuccess) e = hipMalloc(&w->partial, sizeof(float) * (size_t)w->grid_k * (size_t)kMaxRows * (size_t)n);
-    if (e == hipSuccess) e = hipMalloc(&w->arrived, sizeof(unsigned) * (size_t)kRowGroups * (size_t)w->wg_x);
-    if (e == hipSuccess) e = hipMemset(w->arrived, 0, sizeof(unsigned) * (size_t)kRowGroups * (size_t)w->wg_x);
+    if (e == hipSuccess) e = hipMalloc(&w->arrived, sizeof(unsigned) * (size_t)w->wg_x);
+    if (e == hipSuccess) e = hipMemset(w->arrived, 0, sizeof(unsigned) * (size_t)w->wg_x);
     if (e == hipSuccess) e = hipStreamCreate(&w->stream);
     if (e == hipSuccess && !on_device) e = hipMemcpy(w->words, words, wb, hipMemcpyHostToDevice);
     if (e == hipSuccess && !on_device) e = hipMemcpy(w->scales, scales, sb, hipMemcpyHostToDevice);

@@ -38,17 +38,17 @@ def test_rows_and_edges(k, n, bits):
             assert np.array_equal(yd.download(np.float32, (64, n))[:m].view(np.uint32), alone[:m].view(np.uint32)), m
 
 
-# Two or three workgroups along K, and from 17 rows on two row groups: the partial sums of each have an adder of their own, which
-# may start when those of its rows are there and no earlier.  Every call takes other rows, so that a sum read too early is the
-# one of the call before.
-@pytest.mark.parametrize("k,n", [(512, 4096), (640, 2048), (2048, 50304), (444, 544)])
+# Two or three workgroups along K, and from 17 rows on two row groups: whoever adds the partial sums may start when those of its
+# rows are there and no earlier (up to 8 rows the last workgroup of a column group, one of all rows; then a launch of its own).
+# Every call takes other rows, so that a sum read too early is the one of the call before.
+@pytest.mark.parametrize("k,n", [(512, 4096), (640, 2048), (2048, 50304), (444, 544), (4096, 4096), (1024, 17408)])
 def test_row_groups_add_their_own_partial_sums(k, n):
     g = np.random.default_rng(k + n)
     words = g.integers(0, 1 << 32, (k, n // 8), dtype=np.uint32)
     scales = g.uniform(0.001, 0.01, (k, n // 32)).astype(np.float32)
     x = g.standard_normal((96, k)).astype(np.float32)
     with M.PackedWeight(words, scales, k, n, 4) as w, M.PackedWeight(words, scales, k, n, 4) as one:
-        for m, at in ((32, 0), (17, 32), (21, 64), (32, 64), (17, 0), (16, 40), (20, 32), (21, 0)):
+        for m, at in ((32, 0), (17, 32), (8, 60), (21, 64), (32, 64), (9, 11), (17, 0), (4, 90), (16, 40), (8, 33), (20, 32), (21, 0)):
             alone = np.concatenate([one.gemv(x[at + i]).reshape(1, n) for i in range(m)])
             assert np.array_equal(w.gemv(x[at:at + m]).view(np.uint32), alone.view(np.uint32)), (m, at)
         want = orc.q4s_gemv(words, scales, k, n, 4, x[:1])
