@@ -122,7 +122,7 @@ def packed_gemv(M, lib, synth, spec: str) -> int:
     """Times the packed-GEMV op (Q4GemvOps::q4s_gemv, nn/packed_gemv.rs) with device-resident inputs:
     `--packed-gemv K,N,BITS,ROWS[,REPS]` (5120,17408,4,1 is the Q4S weight the reference quotes).  Several copies of the
     weight are used in rotation so that no call finds its weight in the 256 MB cache.  Prints one JSON line:
-    wall-clock microseconds per call (two launches: the product and the sum over the K split) and the packed bytes
+    wall-clock microseconds per call (one launch; two where the partial sums of the K split are many) and the packed bytes
     (values + scales) per second."""
     parts = [int(v) for v in spec.split(",")]
     if len(parts) not in (4, 5) or parts[2] not in (4, 8):

@@ -968,9 +968,6 @@ __global__ __launch_bounds__(256 * WM, GATE_UP ? 2 : 3) void grouped_gemm_q4k_f1
     __shared__ __attribute__((aligned(16))) uint8_t s_raw[L::kBytes];
     __shared__ __attribute__((aligned(16))) float s_as[2][BM];         // activation scale of a 128-element run, per tile row
     __shared__ __attribute__((aligned(16))) _Float16 s_sum[2][BM][GATE_UP ? 16 : 8];   // block sums of one fold: hi halfs, then lo halfs
-    auto s_a = [&](int buf, int plane, int row) -> _Float16 * {
-        return (_Float16 *)(s_raw + (size_t)buf * L::kBuf + ((size_t)plane * BM + row) * kRow);
-    };
 
     int tile, slab;
     if (!xcd_tile(n_tiles, (out_dim + kBN - 1) / kBN, tile, slab)) return;

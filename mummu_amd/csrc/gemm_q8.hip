@@ -6,7 +6,8 @@
 // (dwords of 64 rows a load) kept the address units busy: one line a lane and load, and the int8 form took 170 us for a layer whose
 // bytes take 75, whatever the batch; 16 bytes a lane straight into registers took 237.  Here a row's 136 bytes of a
 // stage (128 elements) come in one piece, 64 neighbouring dwords a load, straight into LDS, two stages ahead: 141 us (OLMoE layer, 19
-// to 100 tokens; 150: 204 -> 153, 512: 350 -> 294), 2.5e-7 off the 64-bit result where the int8 form is by 4.5e-5.
+// to 100 tokens; 150: 204 -> 153, 512: 350 -> 294; each byte is fetched once, 295 MB of 285 at 3.5 TB/s with the vector ALUs busy for 29 %
+// of the cycles and the matrix units for 18, profiles/listed_work_counters.txt), 2.5e-7 off the 64-bit result where the int8 form is by 4.5e-5.
 //
 // x has one scale for its whole row (HAct): an element is off by at most 2^-34 of the row's largest, where the int8 form's is off
 // by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of their own and

@@ -11,8 +11,9 @@
 //   - Whole rounds.  An expert's rows are split evenly, in steps of 64, over as few tiles as hold them, so that the
 //     workgroups of a launch are alike (full tiles and a remainder left a fifth of the launch to stragglers), and a wave
 //     multiplies only as many row blocks as the tile has.
-// What remains is the feed of the LDS (336 of 345 us with the products taken out of the loop and the loads left in was
-// 288) and the power limit: at full rate on random data the matrix cores alone hold 1.7 of their nominal 2.4 GHz.
+// What remains: the loads into LDS and the products with their reads overlap only in part (gate/up / down of 4096 bf16 rows x 8, us in
+// a kernel trace: whole 326 / 199, loads alone 223 / 153, without loads beyond the first two stages 281 / 164), at 1.9 GHz of 2.4.
+// The matrix units are busy for 45 / 34 % of the cycles, the LDS port for 33 / 25 (profiles/listed_work_counters.txt).
 // OLMoE shape, 4096 rows x 8: gate/up 503 -> 345 us, down 262 -> 190 us; 2048: 260 -> 207, 135 -> 112; 1000: 160 -> 141, 84 -> 82.
 #include "device_utils.h"
 #include "kernels.h"

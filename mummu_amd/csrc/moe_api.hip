@@ -1097,8 +1097,9 @@ int mummu_moe_create(const mummu_moe_config *cfg, mummu_moe **out) {
     // type takes) instead of the f16 units
     if (const char *e = getenv("MUMMU_GEMM_Q4K_F16")) h->gemm_q4k_f16 = atoi(e) != 0;
     // MUMMU_GEMM_Q8_F16=1: Q8_0 banks of the batched path take the f16 kernel (every weight exact as two halfs, x and the
-    // activations between the products rounded to halfs as for F16 banks: 1.2 to 1.5 times faster, errors of 1.5e-3
-    // by the reference's measure where the int8 form has 2e-4 - which is why it is not the default)
+    // activations between the products rounded to halfs as for F16 banks: 1.2 to 1.5 times faster than the int8 form, errors of
+    // 1.5e-3 by the reference's measure where that has 2e-4 and the pairs of halfs of gemm_q8.hip 1e-6 - which is why it is not the
+    // default)
     if (const char *e = getenv("MUMMU_GEMM_Q8_F16")) h->gemm_q8_f16 = atoi(e) != 0;
     // MUMMU_GEMM_TILE_ROWS=16 | 32 | 64: rows per tile of the f16-unit Q4_K kernels (default: by expected cost)
     if (const char *e = getenv("MUMMU_GEMM_TILE_ROWS")) {
