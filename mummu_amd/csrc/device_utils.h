@@ -186,6 +186,10 @@ __device__ inline uint32_t lds_offset(const void *shared) {
 __device__ inline void load_to_lds16(uint32_t lds, const uint8_t *base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
 }
+// ... from an address of each lane's own.
+__device__ inline void load_to_lds16(uint32_t lds, const uint8_t *from) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(uniform((int)lds)), "v"(from) : "memory");
+}
 __device__ inline void load_to_lds4(uint32_t lds, const uint8_t *base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
 }

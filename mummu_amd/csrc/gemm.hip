@@ -25,19 +25,15 @@
 
 #include "device_utils.h"
 #include "kernels.h"
+#include "q4k_half.h"
 
 MUMMU_TRACE_UNIT(gemm)
 
 namespace mummu {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
 typedef int int4v __attribute__((ext_vector_type(4)));
 typedef int int16v __attribute__((ext_vector_type(16)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));  // staging registers: first-class vectors stay in VGPRs
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 
 constexpr int kBN = 128;            // output rows per workgroup
 constexpr int kBK = 64;             // K step
@@ -62,32 +58,6 @@ __device__ inline half2v biased_pair(uint32_t t, bool upper) {
     __builtin_memcpy(&h, &u, 4);
     return h;
 }
-
-// Codes at bits 0-3 and 16-19 (4-7 and 20-23 with HIGH) of t as halfs: the code itself, as a subnormal, is code * 2^-24
-// (16 code * 2^-24), which one packed product turns into code * mul.
-template <bool HIGH>
-__device__ inline half2v code_pair(uint32_t t, half2v mul) {
-    const uint32_t u = t & (HIGH ? 0x00F000F0u : 0x000F000Fu);
-    half2v h;
-    __builtin_memcpy(&h, &u, 4);
-    return h * mul;
-}
-// Eight Q4_K codes (the low or high nibbles of two words, in the element order of HAct) times their sub-block's scale, over
-// 2^14 (exact: up to 63 * 15 in units of 2^-14): two masks, a shift and four products a word.
-template <bool HIGH>
-__device__ inline half8 q4k_operand(uint32_t w0, uint32_t w1, half2v mul) {
-    const half2v f[4] = {code_pair<HIGH>(w0, mul), code_pair<HIGH>(w0 >> 8, mul), code_pair<HIGH>(w1, mul), code_pair<HIGH>(w1 >> 8, mul)};
-    half8 o;
-    __builtin_memcpy(&o, f, 16);
-    return o;
-}
-// ... with mul for a sub-block scale sc: sc * 2^10 for the low nibbles, sc * 2^6 for the high ones.
-template <bool HIGH>
-__device__ inline half2v q4k_mul(uint32_t sc) {
-    const _Float16 m = (_Float16)__fmul_rn((float)sc, HIGH ? 64.0f : 1024.0f);
-    return half2v{m, m};
-}
-constexpr float kQ4kUnit = 16384.0f;
 
 // Eight Q8_0 codes (two words of int8) times the block scale d as two halfs each, hi = rn(d * code) and
 // lo = d * code - hi (exact: a 19-bit product, subnormal halfs included, which the vector and the matrix units
@@ -924,367 +894,9 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Q4_K banks on the f16 units
+// Q4_K banks on the f16 units, few rows per expert
 // ---------------------------------------------------------------------------------------
-// A Q4_K weight is d * (sc * q) - dmin * m with q < 16 and sc, m < 64 per 32 elements and d, dmin per 256.
-// sc * q < 1024 is an exact half, so the matrix cores can sum x * (sc * q) over a whole run of
-// sub-blocks with no vector work in between; the f32 accumulator takes d * that sum once per 128
-// elements.  Activations come as pairs of halfs (HAct): the two products of a K step go into the
-// same accumulator.  The offset term is one more instruction per 128 elements: the sums of the four
-// 32-element blocks (hi and lo halfs, K = 8) against the four m.  Per output element and 128 elements
-// of K that leaves three vector operations where the int8 form spends fourteen.
-
-// Only the activation tile goes through LDS.  Wave w owns output columns 32w..32w+31 for every row of the
-// tile, so the weights of those columns are its own: lane (column c, K group g) reads 16 of the 32 quant
-// bytes of a 64-element step of row c straight into registers (low nibbles: elements 16g..16g+15, high
-// nibbles: 32+16g..), turns them into its four B operands and never stores them anywhere.  The K index of
-// an instruction therefore maps to element (kk/2)*32 + 16g + (kk%2)*8 + i of the step, and the A operands
-// are read from the tile at that offset.  The activation tile is double-buffered (one barrier per step),
-// loads run two steps (weights) and one step (activations) ahead of their use.
-template <bool GATE_UP, int MT>
-struct HTileLds {
-    static constexpr int BM = 32 * MT;
-    static constexpr int kRow = 2 * kLds;                     // LDS row (bytes): 64 halfs + 8 of padding
-    static constexpr int kBuf = 2 * BM * kRow;                // hi and lo planes of one K step
-    static constexpr int kC = GATE_UP ? BM * kLdsC * 4 : 0;   // f32 staging of the epilogue (aliases the tiles)
-    static constexpr int kBytes = 2 * kBuf > kC ? 2 * kBuf : kC;
-};
-
-// GATE_UP: A = the token rows of a_in gathered through `sorted`; the epilogue writes silu(g)*u in sorted
-//          order, as HAct (OUT_H: the down banks are Q4_K too) or in the int8 kernels' QAct64.
-// else   : A = a_in rows in sorted order; y[pos, n] = f32 sum.
-// WM: the workgroup has 4 WM waves; wave w owns columns 32 (w % 4) .. +31 of row blocks (w / 4) * MT / WM .. of the
-// tile.  With two waves to a column block each expands the weights of its columns itself (twice the vector work
-// in the workgroup) and keeps half the accumulators, which is what lets two workgroups share a CU without spills.
-template <bool GATE_UP, int MT, int WM, bool OUT_H>
-__global__ __launch_bounds__(256 * WM, GATE_UP ? 2 : 3) void grouped_gemm_q4k_f16_kernel(
-    const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, HAct a_in, const int32_t *__restrict__ sorted, int k_slots,
-    const int32_t *__restrict__ tiles, const int32_t *__restrict__ n_tiles, int in_dim, int out_dim, HAct act_h, QAct64 act_q,
-    float *__restrict__ y_out) {
-    using L = HTileLds<GATE_UP, MT>;
-    constexpr int NB = GATE_UP ? 2 : 1, BM = L::BM, kRow = L::kRow;
-    constexpr int MW = MT / WM, NT = 256 * WM;   // row blocks per wave, threads
-    static_assert(MT % WM == 0, "row blocks split evenly over the wave rows");
-    __shared__ __attribute__((aligned(16))) uint8_t s_raw[L::kBytes];
-    __shared__ __attribute__((aligned(16))) float s_as[2][BM];         // activation scale of a 128-element run, per tile row
-    __shared__ __attribute__((aligned(16))) _Float16 s_sum[2][BM][GATE_UP ? 16 : 8];   // block sums of one fold: hi halfs, then lo halfs
-
-    int tile, slab;
-    if (!xcd_tile(n_tiles, (out_dim + kBN - 1) / kBN, tile, slab)) return;
-    const int e = tiles[3 * tile], p0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-    const int n0 = slab * kBN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t row_bytes = gemm_row_bytes(T_Q4_K, in_dim);
-    const int col = 32 * (wave & 3) + (lane & 31), g = lane >> 5;
-    const int row0 = 32 * MW * (wave >> 2);   // first tile row of this wave
-
-    // Addresses are a uniform base plus a 32-bit byte offset per lane (an expert's bank and the activation planes
-    // are far below 4 GB).  Rows past the tile's end read its last row and columns past the matrix its last column:
-    // their products are never stored.
-    const int b_out = n0 + col < out_dim ? n0 + col : out_dim - 1;
-    const uint8_t *b_base[NB];
-    b_base[0] = w0 + (size_t)e * (size_t)out_dim * row_bytes;
-    if (GATE_UP) b_base[NB - 1] = w1 + (size_t)e * (size_t)out_dim * row_bytes;
-    const uint32_t b_off = (uint32_t)b_out * (uint32_t)row_bytes + 16u * (uint32_t)g;
-
-    auto source_row = [&](int r) -> int {
-        r = r < rows ? r : rows - 1;
-        return GATE_UP ? sorted[p0 + r] / k_slots : p0 + r;
-    };
-    // activation tile: thread -> (plane, row, 8 halfs), passes of 16 WM rows
-    constexpr int A_PASSES = 2 * MT / WM, A_ROWS = 16 * WM;
-    const int a_plane = tid / (NT / 2), a_chunk = tid & 7;
-    const uint8_t *a_base = (const uint8_t *)(a_plane ? a_in.lo : a_in.hi);
-    uint32_t a_off[A_PASSES], a_lds[A_PASSES];
-#pragma unroll
-    for (int p = 0; p < A_PASSES; p++) {
-        const int r = A_ROWS * p + ((tid >> 3) & (A_ROWS - 1));
-        a_off[p] = ((uint32_t)source_row(r) * (uint32_t)in_dim + (uint32_t)a_chunk * 8u) * 2u;
-        a_lds[p] = (uint32_t)(((size_t)a_plane * BM + r) * kRow + a_chunk * 16);
-    }
-    // Activation scales.  ROW (the gate/up side: x comes from quantize_rows_h, one scale for the whole row): the
-    // scale is applied once, in the epilogue, and a super-block is folded into acc in one go.  Otherwise (the down
-    // side: the gate/up epilogue knows only its own 128 columns) every 128-element run has its own scale and is
-    // folded on its own.
-    // Block sums: thread -> (row tid / 4 of the tile, quarter tid % 4 of the run's blocks).  Threads past 4 BM
-    // repeat rows and all four threads of a row store its scale: the same values twice, and no branch in the
-    // loop body - with basic blocks in it the compiler sinks one step's arithmetic into the next and keeps both
-    // steps' accumulators alive.
-    constexpr bool ROW = GATE_UP;
-    constexpr int NSUM = ROW ? 8 : 4;          // block sums per fold
-    const int m_row = (tid >> 2) & (BM - 1), m_blk = tid & 3;
-    const uint32_t src_m = (uint32_t)source_row(m_row);
-    const uint32_t sum_off = (src_m * (uint32_t)(in_dim / 32) + (uint32_t)m_blk * (ROW ? 2u : 1u)) * 4u;
-    const uint32_t scale_off = src_m * (uint32_t)(in_dim / 128) * 4u;
-    if (ROW) s_as[0][m_row] = *(const float *)((const uint8_t *)a_in.scale + scale_off);
-
-    float16v acc[NB][MW], c1[NB][MW];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-        for (int m = 0; m < MW; m++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[b][m][r] = c1[b][m][r] = 0.0f;
-
-    // weights: the raw bytes of the step being multiplied and of the next one; of the current super-block d | dmin
-    // and its eight scales and eight offsets as bytes (sub-blocks 0-3, 4-7); the header of the next super-block
-    // during this one's last step
-    u32x4 raw[2][NB], rh_next[NB];
-    uint32_t dd[NB], sc4[NB][2], mn4[NB][2];
-    // (the header of the NEXT super-block comes with the weights of this one's last step and is unpacked at the end
-    // of that step, a whole step after its load: a value loaded in the loop's last step and first read in the next
-    // iteration is copied between registers at the loop's end, behind a wait for every load in flight)
-    auto load_b = [&](int k0, int st, u32x4 (&dst)[NB]) {
-        const uint32_t o = b_off + (uint32_t)(k0 >> 8) * 144u;
-        const uint32_t oh = b_off - 16u * (uint32_t)g + (k0 + 256 < in_dim ? (uint32_t)(k0 >> 8) * 144u + 144u : 0u);
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            dst[b] = *(const u32x4 *)(b_base[b] + (o + 16u + (uint32_t)st * 32u));
-            if (st == 3) rh_next[b] = *(const u32x4 *)(b_base[b] + oh);
-        }
-    };
-    // ggml get_scale_min_k4 for all eight sub-blocks at once
-    auto unpack_header = [&]() {
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const uint32_t y = rh_next[b][1], z = rh_next[b][2], w = rh_next[b][3];
-            dd[b] = rh_next[b][0];
-            sc4[b][0] = y & 0x3F3F3F3Fu;
-            mn4[b][0] = z & 0x3F3F3F3Fu;
-            sc4[b][1] = (w & 0x0F0F0F0Fu) | ((y >> 2) & 0x30303030u);
-            mn4[b][1] = ((w >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u);
-        }
-    };
-    // activations of one step in registers, then into a tile
-    u32x4 ra[A_PASSES];
-    float rsum[ROW ? 2 : 1] = {}, rscale = 0.0f;
-    auto load_a = [&](int k0, int st) {
-#pragma unroll
-        for (int p = 0; p < A_PASSES; p++) ra[p] = *(const u32x4 *)(a_base + (a_off[p] + (uint32_t)k0 * 2u));
-        if (ROW) {
-            if (st == 0) {
-                const float2 v = *(const float2 *)((const uint8_t *)a_in.ssum + (sum_off + (uint32_t)(k0 >> 5) * 4u));
-                rsum[0] = v.x;
-                rsum[ROW ? 1 : 0] = v.y;
-            }
-        } else if ((st & 1) == 0) {
-            rsum[0] = *(const float *)((const uint8_t *)a_in.ssum + (sum_off + (uint32_t)(k0 >> 5) * 4u));
-            rscale = *(const float *)((const uint8_t *)a_in.scale + (scale_off + (uint32_t)(k0 >> 7) * 4u));
-        }
-    };
-    // sum_buf: which of the two sets of block sums (they alternate per fold)
-    auto store_a = [&](int buf, int st, int sum_buf) {
-#pragma unroll
-        for (int p = 0; p < A_PASSES; p++) *(u32x4 *)(s_raw + (size_t)buf * L::kBuf + a_lds[p]) = ra[p];
-        if (ROW) {
-            if (st == 0) {
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const float v = rsum[ROW ? i : 0];
-                    const _Float16 h = (_Float16)v;
-                    s_sum[sum_buf][m_row][2 * m_blk + i] = h;
-                    s_sum[sum_buf][m_row][8 + 2 * m_blk + i] = (_Float16)__fsub_rn(v, (float)h);
-                }
-            }
-        } else if ((st & 1) == 0) {
-            const _Float16 h = (_Float16)rsum[0];
-            s_sum[sum_buf][m_row][m_blk] = h;
-            s_sum[sum_buf][m_row][4 + m_blk] = (_Float16)__fsub_rn(rsum[0], (float)h);
-            s_as[sum_buf][m_row] = rscale;
-        }
-    };
-
-    const float16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // one 64-element step: st = which step of the super-block, buf = which tile holds its activations
-    auto multiply = [&](int st, int buf, const u32x4 (&rw)[NB]) {
-        half2v ml2[NB], mh2[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            // sub-blocks 2 st (the low nibbles) and 2 st + 1 (the high nibbles)
-            const uint32_t sw = sc4[b][st >> 1] >> (16 * (st & 1));
-            ml2[b] = q4k_mul<false>(sw & 0xFFu);
-            mh2[b] = q4k_mul<true>((sw >> 8) & 0xFFu);
-        }
-        const uint8_t *tile = s_raw + (size_t)buf * L::kBuf + (size_t)(row0 + (lane & 31)) * kRow + 32 * g;
-        // the A operands of instruction group kk + 1 are read from the tile before group kk is issued
-        half8 a_hi[2][MW], a_lo[2][MW];
-        auto read_a = [&](int kk) {
-            const int a_byte = (kk >> 1) * 64 + (kk & 1) * 16;  // element (kk/2)*32 + 16g + (kk%2)*8 of the step
-#pragma unroll
-            for (int m = 0; m < MW; m++) {
-                a_hi[kk & 1][m] = *(const half8 *)(tile + (size_t)(32 * m) * kRow + a_byte);
-                a_lo[kk & 1][m] = *(const half8 *)(tile + (size_t)(BM + 32 * m) * kRow + a_byte);
-            }
-        };
-        const bool first = ROW ? st == 0 : (st & 1) == 0;   // the step that starts a new sum in c1
-        read_a(0);
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            if (kk < 3) read_a(kk + 1);
-            half8 bfrag[NB];
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                const uint32_t w_a = (kk & 1) ? rw[b][2] : rw[b][0], w_b = (kk & 1) ? rw[b][3] : rw[b][1];
-                bfrag[b] = kk < 2 ? q4k_operand<false>(w_a, w_b, ml2[b]) : q4k_operand<true>(w_a, w_b, mh2[b]);
-            }
-            // (the hi products of every block first, then the lo products: instructions that accumulate into the same
-            // registers are NB * MW apart)
-#pragma unroll
-            for (int m = 0; m < MW; m++)
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    c1[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi[kk & 1][m], bfrag[b], (first && kk == 0) ? zero : c1[b][m], 0, 0, 0);
-#pragma unroll
-            for (int m = 0; m < MW; m++)
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    c1[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_lo[kk & 1][m], bfrag[b], c1[b][m], 0, 0, 0);
-        }
-    };
-    // what has been summed into c1 -> acc.  part: which 128-element run of the super-block (the whole of it with
-    // one scale per row); sum_buf: which set of block sums
-    auto fold = [&](int part, int sum_buf) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const float d = __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu)));
-            const float ndmin = -half_bits_to_float((uint16_t)(dd[b] >> 16));
-            // the block offsets m as halfs (exact), in the order of the block sums
-            _Float16 mh[NSUM];
-#pragma unroll
-            for (int j = 0; j < NSUM; j++) {
-                const uint32_t word = ROW ? mn4[b][j >> 2] : mn4[b][part];
-                mh[j] = (_Float16)(float)((word >> (8 * (j & 3))) & 0xFFu);
-            }
-#pragma unroll
-            for (int m = 0; m < MW; m++) {
-                float16v c2;
-                if constexpr (ROW) {
-                    // K = 16: the eight sums' hi halfs from lanes 0-31, their lo halfs from lanes 32-63
-                    const half8 am = *(const half8 *)&s_sum[sum_buf][row0 + 32 * m + (lane & 31)][8 * g];
-                    half8 bm;
-#pragma unroll
-                    for (int j = 0; j < 8; j++) bm[j] = mh[j];
-                    c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, zero, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) acc[b][m][r] = fmaf(ndmin, c2[r], fmaf(d, c1[b][m][r], acc[b][m][r]));
-                } else {
-                    const half4v am = *(const half4v *)&s_sum[sum_buf][row0 + 32 * m + (lane & 31)][4 * g];
-                    const half4v bm = {mh[0], mh[1], mh[2], mh[3]};
-                    c2 = __builtin_amdgcn_mfma_f32_32x32x8f16(am, bm, zero, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float4 s4 = *(const float4 *)&s_as[sum_buf][row0 + 32 * m + 8 * j + 4 * g];
-                        const float sr[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int r = 4 * j + i;
-                            const float u = fmaf(ndmin, c2[r], __fmul_rn(d, c1[b][m][r]));
-                            acc[b][m][r] = fmaf(u, sr[i], acc[b][m][r]);
-                        }
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);  // (one 32 x 32 block at a time: scheduled together they do not fit the registers)
-            }
-        }
-    };
-
-    // prologue: the first header, step 0 into tile 0
-#pragma unroll
-    for (int b = 0; b < NB; b++) rh_next[b] = *(const u32x4 *)(b_base[b] + (b_off - 16u * (uint32_t)g));
-    unpack_header();
-    load_b(0, 0, raw[0]);
-    load_a(0, 0);
-    store_a(0, 0, 0);
-    __syncthreads();
-    MUMMU_TIMER_DECL;
-    // (one step as a generic lambda over a compile-time step index: the register sets are picked by constants)
-    auto step = [&](int sb0, auto st_c) {
-        constexpr int st = decltype(st_c)::value;
-        // (after the last step the "next" one is step 0 again: loaded and stored like any other, never multiplied;
-        // no branch in the loop body)
-        const int k_next = (st == 3 && sb0 + 256 >= in_dim) ? 0 : sb0 + kBK * (st + 1);
-        // block sums alternate between two sets: per super-block with one scale per row, else per 128-element run
-        const int sb_par = (sb0 >> 8) & 1;
-        const int sum_buf = ROW ? sb_par : (st >> 1) & 1;
-        const int sum_buf_next = ROW ? (st == 3 ? sb_par ^ 1 : sb_par) : (((st + 1) & 3) >> 1) & 1;
-        MUMMU_TIMER_MARK(0);
-        // the next step: activations into registers, weights into the other set of registers.  (Loads come back in
-        // the order issued: the activations are wanted at the end of this step, the weights a step later, so the
-        // wait before store_a must not have the weight loads in front of it.)
-        load_a(k_next, (st + 1) & 3);
-        load_b(k_next, (st + 1) & 3, raw[(st + 1) & 1]);
-        MUMMU_CODE_FENCE();  // (the loads stay here, a whole step ahead of their first use)
-        MUMMU_TIMER_MARK(1);
-        multiply(st, st & 1, raw[st & 1]);
-        MUMMU_TIMER_MARK(2);
-        if (ROW ? st == 3 : (st & 1) == 1) fold(st >> 1, sum_buf);
-        if (st == 3) unpack_header();
-        MUMMU_TIMER_MARK(3);
-        MUMMU_CODE_FENCE();
-        // ... and into the tile that the step before this one was read from
-        store_a((st + 1) & 1, (st + 1) & 3, sum_buf_next);
-        MUMMU_TIMER_MARK(4);
-        __syncthreads();
-        MUMMU_TIMER_MARK(5);
-    };
-    for (int sb0 = 0; sb0 < in_dim; sb0 += 256) {
-        step(sb0, std::integral_constant<int, 0>{});
-        step(sb0, std::integral_constant<int, 1>{});
-        step(sb0, std::integral_constant<int, 2>{});
-        step(sb0, std::integral_constant<int, 3>{});
-    }
-    MUMMU_TIMER_STORE;
-
-    if (GATE_UP) {
-        // stage silu(g)*u of the whole tile as f32 (over the activation tiles, no longer needed), then store it in the
-        // form the down product reads
-        float *s_c = (float *)s_raw;
-#pragma unroll
-        for (int m = 0; m < MW; m++)
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-            {
-                // (one scale per row on this side: both products take it here)
-                const float sr = s_as[0][row0 + 32 * m + acc_row(r, lane)];
-                s_c[(row0 + 32 * m + acc_row(r, lane)) * kLdsC + col] =
-                    __fmul_rn(det_silu(__fmul_rn(sr, acc[0][m][r])), __fmul_rn(sr, acc[NB - 1][m][r]));
-            }
-        __syncthreads();
-        if (OUT_H) {
-            const int grp = tid >> 5, l32 = tid & 31;
-#pragma unroll
-            for (int pass = 0; pass < BM / (NT / 32); pass++) {
-                const int row = pass * (NT / 32) + grp;
-                const float4 v = *(const float4 *)&s_c[row * kLdsC + 4 * l32];
-                const bool active = row < rows && n0 < out_dim;
-                hact_store128(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, act_h, (size_t)(p0 + row), out_dim, n0 + 4 * l32);
-            }
-        } else {
-            const int grp = tid >> 4, l16 = tid & 15;
-#pragma unroll
-            for (int pass = 0; pass < 2 * BM / (NT / 16); pass++) {
-                const int task = pass * (NT / 16) + grp, row = task >> 1, cb = task & 1;
-                const float4 v = *(const float4 *)&s_c[row * kLdsC + cb * 64 + 4 * l16];
-                const bool active = row < rows && n0 + cb * 64 < out_dim;
-                quantize_store64(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, act_q, (size_t)(p0 + row), out_dim,
-                                 n0 + cb * 64 + 4 * l16);
-            }
-        }
-    } else {
-        const int n = n0 + col;
-        if (n < out_dim) {
-#pragma unroll
-            for (int m = 0; m < MW; m++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int row = row0 + 32 * m + acc_row(r, lane);
-                    if (row < rows) y_out[(size_t)(p0 + row) * (size_t)out_dim + (size_t)n] = acc[0][m][r];
-                }
-        }
-    }
-}
-
-// The same product for experts with few rows (small batches): 16-row tiles on v_mfma_f32_16x16x32_f16.  Eight
+// The product of gemm_q4k.hip for experts with few rows (small batches): 16-row tiles on v_mfma_f32_16x16x32_f16.  Eight
 // waves, wave w owns output columns 16w..16w+15; a stage is half a super-block (128 elements).  Lane (column c,
 // K group kg) reads 16 of the 64 quant bytes of the stage - the four lanes of a column read 64 consecutive bytes
 // of its row - and supplies, in instruction q of the stage, the eight elements
@@ -1583,19 +1195,13 @@ bool grouped_gemm_supported(const ExpertBanks &b) {
 // that streams its whole weight slab again, so the tile is sized to hold the average expert load
 // plus its spread (binomial: about +-sqrt(avg) per expert, 3.5 sigma here) when that fits; the f16
 // kernel goes up to 128 rows, the int8 kernel (more registers per row) to 64.
-// Tile rows for the f16-unit Q4_K kernels, which come in 16-, 32- and 64-row forms: the one with the smallest
-// expected cost when an expert's rows are spread like a binomial around the average (normal approximation,
-// variance = mean).  A 32-row workgroup costs 0.55 of a 64-row one (measured at 4096 tokens, where both forms run
-// full tiles): the expansion of the weights, the loads and the barriers do not shrink with the rows.  At an
-// average of 64 rows half the experts need a second, almost empty 64-row tile and 32-row tiles win; at 48 one
-// 64-row tile holds nearly every expert and wins; from a few hundred rows on the 64-row form wins by its 9 %.
-// A launch of 16-row tiles costs 0.83-0.89 of one with as many 32-row tiles (32 / 64 tokens over 64 experts: gate/up
-// 46.1 / 50.2 against 56.0 / 55.8 us, down 25.1 / 26.7 against 30.0 / 30.8 us), but every expert that needs a second
-// tile streams its weights again: with 10 % more tiles (96 tokens) the 16-row launches already take 65.9 + 33.9 us
-// against 56.5 + 31.8 us.  So the 16-row form is taken only while next to no expert has more than 16 rows (its
-// expected tiles within 1 % of the 32-row form's: 64 experts x 8 slabs of 16-row tiles are exactly the 512
-// workgroups the chip holds at once, and the first second tiles start a second round - 72 / 80 tokens: 104 / 114 us
-// per layer with 16-row tiles, 105 / 106-112 us with 32-row tiles).
+// Tile rows for the f16-unit Q4_K kernels: 16 (the form for few rows) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what
+// they have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal
+// approximation, variance = mean).  The 16-row form is taken only while next to no expert has more than 16 rows, its expected tiles within
+// 1 % of the other's: 64 experts x 8 slabs of 16-row tiles are exactly the 512 workgroups the chip holds at once, and the first
+// second tiles start a second round.  Layers, 16 / 64 rows, us: OLMoE 24 tokens 78 / 92, 48: 79 / 93, 72: 97 / 93, 96: 99 / 96, 192: 150 / 113;
+// 128 experts of 2048 x 768, 128 tokens 141 / 152, 140: 143 / 154, 160: 160 / 154, 208: 165 / 159.  Lists of 32 rows gained nothing
+// between them (OLMoE 96 tokens 94, 256: 132 against 129, 1000: 331 against 302).
 // With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
 // products together: OLMoE Q4_K with Q6_K downs, 32 / 64 rows: 150 tokens 154 / 206 us, 230: 181 / 208, 260: 225 / 214; the
 // 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013.
@@ -1612,8 +1218,8 @@ int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts, bool int8_down) 
         return t;
     };
     const double e16 = expected_tiles(16.0), e32 = expected_tiles(32.0), e64 = expected_tiles(64.0);
-    if (0.99 * e16 < e32 && 0.99 * 0.55 * e16 < e64) return 16;
-    return (int8_down ? 0.69 : 0.55) * e32 < e64 ? 32 : 64;
+    if (0.99 * e16 < (int8_down ? e32 : e64)) return 16;
+    return int8_down && 0.69 * e32 < e64 ? 32 : 64;
 }
 
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half) {
@@ -1689,30 +1295,16 @@ bool grouped_gemm_q4k_f16_down(const ExpertBanks &b) {
 }
 
 template <bool GATE_UP>
-static hipError_t launch_gemm_q4k_f16(const uint8_t *w0, const uint8_t *w1, HAct a_in, const int32_t *sorted, int k_slots,
-                                      const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows, int in_dim,
-                                      int out_dim, HAct act_h, QAct64 act_q, bool out_h, float *y_out, hipStream_t s) {
+static hipError_t launch_gemm_q4k_f16_m16(const uint8_t *w0, const uint8_t *w1, HAct a_in, const int32_t *sorted, int k_slots,
+                                          const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int in_dim, int out_dim, HAct act_h,
+                                          QAct64 act_q, bool out_h, float *y_out, hipStream_t s) {
     dim3 grid((unsigned)((max_tiles + 7) / 8 * 8) * (unsigned)((out_dim + kBN - 1) / kBN));
-#define MUMMU_H(MT, WM, OUT_H)                                                                                           \
-    launch_kernel(grouped_gemm_q4k_f16_kernel<GATE_UP, MT, WM, OUT_H>, grid, dim3(256 * WM), 0, s, w0, w1, a_in, sorted, k_slots, \
-                  tiles, n_tiles, in_dim, out_dim, act_h, act_q, y_out)
-    if (tile_rows == 64) {
-        if (out_h) MUMMU_H(2, 1, true);
-        else MUMMU_H(2, 1, false);
-    } else if (tile_rows == 32) {
-        if (out_h) MUMMU_H(1, 1, true);
-        else MUMMU_H(1, 1, false);
-    } else if (tile_rows == 16) {
-        if (out_h)
-            launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, true>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles,
-                          n_tiles, in_dim, out_dim, act_h, act_q, y_out);
-        else
-            launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, false>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles,
-                          n_tiles, in_dim, out_dim, act_h, act_q, y_out);
-    } else {
-        return hipErrorInvalidValue;
-    }
-#undef MUMMU_H
+    if (out_h)
+        launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, true>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles, n_tiles,
+                      in_dim, out_dim, act_h, act_q, y_out);
+    else
+        launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, false>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles, n_tiles,
+                      in_dim, out_dim, act_h, act_q, y_out);
     return hipGetLastError();
 }
 
@@ -1770,8 +1362,10 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
         if (!grouped_gemm_q4k_f16(b)) return hipErrorInvalidValue;
         const bool out_h = acth.hi != nullptr;
         if (out_h && !grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
-        return launch_gemm_q4k_f16<true>(b.gate, b.up, xh, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden, b.inter,
-                                         acth, actq, out_h, nullptr, s);
+        if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
+        if (tile_rows > 16) return launch_q4k_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
+        return launch_gemm_q4k_f16_m16<true>(b.gate, b.up, xh, sorted, k_slots, tiles, n_tiles, max_tiles, b.hidden, b.inter, acth, actq,
+                                             out_h, nullptr, s);
     }
     if (b.gate_type == T_F32)
         return launch_gemm_f32<true>(b.gate, b.up, x, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden, b.inter, act32,
@@ -1817,8 +1411,10 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
     }
     if (acth.hi != nullptr) {
         if (!grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
-        return launch_gemm_q4k_f16<false>(b.down, nullptr, acth, nullptr, 1, tiles, n_tiles, max_tiles, tile_rows, b.inter, b.hidden,
-                                          HAct(), QAct64(), false, y, s);
+        if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
+        if (tile_rows > 16) return launch_q4k_down(b, acth, tiles, n_tiles, max_tiles, y, s);
+        return launch_gemm_q4k_f16_m16<false>(b.down, nullptr, acth, nullptr, 1, tiles, n_tiles, max_tiles, b.inter, b.hidden, HAct(),
+                                              QAct64(), false, y, s);
     }
     if (b.down_type == T_F32)
         return launch_gemm_f32<false>(b.down, nullptr, act32, nullptr, 1, tiles, n_tiles, max_tiles, tile_rows, b.inter, b.hidden,

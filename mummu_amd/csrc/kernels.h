@@ -225,6 +225,14 @@ hipError_t launch_wide_gate_up(const ExpertBanks &b, const _Float16 *x16, const 
 hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, const int32_t *n_tiles, int max_tiles,
                             float *y, hipStream_t s);
 
+// gemm_q4k.hip ------------------------------------------------------------------------
+// Q4_K gate and up banks (and down banks) on the f16 units, tiles of up to kQ4kRows rows; the activations go to act_h, or to act_q
+// where that is empty.
+constexpr int kQ4kRows = 64;
+hipError_t launch_q4k_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
+                              int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s);
+hipError_t launch_q4k_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y, hipStream_t s);
+
 // gemm_q8.hip -------------------------------------------------------------------------
 // Q8_0 banks on the f16 units: x and the activations between the two products as pairs of halfs, tiles of 32 rows.
 bool q8_gemm_takes(const ExpertBanks &b);

@@ -139,7 +139,8 @@ __device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_
         m = fmaxf(m, dpp_move<0x4E>(m));
         m = fmaxf(m, dpp_move<0x141>(m));
         m = fmaxf(m, dpp_move<0x140>(m));
-        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        const auto o = __builtin_amdgcn_permlane16_swap(__float_as_int(m), __float_as_int(m), false, false);
+        m = fmaxf(__int_as_float(o[0]), __int_as_float(o[1]));
     }
     float inv, scale;
     hact_scale_of(m, inv, scale);
