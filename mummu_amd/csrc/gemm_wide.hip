@@ -6,14 +6,16 @@
 //   - LDS reads.  A 64 x 128 tile reads one operand per matrix instruction, which keeps the LDS port (128 bytes a clock)
 //     busy all the time at half the matrix rate.  Eight waves of 32 MW x 64 outputs (MW up to 5) read 7 operands for 10.
 //   - The way into LDS.  Both tiles go from global memory straight into LDS, 64 elements of K (whole 128-byte lines: pieces
-//     of 64 bytes come out of the L2 at half the rate, 17 against 34 TB/s) at a time and two stages deep, without registers in
-//     between.
+//     of 64 bytes come out of the L2 at half the rate, 17 against 34 TB/s) at a time, without registers in between, the weights two
+//     stages ahead where the LDS holds them, and never a stage at once: 72 loads behind a barrier fill the address unit's queue, with
+//     all eight waves waiting in front of it.  (Asked for in one go, one stage ahead: 4096 bf16 rows x 8 gate/up / down 620 / 416 k cycles
+//     against 529 / 363, 1500 f16 rows 358 / 206 against 299 / 217.)
 //   - Whole rounds.  An expert's rows are split evenly, in steps of 64, over as few tiles as hold them, so that the
 //     workgroups of a launch are alike (full tiles and a remainder left a fifth of the launch to stragglers), and a wave
 //     multiplies only as many row blocks as the tile has.
-// What remains: the loads into LDS and the products with their reads overlap only in part (gate/up / down of 4096 bf16 rows x 8, us in
-// a kernel trace: whole 326 / 199, loads alone 223 / 153, without loads beyond the first two stages 281 / 164), at 1.9 GHz of 2.4.
-// The matrix units are busy for 45 / 34 % of the cycles, the LDS port for 33 / 25 (profiles/listed_work_counters.txt).
+//   - Weights of bf16 become halfs beside the last products of the group before, not between their read and the next products.
+// What remains: the matrix units are busy for 52 / 38 % of the cycles at 4096 bf16 rows x 8, and the card lowers its clock as they
+// are: 15 % fewer cycles were 7 % of the time (340 / 206 us -> 316 / 194).
 // OLMoE shape, 4096 rows x 8: gate/up 503 -> 345 us, down 262 -> 190 us; 2048: 260 -> 207, 135 -> 112; 1000: 160 -> 141, 84 -> 82.
 #include "device_utils.h"
 #include "kernels.h"
@@ -28,11 +30,15 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWK = 64;                          // K elements of a stage: a line of 128 bytes per row, eight pieces of 16
 constexpr int kWCols = 256;                      // weight rows of a tile
-constexpr int kWATile = kWideRows * kWK * 2;     // bytes of a stage: activation rows, then weight rows
-constexpr int kWStage = kWATile + kWCols * kWK * 2;
-
-// Every load this wave has asked for has landed, every LDS read it has asked for is in its registers; then everybody's.
-__device__ inline void settle() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+constexpr int kWStageB = kWCols * kWK * 2;       // bytes of a stage of weights
+// Stages in LDS, for tiles of 64 MW rows: of the weights, then two of the activations.
+template <int MW>
+struct Ring {
+    static constexpr int kB = MW <= 4 ? 3 : 2, kStageA = 64 * MW * kWK * 2, kAtA = kB * kWStageB;
+    static_assert(kAtA + 2 * kStageA <= 160 * 1024, "the stages fit the LDS");
+};
+constexpr int kWLds = Ring<4>::kAtA + 2 * Ring<4>::kStageA;
+static_assert(kWideRows == 64 * 5 && Ring<5>::kAtA + 2 * Ring<5>::kStageA <= kWLds, "... all of them");
 
 template <int WT>
 __device__ inline half8 weight_operand(u32x4 v) {
@@ -82,18 +88,18 @@ struct Loader {
     uint32_t a_off[MW], b_off[4];
     const uint8_t *a_base, *b_base;
 
-    __device__ void stage(uint32_t at, int step, int wave) const {
-        const uint8_t *ab = a_base + (size_t)step * (kWK * 2), *bb = b_base + (size_t)step * (kWK * 2);
-#pragma unroll
-        for (int i = 0; i < MW; i++) load_to_lds16(at + (uint32_t)(8 * MW * wave + 8 * i) * (kWK * 2), ab, a_off[i]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) load_to_lds16(at + kWATile + (uint32_t)(32 * wave + 8 * i) * (kWK * 2), bb, b_off[i]);
+    __device__ void load_a(uint32_t at, int step, int wave, int i) const {
+        load_to_lds16(at + (uint32_t)(8 * MW * wave + 8 * i) * (kWK * 2), a_base + (size_t)step * (kWK * 2), a_off[i]);
+    }
+    __device__ void load_b(uint32_t at, int step, int wave, int i) const {
+        load_to_lds16(at + (uint32_t)(32 * wave + 8 * i) * (kWK * 2), b_base + (size_t)step * (kWK * 2), b_off[i]);
     }
 };
 
 // A tile of up to 64 MW rows by one slab; wave (wm, wn) multiplies rows 32 MW wm .. by its 64 weight rows.
 template <bool GATE_UP, int WT, int MW>
-__device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int slab, uint8_t *s_lds, const int *s_rows) {
+__device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int slab, uint8_t *s_lds) {
+    using R = Ring<MW>;
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3, g = lane >> 5, lr = lane & 31;
     const uint32_t row_bytes = (uint32_t)p.in_dim * 2u;
@@ -109,7 +115,7 @@ __device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int
         for (int i = 0; i < MW; i++) {
             const int r = 8 * MW * wave + 8 * i + lrow;
             const int rr = r < rows ? r : rows - 1;   // (rows past the tile's end repeat its last: multiplied, never stored)
-            l.a_off[i] = (uint32_t)(GATE_UP ? s_rows[rr] : p0 + rr) * row_bytes + piece;
+            l.a_off[i] = (uint32_t)(GATE_UP ? p.sorted[p0 + rr] / p.k_slots : p0 + rr) * row_bytes + piece;
         }
         // weight rows: gate/up: 32 rows of gate, then 32 of up for each pair of waves; down: 64 rows for each pair
         const int col0 = GATE_UP ? slab * (kWCols / 2) + 32 * (wave >> 1) : slab * kWCols + 32 * wave;
@@ -131,42 +137,70 @@ __device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int
     uint32_t q[4];
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) q[kk] = (uint32_t)((2 * kk + g) ^ (lr & 7)) * 16u;
-    const uint8_t *a_rd = s_lds + (32 * MW * wm + lr) * (kWK * 2), *b_rd = s_lds + kWATile + (64 * wn + lr) * (kWK * 2);
+    const uint8_t *a_rd = s_lds + R::kAtA + (32 * MW * wm + lr) * (kWK * 2), *b_rd = s_lds + (64 * wn + lr) * (kWK * 2);
     // operands of 16 elements of K, read while the ones before are multiplied
     half8 ra[2][MW], rb[2][2];
-    auto read = [&](int slot, int kk) {
-        const uint32_t o = (uint32_t)slot * kWStage + q[kk];
+    u32x4 raw[2];
+    auto read = [&](uint32_t at_a, uint32_t at_b, int kk) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) rb[kk & 1][j] = weight_operand<WT>(*(const u32x4 *)(b_rd + o + 32 * (kWK * 2) * j));
+        for (int j = 0; j < 2; j++) raw[j] = *(const u32x4 *)(b_rd + (at_b + q[kk]) + 32 * (kWK * 2) * j);
 #pragma unroll
-        for (int m = 0; m < MW; m++) ra[kk & 1][m] = *(const half8 *)(a_rd + o + 32 * (kWK * 2) * m);
+        for (int m = 0; m < MW; m++) ra[kk & 1][m] = *(const half8 *)(a_rd + (at_a + q[kk]) + 32 * (kWK * 2) * m);
     };
-    auto multiply = [&](int kk) {
-        __builtin_amdgcn_sched_barrier(0);
+    auto convert = [&](int kk) {
 #pragma unroll
-        for (int m = 0; m < MW; m++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) acc[j][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ra[kk & 1][m], rb[kk & 1][j], acc[j][m], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < 2; j++) rb[kk & 1][j] = weight_operand<WT>(raw[j]);
     };
-    l.stage(lds0, 0, wave);
-    settle();
-    l.stage(lds0 + kWStage, 1, wave);
-    read(0, 0);
-    for (int step = 0; step < n_steps; step++) {
-        const int slot = step & 1;
-        read(slot, 1);
-        multiply(0);
-        read(slot, 2);
-        multiply(1);
-        read(slot, 3);
-        multiply(2);
-        // the next stage has landed and this one has been read by everybody: its slot takes the stage after the next
-        settle();
-        if (step + 2 < n_steps) l.stage(lds0 + (uint32_t)slot * kWStage, step + 2, wave);
-        if (step + 1 < n_steps) read(slot ^ 1, 0);
-        multiply(3);
+    // row block m's two products of group kk
+    auto multiply = [&](int kk, int m) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[j][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ra[kk & 1][m], rb[kk & 1][j], acc[j][m], 0, 0, 0);
+    };
+    // Behind the barrier of a step, beside its last products, the rows of the step after the next are asked for; beside the first
+    // products after that the weights of one step more (tiles of more than 256 rows leave no room for that: of the same step).  All at once
+    // they fill the address unit's queue, and every wave stands before it.  Past the end: the last again, never multiplied.
+    constexpr int kAhead = R::kB == 3 ? 2 : 1;
+    const uint32_t lds_a = lds0 + R::kAtA;
+    auto at_most = [&](int step) { return step < n_steps ? step : n_steps - 1; };
+#pragma unroll
+    for (int i = 0; i < 4; i++) l.load_b(lds0, 0, wave, i);
+#pragma unroll
+    for (int i = 0; i < MW; i++) l.load_a(lds_a, 0, wave, i);
+    if (kAhead == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) l.load_b(lds0 + kWStageB, 1, wave, i);
     }
+#pragma unroll
+    for (int i = 0; i < MW; i++) l.load_a(lds_a + R::kStageA, 1, wave, i);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(MW + (kAhead == 2 ? 4 : 0)) : "memory");
+    read(0, 0, 0);
+    convert(0);
+    uint32_t at_b = 0, free_b = kAhead * kWStageB;   // of this step's weights; of those kAhead on
+    for (int step = 0; step < n_steps; step++) {
+        const uint32_t at_a = (uint32_t)(step & 1) * R::kStageA, next_a = R::kStageA - at_a;
+        const uint32_t next_b = at_b == (R::kB - 1) * kWStageB ? 0u : at_b + kWStageB;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            // the next stage has landed and this one has been read by everybody
+            if (kk == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kAhead == 2 ? 4 : 0) : "memory");
+            read(kk == 3 ? next_a : at_a, kk == 3 ? next_b : at_b, (kk + 1) & 3);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MW; m++) {
+                multiply(kk, m);
+                if (kk == 3) l.load_a(lds_a + at_a, at_most(step + 2), wave, m);
+                if (kk == 0) {
+#pragma unroll
+                    for (int i = m; i < 4; i += MW) l.load_b(lds0 + free_b, at_most(step + kAhead), wave, i);
+                }
+                if (m == MW - 1) convert((kk + 1) & 3);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        free_b = at_b;
+        at_b = next_b;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load into LDS is under way when the workgroup ends)
 
     // element r of an accumulator: row 8 (r / 4) + 4 g + r % 4, column lane % 32
 #pragma unroll
@@ -188,8 +222,7 @@ __device__ inline void wide_tile(const WideArgs &p, int e, int p0, int rows, int
 
 template <bool GATE_UP, int WT>
 __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(WideArgs p) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // [2][kWStage]
-    __shared__ int s_rows[kWideRows];
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // Ring
     // As xcd_tile in gemm.hip: an XCD (workgroup ids equal modulo 8) takes neighbouring tiles with the slab running
     // fastest: the slabs of a tile share its rows in the XCD's L2, the tiles of an expert its weights.
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
@@ -200,16 +233,12 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(WideArgs p) {
     const int tile = (int)(blockIdx.x & 7) * per_xcd + within;
     if (within >= per_xcd || tile >= total) return;
     const int e = uniform(p.tiles[3 * tile]), p0 = uniform(p.tiles[3 * tile + 1]), rows = uniform(p.tiles[3 * tile + 2]);
-    if (GATE_UP) {
-        if ((int)threadIdx.x < rows) s_rows[threadIdx.x] = p.sorted[p0 + threadIdx.x] / p.k_slots;
-        __syncthreads();
-    }
     switch ((rows + kWideUnit - 1) / kWideUnit) {
-    case 1: wide_tile<GATE_UP, WT, 1>(p, e, p0, rows, slab, s_lds, s_rows); break;
-    case 2: wide_tile<GATE_UP, WT, 2>(p, e, p0, rows, slab, s_lds, s_rows); break;
-    case 3: wide_tile<GATE_UP, WT, 3>(p, e, p0, rows, slab, s_lds, s_rows); break;
-    case 4: wide_tile<GATE_UP, WT, 4>(p, e, p0, rows, slab, s_lds, s_rows); break;
-    default: wide_tile<GATE_UP, WT, 5>(p, e, p0, rows, slab, s_lds, s_rows); break;
+    case 1: wide_tile<GATE_UP, WT, 1>(p, e, p0, rows, slab, s_lds); break;
+    case 2: wide_tile<GATE_UP, WT, 2>(p, e, p0, rows, slab, s_lds); break;
+    case 3: wide_tile<GATE_UP, WT, 3>(p, e, p0, rows, slab, s_lds); break;
+    case 4: wide_tile<GATE_UP, WT, 4>(p, e, p0, rows, slab, s_lds); break;
+    default: wide_tile<GATE_UP, WT, 5>(p, e, p0, rows, slab, s_lds); break;
     }
 }
 
@@ -217,7 +246,7 @@ template <bool GATE_UP, int WT>
 hipError_t launch_wide(const WideArgs &p, int max_tiles, hipStream_t s) {
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
     const unsigned n_slabs = (unsigned)((p.out_dim + kCols - 1) / kCols);
-    launch_kernel(wide_gemm_kernel<GATE_UP, WT>, dim3((unsigned)(max_tiles + 7) / 8 * 8 * n_slabs), dim3(512), (size_t)2 * kWStage, s, p);
+    launch_kernel(wide_gemm_kernel<GATE_UP, WT>, dim3((unsigned)(max_tiles + 7) / 8 * 8 * n_slabs), dim3(512), (size_t)kWLds, s, p);
     return hipGetLastError();
 }
 
