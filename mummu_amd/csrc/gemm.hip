@@ -893,246 +893,6 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
     }
 }
 
-// ---------------------------------------------------------------------------------------
-// Q4_K banks on the f16 units, few rows per expert
-// ---------------------------------------------------------------------------------------
-// The product of gemm_q4k.hip for experts with few rows (small batches): 16-row tiles on v_mfma_f32_16x16x32_f16.  Eight
-// waves, wave w owns output columns 16w..16w+15; a stage is half a super-block (128 elements).  Lane (column c,
-// K group kg) reads 16 of the 64 quant bytes of the stage - the four lanes of a column read 64 consecutive bytes
-// of its row - and supplies, in instruction q of the stage, the eight elements
-//     64 (kg / 2) + 16 (kg % 2) + 32 (q / 2) + 8 (q % 2) + 0..7
-// (low nibbles of its bytes for q < 2, high nibbles after), and the activation operands are read from the tile at
-// that offset.  A quarter of the accumulators and half the matrix work of the 32-row form, and twice the waves
-// on a SIMD.
-template <bool GATE_UP, bool OUT_H>
-__global__ __launch_bounds__(512, 4) void grouped_gemm_q4k_f16_m16_kernel(
-    const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, HAct a_in, const int32_t *__restrict__ sorted, int k_slots,
-    const int32_t *__restrict__ tiles, const int32_t *__restrict__ n_tiles, int in_dim, int out_dim, HAct act_h, QAct64 act_q,
-    float *__restrict__ y_out) {
-    constexpr int NB = GATE_UP ? 2 : 1, BM = 16;
-    constexpr int kRow = 2 * 128 + 16;                 // LDS row (bytes): 128 halfs + 16 bytes keep 16-byte reads conflict-free
-    constexpr int kPlane = BM * kRow, kBuf = 2 * kPlane;   // hi plane, lo plane of one stage
-    constexpr int kC = GATE_UP ? BM * kLdsC * 4 : 0;   // f32 staging of the epilogue (aliases the tiles)
-    constexpr int kBytes = 2 * kBuf > kC ? 2 * kBuf : kC;
-    constexpr bool ROW = GATE_UP;                      // one activation scale per row (else per 128 elements = per stage)
-    __shared__ __attribute__((aligned(16))) uint8_t s_raw[kBytes];
-    __shared__ __attribute__((aligned(16))) float s_as[2][BM];
-    // block sums of one fold.  ROW: the super-block's eight hi halfs, then its eight lo halfs; else the stage's four
-    // hi halfs, four lo halfs and eight zeros (the fold is one K = 16 instruction either way)
-    // (rows of 20 halfs: with 16 the rows four apart share their banks)
-    __shared__ __attribute__((aligned(16))) _Float16 s_sum[2][BM][20];
-
-    int tile, slab;
-    if (!xcd_tile(n_tiles, (out_dim + kBN - 1) / kBN, tile, slab)) return;
-    const int e = tiles[3 * tile], p0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-    const int n0 = slab * kBN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t row_bytes = gemm_row_bytes(T_Q4_K, in_dim);
-    const int c = lane & 15, kg = lane >> 4;
-    const int col = 16 * wave + c;
-
-    const int b_out = n0 + col < out_dim ? n0 + col : out_dim - 1;
-    const uint8_t *b_base[NB];
-    b_base[0] = w0 + (size_t)e * (size_t)out_dim * row_bytes;
-    if (GATE_UP) b_base[NB - 1] = w1 + (size_t)e * (size_t)out_dim * row_bytes;
-    const uint32_t h_off = (uint32_t)b_out * (uint32_t)row_bytes;   // the row's first super-block header
-    const uint32_t b_off = h_off + 16u + 16u * (uint32_t)kg;
-
-    auto source_row = [&](int r) -> int {
-        r = r < rows ? r : rows - 1;
-        return GATE_UP ? sorted[p0 + r] / k_slots : p0 + r;
-    };
-    // activation tile: thread -> (plane, row, 8 halfs of the stage's 128)
-    const int a_plane = tid >> 8, a_row = (tid >> 4) & 15, a_chunk = tid & 15;
-    const uint8_t *a_base = (const uint8_t *)(a_plane ? a_in.lo : a_in.hi);
-    const uint32_t a_off = ((uint32_t)source_row(a_row) * (uint32_t)in_dim + (uint32_t)a_chunk * 8u) * 2u;
-    const uint32_t a_lds = (uint32_t)(a_plane * kPlane + a_row * kRow + a_chunk * 16);
-    // block sums: thread -> (row, one of the stage's four blocks); every thread stores (threads past 64 repeat rows)
-    const int m_row = (tid >> 2) & (BM - 1), m_blk = tid & 3;
-    const uint32_t src_m = (uint32_t)source_row(m_row);
-    const uint32_t sum_off = (src_m * (uint32_t)(in_dim / 32) + (uint32_t)m_blk) * 4u;
-    const uint32_t scale_off = src_m * (uint32_t)(in_dim / 128) * 4u;
-    if (ROW) s_as[0][m_row] = *(const float *)((const uint8_t *)a_in.scale + scale_off);
-    if (!ROW) {
-        s_sum[0][m_row][8 + m_blk] = s_sum[0][m_row][12 + m_blk] = (_Float16)0.0f;
-        s_sum[1][m_row][8 + m_blk] = s_sum[1][m_row][12 + m_blk] = (_Float16)0.0f;
-    }
-
-    f32x4 acc[NB], c1[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) acc[b] = c1[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    u32x4 raw[2][NB], rh_next[NB];
-    uint32_t dd[NB], sc4[NB][2], mn4[NB][2];
-    auto load_b = [&](int k0, u32x4 (&dst)[NB]) {
-        const uint32_t o = b_off + (uint32_t)(k0 >> 8) * 144u + (uint32_t)((k0 >> 7) & 1) * 64u;
-#pragma unroll
-        for (int b = 0; b < NB; b++) dst[b] = *(const u32x4 *)(b_base[b] + o);
-    };
-    auto load_header = [&](int k0) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) rh_next[b] = *(const u32x4 *)(b_base[b] + (h_off + (uint32_t)(k0 >> 8) * 144u));
-    };
-    auto unpack_header = [&]() {   // ggml get_scale_min_k4 for all eight sub-blocks at once
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const uint32_t y = rh_next[b][1], z = rh_next[b][2], w = rh_next[b][3];
-            dd[b] = rh_next[b][0];
-            sc4[b][0] = y & 0x3F3F3F3Fu;
-            mn4[b][0] = z & 0x3F3F3F3Fu;
-            sc4[b][1] = (w & 0x0F0F0F0Fu) | ((y >> 2) & 0x30303030u);
-            mn4[b][1] = ((w >> 4) & 0x0F0F0F0Fu) | ((z >> 2) & 0x30303030u);
-        }
-    };
-    u32x4 ra;
-    float rsum = 0.0f, rscale = 0.0f;
-    auto load_a = [&](int k0) {
-        ra = *(const u32x4 *)(a_base + (a_off + (uint32_t)k0 * 2u));
-        rsum = *(const float *)((const uint8_t *)a_in.ssum + (sum_off + (uint32_t)(k0 >> 5) * 4u));
-        if (!ROW) rscale = *(const float *)((const uint8_t *)a_in.scale + (scale_off + (uint32_t)(k0 >> 7) * 4u));
-    };
-    // buf: the tile of the stage; sum_buf / slot: where its block sums go
-    auto store_a = [&](int buf, int sum_buf, int slot) {
-        *(u32x4 *)(s_raw + (size_t)buf * kBuf + a_lds) = ra;
-        if (wave == 0) {   // (every wave holds the same sums: one stores them)
-            const _Float16 h = (_Float16)rsum;
-            s_sum[sum_buf][m_row][slot + m_blk] = h;
-            s_sum[sum_buf][m_row][slot + (ROW ? 8 : 4) + m_blk] = (_Float16)__fsub_rn(rsum, (float)h);
-            if (!ROW) s_as[sum_buf][m_row] = rscale;
-        }
-    };
-
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto multiply = [&](int hs, int buf, const u32x4 (&rw)[NB], bool first) {
-        half2v ml2[NB], mh2[NB];
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            // this lane's bytes belong to sub-blocks 4 hs + 2 (kg / 2) (low nibbles) and the one after (high nibbles)
-            // (hs is a constant at every call: picked with a conditional, an index would send the array to LDS)
-            const uint32_t sw = (hs ? sc4[b][1] : sc4[b][0]) >> (16 * (kg >> 1));
-            ml2[b] = q4k_mul<false>(sw & 0xFFu);
-            mh2[b] = q4k_mul<true>((sw >> 8) & 0xFFu);
-        }
-        const uint8_t *tile_p = s_raw + (size_t)buf * kBuf + (size_t)(lane & 15) * kRow + 128 * (kg >> 1) + 32 * (kg & 1);
-        half8 a_hi[2], a_lo[2];
-        auto read_a = [&](int q) {
-            const int a_byte = 64 * (q >> 1) + 16 * (q & 1);
-            a_hi[q & 1] = *(const half8 *)(tile_p + a_byte);
-            a_lo[q & 1] = *(const half8 *)(tile_p + kPlane + a_byte);
-        };
-        read_a(0);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (q < 3) read_a(q + 1);
-            half8 bfrag[NB];
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                const uint32_t w_a = (q & 1) ? rw[b][2] : rw[b][0], w_b = (q & 1) ? rw[b][3] : rw[b][1];
-                bfrag[b] = q < 2 ? q4k_operand<false>(w_a, w_b, ml2[b]) : q4k_operand<true>(w_a, w_b, mh2[b]);
-            }
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-                c1[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_hi[q & 1], bfrag[b], (first && q == 0) ? zero : c1[b], 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < NB; b++) c1[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_lo[q & 1], bfrag[b], c1[b], 0, 0, 0);
-        }
-    };
-    // what has been summed into c1 -> acc (hs: the stage, for the per-stage fold of the down side)
-    auto fold = [&](int hs, int sum_buf) {
-        const half4v am = *(const half4v *)&s_sum[sum_buf][lane & 15][4 * kg];
-        float sr[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-        if (!ROW) {
-            const float4 s4 = *(const float4 *)&s_as[sum_buf][4 * kg];
-            sr[0] = s4.x, sr[1] = s4.y, sr[2] = s4.z, sr[3] = s4.w;
-        }
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const float d = __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd[b] & 0xFFFFu)));
-            const float ndmin = -half_bits_to_float((uint16_t)(dd[b] >> 16));
-            // K index 4 kg + i of the fold: sub-block (4 kg + i) % 8 with ROW, else 4 hs + i (its K groups 2, 3 meet zeros)
-            // (with one scale per row the word depends on the lane: blended with a mask - a conditional between the two
-            // array elements becomes an indexed load and sends the array to LDS)
-            const uint32_t lane_mask = 0u - (uint32_t)(kg & 1);
-            const uint32_t word = ROW ? (mn4[b][0] ^ ((mn4[b][0] ^ mn4[b][1]) & lane_mask)) : (hs ? mn4[b][1] : mn4[b][0]);
-            half4v bm;
-#pragma unroll
-            for (int i = 0; i < 4; i++) bm[i] = (_Float16)(float)((word >> (8 * i)) & 0xFFu);
-            const f32x4 c2 = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (ROW) {
-                    acc[b][i] = fmaf(ndmin, c2[i], fmaf(d, c1[b][i], acc[b][i]));
-                } else {
-                    const float u = fmaf(ndmin, c2[i], __fmul_rn(d, c1[b][i]));
-                    acc[b][i] = fmaf(u, sr[i], acc[b][i]);
-                }
-            }
-        }
-    };
-
-    // prologue: the first header, stage 0 into tile 0
-    load_header(0);
-    unpack_header();
-    load_a(0);
-    load_b(0, raw[0]);
-    store_a(0, 0, 0);
-    __syncthreads();
-    auto stage = [&](int sb0, auto hs_c) {
-        constexpr int hs = decltype(hs_c)::value;
-        // (after the last stage the "next" one is stage 0 again: loaded and stored like any other, never multiplied)
-        const int sb_next = sb0 + 256 < in_dim ? sb0 + 256 : 0;
-        const int k_next = hs == 0 ? sb0 + 128 : sb_next;
-        const int sb_par = (sb0 >> 8) & 1;
-        load_a(k_next);
-        load_b(k_next, raw[(hs + 1) & 1]);
-        if (hs == 0) load_header(sb_next);   // (a stage before its unpacking: nothing loaded in the loop's last stage is first read in the next iteration)
-        MUMMU_CODE_FENCE();
-        multiply(hs, hs, raw[hs], ROW ? hs == 0 : true);
-        if (ROW ? hs == 1 : true) fold(hs, ROW ? sb_par : hs);
-        if (hs == 1) unpack_header();
-        MUMMU_CODE_FENCE();
-        if (ROW) store_a((hs + 1) & 1, hs == 0 ? sb_par : sb_par ^ 1, hs == 0 ? 4 : 0);
-        else store_a((hs + 1) & 1, (hs + 1) & 1, 0);
-        __syncthreads();
-    };
-    for (int sb0 = 0; sb0 < in_dim; sb0 += 256) {
-        stage(sb0, std::integral_constant<int, 0>{});
-        stage(sb0, std::integral_constant<int, 1>{});
-    }
-
-    if (GATE_UP) {
-        float *s_c = (float *)s_raw;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = 4 * kg + i;
-            const float sr = s_as[0][row];   // (one scale per row on this side: both products take it here)
-            s_c[row * kLdsC + col] = __fmul_rn(det_silu(__fmul_rn(sr, acc[0][i])), __fmul_rn(sr, acc[NB - 1][i]));
-        }
-        __syncthreads();
-        if (OUT_H) {
-            const int row = tid >> 5, l32 = tid & 31;
-            const float4 v = *(const float4 *)&s_c[row * kLdsC + 4 * l32];
-            const bool active = row < rows && n0 < out_dim;
-            hact_store128(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, act_h, (size_t)(p0 + row), out_dim, n0 + 4 * l32);
-        } else {
-            const int grp = tid >> 4, l16 = tid & 15, row = grp >> 1, cb = grp & 1;
-            const float4 v = *(const float4 *)&s_c[row * kLdsC + cb * 64 + 4 * l16];
-            const bool active = row < rows && n0 + cb * 64 < out_dim;
-            quantize_store64(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, act_q, (size_t)(p0 + row), out_dim,
-                             n0 + cb * 64 + 4 * l16);
-        }
-    } else {
-        const int n = n0 + col;
-        if (n < out_dim) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = 4 * kg + i;
-                if (row < rows) y_out[(size_t)(p0 + row) * (size_t)out_dim + (size_t)n] = acc[0][i];
-            }
-        }
-    }
-}
-
 // x [n, d] f32 -> HAct with one scale per row: a workgroup per row finds the row's largest magnitude, then
 // stores the row 1024 elements at a time.
 __global__ __launch_bounds__(256) void quantize_rows_h_kernel(const float *__restrict__ x, int d, HAct q) {
@@ -1195,17 +955,18 @@ bool grouped_gemm_supported(const ExpertBanks &b) {
 // that streams its whole weight slab again, so the tile is sized to hold the average expert load
 // plus its spread (binomial: about +-sqrt(avg) per expert, 3.5 sigma here) when that fits; the f16
 // kernel goes up to 128 rows, the int8 kernel (more registers per row) to 64.
-// Tile rows for the f16-unit Q4_K kernels: 16 (the form for few rows) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what
-// they have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal
-// approximation, variance = mean).  The 16-row form is taken only while next to no expert has more than 16 rows, its expected tiles within
-// 1 % of the other's: 64 experts x 8 slabs of 16-row tiles are exactly the 512 workgroups the chip holds at once, and the first
-// second tiles start a second round.  Layers, 16 / 64 rows, us: OLMoE 24 tokens 78 / 92, 48: 79 / 93, 72: 97 / 93, 96: 99 / 96, 192: 150 / 113;
-// 128 experts of 2048 x 768, 128 tokens 141 / 152, 140: 143 / 154, 160: 160 / 154, 208: 165 / 159.  Lists of 32 rows gained nothing
-// between them (OLMoE 96 tokens 94, 256: 132 against 129, 1000: 331 against 302).
+// Tile rows for the f16-unit Q4_K kernels: 16 (gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what they
+// have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
+// variance = mean).  Layers, 16 / 64 rows, us: in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it
+// weighs: 128 experts of 2048 x 768, 128 tokens 127 / 155, 160: 145 / 158, 208 (1.17 tiles an expert): 148 / 159, 240 (1.4): 162 / 161.  Where a
+// tile per expert fills the chip exactly once, the first second tiles start a second round: OLMoE, 24 tokens 76 / 92, 60: 77 / 93, 64: 96 / 93,
+// 96: 97 / 95, 112 (1.27): 96 / 97.  Lists of 32 rows gained nothing between the two (96 tokens 94, 256: 132 against 129, 1000: 331 against
+// 302).
 // With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
 // products together: OLMoE Q4_K with Q6_K downs, 32 / 64 rows: 150 tokens 154 / 206 us, 230: 181 / 208, 260: 225 / 214; the
 // 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013.
-int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts, bool int8_down) {
+int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8_down) {
+    const int n_experts = b.n_experts;
     const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
     const double sigma = __builtin_sqrt(avg > 1.0 ? avg : 1.0);
     auto expected_tiles = [&](double rows) {
@@ -1218,8 +979,10 @@ int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts, bool int8_down) 
         return t;
     };
     const double e16 = expected_tiles(16.0), e32 = expected_tiles(32.0), e64 = expected_tiles(64.0);
-    if (0.99 * e16 < (int8_down ? e32 : e64)) return 16;
-    return int8_down && 0.69 * e32 < e64 ? 32 : 64;
+    if (int8_down) return 0.99 * e16 < e32 ? 16 : (0.69 * e32 < e64 ? 32 : 64);
+    const double each = (double)n_experts * (double)((b.inter + 127) / 128);   // workgroups of a tile per expert
+    const bool second_round = each * e64 <= 512.0 && each * e16 > 1.01 * 512.0;
+    return !second_round && e16 < 1.25 * e64 ? 16 : 64;
 }
 
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half) {
@@ -1295,20 +1058,6 @@ bool grouped_gemm_q4k_f16_down(const ExpertBanks &b) {
 }
 
 template <bool GATE_UP>
-static hipError_t launch_gemm_q4k_f16_m16(const uint8_t *w0, const uint8_t *w1, HAct a_in, const int32_t *sorted, int k_slots,
-                                          const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int in_dim, int out_dim, HAct act_h,
-                                          QAct64 act_q, bool out_h, float *y_out, hipStream_t s) {
-    dim3 grid((unsigned)((max_tiles + 7) / 8 * 8) * (unsigned)((out_dim + kBN - 1) / kBN));
-    if (out_h)
-        launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, true>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles, n_tiles,
-                      in_dim, out_dim, act_h, act_q, y_out);
-    else
-        launch_kernel(grouped_gemm_q4k_f16_m16_kernel<GATE_UP, false>, grid, dim3(512), 0, s, w0, w1, a_in, sorted, k_slots, tiles, n_tiles,
-                      in_dim, out_dim, act_h, act_q, y_out);
-    return hipGetLastError();
-}
-
-template <bool GATE_UP>
 static hipError_t launch_gemm_f32(const uint8_t *w0, const uint8_t *w1, const float *a_in, const int32_t *sorted, int k_slots,
                                   const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows, int in_dim,
                                   int out_dim, float *act_out, float *y_out, hipStream_t s) {
@@ -1364,8 +1113,7 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
         if (out_h && !grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
         if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
         if (tile_rows > 16) return launch_q4k_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
-        return launch_gemm_q4k_f16_m16<true>(b.gate, b.up, xh, sorted, k_slots, tiles, n_tiles, max_tiles, b.hidden, b.inter, acth, actq,
-                                             out_h, nullptr, s);
+        return launch_q4k_few_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
     }
     if (b.gate_type == T_F32)
         return launch_gemm_f32<true>(b.gate, b.up, x, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden, b.inter, act32,
@@ -1413,8 +1161,7 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
         if (!grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
         if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
         if (tile_rows > 16) return launch_q4k_down(b, acth, tiles, n_tiles, max_tiles, y, s);
-        return launch_gemm_q4k_f16_m16<false>(b.down, nullptr, acth, nullptr, 1, tiles, n_tiles, max_tiles, b.inter, b.hidden, HAct(),
-                                              QAct64(), false, y, s);
+        return launch_q4k_few_down(b, acth, tiles, n_tiles, max_tiles, y, s);
     }
     if (b.down_type == T_F32)
         return launch_gemm_f32<false>(b.down, nullptr, act32, nullptr, 1, tiles, n_tiles, max_tiles, tile_rows, b.inter, b.hidden,

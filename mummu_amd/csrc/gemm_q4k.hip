@@ -43,42 +43,10 @@ constexpr int kLdsBytes = kAtC + 4 * kRows * 4;
 static_assert(kRows == 64 && kRows * kRowC * 4 <= kAtC && kLdsBytes <= 80 * 1024,
               "a lane per row; the epilogue leaves the scales alone; two workgroups share a CU");
 
-struct Args {
-    const uint8_t *w0, *w1;        // gate and up, or down [experts][out_dim][in_dim]
-    HAct a;                        // rows of in_dim: tokens (gate/up, through sorted / k_slots) or sorted positions
-    const int32_t *sorted, *tiles, *n_tiles;
-    int k_slots, in_dim, out_dim;
-    HAct act_h;                    // gate/up: silu(g) * u, sorted positions, in the form the down product reads
-    QAct64 act_q;
-    float *y;                      // down
-};
-
-// x / (1 + e^-x) in f32: the hardware's 2^y and reciprocal (1 ulp each), with what rounding y = -x log2 e lost put back and the
-// reciprocal refined once.  The exponent stops at +-87, where e^-x and its reciprocal are both normal numbers: above, the quotient
-// is x as it is; below, it is x * 0 (a gate of -inf is NaN, as in det_silu).
-__device__ inline float silu_of(float x) {
-    const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
-    const float y = __fmul_rn(c, -1.44269504f);
-    const float lost = __builtin_fmaf(c, -1.44269504f, -y);
-    const float lost2 = __builtin_fmaf(c, -1.92596299e-8f, lost);   // log2 e - 1.44269504f
-    float t = __builtin_amdgcn_exp2f(y);
-    t = __builtin_fmaf(t, __fmul_rn(lost2, 0.693147181f), t);
-    const float den = __fadd_rn(1.0f, t);
-    float r = __builtin_amdgcn_rcpf(den);
-    r = __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
-    return __fmul_rn(x, x < -87.0f ? 0.0f : r);
-}
-
-// The same value, computed again: what is derived from it does not keep a register through the loop.
-__device__ inline int again(int v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 // A tile of up to 32 MW rows by one slab.  Wave w multiplies all rows by its 64 weight rows: columns c and 32 + c of lane
 // (c, g) (gate/up: column 32 w + c of gate and of up).
 template <bool GATE_UP, int MW, bool OUT_H>
-__device__ inline void q4k_tile(const Args &p, int e, int p0, int rows, int slab, uint8_t *s_lds) {
+__device__ inline void q4k_tile(const Q4kArgs &p, int e, int p0, int rows, int slab, uint8_t *s_lds) {
     constexpr bool ROW = GATE_UP;   // one scale per row, applied at the end: a fold takes a whole super-block; else 128 elements
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 31, g = lane >> 5;
     const uint32_t row_bytes = (uint32_t)(p.in_dim / 256) * 144u;
@@ -201,9 +169,7 @@ __device__ inline void q4k_tile(const Args &p, int e, int p0, int rows, int slab
     auto scales = [&](int st) {
 #pragma unroll
         for (int b = 0; b < 2; b++) {
-            const uint32_t sw = head[b].sc4[st >> 1] >> (16 * (st & 1));   // sub-blocks 2 st (the low nibbles) and 2 st + 1
-            ml[b] = q4k_mul<false>(sw & 0xFFu);
-            mh[b] = q4k_mul<true>((sw >> 8) & 0xFFu);
+            head[b].muls(st, ml[b], mh[b]);
         }
     };
     auto decode = [&](int st, int kk) {
@@ -216,17 +182,14 @@ __device__ inline void q4k_tile(const Args &p, int e, int p0, int rows, int slab
     };
     // what has been summed into c1 -> acc.  part: which 128 elements of super-block sb (all of it with one scale per row)
     float fd[2], fm[2];
-    half8 bm[2];
+    std::conditional_t<ROW, half8, half4v> bm[2];
     auto fold_begin = [&](int part) {
 #pragma unroll
         for (int b = 0; b < 2; b++) {
             fd[b] = head[b].d();
             fm[b] = head[b].minus_dmin();
-#pragma unroll
-            for (int j = 0; j < (ROW ? 8 : 4); j++) {
-                const uint32_t word = ROW ? head[b].mn4[j >> 2] : head[b].mn4[part];
-                bm[b][j] = (_Float16)(float)((word >> (8 * (j & 3))) & 0xFFu);
-            }
+            if constexpr (ROW) bm[b] = head[b].offsets();
+            else bm[b] = head[b].offsets(part);
         }
     };
     auto fold = [&](int sb, int part) {
@@ -238,8 +201,7 @@ __device__ inline void q4k_tile(const Args &p, int e, int p0, int rows, int slab
                 float16v c2;
                 if constexpr (ROW) c2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const half8 *)(at + 16 * g), bm[b], zero, 0, 0, 0);
                 else {
-                    const half4v y = {bm[b][0], bm[b][1], bm[b][2], bm[b][3]};
-                    c2 = __builtin_amdgcn_mfma_f32_32x32x8f16(*(const half4v *)(at + 16 * part + 8 * g), y, zero, 0, 0, 0);
+                    c2 = __builtin_amdgcn_mfma_f32_32x32x8f16(*(const half4v *)(at + 16 * part + 8 * g), bm[b], zero, 0, 0, 0);
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -398,7 +360,7 @@ __device__ inline void q4k_tile(const Args &p, int e, int p0, int rows, int slab
 }
 
 template <bool GATE_UP, bool OUT_H>
-__global__ __launch_bounds__(64 * kWaves, 2) void q4k_gemm_kernel(Args p) {
+__global__ __launch_bounds__(64 * kWaves, 2) void q4k_gemm_kernel(Q4kArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];
     // As xcd_tile in gemm.hip: an XCD takes neighbouring tiles with the slab running fastest.
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
@@ -414,7 +376,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q4k_gemm_kernel(Args p) {
 }
 
 template <bool GATE_UP, bool OUT_H>
-hipError_t launch_q4k(const Args &p, int max_tiles, hipStream_t s) {
+hipError_t launch_q4k(const Q4kArgs &p, int max_tiles, hipStream_t s) {
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
     const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)((p.out_dim + kCols - 1) / kCols));
     launch_kernel(q4k_gemm_kernel<GATE_UP, OUT_H>, grid, dim3(64 * kWaves), kLdsBytes, s, p);
@@ -425,12 +387,12 @@ hipError_t launch_q4k(const Args &p, int max_tiles, hipStream_t s) {
 
 hipError_t launch_q4k_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
                               int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s) {
-    const Args p{b.gate, b.up, x, sorted, tiles, n_tiles, k_slots, b.hidden, b.inter, act_h, act_q, nullptr};
+    const Q4kArgs p{b.gate, b.up, x, sorted, tiles, n_tiles, k_slots, b.hidden, b.inter, act_h, act_q, nullptr};
     return act_h.hi != nullptr ? launch_q4k<true, true>(p, max_tiles, s) : launch_q4k<true, false>(p, max_tiles, s);
 }
 
 hipError_t launch_q4k_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y, hipStream_t s) {
-    const Args p{b.down, nullptr, act, nullptr, tiles, n_tiles, 1, b.inter, b.hidden, HAct(), QAct64(), y};
+    const Q4kArgs p{b.down, nullptr, act, nullptr, tiles, n_tiles, 1, b.inter, b.hidden, HAct(), QAct64(), y};
     return launch_q4k<false, true>(p, max_tiles, s);
 }
 

@@ -189,7 +189,7 @@ hipError_t launch_identity_tiles(int n, int tile_rows, int expert, int32_t *sort
 bool grouped_gemm_supported(const ExpertBanks &b);
 bool grouped_gemm_quantized(const ExpertBanks &b);
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half = false);
-int grouped_gemm_tile_rows_q4k_f16(int n_assign, int n_experts, bool int8_down = false);   // (the f16-unit Q4_K kernels: 16, 32 or 64)
+int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8_down = false);   // (the f16-unit Q4_K kernels: 16, 32 or 64)
 // x [n, d] f32 -> QAct64 (d % 64 == 0).
 hipError_t launch_quantize_rows64(const float *x, int n, int d, QAct64 q, hipStream_t s);
 // Q4_K banks can take the f16 units instead, against activations held as pairs of halfs (HAct: xh tokens x
@@ -232,6 +232,13 @@ constexpr int kQ4kRows = 64;
 hipError_t launch_q4k_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
                               int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s);
 hipError_t launch_q4k_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y, hipStream_t s);
+
+// gemm_q4k_few.hip: the same on tiles of up to kQ4kFewRows rows.
+constexpr int kQ4kFewRows = 16;
+hipError_t launch_q4k_few_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles,
+                                  const int32_t *n_tiles, int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s);
+hipError_t launch_q4k_few_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y,
+                               hipStream_t s);
 
 // gemm_q8.hip -------------------------------------------------------------------------
 // Q8_0 banks on the f16 units: x and the activations between the two products as pairs of halfs, tiles of 32 rows.

@@ -545,9 +545,9 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         const bool hf = hp.hf, hf_down = hp.hf_down;
         // Q8_0 banks through the f16 kernel: x as halfs, like the f16 banks
         const bool q8h = h->gemm_q8_f16 && grouped_gemm_q8_f16(b);
-        int tile_rows = hf_down ? grouped_gemm_tile_rows_q4k_f16(na, b.n_experts) : grouped_gemm_tile_rows(b, na, b.n_experts, q8h);
+        int tile_rows = hf_down ? grouped_gemm_tile_rows_q4k_f16(b, na) : grouped_gemm_tile_rows(b, na, b.n_experts, q8h);
         // (gate/up alone on the f16 units: the int8 down product takes a tile of 16 rows like one of 32)
-        if (hf && !hf_down) tile_rows = grouped_gemm_tile_rows_q4k_f16(na, b.n_experts, true);
+        if (hf && !hf_down) tile_rows = grouped_gemm_tile_rows_q4k_f16(b, na, true);
         if (hf_down && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
         if (hp.q8) tile_rows = 32;
         const bool wide = wide_gemm_takes(b, (int)n, na);

@@ -4,7 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "device_utils.h"
+#include "qact.h"
 
 namespace mummu {
 
@@ -32,12 +35,6 @@ __device__ inline half8 q4k_operand(uint32_t w0, uint32_t w1, half2v mul) {
     __builtin_memcpy(&o, f, 16);
     return o;
 }
-// ... with mul for a sub-block scale sc: sc * 2^10 for the low nibbles, sc * 2^6 for the high ones.
-template <bool HIGH>
-__device__ inline half2v q4k_mul(uint32_t sc) {
-    const _Float16 m = (_Float16)__fmul_rn((float)sc, HIGH ? 64.0f : 1024.0f);
-    return half2v{m, m};
-}
 constexpr float kQ4kUnit = 16384.0f;
 
 // The first 16 bytes of a super-block: d | dmin, and (ggml get_scale_min_k4 for all eight sub-blocks at once) the scales and
@@ -51,8 +48,62 @@ struct Q4kHeader {
         sc4[1] = (h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u);
         mn4[1] = ((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u);
     }
+    // Bytes 0, 1 (or 2, 3) of t as halfs: a byte under 0x64 is the half 1024 + byte.
+    __device__ static half2v pair(uint32_t t, bool upper) {
+        const uint32_t u = __builtin_amdgcn_perm(0x64646464u, t, upper ? 0x04030402u : 0x04010400u);
+        half2v h;
+        __builtin_memcpy(&h, &u, 4);
+        return h - half2v{(_Float16)1024.0f, (_Float16)1024.0f};
+    }
+    // mul of q4k_operand for step st: of sub-block 2 st (the low nibbles) sc * 2^10, of 2 st + 1 (the high ones) sc * 2^6.
+    __device__ void muls(int st, half2v &low, half2v &high) const {
+        const half2v m = pair(sc4[st >> 1], st & 1) * half2v{(_Float16)1024.0f, (_Float16)64.0f};
+        low = half2v{m[0], m[0]};
+        high = half2v{m[1], m[1]};
+    }
+    // The block offsets m as halfs (exact), in the order of the block sums: of four sub-blocks, of all.
+    __device__ half4v offsets(int part) const {
+        const half2v a = pair(mn4[part], false), b = pair(mn4[part], true);
+        return half4v{a[0], a[1], b[0], b[1]};
+    }
+    __device__ half8 offsets() const {
+        const half4v a = offsets(0), b = offsets(1);
+        return half8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    }
     __device__ float d() const { return __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd & 0xFFFFu))); }
     __device__ float minus_dmin() const { return -half_bits_to_float((uint16_t)(dd >> 16)); }
 };
+
+struct Q4kArgs {
+    const uint8_t *w0, *w1;        // gate and up, or down [experts][out_dim][in_dim]
+    HAct a;                        // rows of in_dim: tokens (gate/up, through sorted / k_slots) or sorted positions
+    const int32_t *sorted, *tiles, *n_tiles;
+    int k_slots, in_dim, out_dim;
+    HAct act_h;                    // gate/up: silu(g) * u, sorted positions, in the form the down product reads
+    QAct64 act_q;
+    float *y;                      // down
+};
+
+// x / (1 + e^-x) in f32: the hardware's 2^y and reciprocal (1 ulp each), with what rounding y = -x log2 e lost put back and the
+// reciprocal refined once.  The exponent stops at +-87, where e^-x and its reciprocal are both normal numbers: above, the quotient
+// is x as it is; below, it is x * 0 (a gate of -inf is NaN, as in det_silu).
+__device__ inline float silu_of(float x) {
+    const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
+    const float y = __fmul_rn(c, -1.44269504f);
+    const float lost = __builtin_fmaf(c, -1.44269504f, -y);
+    const float lost2 = __builtin_fmaf(c, -1.92596299e-8f, lost);   // log2 e - 1.44269504f
+    float t = __builtin_amdgcn_exp2f(y);
+    t = __builtin_fmaf(t, __fmul_rn(lost2, 0.693147181f), t);
+    const float den = __fadd_rn(1.0f, t);
+    float r = __builtin_amdgcn_rcpf(den);
+    r = __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
+    return __fmul_rn(x, x < -87.0f ? 0.0f : r);
+}
+
+// The same value, computed again: what is derived from it does not keep a register through the loop.
+__device__ inline int again(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 }  // namespace mummu

@@ -1,4 +1,4 @@
-"""The grouped GEMM of Q4_K banks on tiles of up to 64 rows: experts whose rows end just before, at and just after each half of a tile,
+"""The grouped GEMMs of Q4_K banks on tiles of up to 64 and of up to 16 rows: experts whose rows end just before, at and just after each half of a tile,
 among experts without rows, against the f64 product of the dequantized weights.  One super-block to a row (the shortest loop over
 K), an odd number of them, and a last slab of columns that is half a slab.  The tolerance is the 3e-5 of the other
 Q4_K forms on these units."""
@@ -11,12 +11,13 @@ from oracle import binding as orc
 
 pytestmark = pytest.mark.gpu
 
-COUNTS = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 0, 2]
+COUNTS = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 0, 2]
 
 
-@pytest.mark.parametrize("down", [M.Q4_K, M.Q8_0])
+@pytest.mark.parametrize("down,tile_rows", [(M.Q4_K, 64), (M.Q4_K, 16), (M.Q8_0, 64)])
 @pytest.mark.parametrize("H,I", [(256, 256), (768, 512), (2048, 768)])
-def test_every_tile_edge_matches_the_f64_reference(H, I, down):
+def test_every_tile_edge_matches_the_f64_reference(monkeypatch, H, I, down, tile_rows):
+    monkeypatch.setenv("MUMMU_GEMM_TILE_ROWS", str(tile_rows))
     E, n = len(COUNTS), sum(COUNTS)
     rng = np.random.Generator(np.random.PCG64(H))
     gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (31, 32))
