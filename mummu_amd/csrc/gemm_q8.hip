@@ -2,21 +2,29 @@
 // is a half as it is, and a block's 32 products are summed by v_mfma_f32_32x32x16_f16 into one f32 accumulator, hi and lo
 // halfs alike; what is left for the vector ALUs is one multiply-add per output and block, with the block's scale.
 //
-// What bounds it: the stream of the weights, if it gets into the CU.  Blocks of 34 bytes loaded by the lanes that multiply them
-// (dwords of 64 rows a load) kept the address units busy: one line a lane and load, and the int8 form took 170 us for a layer whose
-// bytes take 75, whatever the batch; 16 bytes a lane straight into registers took 237.  Here a row's 136 bytes of a
-// stage (128 elements) come in one piece, 64 neighbouring dwords a load, straight into LDS, two stages ahead: 141 us (OLMoE layer, 19
-// to 100 tokens; 150: 204 -> 153, 512: 350 -> 294; each byte is fetched once, 295 MB of 285 at 3.5 TB/s with the vector ALUs busy for 29 %
-// of the cycles and the matrix units for 18, profiles/listed_work_counters.txt), 2.5e-7 off the 64-bit result where the int8 form is by 4.5e-5.
+// What bounds it: the stream of the weights and, not wholly beside it, the CU's own work (with every tile on one expert's weights, out
+// of L2, gate/up of the layer below still takes 59 us of its 75; its bytes take 50).  Blocks of 34 bytes loaded by the lanes that
+// multiply them kept the address units busy (int8 form: 170 us for a layer whose bytes take 75), 16 bytes a lane straight into
+// registers took 237.  Here a stage of a row (128 elements, 136 bytes) comes as the aligned pieces of 16 bytes that hold it, straight into LDS,
+// two stages ahead, the loads dealt over the products of a stage: a burst behind the barrier stalls all waves at the address units.
+// A workgroup fills a CU's LDS, so what it does outside the loop is not hidden by another: it takes several items, and loads for the
+// next while it stores the last.  A piece read by 16 lanes, 9 pieces a row, meets all banks of LDS; codes taken from there by dwords
+// met a quarter.  OLMoE layer, 150 tokens, gate/up + down, us: dwords loaded in a burst 86 + 47; pieces, dealt 80.5 + 45.5; several items 75.2 +
+// 42.5; whole pieces read 74 + 41 (the layer: 152, 147, 142, 139.5; 16 tokens 134 -> 117, 512: 296 -> 255, 1000: 491 -> 412).
+// Fetched once: 296 MB of 285.  Tried: half the rows of a stage and two workgroups a CU (84.7 + 60.2: more streams than L2 holds lines
+// for, 385 MB); a wave for one block of a stage and 128 columns, a quarter of the reads of rows (81.1 + 54.8: sums exchanged at the end).
+// Off the 64-bit result by 2.5e-7 where the int8 form is by 4.5e-5.
 //
 // x has one scale for its whole row (HAct): an element is off by at most 2^-34 of the row's largest, where the int8 form's is off
 // by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of their own and
 // meet weights of 0: a block 2^20 (2^26) above the rest 1.0e-4 (6.4e-3) off the 64-bit result, the int8 form 4.6e-5.  A single element
 // 2^20 above it, its weights 0: 5.0e-5, the int8 form, which loses its 63 neighbours, 2.4e-1; weights as they come: 3.3e-7 and 3.1e-5.
 //
-// A workgroup has 256 weight rows (128 of gate and 128 of up), a wave 32 of them, which it loads for itself; the activation tile is
-// shared.  Lane (column c, K group g) reads 16 of a block's 32 codes, so element 16 g + 8 kk + i of the block is the K index
+// An item is a tile by 256 weight rows (128 of gate and 128 of up), a wave has 32 of them, which it loads for itself; the activation tile
+// is shared.  Lane (column c, K group g) reads 16 of a block's 32 codes, so element 16 g + 8 kk + i of the block is the K index
 // 8 g + i of its product kk, and the A operands are read from the tile to match.
+#include <type_traits>
+
 #include "device_utils.h"
 #include "kernels.h"
 #include "qact.h"
@@ -32,13 +40,14 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 constexpr int kRows = 32;                    // rows of a tile
 constexpr int kWaves = 8, kWCols = 32 * kWaves;
 constexpr int kStep = 128, kBlocks = 4;      // K elements and blocks of a stage
-constexpr int kRowW = 136;                   // bytes of a weight row's stage, in memory and in LDS
-constexpr int kWLoads = 32 * kRowW / 256;    // loads of a wave's weights: 64 dwords each
-constexpr int kWaveW = 32 * kRowW, kStageW = kWaves * kWaveW, kRing = 3;
+constexpr int kRowW = 136;                   // bytes of a weight row's stage
+constexpr int kWLoads = 5;                   // loads of a wave's weights: 64 pieces of 16 bytes each
+constexpr int kWaveW = kWLoads * 1024, kStageW = kWaves * kWaveW, kRing = 3;
 constexpr int kPlane = kRows * kStep * 2, kStageA = 2 * kPlane;   // hi, lo: [row][16 pieces of 16 bytes]
 constexpr int kLdsBytes = kRing * kStageW + 2 * kStageA;
+constexpr int kCusOfXcd = 32;               // (a workgroup fills a CU)
 constexpr int kRowC = 128 + 4;               // f32 row of the gate/up epilogue
-static_assert(32 * kRowW % 256 == 0 && 2 * kRows * kRowC * 4 <= kLdsBytes, "whole loads; the epilogue fits the stages");
+static_assert(2 * kRows * kRowC * 4 <= kStageW, "the epilogue fits a stage's weights");
 
 // Eight codes as halfs, in the element order of HAct: a byte b ^ 0x80 under 0x64 is the half 1024 + 128 + b.
 __device__ inline half8 q8_codes(uint32_t w0, uint32_t w1) {
@@ -57,145 +66,263 @@ __device__ inline half8 q8_codes(uint32_t w0, uint32_t w1) {
 
 // GATE_UP: a = the token rows gathered through `sorted`, one scale per row; silu(g) * u leaves as HAct in sorted order.
 // else   : a in sorted order, a scale per 128 elements; y[pos, n] = f32 sum.
-template <bool GATE_UP>
+// PIECES: the aligned pieces of 16 bytes that hold a row's 136 of a stage: nine where rows begin at a multiple of 16 (stages then begin
+// there or 8 past it), else ten.
+template <bool GATE_UP, int PIECES>
 __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, HAct a,
                                                                          const int32_t *__restrict__ sorted, int k_slots,
                                                                          const int32_t *__restrict__ tiles, const int32_t *__restrict__ n_tiles,
                                                                          int in_dim, int out_dim, HAct act, float *__restrict__ y) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // [kRing][kStageW], then [2][kStageA]
-    __shared__ __attribute__((aligned(16))) float s_as[2][64];        // row scales (gate/up: [0], else of a stage), twice
-    // as xcd_tile in gemm.hip: an XCD takes neighbouring tiles, the slab running fastest
+    __shared__ __attribute__((aligned(16))) float s_as[2][64];        // row scales (gate/up: of an item, else of a stage), twice
+    __shared__ int32_t s_idx[2][64];                                  // an item's entries of `sorted`, twice
+    // as xcd_tile in gemm.hip: an XCD takes neighbouring tiles, the slab running fastest; here a workgroup takes every
+    // gridDim.x / 8 -th of its XCD's items, and its loads run on from one into the next
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
     const int n_slabs = (out_dim + kCols - 1) / kCols;
-    const int total = *n_tiles, per_xcd = (total + 7) >> 3;
-    const int item = (int)(blockIdx.x >> 3), within = item / n_slabs, slab = item - within * n_slabs;
-    const int tile = (int)(blockIdx.x & 7) * per_xcd + within;
-    if (within >= per_xcd || tile >= total) return;
-    const int e = uniform(tiles[3 * tile]), p0 = uniform(tiles[3 * tile + 1]), rows = uniform(tiles[3 * tile + 2]);
+    const int total = *n_tiles, per_xcd = (total + 7) >> 3, tile0 = (int)(blockIdx.x & 7) * per_xcd;
+    const int n_items = n_slabs * (total - tile0 < per_xcd ? total - tile0 : per_xcd), apart = (int)(gridDim.x >> 3);
+    const int first_item = (int)(blockIdx.x >> 3);
+    if (first_item >= n_items) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 31, g = lane >> 5;
     const uint32_t row_bytes = (uint32_t)(in_dim / kStep) * kRowW;
     const uint32_t lds0 = lds_offset(s_lds);
-    const uint32_t lds_as = lds_offset(s_as);
+    const uint32_t lds_as = lds_offset(s_as), lds_idx = lds_offset(s_idx);
     const int n_steps = in_dim / kStep;
-
+    auto expert_of = [&](int item) { return uniform(tiles[3 * (tile0 + item / n_slabs)]); };
+    auto start_of = [&](int item) { return uniform(tiles[3 * (tile0 + item / n_slabs) + 1]); };
+    auto rows_of = [&](int item) { return uniform(tiles[3 * (tile0 + item / n_slabs) + 2]); };
     // this wave's weight rows: first .. first + 31 of gate (waves 0-3), up (4-7) or down
-    const int first = slab * kCols + 32 * (GATE_UP ? wave & 3 : wave);
-    const uint8_t *w_base = uniform((GATE_UP && wave >= 4 ? w1 : w0) + (size_t)e * (size_t)out_dim * row_bytes);
-    // (columns past the matrix repeat its last, rows past the tile's end its last: multiplied, never stored)
-    uint32_t w_off[kWLoads];
+    auto first_of = [&](int item) { return item % n_slabs * kCols + 32 * (GATE_UP ? wave & 3 : wave); };
+
+    // Where the loads stand: an item and its stage, for the weights (two stages ahead of the products) and for the rows (one).
+    // Past the last item they stay at its last stage, never multiplied.
+    int w_item = first_item, w_step = 0, a_item = first_item, a_step = 0, w_flip = 0, a_flip = 0;
+    const uint8_t *w_base = nullptr;
+    uint32_t w_off[kWLoads], a_off = 0, s_off = 0;
+    // (columns past the matrix repeat its last, rows past the tile's end its last: multiplied, never stored; the lanes past the
+    // last piece repeat it)
+    auto set_w = [&]() {
+        const int first = first_of(w_item);
+        w_base = uniform((GATE_UP && wave >= 4 ? w1 : w0) + (size_t)expert_of(w_item) * (size_t)out_dim * row_bytes);
 #pragma unroll
-    for (int j = 0; j < kWLoads; j++) {
-        const int d = 64 * j + lane, col = first + d / (kRowW / 4);
-        w_off[j] = (uint32_t)(col < out_dim ? col : out_dim - 1) * row_bytes + (uint32_t)(d % (kRowW / 4)) * 4u;
-    }
-    auto source_row = [&](int r) {
-        r = r < rows ? r : rows - 1;
-        return (uint32_t)(GATE_UP ? sorted[p0 + r] / k_slots : p0 + r);
+        for (int j = 0; j < kWLoads; j++) {
+            const int piece = 64 * j + lane < 32 * PIECES ? 64 * j + lane : 32 * PIECES - 1, col = first + piece / PIECES;
+            w_off[j] = ((uint32_t)(col < out_dim ? col : out_dim - 1) * row_bytes & ~15u) + (uint32_t)(piece % PIECES) * 16u;
+        }
+        if (GATE_UP) {
+            const int rows = rows_of(w_item);
+            load_to_lds4(lds_idx + (uint32_t)w_flip * 256u, (const uint8_t *)(sorted + start_of(w_item)), (uint32_t)(c < rows ? c : rows - 1) * 4u);
+        }
     };
     // Activation pieces: load `wave` of each plane holds four rows.  Piece q of row r lies at q ^ (r % 16): sixteen lanes that read
     // the same piece of neighbouring rows meet all banks.
     const int a_row = 4 * wave + (lane >> 4);
-    const uint32_t a_off = source_row(a_row) * (uint32_t)in_dim * 2u + (uint32_t)((lane & 15) ^ (a_row & 15)) * 16u;
-    const uint32_t s_off = source_row(c) * (uint32_t)(in_dim / 128) * 4u;
-    auto load_w = [&](int step) {
-        const uint32_t at = lds0 + (uint32_t)(step % kRing) * kStageW + (uint32_t)wave * kWaveW;
-        const uint8_t *base = w_base + (size_t)step * kRowW;
-#pragma unroll
-        for (int j = 0; j < kWLoads; j++) load_to_lds4(at + 256 * j, base, w_off[j]);
+    auto set_a = [&]() {
+        auto source_row = [&](int r) {
+            if (GATE_UP) return (uint32_t)(s_idx[a_flip][r] / k_slots);
+            const int rows = rows_of(a_item);
+            return (uint32_t)(start_of(a_item) + (r < rows ? r : rows - 1));
+        };
+        a_off = source_row(a_row) * (uint32_t)in_dim * 2u + (uint32_t)((lane & 15) ^ (a_row & 15)) * 16u;
+        s_off = source_row(c) * (uint32_t)(in_dim / 128) * 4u;
+        if (GATE_UP) load_to_lds4(lds_as + (uint32_t)a_flip * 256u, (const uint8_t *)a.scale, s_off);
     };
-    auto load_a = [&](int step) {
-        const uint32_t at = lds0 + kRing * kStageW + (uint32_t)(step & 1) * kStageA + (uint32_t)wave * 1024u;
-        load_to_lds16(at, (const uint8_t *)a.hi + (size_t)step * (kStep * 2), a_off);
-        load_to_lds16(at + kPlane, (const uint8_t *)a.lo + (size_t)step * (kStep * 2), a_off);
-        if (!GATE_UP) load_to_lds4(lds_as + (uint32_t)(step & 1) * 256u, (const uint8_t *)a.scale + (size_t)step * 4, s_off);   // (every wave the same)
+    auto next_w = [&]() {
+        if (++w_step < n_steps) return;
+        if (w_item + apart < n_items) {
+            w_item += apart, w_step = 0, w_flip ^= 1;
+            set_w();
+        } else {
+            w_step = n_steps - 1;
+        }
     };
-    if (GATE_UP && tid < 64) s_as[0][tid] = *(const float *)((const uint8_t *)a.scale + s_off);
+    auto next_a = [&]() {
+        if (++a_step < n_steps) return;
+        if (a_item + apart < n_items) {
+            a_item += apart, a_step = 0, a_flip ^= 1;
+            set_a();
+        } else {
+            a_step = n_steps - 1;
+        }
+    };
+    // one load each
+    auto load_w = [&](uint32_t slot, int j) {
+        load_to_lds16(lds0 + slot + (uint32_t)wave * kWaveW + 1024 * j, w_base + ((size_t)(w_step >> 1) * (2 * kRowW) + (size_t)(w_step & 1) * (kRowW - 8)),
+                      w_off[j]);
+    };
+    auto load_a = [&](int which, int i) {
+        const uint32_t at = lds0 + kRing * kStageW + (uint32_t)which * kStageA + (uint32_t)wave * 1024u;
+        if (i == 0) load_to_lds16(at, (const uint8_t *)a.hi + (size_t)a_step * (kStep * 2), a_off);
+        else if (i == 1) load_to_lds16(at + kPlane, (const uint8_t *)a.lo + (size_t)a_step * (kStep * 2), a_off);
+        else load_to_lds4(lds_as + (uint32_t)which * 256u, (const uint8_t *)a.scale + (size_t)a_step * 4, s_off);   // (every wave the same)
+    };
+    constexpr int kALoads = GATE_UP ? 2 : 3;
+    set_w();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    set_a();
+#pragma unroll
+    for (int j = 0; j < kWLoads; j++) load_w(0, j);
+#pragma unroll
+    for (int i = 0; i < kALoads; i++) load_a(0, i);
+    next_w();
+#pragma unroll
+    for (int j = 0; j < kWLoads; j++) load_w(kStageW, j);
 
     const float16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    float16v acc = zero;
-    load_w(0);
-    load_a(0);
-    if (n_steps > 1) load_w(1);
-    for (int step = 0; step < n_steps; step++) {
-        // everything but the next stage's weights is there, for this wave; then, the activations, for everybody, who are also
-        // done with the tile of the step before
-        if (step + 1 < n_steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (step + 1 < n_steps) load_a(step + 1);
-        if (step + 2 < n_steps) load_w(step + 2);
-        const uint8_t *ws = s_lds + (uint32_t)(step % kRing) * kStageW + (uint32_t)wave * kWaveW + (uint32_t)c * kRowW + 16u * (uint32_t)g;
-        const uint8_t *ds = ws - 16u * (uint32_t)g;
-        const uint8_t *as = s_lds + kRing * kStageW + (uint32_t)(step & 1) * kStageA + (uint32_t)c * (kStep * 2);
-        float16v run = zero;
+    // what a block's products take: 16 codes and the scale, the rows' pieces; of this block and of the next
+    uint32_t v[2][8];
+    float d[2];
+    half8 hi[2][2], lo[2][2];
+    const uint32_t w_rd = (uint32_t)wave * kWaveW + (uint32_t)c * (16 * PIECES) + (PIECES == 9 ? 0u : (uint32_t)c * row_bytes & 8u);
+    auto read = [&](uint32_t slot, int odd, int which, int blk) {   // (odd: of the stage, known where PIECES is 9)
+        const uint8_t *ds = s_lds + slot + w_rd + 8u * (uint32_t)odd;
+        const int at = 34 * blk + 2, n = blk & 1;
+        if (PIECES == 9) {
+            // (sixteen lanes that read a piece each, rows of 9 pieces apart, meet all banks)
+            const uint8_t *from = s_lds + slot + w_rd + 16u * (uint32_t)g + (uint32_t)((at + 8 * odd) & ~15);
+            __builtin_memcpy(v[n], __builtin_assume_aligned(from, 16), 16);
+            if ((at + 8 * odd) & 15) __builtin_memcpy(v[n] + 4, __builtin_assume_aligned(from + 16, 16), 16);
+        } else {
 #pragma unroll
-        for (int blk = 0; blk < kBlocks; blk++) {
-            // 16 codes from byte 34 blk + 2 on: two bytes into a dword in every other block
-            constexpr int kDwords = 5;
-            uint32_t v[kDwords], q[4];
-            const int at = 34 * blk + 2, off = at & ~3;
-#pragma unroll
-            for (int i = 0; i < ((at & 2) ? 5 : 4); i++) v[i] = *(const uint32_t *)(ws + off + 4 * i);
-#pragma unroll
-            for (int i = 0; i < 4; i++) q[i] = (at & 2) ? __builtin_amdgcn_alignbyte(v[i + 1], v[i], 2) : v[i];
-            const float d = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
-            const half8 w[2] = {q8_codes(q[0], q[1]), q8_codes(q[2], q[3])};
-            float16v s = zero;
-#pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                const uint8_t *piece = as + (uint32_t)(((4 * blk + 2 * g + kk) ^ (c & 15)) * 16);
-                const half8 hi = *(const half8 *)piece, lo = *(const half8 *)(piece + kPlane);
-                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, w[kk], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, w[kk], s, 0, 0, 0);
-            }
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                if (GATE_UP) acc[r] = fmaf(d, s[r], acc[r]);
-                else run[r] = blk == 0 ? __fmul_rn(d, s[r]) : fmaf(d, s[r], run[r]);
-            }
+            for (int i = 0; i < ((at & 2) ? 5 : 4); i++) v[n][i] = *(const uint32_t *)(ds + 16u * (uint32_t)g + (at & ~3) + 4 * i);
         }
-        if (!GATE_UP) {
+        d[n] = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
+        const uint8_t *as = s_lds + kRing * kStageW + (uint32_t)which * kStageA + (uint32_t)c * (kStep * 2);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float4 s4 = *(const float4 *)&s_as[step & 1][8 * j + 4 * g];
-                const float sr[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[4 * j + i] = fmaf(run[4 * j + i], sr[i], acc[4 * j + i]);
-            }
+        for (int kk = 0; kk < 2; kk++) {
+            const uint8_t *piece = as + (uint32_t)(((4 * blk + 2 * g + kk) ^ (c & 15)) * 16);
+            hi[n][kk] = *(const half8 *)piece;
+            lo[n][kk] = *(const half8 *)(piece + kPlane);
         }
-    }
-
+    };
+    // a block's sum -> acc, or (down) the 128 elements' sum
+    float16v acc = zero, run = zero, s[2] = {zero, zero};
+    float fd = 0.0f;
+    auto fold = [&](int n, int blk) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            if (GATE_UP) acc[r] = fmaf(fd, s[n][r], acc[r]);
+            else run[r] = blk == 0 ? __fmul_rn(fd, s[n][r]) : fmaf(fd, s[n][r], run[r]);
+        }
+    };
+    // the stage's row scales, read in front of its last barrier: the stage after the next lands in their place
+    float4 sr[4] = {};
+    auto read_scales = [&](int which) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) sr[j] = *(const float4 *)&s_as[which][8 * j + 4 * g];
+    };
+    auto fold_run = [&]() {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float f[4] = {sr[j].x, sr[j].y, sr[j].z, sr[j].w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[4 * j + i] = fmaf(run[4 * j + i], f[i], acc[4 * j + i]);
+        }
+    };
     // element r of an accumulator: row 8 (r / 4) + 4 g + r % 4, column lane % 32
     auto acc_row = [&](int r) { return 8 * (r >> 2) + 4 * g + (r & 3); };
-    if (GATE_UP) {
-        __syncthreads();   // (the stages are done with)
-        float *s_c = (float *)s_lds;   // [gate, up][row][kRowC]
+
+    // the first stage is there; its first block
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
+    read(0, 0, 0, 0);
+    uint32_t slot = 0;   // of the stage's weights
+    int which = 0;       // of its rows
+    for (int item = first_item, flip = 0; item < n_items; item += apart, flip ^= 1) {
+        auto stage = [&](int step, auto odd) {
+            const uint32_t slot1 = slot == (kRing - 1) * kStageW ? 0 : slot + kStageW, slot2 = slot1 == (kRing - 1) * kStageW ? 0 : slot1 + kStageW;
+            next_a();
+            next_w();
 #pragma unroll
-        for (int r = 0; r < 16; r++) s_c[((wave >> 2) * kRows + acc_row(r)) * kRowC + 32 * (wave & 3) + c] = __fmul_rn(s_as[0][acc_row(r)], acc[r]);
-        __syncthreads();
+            for (int blk = 0; blk < kBlocks; blk++) {
+                const int n = blk & 1;
+                // In front of a stage's last products: everything but the weights of the stage after the next is there, for this
+                // wave; then, the activations, for everybody, who have also read this stage's.
+                if (blk == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
+                // beside the first three, a few at a time: the next step's rows, then the weights of the one after
+                if (blk == 0) {
 #pragma unroll
-        for (int pass = 0; pass < kRows / 16; pass++) {
-            const int row = 16 * pass + (tid >> 5), at = row * kRowC + 4 * (tid & 31);
-            const float4 gv = *(const float4 *)&s_c[at], uv = *(const float4 *)&s_c[kRows * kRowC + at];
-            const float4 v = make_float4(__fmul_rn(det_silu(gv.x), uv.x), __fmul_rn(det_silu(gv.y), uv.y), __fmul_rn(det_silu(gv.z), uv.z),
-                                         __fmul_rn(det_silu(gv.w), uv.w));
-            const bool active = row < rows;
-            hact_store128(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, act, (size_t)(p0 + row), out_dim, slab * kCols + 4 * (tid & 31));
+                    for (int i = 0; i < kALoads; i++) load_a(which ^ 1, i);
+                } else if (blk < 3) {
+#pragma unroll
+                    for (int j = 3 * blk - 3; j < 3 * blk && j < kWLoads; j++) load_w(slot2, j);
+                }
+                const float now = d[n];
+                uint32_t q[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    // (codes begin two bytes into a dword in every other block)
+                    const int at = 34 * blk + 2, j = i + (PIECES == 9 ? ((at + 8 * odd) & 15) >> 2 : 0);
+                    q[i] = (at & 2) ? __builtin_amdgcn_alignbyte(v[n][j + 1], v[n][j], 2) : v[n][j];
+                }
+                const half8 w[2] = {q8_codes(q[0], q[1]), q8_codes(q[2], q[3])};
+                const half8 h[2] = {hi[n][0], hi[n][1]}, l[2] = {lo[n][0], lo[n][1]};
+                if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1);
+                else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0);
+#pragma unroll
+                for (int kk = 0; kk < 2; kk++) {
+                    s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[kk], w[kk], kk == 0 ? zero : s[n], 0, 0, 0);
+                    s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l[kk], w[kk], s[n], 0, 0, 0);
+                }
+                // the block before this one, while these are multiplied
+                fold(n ^ 1, (blk + 3) & 3);
+                if (!GATE_UP && blk == 0) fold_run();
+                if (!GATE_UP && blk == 2) read_scales(which);
+                fd = now;
+            }
+            slot = slot1;
+            which ^= 1;
+        };
+        for (int step = 0; step < n_steps;) {
+            stage(step++, std::integral_constant<int, 0>());
+            if (PIECES == 9) stage(step++, std::integral_constant<int, 1>());   // (stages come in pairs)
         }
-    } else if (first + c < out_dim) {
+        fold(1, 3);
+        if (!GATE_UP) fold_run();
+        const int p0 = start_of(item), rows = rows_of(item);
+        if (GATE_UP) {
+            // (the last stage's weights are read: their place is free until the loads beside the next item's products)
+            float *s_c = (float *)(s_lds + (slot == 0 ? (kRing - 1) * kStageW : slot - kStageW));   // [gate, up][row][kRowC]
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-            if (acc_row(r) < rows) y[(size_t)(p0 + acc_row(r)) * (size_t)out_dim + (size_t)(first + c)] = acc[r];
+            for (int r = 0; r < 16; r++) s_c[((wave >> 2) * kRows + acc_row(r)) * kRowC + 32 * (wave & 3) + c] = __fmul_rn(s_as[flip][acc_row(r)], acc[r]);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+            for (int pass = 0; pass < kRows / 16; pass++) {
+                const int row = 16 * pass + (tid >> 5), at = row * kRowC + 4 * (tid & 31);
+                const float4 gv = *(const float4 *)&s_c[at], uv = *(const float4 *)&s_c[kRows * kRowC + at];
+                const float4 r = make_float4(__fmul_rn(det_silu(gv.x), uv.x), __fmul_rn(det_silu(gv.y), uv.y), __fmul_rn(det_silu(gv.z), uv.z),
+                                             __fmul_rn(det_silu(gv.w), uv.w));
+                const bool active = row < rows;
+                hact_store128(active ? r : make_float4(0.f, 0.f, 0.f, 0.f), active, act, (size_t)(p0 + row), out_dim,
+                              item % n_slabs * kCols + 4 * (tid & 31));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else {
+            const int col = first_of(item) + c;
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (col < out_dim && acc_row(r) < rows) y[(size_t)(p0 + acc_row(r)) * (size_t)out_dim + (size_t)col] = acc[r];
+        }
+        acc = run = s[1] = zero;
+        fd = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) sr[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load into LDS is under way when the workgroup ends)
 }
 
 template <bool GATE_UP>
 hipError_t launch_q8(const uint8_t *w0, const uint8_t *w1, HAct a, const int32_t *sorted, int k_slots, const int32_t *tiles,
                      const int32_t *n_tiles, int max_tiles, int in_dim, int out_dim, HAct act, float *y, hipStream_t s) {
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
-    const dim3 grid((unsigned)((max_tiles + 7) / 8 * 8) * (unsigned)((out_dim + kCols - 1) / kCols));
-    launch_kernel(grouped_gemm_q8_kernel<GATE_UP>, grid, dim3(64 * kWaves), kLdsBytes, s, w0, w1, a, sorted, k_slots, tiles, n_tiles, in_dim,
-                  out_dim, act, y);
+    const int per_xcd = (max_tiles + 7) / 8 * ((out_dim + kCols - 1) / kCols);
+    const dim3 grid(8u * (unsigned)(per_xcd < kCusOfXcd ? per_xcd : kCusOfXcd));
+    if (in_dim % (2 * kStep) == 0)
+        launch_kernel(grouped_gemm_q8_kernel<GATE_UP, 9>, grid, dim3(64 * kWaves), kLdsBytes, s, w0, w1, a, sorted, k_slots, tiles, n_tiles,
+                      in_dim, out_dim, act, y);
+    else
+        launch_kernel(grouped_gemm_q8_kernel<GATE_UP, 10>, grid, dim3(64 * kWaves), kLdsBytes, s, w0, w1, a, sorted, k_slots, tiles, n_tiles,
+                      in_dim, out_dim, act, y);
     return hipGetLastError();
 }
 

@@ -30,6 +30,9 @@ const char *const kSlotNames[K_SLOTS] = {"router", "router_logits", "route_topk"
                                          "down", "combine", "rmsnorm", "dispatch", "gemm_gate_up", "gemm_down", "shared_expert",
                                          "decode_layer"};
 
+// Kernels read a bank's rows in whole aligned pieces of 16 bytes: up to 24 bytes past its last row.
+constexpr size_t kBankSlack = 32;
+
 struct Layer {
     void *router = nullptr;
     int router_type = 0;
@@ -497,21 +500,19 @@ struct HalfPlan {
 };
 
 // Which Q8_0 batches take the 32-row tiles of gemm_q8.hip and which the int8 form's 64-row ones, by the rows of an expert.  Layers of
-// 64 / 128 / 512 experts (hidden x inter 2048 x 1024, 2048 x 768, 2560 x 640) and 16 (4096 x 1792), us here / int8:
-//   up to 33 rows next to none needs a second tile: 16 rows 142 / 179, 216 / 271, 917 / 990, 236 / 315; 33: 224 / 217, 331 / 363, 1386 /
-//   1400, 324 / 364.
-//   While a tile of 64 holds every expert the int8 form reads the weights once: 40 rows 237 / 228, 372 / 374, 1595 / 1477, 364 / 428;
-//   42: 237 / 228, 378 / 384.
-//   Beyond, some need a second one.  In a launch of a few rounds of workgroups that is another round for all: 44 rows 238 / 311, 381 /
-//   383, 381 / 448; 64: 289 / 347, 473 / 530, 496 / 562; 80: 334 / 387, 564 / 622, 517 / 577.  In one of many rounds it costs what it
-//   weighs, and the two are nearly alike from where half the experts do: 512 experts, 52 rows 1889 / 1778, 64: 2277 / 2254, 80: 2743 / 2746.
-//   From 90 rows on the weights are read more often here: 96 rows 392 / 376, 636 / 632, 607 / 602; 128: 495 / 495, 785 / 775, 759 / 858;
-//   160: 575 / 556, 973 / 937, 937 / 923.  Up to 190 the pairs of halfs, a hundred times nearer the 64-bit result, are kept for these few
-//   per cent; at 256 rows it is 6 (871 / 823, 1394 / 1299, 1307 / 1245).
+// 64 / 128 experts (hidden x inter 2048 x 1024, 2048 x 768), 16 (4096 x 1792) and 512 (2560 x 640, whose rows come in ten pieces), us here / int8:
+//   up to 33 rows next to none needs a second tile: 16 rows 138 / 181, 201 / 273, 232 / 316, 844 / 985; 33: 201 / 218, 291 / 364, 301 / 379, 1279 / 1400.
+//   While a tile of 64 holds every expert the int8 form reads the weights once: 40 rows 207 / 225, 319 / 376, 329 / 419, 1496 / 1509.  A layer on
+//   its own is still faster here, by what the int8 form waits; where other streams fill that (three of them, 64 experts, 37 rows: 179 / 176 a
+//   layer) it is not, and the bytes decide.
+//   Beyond, some need a second one: 54 rows 512 experts 1777 / 1841; 64: 257 / 353, 405 / -, 449 / 548, 2142 / 2250; 128: 424 / 512, 670 / -, 636 / 808.
+//   From 190 rows on: 192 rows 572 / 665, 934 / 1066, 951 / 1062; 512: 1361 / 1462, -, 2208 / 2331 (three streams 1400 / 1399), a hundred times nearer the
+//   64-bit result.  Rows in ten pieces are behind there (512 experts, 128 rows 3998 / 3861, 160: 4995 / 4686) and keep the int8 form.
 bool q8_gemm_should(const ExpertBanks &b, size_t n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const size_t workgroups = (size_t)b.n_experts * (size_t)(b.inter / 128);   // of a gate/up launch with a tile per expert
-    return avg <= 33.0 || (avg + (workgroups <= 1024 ? 3.2 : 2.2) * __builtin_sqrt(avg) >= 64.0 && avg <= 190.0);
+    const bool nine_pieces = b.hidden % 256 == 0 && b.inter % 256 == 0;
+    return avg <= 33.0 || (avg + (workgroups <= 1024 ? 3.2 : 2.2) * __builtin_sqrt(avg) >= 64.0 && (avg <= 190.0 || nine_pieces));
 }
 
 // (one_expert: all n rows go to the same one)
@@ -1215,9 +1216,9 @@ int mummu_moe_load_layer(mummu_moe *h, int layer, const void *router, int router
     const size_t ub = (size_t)E * (size_t)I * row_bytes_of(up_type, H);
     const size_t db = (size_t)E * (size_t)H * row_bytes_of(down_type, I);
     HIPCHK(h, hipMalloc(&L.router, rb));
-    HIPCHK(h, hipMalloc(&L.gate, gb));
-    HIPCHK(h, hipMalloc(&L.up, ub));
-    HIPCHK(h, hipMalloc(&L.down, db));
+    HIPCHK(h, hipMalloc(&L.gate, gb + kBankSlack));
+    HIPCHK(h, hipMalloc(&L.up, ub + kBankSlack));
+    HIPCHK(h, hipMalloc(&L.down, db + kBankSlack));
     HIPCHK(h, hipMalloc(&L.hits, sizeof(unsigned long long) * (size_t)E));
     HIPCHK(h, hipMemcpy(L.router, router, rb, hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(L.gate, gate, gb, hipMemcpyHostToDevice));
@@ -1285,9 +1286,9 @@ int mummu_moe_load_shared_expert(mummu_moe *h, int layer, int inter, const void 
     L.sh_bytes = 0;
     const size_t gb = (size_t)inter * row_bytes_of(gate_type, H), db = (size_t)H * row_bytes_of(down_type, inter);
     const size_t vb = gate_vec ? (size_t)H * (size_t)block_bytes(gate_vec_type) : 0;
-    HIPCHK(h, hipMalloc(&L.sh_gate, gb));
-    HIPCHK(h, hipMalloc(&L.sh_up, gb));
-    HIPCHK(h, hipMalloc(&L.sh_down, db));
+    HIPCHK(h, hipMalloc(&L.sh_gate, gb + kBankSlack));
+    HIPCHK(h, hipMalloc(&L.sh_up, gb + kBankSlack));
+    HIPCHK(h, hipMalloc(&L.sh_down, db + kBankSlack));
     HIPCHK(h, hipMemcpy(L.sh_gate, gate, gb, hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(L.sh_up, up, gb, hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(L.sh_down, down, db, hipMemcpyHostToDevice));

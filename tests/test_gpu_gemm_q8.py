@@ -104,3 +104,24 @@ def test_the_form_by_rows_per_expert(E, I, rows, pairs):
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids[:E], w[:E], x[:E])
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err <= 2e-3 and (err <= 3e-6) == pairs, err
+
+
+# More items (tiles by 128 rows of gate and up, or 256 of down) than workgroups, so that loads run on from one item into the next:
+# rows of one, two, three, five and eight stages, a last slab that is half one; and more rows per expert than ragged shapes
+# keep in this form.
+@pytest.mark.parametrize("H,I,scale", [(128, 384, 1), (768, 128, 1), (640, 384, 1), (1024, 256, 1), (512, 768, 1), (256, 512, 8)])
+def test_workgroups_of_several_items_match_the_f64_reference(H, I, scale):
+    counts = np.array([0, 1, 16, 31, 32, 33, 64, 65, 0, 2] * (8 if scale == 1 else 2)) * scale
+    E = len(counts)
+    gate, up = (synth.random_bank_fast(M.Q8_0, [H, I, E], seed) for seed in (11, 12))
+    down = synth.random_bank_fast(M.Q8_0, [I, H, E], 13)
+    g = np.random.default_rng(H + I)
+    ids = g.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    n = len(ids)
+    x, w = g.standard_normal((n, H)).astype(np.float32) * np.exp2(g.integers(-12, 1, (n, 1))).astype(np.float32), g.random((n, 1)).astype(np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got, again = m.apply_routing(0, ids, w, x), m.apply_routing(0, ids, w, x)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids, w, x)
+    assert orc.rel_err(got, want, mag).max() <= 3e-5
