@@ -186,6 +186,11 @@ __device__ inline uint32_t lds_offset(const void *shared) {
 __device__ inline void load_to_lds16(uint32_t lds, const uint8_t *base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(uniform((int)lds)), "v"(off), "s"(uniform(base)) : "memory");
 }
+// ... by the lanes of `low` (0-31) and `high` (32-63), of a whole wave.  (No branch: what stands around it can be moved together.)
+__device__ inline void load_to_lds16_if(uint32_t low, uint32_t high, uint32_t lds, const uint8_t *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(uniform((int)lds)),
+                 "v"(off), "s"(uniform(base)), "s"(uniform((int)low)), "s"(uniform((int)high)) : "memory");
+}
 // ... from an address of each lane's own.
 __device__ inline void load_to_lds16(uint32_t lds, const uint8_t *from) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(uniform((int)lds)), "v"(from) : "memory");

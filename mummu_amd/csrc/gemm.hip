@@ -951,10 +951,18 @@ bool grouped_gemm_supported(const ExpertBanks &b) {
     return (f16 || grouped_gemm_quantized(b)) && b.hidden % kBK == 0 && b.inter % kBK == 0;
 }
 
-// Rows per tile.  An expert with one row more than a tile holds runs a second, almost empty tile
-// that streams its whole weight slab again, so the tile is sized to hold the average expert load
-// plus its spread (binomial: about +-sqrt(avg) per expert, 3.5 sigma here) when that fits; the f16
-// kernel goes up to 128 rows, the int8 kernel (more registers per row) to 64.
+// Tiles of `rows` rows that experts of `avg` rows on average, give or take its root, make: each.
+static double expected_tiles(double avg, double rows) {
+    const double sigma = __builtin_sqrt(avg > 1.0 ? avg : 1.0);
+    double t = 0.0;
+    for (int j = 0; j < 1024; j++) {
+        const double p = 0.5 * erfc(((double)j * rows + 0.5 - avg) / (sigma * 1.4142135623730951));
+        t += p;
+        if (p < 1e-6) break;
+    }
+    return t;
+}
+
 // Tile rows for the f16-unit Q4_K kernels: 16 (gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what they
 // have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
 // variance = mean).  Layers, 16 / 64 rows, us: in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it
@@ -963,28 +971,35 @@ bool grouped_gemm_supported(const ExpertBanks &b) {
 // 96: 97 / 95, 112 (1.27): 96 / 97.  Lists of 32 rows gained nothing between the two (96 tokens 94, 256: 132 against 129, 1000: 331 against
 // 302).
 // With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
-// products together: OLMoE Q4_K with Q6_K downs, 32 / 64 rows: 150 tokens 154 / 206 us, 230: 181 / 208, 260: 225 / 214; the
-// 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013.
+// products together: the 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013 us.
 int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8_down) {
     const int n_experts = b.n_experts;
     const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
-    const double sigma = __builtin_sqrt(avg > 1.0 ? avg : 1.0);
-    auto expected_tiles = [&](double rows) {
-        double t = 0.0;
-        for (int j = 0; j < 1024; j++) {
-            const double p = 0.5 * erfc(((double)j * rows + 0.5 - avg) / (sigma * 1.4142135623730951));
-            t += p;
-            if (p < 1e-6) break;
-        }
-        return t;
-    };
-    const double e16 = expected_tiles(16.0), e32 = expected_tiles(32.0), e64 = expected_tiles(64.0);
+    const double e16 = expected_tiles(avg, 16.0), e32 = expected_tiles(avg, 32.0), e64 = expected_tiles(avg, 64.0);
     if (int8_down) return 0.99 * e16 < e32 ? 16 : (0.69 * e32 < e64 ? 32 : 64);
     const double each = (double)n_experts * (double)((b.inter + 127) / 128);   // workgroups of a tile per expert
     const bool second_round = each * e64 <= 512.0 && each * e16 > 1.01 * 512.0;
     return !second_round && e16 < 1.25 * e64 ? 16 : 64;
 }
 
+// With a Q6_K down product on the f16 units, whose 32-row form multiplies tiles of 16 as well.  us a layer by tiles of 16 / 32 / 64 rows, OLMoE
+// shape, 128 experts of 2048 x 768 and 16 of 4096 x 1792: 8 rows per expert 101 / 112 / 129, 159 / 175 / 196, 94 / 107 / 121; 16 rows - / 118 / 132,
+// - / 183 / 206, - / 202 / 218; 18: - / 149 / 139, - / 193 / 214, - / 204 / 219; 38 (the first alone): 227 / 197 / 168.  Tiles of 16 as long as next to no
+// expert needs two, and no launch a second round of workgroups for them (10 rows: 128 / 112, 180 / 178, 237 / 200).
+int grouped_gemm_tile_rows_q6k_down(const ExpertBanks &b, int n_assign) {
+    const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
+    const double e16 = expected_tiles(avg, 16.0), e32 = expected_tiles(avg, 32.0);
+    // (workgroups of a tile per expert in the two launches, of which a CU holds two and one)
+    const double gate_up = (double)b.n_experts * (double)((b.inter + 127) / 128), down = (double)b.n_experts * (double)((b.hidden + 255) / 256);
+    auto second_round = [&](double each, double at_once) { return each * e32 <= at_once && each * e16 > 1.01 * at_once; };
+    if (e16 < 1.1 * e32 && !second_round(gate_up, 512.0) && !second_round(down, 256.0)) return 16;
+    return avg <= 16.0 ? 32 : 64;
+}
+
+// Rows per tile.  An expert with one row more than a tile holds runs a second, almost empty tile
+// that streams its whole weight slab again, so the tile is sized to hold the average expert load
+// plus its spread (binomial: about +-sqrt(avg) per expert, 3.5 sigma here) when that fits; the f16
+// kernel goes up to 128 rows, the int8 kernel (more registers per row) to 64.
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half) {
     const int max_rows = ((grouped_gemm_quantized(b) && !q8_half) || b.gate_type == T_F32) ? 64 : 128;
     const double avg = (double)n_assign / (double)n_experts;
@@ -1057,6 +1072,10 @@ bool grouped_gemm_q4k_f16_down(const ExpertBanks &b) {
     return grouped_gemm_q4k_f16(b) && b.down_type == T_Q4_K && b.inter % 256 == 0 && b.hidden % 128 == 0;
 }
 
+bool grouped_gemm_q6k_down(const ExpertBanks &b) {
+    return grouped_gemm_q4k_f16(b) && b.down_type == T_Q6_K && b.inter % 256 == 0 && b.hidden % 32 == 0;
+}
+
 template <bool GATE_UP>
 static hipError_t launch_gemm_f32(const uint8_t *w0, const uint8_t *w1, const float *a_in, const int32_t *sorted, int k_slots,
                                   const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows, int in_dim,
@@ -1110,7 +1129,7 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
     if (xh.hi != nullptr && xh.lo != nullptr) {
         if (!grouped_gemm_q4k_f16(b)) return hipErrorInvalidValue;
         const bool out_h = acth.hi != nullptr;
-        if (out_h && !grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
+        if (out_h && !grouped_gemm_q4k_f16_down(b) && !grouped_gemm_q6k_down(b)) return hipErrorInvalidValue;
         if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
         if (tile_rows > 16) return launch_q4k_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
         return launch_q4k_few_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
@@ -1156,6 +1175,10 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
     if (acth.hi != nullptr && b.down_type == T_Q8_0) {
         if (!q8_gemm_takes(b) || tile_rows != 32) return hipErrorInvalidValue;
         return launch_q8_down(b, acth, tiles, n_tiles, max_tiles, y, s);
+    }
+    if (acth.hi != nullptr && b.down_type == T_Q6_K) {
+        if (!grouped_gemm_q6k_down(b) || tile_rows > 64) return hipErrorInvalidValue;
+        return launch_q6k_down(b, acth, tiles, n_tiles, max_tiles, tile_rows, y, s);
     }
     if (acth.hi != nullptr) {
         if (!grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;

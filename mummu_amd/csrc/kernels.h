@@ -198,6 +198,8 @@ hipError_t launch_quantize_rows64(const float *x, int n, int d, QAct64 q, hipStr
 // down bank of another type the gate/up launch still writes actq.
 bool grouped_gemm_q4k_f16(const ExpertBanks &b);
 bool grouped_gemm_q4k_f16_down(const ExpertBanks &b);
+int grouped_gemm_tile_rows_q6k_down(const ExpertBanks &b, int n_assign);
+bool grouped_gemm_q6k_down(const ExpertBanks &b);   // Q4_K gate/up on the f16 units with a Q6_K down product there (gemm_q6k.hip)
 // Q8_0 banks (gate, up and down) can take the f16 kernel of the f16 banks instead: x as halfs in xh.hi alone, every
 // weight as two halfs made inside the kernel, act16 between the two products.  The launchers take that form with
 // q8_half set (tile rows from grouped_gemm_tile_rows(..., true): up to 128).
@@ -239,6 +241,9 @@ hipError_t launch_q4k_few_gate_up(const ExpertBanks &b, HAct x, const int32_t *s
                                   const int32_t *n_tiles, int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s);
 hipError_t launch_q4k_few_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y,
                                hipStream_t s);
+// gemm_q6k.hip: Q6_K down banks, act in sorted order, tiles of up to 32 or 64 rows.
+hipError_t launch_q6k_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows, float *y,
+                           hipStream_t s);
 
 // gemm_q8.hip -------------------------------------------------------------------------
 // Q8_0 banks on the f16 units: x and the activations between the two products as pairs of halfs, tiles of 32 rows.

@@ -492,10 +492,10 @@ int batched_from(const mummu_moe *h, const Layer &L) {
     return grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
 }
 
-// Q4_K and Q8_0 banks on the f16 units (batched path): whether gate/up (hf) and down (hf_down) take that form for this batch,
+// Q4_K and Q8_0 banks on the f16 units (batched path): whether gate/up (hf) and down (hf_down; q6: of Q6_K) take that form for this batch,
 // and where x goes as pairs of halfs: the (not yet written) buffer of the down product's output.
 struct HalfPlan {
-    bool hf = false, hf_down = false, q8 = false;
+    bool hf = false, hf_down = false, q8 = false, q6 = false;
     HAct xh;
 };
 
@@ -524,6 +524,7 @@ HalfPlan half_plan(const mummu_moe *h, const ExpertBanks &b, int64_t n, int k, b
     p.q8 = small32 && q8_half_pairs(h, b) && (one_expert || q8_gemm_should(b, na));
     p.hf = p.q8 || (h->gemm_q4k_f16 && small32 && grouped_gemm_q4k_f16(b));
     p.hf_down = p.q8 || (p.hf && grouped_gemm_q4k_f16_down(b));
+    p.q6 = p.hf && !one_expert && grouped_gemm_q6k_down(b);
     // x as pairs of halfs borrows h->y (the down product's output, written only after the gate/up launch has read x) and
     // the scale / sum arrays of the 16-bit form (unused on this path): run_experts keeps the order quantize -> gate/up ->
     // down on one stream, and nothing else may hold h->y across the gate/up launch
@@ -549,7 +550,8 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         int tile_rows = hf_down ? grouped_gemm_tile_rows_q4k_f16(b, na) : grouped_gemm_tile_rows(b, na, b.n_experts, q8h);
         // (gate/up alone on the f16 units: the int8 down product takes a tile of 16 rows like one of 32)
         if (hf && !hf_down) tile_rows = grouped_gemm_tile_rows_q4k_f16(b, na, true);
-        if (hf_down && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
+        if (hp.q6) tile_rows = grouped_gemm_tile_rows_q6k_down(b, na);
+        if ((hf_down || hp.q6) && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
         if (hp.q8) tile_rows = 32;
         const bool wide = wide_gemm_takes(b, (int)n, na);
         if (wide) tile_rows = kWideRows;
@@ -558,7 +560,7 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         // (f16 / bf16 banks: x as halfs in the same buffer)
         const bool half_banks = b.gate_type == T_F16 || b.gate_type == T_BF16 || q8h;
         const HAct xh = hf ? hp.xh : (half_banks ? HAct{(_Float16 *)h->y, nullptr, nullptr, nullptr} : HAct());
-        const HAct acth = hf_down ? HAct{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum} : HAct();
+        const HAct acth = hf_down || hp.q6 ? HAct{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum} : HAct();
         if (hf && !xh_done) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows_h(x, (int)n, b.hidden, xh, s));
         else if (hf) {}   // (the router launch wrote them)
         else if (half_banks) LAUNCH(h, K_QUANTIZE, s, launch_convert_rows_f16(x, (int)n, b.hidden, xh.hi, s));
