@@ -1,0 +1,31 @@
+"""Router logits of many tokens, four by four experts to a wave: bit for bit the oracle's fixed summation order, at token and expert counts
+that end inside a tile, on one to four passes over the experts, for every router type."""
+import numpy as np
+import pytest
+
+from mummu_amd import moe as M
+from mummu_amd import synth
+from oracle import binding as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,E,n", [(512, 3, 9), (512, 130, 12), (2560, 512, 67), (1024, 129, 33), (512, 512, 600), (512, 501, 1101), (8192, 17, 10)])
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
+    rng = np.random.Generator(np.random.PCG64(H + E + n))
+    w = rng.standard_normal((E, H), dtype=np.float32) * np.float32(0.05)
+    w[0, :64] = 1e-6   # (subnormal halfs)
+    if kind == "f16":
+        w, t, ot = w.astype(np.float16), M.F16, orc.F16
+    elif kind == "bf16":
+        w, t, ot = (w.view(np.uint32) >> 16).astype(np.uint16), M.BF16, orc.BF16
+    else:
+        t, ot = M.F32, orc.F32
+    x = rng.standard_normal((n, H), dtype=np.float32)
+    bank = synth.random_bank_fast(M.Q8_0, [H, 32, E], 1)
+    with M.SparseMoe(M.SparseMoeConfig(H, 32, E, 2), max_tokens=n) as m:
+        m.load_layer(0, w, t, bank, M.Q8_0, bank, M.Q8_0, synth.random_bank_fast(M.Q8_0, [32, H, E], 2), M.Q8_0)
+        got = np.asarray(m.route(x, 2, True, return_logits=True)[-1]).reshape(n, E)
+    want = orc.router_logits(x, w, ot, E).reshape(n, E)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
