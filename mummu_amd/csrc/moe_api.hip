@@ -595,7 +595,7 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
     return MUMMU_OK;
 }
 
-// Rows from which one expert alone takes the grouped GEMM pair of the f16 units: the per-row kernels decode every weight again
+// Rows from which one expert alone takes the grouped GEMM pair of the f16 units (between the two, one_expert_few): the per-row kernels decode every weight again
 // for each few rows, a GEMM of one expert has few workgroups and the latency of its loop over K.  Host call, OLMoE Q4_K, the
 // former / the latter: 48 rows 76.8 / 79.4 us, 64: 91.9 / 88.8, 128: 173 / 149, 512: 477 / 323; Q8_0 64: 121 / 106,
 // 128: 223 / 143, 512: 789 / 353.  On the device alone the lines cross at 53 rows there, and for 2048 x 768 / 2560 x 768 / 4096 x 1792 at
@@ -615,10 +615,25 @@ int one_expert_tile_rows(const ExpertBanks &b, int rows) {
     return 64;
 }
 
+// Which calls of one Q4_K expert take the kernels of gemm_q4k_one.hip: from where the per-row kernels, whose time goes with rows and weights, take
+// longer than a round trip, to where the GEMM pair does better.  Host call, hidden x inter, per-row kernels (from 64 rows on the GEMM) / these:
+// 1024 x 512 24 rows 39 / 43 us, 56: 52 / 56, 64: 59 / 61, 128: 79 / 75; 2048 x 768 24: 50 / 51, 48: 76 / 65; 2048 x 1024 16: 48 / 47, 24: 53 / 53, 48: 80 / 66,
+// 64: 92 / 78, 72: 98 / 97; 2560 x 768 16: 52 / 49, 32: 75 / 62, 80: 115 / 105, 96: 124 / 120; 4096 x 1792 8: 56 / 54, 32: 119 / 89, 56: 193 / 140, 64: 147 /
+// 153.  (1.0e-7 off the 64-bit result as the GEMM pair is, the per-row kernels 2.8e-5.)
+bool one_expert_few(const ExpertBanks &b, int rows) {
+    const int workgroups = (rows + 15) / 16 * (b.inter / 16);   // of the gate/up launch; 256 are one to a CU
+    return (size_t)rows * (size_t)b.hidden * (size_t)b.inter >= 45000000 && (rows < kOneExpertGemm || workgroups <= 256);
+}
+
 // One expert's SwiGLU on `rows` rows (at most the workspace's tokens), in order, into out.
 int run_one_expert(mummu_moe *h, const Layer &L, int expert, const float *x, int rows, float *out, hipStream_t s) {
     const ExpertBanks b = banks_of(h, L);
     const HalfPlan hp = half_plan(h, b, rows, 1, true);
+    if (hp.hf_down && !hp.q8 && one_expert_few(b, rows)) {
+        LAUNCH(h, K_GATE_UP, s, launch_q4k_one_gate_up(b, expert, x, rows, h->act, s));
+        LAUNCH(h, K_DOWN, s, launch_q4k_one_down(b, expert, h->act, rows, out, s));
+        return MUMMU_OK;
+    }
     if (hp.hf_down && rows >= kOneExpertGemm) {
         const int tile_rows = hp.q8 ? 32 : one_expert_tile_rows(b, rows), tiles = (rows + tile_rows - 1) / tile_rows;
         const HAct acth{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum};
