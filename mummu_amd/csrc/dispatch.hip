@@ -8,8 +8,8 @@
 // every expert's segment lists its assignments in ascending a = token*k + slot, which is that
 // order.
 //
-// Two small launches over chunks of 1024 assignments (one fused launch of one workgroup when there is a single
-// chunk, where the launches themselves are most of the time):
+// Two small launches over chunks of 1024 assignments (one fused launch of one workgroup for up to three
+// chunks, where the launches themselves are most of the time):
 //   count   per chunk: every assignment's rank among the chunk's assignments to the same expert
 //           (wave ballots, then a prefix over the workgroup's 16 waves in LDS) and the chunk's
 //           per-expert counts
@@ -48,14 +48,29 @@ __device__ inline void write_tiles(int32_t *__restrict__ tiles, int at, int n, i
     }
 }
 
+// Rank of this lane among the lanes of its wave with the same expert, whose number the first of them leaves in counts[e] (e < 0: no
+// expert).  The lanes of an expert by a ballot per bit of its number: six to nine steps, where one per distinct expert of 64
+// assignments, some forty, kept the four waves of a SIMD busy for two thirds of the launch (count, 1200 assignments to 64 experts 9.0 -> 5.0 us; the fused form, 216
+// to 128 10.4 -> 4.7, 640 to 512 13.1 -> 5.2).
+__device__ inline int rank_in_wave(int e, int n_experts, int lane, int *counts) {
+    unsigned long long same = __ballot(e >= 0);
+    for (int bit = 1; bit < n_experts; bit <<= 1) {
+        const unsigned long long set = __ballot((e & bit) != 0);
+        same &= e & bit ? set : ~set;
+    }
+    const int rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+    if (e >= 0 && rank == 0) counts[e] = __builtin_popcountll(same);
+    return rank;
+}
+
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_count_kernel(const int32_t *__restrict__ ids, int n_assign,
                                                                           int n_experts, int32_t *__restrict__ rank_out,
                                                                           int32_t *__restrict__ counts,
                                                                           int32_t *__restrict__ flags) {
-    __shared__ int s_wave[kDispatchWaves][kDispatchMaxExperts];  // per-wave counts of this chunk
+    __shared__ __attribute__((aligned(16))) int s_wave[kDispatchWaves][kDispatchMaxExperts];  // per-wave counts of this chunk
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int chunk = blockIdx.x;
-    for (int i = tid; i < kDispatchWaves * n_experts; i += kDispatchThreads) s_wave[i / n_experts][i % n_experts] = 0;
+    for (int i = tid; i < kDispatchWaves * kDispatchMaxExperts / 4; i += kDispatchThreads) ((int4 *)s_wave)[i] = make_int4(0, 0, 0, 0);
     __syncthreads();
     const int a = chunk * kDispatchThreads + tid;
     int e = a < n_assign ? ids[a] : -1;
@@ -63,19 +78,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_count_kernel(const 
         atomicAdd(&flags[FLAG_BAD_ID], 1);
         e = -1;
     }
-    // rank among the lanes of this wave that hold the same expert, and that group's size
-    int rank = 0;
-    unsigned long long todo = __ballot(e >= 0);
-    while (todo) {
-        const int leader = (int)__builtin_ctzll(todo);
-        const int le = __shfl(e, leader, 64);
-        const unsigned long long same = __ballot(e == le);
-        if (e == le) {
-            rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
-            if (rank == 0) s_wave[wave][e] = __builtin_popcountll(same);
-        }
-        todo &= ~same;
-    }
+    const int rank = rank_in_wave(e, n_experts, lane, s_wave[wave]);
     __syncthreads();
     if (e >= 0) {
         int before = 0;
@@ -105,6 +108,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
     const int e = tid;
     int total = 0, before = 0;
     if (e < n_experts) {
+#pragma unroll 8
         for (int c = 0; c < n_chunks; c++) {
             const int v = counts[(size_t)c * n_experts + e];
             before += c < chunk ? v : 0;
@@ -157,15 +161,15 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
 // The three steps above in one launch of one workgroup, for batches of at most kFusedChunks
 // chunks: the per-chunk counts never leave LDS and every thread keeps its assignments' experts and
 // ranks in registers between the steps.  Same outputs, element for element.  One workgroup takes
-// about 7 us per chunk against 10 us for the two launches whatever the size, so this form only
-// serves a single chunk (up to 1024 assignments).
-constexpr int kFusedChunks = 1;
+// 4.7 us for one chunk, 7.3 for two, 8.5 for three and 21.7 for eight, the two launches 10 us and the gap between them
+// whatever the size.
+constexpr int kFusedChunks = 3;
 
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
     const int32_t *__restrict__ ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *__restrict__ offsets,
     int32_t *__restrict__ sorted, int32_t *__restrict__ inv, int32_t *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     unsigned long long *__restrict__ hits, int32_t *__restrict__ flags) {
-    __shared__ int s_wave[kDispatchWaves][kDispatchMaxExperts];   // per-wave counts of the current chunk
+    __shared__ __attribute__((aligned(16))) int s_wave[kDispatchWaves][kDispatchMaxExperts];   // per-wave counts of the current chunk
     __shared__ int s_chunk[kFusedChunks][kDispatchMaxExperts];    // per-chunk counts, then exclusive running counts
     __shared__ int s_off[kDispatchMaxExperts];
     __shared__ int s_carry[kDispatchMaxExperts / 64][2];
@@ -177,7 +181,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
         my_e[c] = -1;
         my_rank[c] = 0;
         if (c >= chunks) continue;  // uniform over the workgroup
-        for (int i = tid; i < kDispatchWaves * n_experts; i += kDispatchThreads) s_wave[i / n_experts][i % n_experts] = 0;
+        for (int i = tid; i < kDispatchWaves * kDispatchMaxExperts / 4; i += kDispatchThreads) ((int4 *)s_wave)[i] = make_int4(0, 0, 0, 0);
         __syncthreads();
         const int a = c * kDispatchThreads + tid;
         int e = a < n_assign ? ids[a] : -1;
@@ -185,18 +189,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
             atomicAdd(&flags[FLAG_BAD_ID], 1);
             e = -1;
         }
-        int rank = 0;
-        unsigned long long todo = __ballot(e >= 0);
-        while (todo) {
-            const int leader = (int)__builtin_ctzll(todo);
-            const int le = __shfl(e, leader, 64);
-            const unsigned long long same = __ballot(e == le);
-            if (e == le) {
-                rank = __builtin_popcountll(same & ((1ull << lane) - 1ull));
-                if (rank == 0) s_wave[wave][e] = __builtin_popcountll(same);
-            }
-            todo &= ~same;
-        }
+        const int rank = rank_in_wave(e, n_experts, lane, s_wave[wave]);
         __syncthreads();
         if (e >= 0) {
             int before = 0;
