@@ -203,7 +203,7 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * for one or two elements (every gate pre-activation far below zero) has outputs orders of magnitude below the
  * batch's, and relative to THAT magnitude single elements come out up to 4e-3 off (2e-8 of the batch's typical
  * output).  F32 / F16 / BF16 banks do not take this path (f32 or f16 products).
- * Two exceptions on the batched path.  Q4_K gate/up (and down) banks: a Q4_K weight is d * (sc * q) - dmin * m
+ * Two exceptions on the batched path.  Q4_K gate/up banks (and Q4_K or Q6_K down banks behind them, whose codes are halfs as they are): a Q4_K weight is d * (sc * q) - dmin * m
  * with sc * q < 1024 an exact half, so their grouped GEMM runs on the f16 matrix units against activations held
  * as PAIRS of halfs, x = 2^e * (hi + lo), hi = f16(x / 2^e), lo = f16(x / 2^e - hi), 2^e one power of two per row
  * (per 128 elements between the two products): 22 significant bits per element down to 2^-13 of the row's largest, an
@@ -212,7 +212,8 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * infinity.)  Q8_0 banks (gate, up and down, hidden and inter multiples of 128) are held against the same pairs where that form is
  * the faster one, by the rows an expert has; 2.5e-7 off the 64-bit result where the integer form is by 4.5e-5.  Its one corner: a row
  * whose large elements fill blocks of 64 of their own AND meet weights of 0 keeps less of its small ones than the integer form
- * (elements 2^-20 of the row's largest 2^-13 of themselves, 2^-26 2^-7).  mummu_expert_run takes these forms from 64 rows on.
+ * (elements 2^-20 of the row's largest 2^-13 of themselves, 2^-26 2^-7).  mummu_expert_run takes these forms from 64 rows on,
+ * a Q4_K expert from some ten rows of a large one on (there with a power of two per row and 256 elements).
  * The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
  * integer form above; MUMMU_GEMM_TILE_ROWS=16, 32 or 64 fixes the rows per tile of these kernels (by default the
  * library picks the form with the smallest expected cost for the batch: same results, different speed).
