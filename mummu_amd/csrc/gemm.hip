@@ -602,7 +602,10 @@ struct QTileLds {
 // of one step: the same registers keep twice the bytes in flight, which is what a launch that
 // streams its weights with few rows per expert is short of; the arithmetic and its order per
 // output element are the same.
-template <int WT, bool GATE_UP, int MT, int KS>
+// HALF (down, MT 1): the tiles have up to 16 rows, which are the first eight elements of an accumulator: nothing is put together for the
+// others, which was 28 % of the instructions (Q5_1, 512 experts of 2560 x 640, 64 / 300 tokens: 141 / 206 -> 124 / 171 us).  A test of the rows in
+// the loop instead was slower.
+template <int WT, bool GATE_UP, int MT, int KS, bool HALF = false>
 __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
     const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, QAct64 a_in, const int32_t *__restrict__ sorted,
     int k_slots, const int32_t *__restrict__ tiles, const int32_t *__restrict__ n_tiles, int in_dim, int out_dim,
@@ -613,7 +616,8 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
     __shared__ __attribute__((aligned(16))) float s_as[KS][BM];   // activation scale of each K step, per tile row
     __shared__ float s_am[BM][2 * KS];                            // activation ssum of their blocks
     constexpr bool OFFSET = gemm_has_offset(WT), SUB16 = gemm_sub16(WT);
-    constexpr int NSC = SUB16 ? 4 : 2;
+    constexpr int NSC = SUB16 ? 4 : 2, ROWS4 = HALF ? 2 : 4;   // (runs of four rows of an accumulator)
+    static_assert(!HALF || (!GATE_UP && MT == 1), "tiles of 16 rows");
     __shared__ float s_bd[NB][kBN][NSC * KS];                     // weight scales of the K steps (per 32 or per 16 elements)
     __shared__ float s_bm[NB][kBN][2 * KS];                       // weight block offsets (types that have one)
     auto s_a = [&](int plane, int row) -> uint8_t * { return s_raw + ((size_t)plane * BM + row) * kRow; };
@@ -775,7 +779,7 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
                     const int16v ch1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah1, bq1, zero, 0, 0, 0);
                     const int16v cl1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(al1, bq1, zero, 0, 0, 0);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
+                    for (int j = 0; j < ROWS4; j++) {
                         // accumulator rows 8j..8j+7 of this 32-row block: past the tile's rows there is
                         // nothing to scale (ragged experts leave most of a tile empty at small batches)
                         if (GATE_UP && 32 * m + 8 * j >= rows) continue;  // (the down kernel measures faster without the test)
@@ -833,14 +837,14 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
                         const int16v ch = __builtin_amdgcn_mfma_i32_32x32x16_i8(ah, bq[j], zero, 0, 0, 0);
                         const int16v cl = __builtin_amdgcn_mfma_i32_32x32x16_i8(al, bq[j], zero, 0, 0, 0);
 #pragma unroll
-                        for (int r = 0; r < 16; r++) {
+                        for (int r = 0; r < 4 * ROWS4; r++) {
                             if (GATE_UP && 32 * m + 8 * (r >> 2) >= rows) continue;  // rows past the tile's: nothing to scale
                             const float f = (float)((ch[r] << 8) + cl[r]);
                             t[r] = j == 0 ? __fmul_rn(dj[0], f) : fmaf(dj[j], f, t[r]);
                         }
                     }
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
+                    for (int j = 0; j < ROWS4; j++) {
                         const float4 s4 = *(const float4 *)&s_as[sub][32 * m + 8 * j + 4 * g];
                         const float sr[4] = {s4.x, s4.y, s4.z, s4.w};
                         if (!GATE_UP || 32 * m + 8 * j < rows) {
@@ -885,7 +889,7 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
+                for (int r = 0; r < 4 * ROWS4; r++) {
                     const int row = 32 * m + acc_row(r, lane);
                     if (row < rows) y_out[(size_t)(p0 + row) * (size_t)out_dim + (size_t)n] = acc[0][m][r];
                 }
@@ -1029,6 +1033,14 @@ static hipError_t launch_gemm_q(const uint8_t *w0, const uint8_t *w1, QAct64 a_i
     // small tiles (few rows per expert: the launch is a stream of weights) also keep two stages of loads in flight
     if (tile_rows == 64 && ks2) MUMMU_Q(2, 2);
     else if (tile_rows == 64) MUMMU_Q(2, 1);
+    else if (!GATE_UP && tile_rows == 16) {
+#define MUMMU_Q16(KS)                                                                                                   \
+    launch_kernel(grouped_gemm_q_kernel<WT, false, 1, KS, true>, grid, block, 0, s, w0, w1, a_in, sorted, k_slots, tiles, n_tiles, in_dim, \
+                  out_dim, act_out, y_out)
+        if (ks2) MUMMU_Q16(2);
+        else MUMMU_Q16(1);
+#undef MUMMU_Q16
+    }
     else if (ks2) MUMMU_Q(1, 2);
     else MUMMU_Q(1, 1);
 #undef MUMMU_Q

@@ -35,6 +35,28 @@ def test_every_tile_edge_matches_the_f64_reference(monkeypatch, H, I, down, tile
     assert orc.rel_err(got, want, mag).max() <= (2e-3 if down == M.Q8_0 else 3e-5)
 
 
+# Lists of 16-row tiles in front of down banks of other types, which put together eight elements of an accumulator: every row count of a tile.
+@pytest.mark.parametrize("name", ["Q4_0", "Q4_1", "Q5_0", "Q5_1", "Q8_0", "Q5_K", "Q6_K"])
+@pytest.mark.parametrize("H,I", [(256, 256), (512, 640)])
+def test_tiles_of_16_rows_in_front_of_other_down_banks(name, H, I):
+    down = getattr(M, name)
+    if down in (M.Q5_K, M.Q6_K) and I % 256:
+        pytest.skip("rows of whole super-blocks")
+    counts = list(range(17)) * 2
+    E, n = len(counts), sum(counts)
+    rng = np.random.Generator(np.random.PCG64(H + I))
+    gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (51, 52))
+    downs = synth.random_bank_fast(down, [I, H, E], 53)
+    ids = np.repeat(np.arange(E), counts)[rng.permutation(n)].astype(np.int32)[:, None]
+    x, w = rng.standard_normal((n, H), dtype=np.float32), rng.random((n, 1), dtype=np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q4_K, up, M.Q4_K, downs, down)
+        got, again = m.apply_routing(0, ids, w, x), m.apply_routing(0, ids, w, x)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, downs, orc.Q4_K, orc.Q4_K, getattr(orc, name)), ids, w, x)
+    assert orc.rel_err(got, want, mag).max() <= (3e-5 if down == M.Q6_K else 2e-3)   # (experts.rs:1264-1271)
+
+
 def test_gates_beyond_the_exponential():
     # gates from -2000 to 2000, e^-x past the largest f32 among them: the wide gates pass, the others leave nothing
     H, I, E, n = 256, 256, 2, 80
