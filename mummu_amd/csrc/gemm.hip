@@ -975,13 +975,14 @@ static double expected_tiles(double avg, double rows) {
 // 96: 97 / 95, 112 (1.27): 96 / 97.  Lists of 32 rows gained nothing between the two (96 tokens 94, 256: 132 against 129, 1000: 331 against
 // 302).
 // With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
-// products together: the 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013 us.
+// products together: the 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013 us.  One of 16-row tiles costs 0.7 of that, unless it is
+// the first second tiles that start a second round: 520 / 600 / 680 / 760 tokens, 16 / 32 rows 479 / 537, 489 / 546, 516 / 557, 547 / 570.
 int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8_down) {
     const int n_experts = b.n_experts;
     const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
     const double e16 = expected_tiles(avg, 16.0), e32 = expected_tiles(avg, 32.0), e64 = expected_tiles(avg, 64.0);
-    if (int8_down) return 0.99 * e16 < e32 ? 16 : (0.69 * e32 < e64 ? 32 : 64);
     const double each = (double)n_experts * (double)((b.inter + 127) / 128);   // workgroups of a tile per expert
+    if (int8_down) return (each * e32 <= 512.0 && each * e16 > 1.01 * 512.0 ? 0.99 : 0.7) * e16 < e32 ? 16 : (0.69 * e32 < e64 ? 32 : 64);
     const bool second_round = each * e64 <= 512.0 && each * e16 > 1.01 * 512.0;
     return !second_round && e16 < 1.25 * e64 ? 16 : 64;
 }
