@@ -34,6 +34,8 @@ hipError_t launch_route_topk(const float *logits, int n, int n_experts, int k, i
 // Both of the above in ONE launch (num_experts <= 128), plus (xq.hi != nullptr) the 16-bit
 // quantization of x for the integer expert products.
 bool router_fused_supported(int n_experts);
+// ... and whether launch_router_logits and launch_route_topk, one after the other, do better there.
+bool router_split_should(int n, int hidden, int n_experts, const float *x, const void *w);
 hipError_t launch_router_fused(const float *x, const void *w, int wtype, int n, int hidden, int n_experts, int k,
                                int flavour, int norm, float *logits, int32_t *ids, float *weights,
                                unsigned long long *hits, int32_t *flags, QAct xq, hipStream_t s, HAct xh = HAct());

@@ -860,7 +860,7 @@ int routed_impl(mummu_moe *h, int layer, const float *x, int64_t n, int k, int n
     const bool want_xq = is_quant_type(L.gate_type) && H % 64 == 0 && !batched;
     const QAct xq = want_xq ? h->xq : QAct();
     if (norm_gamma && !decode_three_launches(h, L, n, k)) return fail(h, MUMMU_ERR_ARG, "fused RmsNorm outside the decode form");
-    if (n > 8 && router_fused_supported(E)) {
+    if (n > 8 && router_fused_supported(E) && !(batched && !want_xq && router_split_should((int)n, H, E, x, L.router))) {
         // many tokens: one workgroup per token tile does logits, routing and quantization
         // on the batched path the dispatch adds the per-expert row counts to the hit counters
         // ... and on the batched path with Q4_K banks on the f16 units it writes x as pairs of halfs beside the routing
@@ -907,9 +907,9 @@ int routed_impl(mummu_moe *h, int layer, const float *x, int64_t n, int k, int n
             return MUMMU_OK;
         }
         LAUNCH(h, K_ROUTE_TOPK, s,
-               launch_route_topk(h->logits, (int)n, E, k, h->cfg.router_flavour, norm, h->ids, h->weights, L.hits, h->flags, s));
+               launch_route_topk(h->logits, (int)n, E, k, h->cfg.router_flavour, norm, h->ids, h->weights, batched ? nullptr : L.hits, h->flags, s));
     }
-    return run_experts(h, L, x, want_xq, n, k, residual, out, s);
+    return run_experts(h, L, x, want_xq, n, k, residual, out, s, batched);   // (batched: the dispatch counts the rows an expert serves)
 }
 
 // The block: the routed experts, plus (when the layer has one) the shared expert every token

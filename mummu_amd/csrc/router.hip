@@ -615,6 +615,15 @@ static hipError_t launch_router_block_t(const float *x, const void *w, int n, in
 
 bool router_fused_supported(int n_experts) { return n_experts <= 128; }
 
+// Which batches take the tiles of router_tile_kernel and a launch for the routing instead: the streaming form turns an expert's row into
+// floats for each token or two, the tiles for four, which pays from where a wave has many rows to walk.  Layers, us, one launch / two: 128 experts
+// of 2048 x 768, 300 tokens 178 / 168, 600: 236 / 210, 1500: 405 / 375, 4096: 889 / 837; 64 of 2048 x 1024, 512: 192 / 195, 2000: 504 / 505, 2500: 633 /
+// 621, 4096: 950 / 947, three streams alike.  (Up to 256 tokens the one launch also converts x.)
+bool router_split_should(int n, int hidden, int n_experts, const float *x, const void *w) {
+    const bool tiles = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && hidden % 512 == 0 && hidden <= kTileMaxHidden;
+    return tiles && n > 256 && n_experts > 64;
+}
+
 // Which batches the router launch also converts x for: the streaming form with a workgroup per token, while those
 // workgroups leave the chip room (up to 256 tokens the extra workgroups save the 4 us launch of their own: 32 / 128 /
 // 256 tokens 110.6 / 119.5 / 157.0 -> 107.1 / 115.8 / 155.3 us per layer; from 512 on the router launch grows by what

@@ -29,3 +29,24 @@ def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
         got = np.asarray(m.route(x, 2, True, return_logits=True)[-1]).reshape(n, E)
     want = orc.router_logits(x, w, ot, E).reshape(n, E)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+# Batches of up to 128 experts on either side of the line from which they take these tiles and a launch for the routing: the oracle's routing
+# bit for bit, every row served counted once.
+@pytest.mark.parametrize("E,n", [(128, 256), (128, 257), (65, 300), (64, 300), (128, 2100)])
+def test_routing_and_hits_of_a_batch(E, n):
+    H, I, k = 512, 64, 2
+    rng = np.random.Generator(np.random.PCG64(E + n))
+    router = (rng.standard_normal((E, H), dtype=np.float32) * np.float32(0.05)).astype(np.float16)
+    x = rng.standard_normal((n, H), dtype=np.float32)
+    bank = synth.random_bank_fast(M.Q8_0, [H, I, E], 1)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, k), max_tokens=n) as m:
+        m.load_layer(0, router, M.F16, bank, M.Q8_0, bank, M.Q8_0, synth.random_bank_fast(M.Q8_0, [I, H, E], 2), M.Q8_0)
+        m.take_hits(0)
+        m.forward(x, k, True)
+        ids, w = m.last_routing(n, k)
+        hits = np.asarray(m.take_hits(0))
+    oids, ow = orc.route_olmoe(orc.router_logits(x, router, orc.F16, E), n, E, k, True)
+    assert np.array_equal(ids, oids.astype(np.int32).reshape(n, k))
+    assert np.array_equal(w.view(np.uint32), ow.reshape(n, k).view(np.uint32))
+    assert np.array_equal(hits, np.bincount(ids.ravel(), minlength=E))
