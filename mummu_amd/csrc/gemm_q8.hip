@@ -118,7 +118,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     // Activation pieces: load `wave` of each plane holds four rows.  Piece q of row r lies at q ^ (r % 16): sixteen lanes that read
     // the same piece of neighbouring rows meet all banks.
     const int a_row = 4 * wave + (lane >> 4);
+    // An item of up to 16 rows has its low halfs' rows behind its high halfs' in one A operand: half the products and row reads, a row's
+    // two parts summed at the end.  OLMoE layer, three streams, 16 / 64 / 100 tokens 89.0 / 103.2 / 105.9 -> 86.3 / 100.8 / 104.1 us, 150 (a third of
+    // the tiles) the same; off the 64-bit result by 2.43e-7 where one sum for both is by 2.52e-7.
+    const uint32_t a_full = (uint32_t)c * (kStep * 2), a_half = (uint32_t)(c & 15) * (kStep * 2) + (uint32_t)(c >> 4) * kPlane;
+    uint32_t a_rd = 0;   // of the item whose rows are being loaded
     auto set_a = [&]() {
+        a_rd = rows_of(a_item) > 16 ? a_full : a_half;
         auto source_row = [&](int r) {
             if (GATE_UP) return (uint32_t)(s_idx[a_flip][r] / k_slots);
             const int rows = rows_of(a_item);
@@ -175,7 +181,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     float d[2];
     half8 hi[2][2], lo[2][2];
     const uint32_t w_rd = (uint32_t)wave * kWaveW + (uint32_t)c * (16 * PIECES) + (PIECES == 9 ? 0u : (uint32_t)c * row_bytes & 8u);
-    auto read = [&](uint32_t slot, int odd, int which, int blk) {   // (odd: of the stage, known where PIECES is 9)
+    auto read = [&](uint32_t slot, int odd, int which, int blk, uint32_t rd, bool both) {   // (odd: of the stage, known where PIECES is 9)
         const uint8_t *ds = s_lds + slot + w_rd + 8u * (uint32_t)odd;
         const int at = 34 * blk + 2, n = blk & 1;
         if (PIECES == 9) {
@@ -188,12 +194,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
             for (int i = 0; i < ((at & 2) ? 5 : 4); i++) v[n][i] = *(const uint32_t *)(ds + 16u * (uint32_t)g + (at & ~3) + 4 * i);
         }
         d[n] = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
-        const uint8_t *as = s_lds + kRing * kStageW + (uint32_t)which * kStageA + (uint32_t)c * (kStep * 2);
+        const uint8_t *as = s_lds + kRing * kStageW + (uint32_t)which * kStageA + rd;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             const uint8_t *piece = as + (uint32_t)(((4 * blk + 2 * g + kk) ^ (c & 15)) * 16);
             hi[n][kk] = *(const half8 *)piece;
-            lo[n][kk] = *(const half8 *)(piece + kPlane);
+            if (both) lo[n][kk] = *(const half8 *)(piece + kPlane);
         }
     };
     // a block's sum -> acc, or (down) the 128 elements' sum
@@ -208,9 +214,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     };
     // the stage's row scales, read in front of its last barrier: the stage after the next lands in their place
     float4 sr[4] = {};
-    auto read_scales = [&](int which) {
+    auto read_scales = [&](int which, bool half) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) sr[j] = *(const float4 *)&s_as[which][8 * j + 4 * g];
+        for (int j = 0; j < 4; j++) sr[j] = *(const float4 *)&s_as[which][8 * (half ? j & 1 : j) + 4 * g];
     };
     auto fold_run = [&]() {
 #pragma unroll
@@ -225,11 +231,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
 
     // the first stage is there; its first block
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
-    read(0, 0, 0, 0);
+    read(0, 0, 0, 0, a_rd, true);
     uint32_t slot = 0;   // of the stage's weights
     int which = 0;       // of its rows
     for (int item = first_item, flip = 0; item < n_items; item += apart, flip ^= 1) {
-        auto stage = [&](int step, auto odd) {
+        auto stage = [&](int step, auto odd, auto half) {
+            const uint32_t rd = half ? a_half : a_full;
             const uint32_t slot1 = slot == (kRing - 1) * kStageW ? 0 : slot + kStageW, slot2 = slot1 == (kRing - 1) * kStageW ? 0 : slot1 + kStageW;
             next_a();
             next_w();
@@ -257,29 +264,37 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
                 }
                 const half8 w[2] = {q8_codes(q[0], q[1]), q8_codes(q[2], q[3])};
                 const half8 h[2] = {hi[n][0], hi[n][1]}, l[2] = {lo[n][0], lo[n][1]};
-                if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1);
-                else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0);
+                if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1, rd, !half);
+                else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0, a_rd, true);
 #pragma unroll
                 for (int kk = 0; kk < 2; kk++) {
                     s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[kk], w[kk], kk == 0 ? zero : s[n], 0, 0, 0);
-                    s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l[kk], w[kk], s[n], 0, 0, 0);
+                    if (!half) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l[kk], w[kk], s[n], 0, 0, 0);
                 }
                 // the block before this one, while these are multiplied
                 fold(n ^ 1, (blk + 3) & 3);
                 if (!GATE_UP && blk == 0) fold_run();
-                if (!GATE_UP && blk == 2) read_scales(which);
+                if (!GATE_UP && blk == 2) read_scales(which, half);
                 fd = now;
             }
             slot = slot1;
             which ^= 1;
         };
-        for (int step = 0; step < n_steps;) {
-            stage(step++, std::integral_constant<int, 0>());
-            if (PIECES == 9) stage(step++, std::integral_constant<int, 1>());   // (stages come in pairs)
-        }
+        const int p0 = start_of(item), rows = rows_of(item);
+        auto stages = [&](auto half) {
+            for (int step = 0; step < n_steps;) {
+                stage(step++, std::integral_constant<int, 0>(), half);
+                if (PIECES == 9) stage(step++, std::integral_constant<int, 1>(), half);   // (stages come in pairs)
+            }
+        };
+        if (rows > 16) stages(std::integral_constant<bool, false>());
+        else stages(std::integral_constant<bool, true>());
         fold(1, 3);
         if (!GATE_UP) fold_run();
-        const int p0 = start_of(item), rows = rows_of(item);
+        if (rows <= 16) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) acc[r] += acc[r + 8];
+        }
         if (GATE_UP) {
             // (the last stage's weights are read: their place is free until the loads beside the next item's products)
             float *s_c = (float *)(s_lds + (slot == 0 ? (kRing - 1) * kStageW : slot - kStageW));   // [gate, up][row][kRowC]

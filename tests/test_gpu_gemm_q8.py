@@ -125,3 +125,22 @@ def test_workgroups_of_several_items_match_the_f64_reference(H, I, scale):
     assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids, w, x)
     assert orc.rel_err(got, want, mag).max() <= 3e-5
+
+
+# Tiles of up to 16 rows (both halfs of a row in one product) beside fuller ones, a workgroup going from one kind to the other.
+@pytest.mark.parametrize("H,I", [(128, 256), (640, 384), (1024, 256)])
+def test_tiles_of_up_to_16_rows_match_the_f64_reference(H, I):
+    counts = np.array([16, 17, 15, 32, 1, 24, 48, 49] * 32)
+    E = len(counts)
+    gate, up = (synth.random_bank_fast(M.Q8_0, [H, I, E], seed) for seed in (21, 22))
+    down = synth.random_bank_fast(M.Q8_0, [I, H, E], 23)
+    g = np.random.default_rng(H)
+    ids = g.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    n = len(ids)
+    x, w = g.standard_normal((n, H)).astype(np.float32), np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got = m.apply_routing(0, ids, w, x)
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids, w, x)
+    assert orc.rel_err(got, want, mag).max() <= 3e-5
+    assert np.linalg.norm(got - want) <= 3e-6 * np.linalg.norm(want)
