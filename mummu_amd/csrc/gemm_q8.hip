@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "device_utils.h"
+#include "gemm_q8_lds.h"
 #include "kernels.h"
 #include "qact.h"
 
@@ -37,14 +38,8 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
-constexpr int kRows = 32;                    // rows of a tile
-constexpr int kWaves = 8, kWCols = 32 * kWaves;
-constexpr int kStep = 128, kBlocks = 4;      // K elements and blocks of a stage
-constexpr int kRowW = 136;                   // bytes of a weight row's stage
-constexpr int kWLoads = 5;                   // loads of a wave's weights: 64 pieces of 16 bytes each
-constexpr int kWaveW = kWLoads * 1024, kStageW = kWaves * kWaveW, kRing = 3;
-constexpr int kPlane = kRows * kStep * 2, kStageA = 2 * kPlane;   // hi, lo: [row][16 pieces of 16 bytes]
-constexpr int kLdsBytes = kRing * kStageW + 2 * kStageA;
+using namespace q8;
+
 constexpr int kCusOfXcd = 32;               // (a workgroup fills a CU)
 constexpr int kRowC = 128 + 4;               // f32 row of the gate/up epilogue
 static_assert(2 * kRows * kRowC * 4 <= kStageW, "the epilogue fits a stage's weights");
@@ -73,7 +68,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
                                                                          const int32_t *__restrict__ sorted, int k_slots,
                                                                          const int32_t *__restrict__ tiles, const int32_t *__restrict__ n_tiles,
                                                                          int in_dim, int out_dim, HAct act, float *__restrict__ y) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // [kRing][kStageW], then [2][kStageA]
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];   // (gemm_q8_lds.h)
     __shared__ __attribute__((aligned(16))) float s_as[2][64];        // row scales (gate/up: of an item, else of a stage), twice
     __shared__ int32_t s_idx[2][64];                                  // an item's entries of `sorted`, twice
     // as xcd_tile in gemm.hip: an XCD takes neighbouring tiles, the slab running fastest; here a workgroup takes every
@@ -115,16 +110,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
             load_to_lds4(lds_idx + (uint32_t)w_flip * 256u, (const uint8_t *)(sorted + start_of(w_item)), (uint32_t)(c < rows ? c : rows - 1) * 4u);
         }
     };
-    // Activation pieces: load `wave` of each plane holds four rows.  Piece q of row r lies at q ^ (r % 16): sixteen lanes that read
-    // the same piece of neighbouring rows meet all banks.
+    // Activation pieces: load `wave` of each plane holds four rows.
     const int a_row = 4 * wave + (lane >> 4);
     // An item of up to 16 rows has its low halfs' rows behind its high halfs' in one A operand: half the products and row reads, a row's
     // two parts summed at the end.  OLMoE layer, three streams, 16 / 64 / 100 tokens 89.0 / 103.2 / 105.9 -> 86.3 / 100.8 / 104.1 us, 150 (a third of
     // the tiles) the same; off the 64-bit result by 2.43e-7 where one sum for both is by 2.52e-7.
-    const uint32_t a_full = (uint32_t)c * (kStep * 2), a_half = (uint32_t)(c & 15) * (kStep * 2) + (uint32_t)(c >> 4) * kPlane;
-    uint32_t a_rd = 0;   // of the item whose rows are being loaded
+    const uint32_t a_full = row_read(c, false), a_half = row_read(c, true);
+    uint32_t a_rd = a_full, a_low = row_low(false);   // of the item whose rows are being loaded
     auto set_a = [&]() {
-        a_rd = rows_of(a_item) > 16 ? a_full : a_half;
+        const bool few = rows_of(a_item) <= 16;
+        a_rd = few ? a_half : a_full, a_low = row_low(few);
         auto source_row = [&](int r) {
             if (GATE_UP) return (uint32_t)(s_idx[a_flip][r] / k_slots);
             const int rows = rows_of(a_item);
@@ -158,7 +153,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
                       w_off[j]);
     };
     auto load_a = [&](int which, int i) {
-        const uint32_t at = lds0 + kRing * kStageW + (uint32_t)which * kStageA + (uint32_t)wave * 1024u;
+        const uint32_t at = lds0 + rows_at(which) + (uint32_t)wave * 1024u;
         if (i == 0) load_to_lds16(at, (const uint8_t *)a.hi + (size_t)a_step * (kStep * 2), a_off);
         else if (i == 1) load_to_lds16(at + kPlane, (const uint8_t *)a.lo + (size_t)a_step * (kStep * 2), a_off);
         else load_to_lds4(lds_as + (uint32_t)which * 256u, (const uint8_t *)a.scale + (size_t)a_step * 4, s_off);   // (every wave the same)
@@ -181,7 +176,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     float d[2];
     half8 hi[2][2], lo[2][2];
     const uint32_t w_rd = (uint32_t)wave * kWaveW + (uint32_t)c * (16 * PIECES) + (PIECES == 9 ? 0u : (uint32_t)c * row_bytes & 8u);
-    auto read = [&](uint32_t slot, int odd, int which, int blk, uint32_t rd, bool both) {   // (odd: of the stage, known where PIECES is 9)
+    auto read = [&](uint32_t slot, int odd, int which, int blk, uint32_t rd, uint32_t low, bool both) {   // (odd: of the stage, known where PIECES is 9)
         const uint8_t *ds = s_lds + slot + w_rd + 8u * (uint32_t)odd;
         const int at = 34 * blk + 2, n = blk & 1;
         if (PIECES == 9) {
@@ -194,12 +189,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
             for (int i = 0; i < ((at & 2) ? 5 : 4); i++) v[n][i] = *(const uint32_t *)(ds + 16u * (uint32_t)g + (at & ~3) + 4 * i);
         }
         d[n] = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
-        const uint8_t *as = s_lds + kRing * kStageW + (uint32_t)which * kStageA + rd;
+        const uint8_t *as = s_lds + rows_at(which);
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
-            const uint8_t *piece = as + (uint32_t)(((4 * blk + 2 * g + kk) ^ (c & 15)) * 16);
-            hi[n][kk] = *(const half8 *)piece;
-            if (both) lo[n][kk] = *(const half8 *)(piece + kPlane);
+            const uint32_t piece = row_piece(c, g, blk, kk);
+            hi[n][kk] = *(const half8 *)(as + rd + piece);
+            if (both) lo[n][kk] = *(const half8 *)(as + rd + piece + low);
         }
     };
     // a block's sum -> acc, or (down) the 128 elements' sum
@@ -231,7 +226,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
 
     // the first stage is there; its first block
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
-    read(0, 0, 0, 0, a_rd, true);
+    read(0, 0, 0, 0, a_rd, a_low, true);
     uint32_t slot = 0;   // of the stage's weights
     int which = 0;       // of its rows
     for (int item = first_item, flip = 0; item < n_items; item += apart, flip ^= 1) {
@@ -264,8 +259,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
                 }
                 const half8 w[2] = {q8_codes(q[0], q[1]), q8_codes(q[2], q[3])};
                 const half8 h[2] = {hi[n][0], hi[n][1]}, l[2] = {lo[n][0], lo[n][1]};
-                if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1, rd, !half);
-                else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0, a_rd, true);
+                if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1, rd, row_low(half), !half);
+                else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0, a_rd, a_low, true);
 #pragma unroll
                 for (int kk = 0; kk < 2; kk++) {
                     s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[kk], w[kk], kk == 0 ? zero : s[n], 0, 0, 0);
