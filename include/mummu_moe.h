@@ -210,9 +210,10 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * absolute error of at most 2^-34 of that largest one below.  That form measures 2e-6 by the reference's measure and has no
  * such corner; it is also the faster one.  (A row that holds an infinity comes out NaN in that form, where f32 products give an
  * infinity.)  Q8_0 banks (gate, up and down, hidden and inter multiples of 128) are held against the same pairs where that form is
- * the faster one, by the rows an expert has; 2.5e-7 off the 64-bit result where the integer form is by 4.5e-5.  Its one corner: a row
- * whose large elements fill blocks of 64 of their own AND meet weights of 0 keeps less of its small ones than the integer form
- * (elements 2^-20 of the row's largest 2^-13 of themselves, 2^-26 2^-7).  mummu_expert_run takes these forms from 64 rows on,
+ * the faster one, by the rows an expert has; 2.5e-7 off the 64-bit result where the integer form is by 4.5e-5; the absolute error is
+ * at most 2^-39 of the row's largest there.  Its one corner: a row whose large elements are more than 2^24 above the rest, fill blocks of 64
+ * of their own AND meet weights of 0 keeps less of its small ones than the integer form (elements 2^-26 of the largest 2^-13 of
+ * themselves, where that keeps 2^-16 of each block's largest).  mummu_expert_run takes these forms from 64 rows on,
  * a Q4_K expert from some ten rows of a large one on (there with a power of two per row and 256 elements).
  * The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
  * integer form above; MUMMU_GEMM_TILE_ROWS=16, 32 or 64 fixes the rows per tile of these kernels (by default the

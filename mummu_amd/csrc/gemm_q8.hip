@@ -15,10 +15,12 @@
 // for, 385 MB); a wave for one block of a stage and 128 columns, a quarter of the reads of rows (81.1 + 54.8: sums exchanged at the end).
 // Off the 64-bit result by 2.5e-7 where the int8 form is by 4.5e-5.
 //
-// x has one scale for its whole row (HAct): an element is off by at most 2^-34 of the row's largest, where the int8 form's is off
-// by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of their own and
-// meet weights of 0: a block 2^20 (2^26) above the rest 1.0e-4 (6.4e-3) off the 64-bit result, the int8 form 4.6e-5.  A single element
-// 2^20 above it, its weights 0: 5.0e-5, the int8 form, which loses its 63 neighbours, 2.4e-1; weights as they come: 3.3e-7 and 3.1e-5.
+// x has one scale for its whole row (HAct, the largest element lifted to 2^15): an element is off by at most 2^-39 of the row's largest, where
+// the int8 form's is off by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of
+// their own, more than 2^24 above the rest, and meet weights of 0: such a block 2^20 / 2^23 / 2^24 / 2^26 above 3.1e-6 / 2.5e-5 / 4.9e-5 / 2.0e-4
+// off the 64-bit result, the int8 form 4.8e-5 each time (with the largest at 2^10, as Q4_K rows have it for their sums' sake, 9.9e-5 / 7.9e-4 / 1.6e-3 /
+// 6.4e-3).  A single element 2^20 above, its weights 0: 1.6e-6, the int8 form, which loses its 63 neighbours, 4.7e-1; no element above: 1.7e-7
+// and 4.8e-5.
 //
 // An item is a tile by 256 weight rows (128 of gate and 128 of up), a wave has 32 of them, which it loads for itself; the activation tile
 // is shared.  Lane (column c, K group g) reads 16 of a block's 32 codes, so element 16 g + 8 kk + i of the block is the K index
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
                                              __fmul_rn(det_silu(gv.w), uv.w));
                 const bool active = row < rows;
                 hact_store128(active ? r : make_float4(0.f, 0.f, 0.f, 0.f), active, act, (size_t)(p0 + row), out_dim,
-                              item % n_slabs * kCols + 4 * (tid & 31));
+                              item % n_slabs * kCols + 4 * (tid & 31), kHActLift);
             }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         } else {

@@ -507,7 +507,8 @@ struct HalfPlan {
 //   layer) it is not, and the bytes decide.
 //   Beyond, some need a second one: 54 rows 512 experts 1777 / 1841; 64: 257 / 353, 405 / -, 449 / 548, 2142 / 2250; 128: 424 / 512, 670 / -, 636 / 808.
 //   From 190 rows on: 192 rows 572 / 665, 934 / 1066, 951 / 1062; 512: 1361 / 1462, -, 2208 / 2331 (three streams 1400 / 1399), a hundred times nearer the
-//   64-bit result.  Rows in ten pieces are behind there (512 experts, 128 rows 3998 / 3861, 160: 4995 / 4686) and keep the int8 form.
+//   64-bit result (but for rows with a block of 64 that is more than 2^24 above the rest and meets weights of 0, where one scale a row keeps less
+//   than one per 64 elements: gemm_q8.hip).  Rows in ten pieces are behind there (512 experts, 128 rows 3998 / 3861, 160: 4995 / 4686) and keep the int8 form.
 bool q8_gemm_should(const ExpertBanks &b, size_t n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const size_t workgroups = (size_t)b.n_experts * (size_t)(b.inter / 128);   // of a gate/up launch with a tile per expert
@@ -528,7 +529,7 @@ HalfPlan half_plan(const mummu_moe *h, const ExpertBanks &b, int64_t n, int k, b
     // x as pairs of halfs borrows h->y (the down product's output, written only after the gate/up launch has read x) and
     // the scale / sum arrays of the 16-bit form (unused on this path): run_experts keeps the order quantize -> gate/up ->
     // down on one stream, and nothing else may hold h->y across the gate/up launch
-    if (p.hf) p.xh = HAct{(_Float16 *)h->y, (_Float16 *)h->y + (size_t)n * b.hidden, h->xq.scale, (float *)h->xq.sum};
+    if (p.hf) p.xh = HAct{(_Float16 *)h->y, (_Float16 *)h->y + (size_t)n * b.hidden, h->xq.scale, (float *)h->xq.sum, p.q8 ? kHActLift : 0};
     return p;
 }
 
@@ -603,7 +604,8 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
 // 220 / 84 (Q8_0).  Only banks that are Q4_K or Q8_0 throughout: their GEMM holds rows as pairs of halfs (1.0e-7
 // and 2.5e-7 off the 64-bit result, the per-row kernels 2.8e-5 and 3.3e-5), the int8 GEMM of the other types a scale per 64
 // elements, where the per-row kernels have one per 16.  (One scale per row there, one per 16 elements in the per-row kernels: a row
-// whose large elements fill blocks of 16 and meet weights of 0 keeps more of its small ones in the latter, see gemm_q8.hip.)
+// whose large elements are more than 2^18 (Q4_K) or 2^23 (Q8_0) above the rest, fill blocks of 16 and meet weights of 0 keeps more of its small
+// ones in the latter, see gemm_q8.hip.)
 constexpr int kOneExpertGemm = 64;
 
 // The Q4_K form's tiles: the smallest whose launch is at most one workgroup per CU (512 rows of OLMoE, tiles of 16 / 32 / 64 rows: 323 / 330 /

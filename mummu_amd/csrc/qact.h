@@ -105,7 +105,9 @@ __device__ inline void quantize_store64(float4 v, bool active, const QAct64 &q, 
 // halfs, x = scale * (hi + lo) with hi = f16(x / scale), lo = f16(x / scale - hi), and a power-of-two
 // scale chosen so that the largest |x / scale| it covers lies in [2^9, 2^10): 22 significant bits per
 // element down to 2^-13 of that largest one, an absolute error of at most 2^-34 of it below, and
-// sums of 32 scaled elements stay below 2^15, inside a half's range.  The scale array has one entry per
+// sums of 32 scaled elements stay below 2^15, inside a half's range.  Q8_0 banks have no offsets, so nothing takes the sums as
+// halfs there: the largest one lies 2^kHActLift higher, below 2^15, and the error under 2^-18 of it is at most 2^-39 of it - no more than
+// 16 bits a block have wherever a block's largest element is at least 2^-23 of its row's.  The scale array has one entry per
 // 128 elements; a producer that sees whole rows (quantize_rows_h) writes the same scale into all of a
 // row's entries, one that sees 128 columns at a time (the gate/up epilogue) a scale per entry.
 //   hi, lo : f16 [rows][D]      scale : f32 [rows][D/128]      ssum : f32 [rows][D/32], sum of x / scale
@@ -115,14 +117,16 @@ struct HAct {
     _Float16 *lo = nullptr;
     float *scale = nullptr;
     float *ssum = nullptr;
+    int lift = 0;   // for the rows written into it: the largest element lies in [2^9, 2^10) * 2^lift
 };
+constexpr int kHActLift = 5;
 
-// The scale for a largest magnitude m = f * 2^ex, f in [0.5, 1): x / scale = x * 2^(10 - ex).
+// The scale for a largest magnitude m = f * 2^ex, f in [0.5, 1): x / scale = x * 2^(10 + lift - ex).
 // A non-finite m (exponent 255) gives hi = inf and lo = inf - inf = NaN for an infinite element: a row that holds an
 // infinity comes out NaN where the reference's f32 product gives an infinity (non-finite rows are outside what the
 // parity tests pin).
-__device__ inline void hact_scale_of(float m, float &inv, float &scale) {
-    int ex = (int)((__float_as_uint(m) >> 23) & 255u) - 126;
+__device__ inline void hact_scale_of(float m, float &inv, float &scale, int lift = 0) {
+    int ex = (int)((__float_as_uint(m) >> 23) & 255u) - 126 - lift;
     ex = ex < -116 ? -116 : ex;
     inv = __uint_as_float((uint32_t)(137 - ex) << 23);
     scale = __uint_as_float((uint32_t)(117 + ex) << 23);
@@ -131,7 +135,7 @@ __device__ inline void hact_scale_of(float m, float &inv, float &scale) {
 // Store 128 consecutive activations held four per lane in an aligned 32-lane group (lane i holds
 // elements 4i..4i+3; an inactive group holds zeros).  elem0: this lane's first element in the row.
 // row_max < 0: the scale comes from these 128 elements; else from row_max, the largest magnitude of the row.
-__device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_t row, int d, int elem0, float row_max = -1.0f) {
+__device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_t row, int d, int elem0, int lift = 0, float row_max = -1.0f) {
     float m = row_max;
     if (row_max < 0.0f) {
         m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
@@ -143,7 +147,7 @@ __device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_
         m = fmaxf(__int_as_float(o[0]), __int_as_float(o[1]));
     }
     float inv, scale;
-    hact_scale_of(m, inv, scale);
+    hact_scale_of(m, inv, scale, lift);
     const float f[4] = {__fmul_rn(v.x, inv), __fmul_rn(v.y, inv), __fmul_rn(v.z, inv), __fmul_rn(v.w, inv)};
     _Float16 hi[4], lo[4];
     float sum = 0.0f;
@@ -189,7 +193,7 @@ __device__ inline void hact_quantize_row(const float *__restrict__ x, int d, con
     for (int e0 = tid * 4; e0 - tid * 4 < d; e0 += NT * 4) {   // (whole 32-lane groups run together: d is a multiple of 128)
         const bool active = e0 < d;
         const float4 v = active ? *(const float4 *)(xr + e0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        hact_store128(v, active, q, (size_t)row, d, e0, m);
+        hact_store128(v, active, q, (size_t)row, d, e0, q.lift, m);
     }
 }
 

@@ -36,19 +36,19 @@ def test_tile_edges_match_the_f64_reference(H, I):
         assert orc.rel_err(y, want, mag).max() <= 3e-5
 
 
-def outlier_case(wide_block):
-    # Rows with one element (or one block of 64) standing out by 2^20; the weights that meet it are 0, so that what comes out is
+def outlier_case(wide_block, n=130, factor=2.0 ** 20):
+    # Rows with one element (or one block of 64) standing out by `factor`; the weights that meet it are 0, so that what comes out is
     # made of the small ones.
-    H, I, E, n = 512, 256, 4, 130
+    H, I, E = 512, 256, 4
     banks = [np.frombuffer(synth.random_bank_fast(M.Q8_0, ne, s), np.uint8).copy() for s, ne in ((1, [H, I, E]), (2, [H, I, E]), (3, [I, H, E]))]
     x = np.random.default_rng(9).standard_normal((n, H)).astype(np.float32)
     blocks = [b.reshape(-1, H // 32, 34) for b in banks[:2]]
     if wide_block:
-        x[:, :64] *= np.float32(2.0 ** 20)
+        x[:, :64] *= np.float32(factor)
         for b in blocks:
             b[:, :2, 2:] = 0
     else:
-        x[:, 7] = np.float32(2.0 ** 20) * np.sign(x[:, 7])
+        x[:, 7] = np.float32(factor) * np.sign(x[:, 7])
         for b in blocks:
             b[:, 0, 2 + 7] = 0
     return H, I, E, n, banks, x
@@ -77,7 +77,7 @@ def test_rows_with_one_element_standing_out_keep_their_small_elements(factor):
 def test_the_limit_of_one_scale_per_row(wide_block):
     # An element is off by at most 2^-34 of its row's largest (2^20 times up to 4.5 here), at random: at most 2^-11.8 of an element of
     # 1, by root mean square a quarter of that (rows' largest are half of it, errors are uniform), in gate and up alike, whose product
-    # carries both: 2^-12 of the result in norm.
+    # carries both: 2^-12 of the result in norm.  (That is with the row's largest below 2^10; it lies 2^5 higher, so 2^-17 comes out.)
     H, I, E, n, (gate, up, down), x = outlier_case(wide_block)
     ids, w = (np.arange(n, dtype=np.int32) % E)[:, None], np.ones((n, 1), np.float32)
     with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
@@ -87,6 +87,21 @@ def test_the_limit_of_one_scale_per_row(wide_block):
     for y, e in ((got, ids), (alone, np.ones((n, 1)))):
         want, _ = orc.moe_ref_f64(banks, e.astype(np.uint32), w, x)
         assert np.linalg.norm(y - want) <= 2.0 ** -12 * np.linalg.norm(want)
+
+
+# Blocks of 64 that stand out by up to 2^23 and meet no weight cost the rest of their row no more than 16 bits for each 64 elements do
+# (4.6e-5): an element is off by at most 2^-39 of its row's largest (below 2^25.2 here), by root mean square 2^-15.8, at most 2^-14.8
+# where the largest passes a power of two, in gate and up alike: 2^-14 of the result in norm.  Few rows per expert, and more than 190.
+@pytest.mark.parametrize("rows", [32, 200])
+@pytest.mark.parametrize("factor", [2.0 ** 16, 2.0 ** 23])
+def test_blocks_standing_out_cost_no_more_than_a_scale_per_64(rows, factor):
+    H, I, E, n, (gate, up, down), x = outlier_case(True, 4 * rows, factor)
+    ids, w = (np.arange(n, dtype=np.int32) % E)[:, None], np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got = m.apply_routing(0, ids, w, x)
+    want, _ = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids, w, x)
+    assert np.linalg.norm(got - want) <= 2.0 ** -14 * np.linalg.norm(want)
 
 
 # Which form takes a batch shows in its error: 2.5e-7 for pairs of halfs, 4.5e-5 for 16 bits per 64 elements.
