@@ -214,7 +214,8 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * at most 2^-39 of the row's largest there.  Its one corner: a row whose large elements are more than 2^24 above the rest, fill blocks of 64
  * of their own AND meet weights of 0 keeps less of its small ones than the integer form (elements 2^-26 of the largest 2^-13 of
  * themselves, where that keeps 2^-16 of each block's largest).  mummu_expert_run takes these forms from 64 rows on,
- * a Q4_K expert from some ten rows of a large one on (there with a power of two per row and 256 elements).
+ * a Q4_K expert from some ten rows of a large one on (there with a power of two per row and 256 elements, and an absolute error of at most
+ * 2^-39 of the largest of those, where the per-row kernels' is 2^-16 of the largest of 16).
  * The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
  * integer form above; MUMMU_GEMM_TILE_ROWS=16, 32 or 64 fixes the rows per tile of these kernels (by default the
  * library picks the form with the smallest expected cost for the batch: same results, different speed).

@@ -5,6 +5,11 @@
 // rows of each matrix, so that a launch is one round trip to memory: weights and rows come straight into the registers that multiply
 // them, the rows become pairs of halfs there (a scale per row and super-block), and the waves' sums meet in LDS in ascending order.
 //
+// A row's scale covers a super-block, the per-row kernels' one 16 elements: those keep more of what stands beside sub-blocks that are more than
+// 2^23 above it and meet weights of 0 (off the 64-bit result, such a sub-block 2^20 / 2^23 / 2^26 above: 3.6e-6 / 1.9e-5 / 2.2e-4, those 1.8e-5 each
+// time; none above: 1.1e-7).  The largest element lies below 2^15 for that (below 2^10, with room for the sums of 32 as halfs: 1.1e-4 / 5.6e-4 /
+// 5.7e-3); the sums are of elements over 2^5 again.
+//
 // OLMoE shape, 48 rows: quantizing, gate/up and down by the per-row kernels 3.5 + 17.8 + 10.0 us -> 9.8 + 9.0, half of it the launch and the way
 // to memory and back, half the instructions of a wave, two to a SIMD; the host call 77 -> 66 us.
 #include "device_utils.h"
@@ -70,8 +75,9 @@ __global__ __launch_bounds__(64 * kWaves, 4) void q4k_one_kernel(OneArgs p) {
         m = fmaxf(m, __shfl_xor(m, 16, 64));
         m = fmaxf(m, __shfl_xor(m, 32, 64));
         float inv, scale;
-        hact_scale_of(m, inv, scale);
-        // (element order of HAct; sums of 32 elements, hi and lo halfs of the first four in lanes c, of c + 32, of the others beside them)
+        hact_scale_of(m, inv, scale, kHActLift);
+        scale = __fmul_rn(scale, (float)(1 << kHActLift));   // (of the sums; d takes the elements' lift)
+        // (element order of HAct; sums of 32 elements, over 2^kHActLift again to be halfs, hi and lo halfs of the first four in lanes c, of c + 32, of the others beside them)
         half8 hi[8], lo[8];
         half4v am;
 #pragma unroll
@@ -83,7 +89,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void q4k_one_kernel(OneArgs p) {
             for (int q = 0; q < 8; q++) {
                 hi[i][q] = (_Float16)f[q];
                 lo[i][q] = (_Float16)__fsub_rn(f[q], (float)hi[i][q]);
-                sum = __fadd_rn(sum, f[q]);
+                sum = fmaf(f[q], 1.0f / (1 << kHActLift), sum);
             }
             sum = __fadd_rn(sum, __shfl_xor(sum, 16, 64));
             sum = __fadd_rn(sum, __shfl_xor(sum, 32, 64));
@@ -111,7 +117,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void q4k_one_kernel(OneArgs p) {
             }
             head.mn4[0] = kg & 1 ? head.mn4[1] : head.mn4[0];
             const f32x4 c2 = __builtin_amdgcn_mfma_f32_16x16x16f16(am, head.offsets(0), zero, 0, 0, 0);
-            const float fd = head.d(), fm = head.minus_dmin();
+            const float fd = head.d(kHActLift), fm = head.minus_dmin();
 #pragma unroll
             for (int r = 0; r < 4; r++) acc[j][r] = fmaf(fmaf(fm, c2[r], __fmul_rn(fd, c1[r])), sr[r], acc[j][r]);
         }

@@ -621,7 +621,8 @@ int one_expert_tile_rows(const ExpertBanks &b, int rows) {
 // longer than a round trip, to where the GEMM pair does better.  Host call, hidden x inter, per-row kernels (from 64 rows on the GEMM) / these:
 // 1024 x 512 24 rows 39 / 43 us, 56: 52 / 56, 64: 59 / 61, 128: 79 / 75; 2048 x 768 24: 50 / 51, 48: 76 / 65; 2048 x 1024 16: 48 / 47, 24: 53 / 53, 48: 80 / 66,
 // 64: 92 / 78, 72: 98 / 97; 2560 x 768 16: 52 / 49, 32: 75 / 62, 80: 115 / 105, 96: 124 / 120; 4096 x 1792 8: 56 / 54, 32: 119 / 89, 56: 193 / 140, 64: 147 /
-// 153.  (1.0e-7 off the 64-bit result as the GEMM pair is, the per-row kernels 2.8e-5.)
+// 153.  (1.0e-7 off the 64-bit result as the GEMM pair is, the per-row kernels 2.8e-5; sub-blocks 2^23 above the rest that meet weights of 0 turn
+// that round, see gemm_q4k_one.hip.)
 bool one_expert_few(const ExpertBanks &b, int rows) {
     const int workgroups = (rows + 15) / 16 * (b.inter / 16);   // of the gate/up launch; 256 are one to a CU
     return (size_t)rows * (size_t)b.hidden * (size_t)b.inter >= 45000000 && (rows < kOneExpertGemm || workgroups <= 256);

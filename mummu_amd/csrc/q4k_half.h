@@ -70,7 +70,7 @@ struct Q4kHeader {
         const half4v a = offsets(0), b = offsets(1);
         return half8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
     }
-    __device__ float d() const { return __fmul_rn(kQ4kUnit, half_bits_to_float((uint16_t)(dd & 0xFFFFu))); }
+    __device__ float d(int lift = 0) const { return __fmul_rn(kQ4kUnit / (float)(1 << lift), half_bits_to_float((uint16_t)(dd & 0xFFFFu))); }
     __device__ float minus_dmin() const { return -half_bits_to_float((uint16_t)(dd >> 16)); }
 };
 
