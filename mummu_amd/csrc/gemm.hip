@@ -1076,17 +1076,17 @@ bool grouped_gemm_q8_f16(const ExpertBanks &b) {
 }
 
 bool grouped_gemm_q4k_f16(const ExpertBanks &b) {
-    // (one expert's matrix is addressed with 32-bit byte offsets)
+    // (one expert's matrix is addressed with 32-bit byte offsets; slabs are whole: 128 rows of gate and of up, 256 of down)
     return b.gate_type == T_Q4_K && b.up_type == T_Q4_K && b.hidden % 256 == 0 && b.inter % 128 == 0 &&
            (size_t)b.hidden * (size_t)b.inter < (1ull << 32);
 }
 
 bool grouped_gemm_q4k_f16_down(const ExpertBanks &b) {
-    return grouped_gemm_q4k_f16(b) && b.down_type == T_Q4_K && b.inter % 256 == 0 && b.hidden % 128 == 0;
+    return grouped_gemm_q4k_f16(b) && b.down_type == T_Q4_K && b.inter % 256 == 0;
 }
 
 bool grouped_gemm_q6k_down(const ExpertBanks &b) {
-    return grouped_gemm_q4k_f16(b) && b.down_type == T_Q6_K && b.inter % 256 == 0 && b.hidden % 32 == 0;
+    return grouped_gemm_q4k_f16(b) && b.down_type == T_Q6_K && b.inter % 256 == 0;
 }
 
 template <bool GATE_UP>

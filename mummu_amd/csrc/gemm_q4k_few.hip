@@ -59,8 +59,7 @@ __device__ inline void q4k_few_tile(const Q4kArgs &p, int e, int p0, int rows, i
     {
         const uint8_t *m0 = p.w0 + (size_t)e * (size_t)p.out_dim * row_bytes;
         const uint8_t *m1 = (GATE_UP ? p.w1 : p.w0) + (size_t)e * (size_t)p.out_dim * row_bytes;
-        int first = GATE_UP ? slab * (kWCols / 2) + 32 * wave : slab * kWCols + 64 * wave;
-        if (!GATE_UP && first >= p.out_dim) first = p.out_dim - 64;   // (columns past the matrix: multiplied, never stored)
+        const int first = GATE_UP ? slab * (kWCols / 2) + 32 * wave : slab * kWCols + 64 * wave;
         w_base[0] = uniform(m0 + (size_t)first * row_bytes);
         w_base[1] = uniform(m1 + (size_t)(first + (GATE_UP ? 0 : 32)) * row_bytes);
 #pragma unroll
@@ -233,7 +232,7 @@ __device__ inline void q4k_few_tile(const Q4kArgs &p, int e, int p0, int rows, i
                                  slab * 128 + cb * 64 + 4 * c);
             }
         }
-    } else if (slab * kWCols + 64 * wave < p.out_dim) {
+    } else {
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -247,7 +246,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q4k_few_kernel(Q4kArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];
     // As xcd_tile in gemm.hip: an XCD takes neighbouring tiles with the slab running fastest.
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
-    const int n_slabs = (p.out_dim + kCols - 1) / kCols;
+    const int n_slabs = p.out_dim / kCols;   // (whole: grouped_gemm_q4k_f16)
     const int total = *p.n_tiles, per_xcd = (total + 7) >> 3;
     const int item = (int)(blockIdx.x >> 3);
     const int within = item / n_slabs, slab = item - within * n_slabs;
@@ -260,7 +259,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q4k_few_kernel(Q4kArgs p) {
 template <bool GATE_UP, bool OUT_H>
 hipError_t launch_q4k_few(const Q4kArgs &p, int max_tiles, hipStream_t s) {
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols;
-    const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)((p.out_dim + kCols - 1) / kCols));
+    const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)(p.out_dim / kCols));
     launch_kernel(q4k_few_kernel<GATE_UP, OUT_H>, grid, dim3(64 * kWaves), kLdsBytes, s, p);
     return hipGetLastError();
 }

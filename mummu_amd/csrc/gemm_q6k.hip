@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q6k_down_kernel(const uint8_t 
     static_assert(!HALF || MT == 1, "tiles of 16 rows");
     // as xcd_tile in gemm.hip: an XCD takes neighbouring tiles, the slab running fastest; a workgroup takes every gridDim.x / 8 -th of its
     // XCD's items, and its loads run on from one into the next
-    const int n_slabs = (out_dim + kCols - 1) / kCols;
+    const int n_slabs = out_dim / kCols;   // (whole: grouped_gemm_q4k_f16)
     const int total = *n_tiles, per_xcd = (total + 7) >> 3, tile0 = (int)(blockIdx.x & 7) * per_xcd;
     const int n_items = n_slabs * (total - tile0 < per_xcd ? total - tile0 : per_xcd), apart = (int)(gridDim.x >> 3);
     const int first_item = (int)(blockIdx.x >> 3);
@@ -78,9 +78,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q6k_down_kernel(const uint8_t 
         w_base = uniform(w + (size_t)tile_of(w_item, 0) * (size_t)out_dim * row_bytes);
         const int at_lane = again(lane);
 #pragma unroll
-        for (int j = 0; j < kWLoads; j++) {   // (columns past the matrix repeat its last)
+        for (int j = 0; j < kWLoads; j++) {
             const int p = 64 * j + at_lane < 32 * kPieces ? 64 * j + at_lane : 0, col = first + p / kPieces;
-            w_off[j] = (uint32_t)(col < out_dim ? col : out_dim - 1) * row_bytes + (uint32_t)(p % kPieces) * 16u;
+            w_off[j] = (uint32_t)col * row_bytes + (uint32_t)(p % kPieces) * 16u;
         }
     };
     // Activation pieces: a load holds four rows of a plane, waves 0-3 load hi, 4-7 lo.  Piece q of row r lies at q ^ (r % 16): sixteen lanes
@@ -258,18 +258,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q6k_down_kernel(const uint8_t 
         for (int m = 0; m < MT; m++) fold_run(m, (which + 3) & 3);
         // element r of an accumulator: row 8 (r / 4) + 4 g + r % 4, column lane % 32
         const int p0 = tile_of(item, 1), rows = tile_of(item, 2), col = item % n_slabs * kCols + 32 * wave + again(c), g4 = 4 * again(g);
-        if (col < out_dim) {
-            float *to = y + (size_t)(p0 + g4) * (size_t)out_dim + (size_t)col;
+        float *to = y + (size_t)(p0 + g4) * (size_t)out_dim + (size_t)col;
 #pragma unroll
-            for (int m = 0; m < MT; m++)
+        for (int m = 0; m < MT; m++)
 #pragma unroll
-                for (int j = 0; j < ROWS / 4; j++) {
+            for (int j = 0; j < ROWS / 4; j++) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++, to += out_dim)
-                        if (32 * m + 8 * j + g4 + r < rows) *to = acc[m][4 * j + r];
-                    to += 4 * (size_t)out_dim;
-                }
-        }
+                for (int r = 0; r < 4; r++, to += out_dim)
+                    if (32 * m + 8 * j + g4 + r < rows) *to = acc[m][4 * j + r];
+                to += 4 * (size_t)out_dim;
+            }
 #pragma unroll
         for (int m = 0; m < MT; m++) acc[m] = run[m] = zero;
         s[1] = zero;
@@ -281,7 +279,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q6k_down_kernel(const uint8_t 
 template <int MT, bool HALF>
 hipError_t launch_q6k(const uint8_t *w, HAct a, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int in_dim, int out_dim, float *y,
                       hipStream_t s) {
-    const int per_xcd = (max_tiles + 7) / 8 * ((out_dim + kCols - 1) / kCols);
+    const int per_xcd = (max_tiles + 7) / 8 * (out_dim / kCols);
     const dim3 grid(8u * (unsigned)(per_xcd < kCusOfXcd ? per_xcd : kCusOfXcd));
     launch_kernel(q6k_down_kernel<MT, HALF>, grid, dim3(64 * kWaves), lds_bytes(MT), s, w, a, tiles, n_tiles, in_dim, out_dim, y);
     return hipGetLastError();

@@ -1,7 +1,7 @@
 """The grouped GEMMs of Q4_K banks on tiles of up to 64 and of up to 16 rows: experts whose rows end just before, at and just after each half of a tile,
 among experts without rows, against the f64 product of the dequantized weights.  One super-block to a row (the shortest loop over
-K), an odd number of them, and a last slab of columns that is half a slab.  The tolerance is the 3e-5 of the other
-forms on these units; Q6_K downs likewise."""
+K), an odd number of them, one to eight slabs of columns, which are whole (hidden and inter are multiples of 256 here).  The tolerance is
+the 3e-5 of the other forms on these units; Q6_K downs likewise."""
 import numpy as np
 import pytest
 
