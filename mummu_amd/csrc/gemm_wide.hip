@@ -16,7 +16,8 @@
 //   - Weights of bf16 become halfs beside the last products of the group before, not between their read and the next products.
 // What remains: the matrix units are busy for 52 / 38 % of the cycles at 4096 bf16 rows x 8, and the card lowers its clock as they
 // are: 15 % fewer cycles were 7 % of the time (340 / 206 us -> 316 / 194).
-// OLMoE shape, 4096 rows x 8: gate/up 503 -> 345 us, down 262 -> 190 us; 2048: 260 -> 207, 135 -> 112; 1000: 160 -> 141, 84 -> 82.
+// OLMoE shape, grouped_gemm_f16_kernel -> the loads in one go -> now, 4096 bf16 rows x 8: gate/up 503 -> 340 -> 316 us, down 262 -> 206 -> 194 (a trace of
+// it on its own; by events between launches 285 / 180, f16 270 / 174).
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -262,7 +263,7 @@ bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign) {
           (size_t)n_assign * (size_t)b.inter * 2 < (1ull << 32)))
         return false;
     // Up to 64 rows per expert either kernel streams the weights once, and the smaller workgroups of grouped_gemm_f16_kernel,
-    // several to a CU, do it better (OLMoE layers, 64 rows: 207 us there, 237 us here; 72: 256 / 245, 80: 260 / 249, 128: 325 / 276; 512
+    // several to a CU, do it better (this kernel with its loads still in one go; OLMoE layers, 64 rows: 207 us there, 237 us here; 72: 256 / 245, 80: 260 / 249, 128: 325 / 276; 512
     // experts of 2560 x 640, 64: 1852 / 1907, 72: 2195 / 2018; 128 of 2048 x 768, 64: 366 / 354, 72: 427 / 381; 16 of 4096 x 1792, 64: 411 /
     // 402, 72: 428 / 417, 128: 568 / 490).
     // One workgroup fills a CU here, so the line also asks for about as many of them as there are CUs.  The one smaller launch that

@@ -93,16 +93,23 @@ struct mummu_moe {
     int32_t *offsets = nullptr, *sorted = nullptr, *inv = nullptr, *tiles = nullptr, *n_tiles = nullptr, *disp_scratch = nullptr;
     void *act16 = nullptr;       // f16 [pairs, inter]
     int max_tiles = 0;
-    // batches at least this large take dispatch + grouped GEMM (measured crossovers on the OLMoE shape:
-    // the 16-bit float decode kernels lose from 7 tokens on, the f32 ones from 10, the integer ones from 19)
+    // Batches at least this large take dispatch + grouped GEMM.  Crossovers of the OLMoE shape with the batched kernels of their time (16-bit
+    // float banks lose on the decode kernels from 7 tokens on, f32 from 10, Q8_0 from 13, Q4_K from 18, the others from 19); with the present ones
+    // the lines of the block types are late, but for 128 experts.  us of a block by the decode / batched kernels, a call and the wait for it
+    // (three streams of calls, a pass):
+    //   Q4_K        64 experts (2048 x 1024, top-8)    10 tokens 72 / 82 (47 / 47), 13: 84 / 83 (57 / 50), 17: 97 / 86 (72 / 56)
+    //               128 (2048 x 768, top-8)            13: 85 / 95 (55 / 56), 18: 100 / 112 (71 / 66), 24: 118 / 121 (90 / 73)
+    //               16 (4096 x 1792, top-2)            8: 88 / 90 (62 / 49), 12: 105 / 95 (75 / 52), 17: 131 / 97 (99 / 54)
+    //               512 (2560 x 768, top-10)           8: 170 / 118 (148 / 76), 17: 325 / 172 (297 / 125)
+    //   Q4_K + Q6_K 64                                 14: 98 / 103 (71 / 70), 16: 105 / 105 (78 / 74), 18: 113 / 105 (87 / 75)
+    //               128                                18: 115 / 132 (85 / 86), 24: 136 / 146 (106 / 96)
+    //   Q4_K + Q5_1 512 (2560 x 640, top-10)           8: 144 / 112 (123 / 69), 18: 285 / 170 (262 / 121)
+    //   Q8_0        64                                 8: 108 / 116 (84 / 69), 10: 129 / 116 (100 / 77), 12: 144 / 118 (114 / 80)
+    //               128                                8: 95 / 114 (71 / 70), 10: 122 / 119 (89 / 77), 12: 137 / 129 (104 / 86)
+    //               16                                 8: 125 / 112 (97 / 78), 12: 179 / 119 (143 / 83)
     int gemm_min_f16 = 7, gemm_min_quant = 19, gemm_min_f32 = 10;
-    // Q8_0 banks on the f16 units: us of the batched against the decode kernels at 10 / 12 / 13 / 14 / 18 tokens, 64 experts (2048 x
-    // 1024, top-8) 121 / 125 / 127 / 127 / 132 against 109 / 129 / 138 / 145 / 175, 16 (4096 x 1792, top-2) 112 / 113 / 114 / 114 / 120
-    // against 126 / 143 / 163 / 173 / 222, 512 (2560 x 640, top-10) 174 / 219 / 223 / 230 / 285 against 206 / 245 / 264 / 277 / 352.  The
-    // line is late for the last and early for 128 experts (2048 x 768, top-8: 119 / 133 / 137 / 141 / 171 against 97 / 116 / 127 / 136 /
-    // 162, alike from 19), where the batched kernels' results are a hundred times nearer the 64-bit ones.
     int gemm_min_q8 = 13;
-    int gemm_min_q4k = 18;   // Q4_K banks on the f16 units (17 tokens: 88.8 us either way; 18: 89.1 against 92.6 us)
+    int gemm_min_q4k = 18;
     int gemm_q4k_f16 = 1;        // Q4_K banks of the batched path on the f16 units (0: the int8 form)
     int gemm_q8_f16 = 0;         // 1: Q8_0 banks of the batched path through the f16 kernel (x and activations as halfs)
     int gemm_tile_rows = 0;          // 0: chosen per batch; else forced (f16-unit Q4_K kernels)
