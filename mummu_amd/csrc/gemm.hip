@@ -131,6 +131,10 @@ __global__ __launch_bounds__(256) void grouped_gemm_f16_kernel(
     if (!xcd_tile(n_tiles, (out_dim + kBN - 1) / kBN, tile, slab)) return;
     const int e = tiles[3 * tile], p0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
     const int n0 = slab * kBN;
+    // An expert with one tile: every line of its weights is read once, past the caches' order of use ("nt"), where they would push out
+    // the rows that the slabs of a tile share (OLMoE f16, a layer, us, without / with: 20 tokens 128 / 118, 128: 147 / 132, 512: 179 / 164; gate/up at
+    // 512 fetched 632 MB for 537 of weights).  Lines that a second tile reads again lose by it, and those read in pieces (Q8_0).
+    const bool once = !Q8 && (tile == 0 || tiles[3 * tile - 3] != e) && (tile + 1 == *n_tiles || tiles[3 * tile + 3] != e);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     static_assert(WT == T_F16 || WT == T_BF16 || WT == T_Q8_0, "banks this kernel reads");
     const size_t row_bytes = Q8 ? (size_t)(in_dim / 32) * 34 : (size_t)in_dim * 2;
@@ -174,7 +178,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_f16_kernel(
 
     u32x4 rb[NB][4];
     u32x4 ra16[A_PASSES];
-    auto fetch = [&](int k0) {
+    auto fetch = [&](int k0, auto read_once) {
 #pragma unroll
         for (int b = 0; b < NB; b++)
 #pragma unroll
@@ -189,7 +193,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_f16_kernel(
                     __builtin_memcpy(&db, p - (2 + 8 * (b_chunk & 3)), 2);
                     rb[b][i] = u32x4{c0, c1, (uint32_t)db, 0u};
                 } else {
-                    rb[b][i] = *(const u32x4 *)(b_ptr[b][i] + (size_t)k0 * 2);
+                    const u32x4 *from = (const u32x4 *)(b_ptr[b][i] + (size_t)k0 * 2);
+                    rb[b][i] = read_once ? __builtin_nontemporal_load(from) : *from;
                 }
             }
 #pragma unroll
@@ -205,67 +210,71 @@ __global__ __launch_bounds__(256) void grouped_gemm_f16_kernel(
     const int n_slabs = (out_dim + kBN - 1) / kBN;
     const int rot = (slab * (n_steps / n_slabs > 0 ? n_steps / n_slabs : 1)) % n_steps;
     auto step_k0 = [&](int step) { return ((step + rot) % n_steps) * kBK; };
-    fetch(step_k0(0));
-
     MUMMU_TIMER_DECL;
-    for (int step = 0; step < n_steps; step++) {
-        MUMMU_TIMER_MARK(0);
-        // registers -> LDS
+    auto multiply = [&](auto read_once) {
+        fetch(step_k0(0), read_once);
+
+        for (int step = 0; step < n_steps; step++) {
+            MUMMU_TIMER_MARK(0);
+            // registers -> LDS
 #pragma unroll
-        for (int b = 0; b < NB; b++)
+            for (int b = 0; b < NB; b++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                u32x4 v = rb[b][i];
-                if constexpr (Q8) {
-                    *(uint2 *)&s_q[b][(tid >> 3) + 32 * i][b_chunk * 8] = make_uint2(v[0], v[1]);
-                    if ((b_chunk & 3) == 0) {
-                        const uint16_t db = (uint16_t)v[2];
-                        __builtin_memcpy(&s_d[b][(tid >> 3) + 32 * i][b_chunk >> 2], &db, 2);
+                for (int i = 0; i < 4; i++) {
+                    u32x4 v = rb[b][i];
+                    if constexpr (Q8) {
+                        *(uint2 *)&s_q[b][(tid >> 3) + 32 * i][b_chunk * 8] = make_uint2(v[0], v[1]);
+                        if ((b_chunk & 3) == 0) {
+                            const uint16_t db = (uint16_t)v[2];
+                            __builtin_memcpy(&s_d[b][(tid >> 3) + 32 * i][b_chunk >> 2], &db, 2);
+                        }
+                        continue;
                     }
-                    continue;
-                }
-                if (BF16) {
+                    if (BF16) {
 #pragma unroll
-                    for (int q = 0; q < 4; q++) v[q] = pack_half2(__uint_as_float(v[q] << 16), __uint_as_float(v[q] & 0xFFFF0000u));
+                        for (int q = 0; q < 4; q++) v[q] = pack_half2(__uint_as_float(v[q] << 16), __uint_as_float(v[q] & 0xFFFF0000u));
+                    }
+                    *(u32x4 *)&s_b[b][(tid >> 3) + 32 * i][b_chunk * 8] = v;
                 }
-                *(u32x4 *)&s_b[b][(tid >> 3) + 32 * i][b_chunk * 8] = v;
+#pragma unroll
+            for (int p = 0; p < A_PASSES; p++) *(u32x4 *)&s_a[a_row[p]][a_col] = ra16[p];
+            MUMMU_TIMER_MARK(1);
+            __syncthreads();
+            MUMMU_TIMER_MARK(2);
+            if (step + 1 < n_steps) fetch(step_k0(step + 1), read_once);
+            MUMMU_TIMER_MARK(3);
+            // multiply: wave owns columns 32*wave .. +31
+#pragma unroll
+            for (int kk = 0; kk < kBK / 16; kk++) {
+                half8 bfrag[NB], bfrag_lo[NB];
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    if constexpr (Q8) {
+                        const uint2 c = *(const uint2 *)&s_q[b][32 * wave + (lane & 31)][kk * 16 + (lane >> 5) * 8];
+                        q8_half_planes(c.x, c.y, s_d[b][32 * wave + (lane & 31)][kk >> 1], bfrag[b], bfrag_lo[b]);
+                    } else {
+                        bfrag[b] = *(const half8 *)&s_b[b][32 * wave + (lane & 31)][kk * 16 + (lane >> 5) * 8];
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    const half8 afrag = *(const half8 *)&s_a[32 * m + (lane & 31)][kk * 16 + (lane >> 5) * 8];
+#pragma unroll
+                    for (int b = 0; b < NB; b++) acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag, bfrag[b], acc[b][m], 0, 0, 0);
+                    if constexpr (Q8) {
+#pragma unroll
+                        for (int b = 0; b < NB; b++)
+                            acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag, bfrag_lo[b], acc[b][m], 0, 0, 0);
+                    }
+                }
             }
-#pragma unroll
-        for (int p = 0; p < A_PASSES; p++) *(u32x4 *)&s_a[a_row[p]][a_col] = ra16[p];
-        MUMMU_TIMER_MARK(1);
-        __syncthreads();
-        MUMMU_TIMER_MARK(2);
-        if (step + 1 < n_steps) fetch(step_k0(step + 1));
-        MUMMU_TIMER_MARK(3);
-        // multiply: wave owns columns 32*wave .. +31
-#pragma unroll
-        for (int kk = 0; kk < kBK / 16; kk++) {
-            half8 bfrag[NB], bfrag_lo[NB];
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                if constexpr (Q8) {
-                    const uint2 c = *(const uint2 *)&s_q[b][32 * wave + (lane & 31)][kk * 16 + (lane >> 5) * 8];
-                    q8_half_planes(c.x, c.y, s_d[b][32 * wave + (lane & 31)][kk >> 1], bfrag[b], bfrag_lo[b]);
-                } else {
-                    bfrag[b] = *(const half8 *)&s_b[b][32 * wave + (lane & 31)][kk * 16 + (lane >> 5) * 8];
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-                const half8 afrag = *(const half8 *)&s_a[32 * m + (lane & 31)][kk * 16 + (lane >> 5) * 8];
-#pragma unroll
-                for (int b = 0; b < NB; b++) acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag, bfrag[b], acc[b][m], 0, 0, 0);
-                if constexpr (Q8) {
-#pragma unroll
-                    for (int b = 0; b < NB; b++)
-                        acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag, bfrag_lo[b], acc[b][m], 0, 0, 0);
-                }
-            }
+            MUMMU_TIMER_MARK(4);
+            __syncthreads();
+            MUMMU_TIMER_MARK(5);
         }
-        MUMMU_TIMER_MARK(4);
-        __syncthreads();
-        MUMMU_TIMER_MARK(5);
-    }
+    };
+    if (once) multiply(std::true_type());
+    else multiply(std::false_type());
     MUMMU_TIMER_STORE;
 
     const int n = n0 + 32 * wave + (lane & 31);
