@@ -1,0 +1,283 @@
+// Grouped GEMM of Q4_K banks on the f16 units for a few rows per expert: the operands and arithmetic of gemm_q4k.hip on tiles of up to 8 or
+// 16 rows (v_mfma_f32_16x16x32_f16).  A wave keeps ONE super-block of K of the tile's rows in registers and takes the weights of 16 columns
+// after 16 of it from memory straight into the registers that multiply them; the waves of a workgroup have the super-blocks of a row side by
+// side, so that together they read whole rows front to back, and their sums meet in LDS in ascending order.  Tiles of 8 rows hold the high
+// halfs in the operand's first eight rows and the low ones in the others: one product where 16 rows take two.
+//
+// What bounds it: the vector ALUs and the stream, neither wholly beside the other.  Every line of the weights is fetched once (128 experts of 2048 x 768, 27
+// tokens: 177 MB where the 144-byte pieces of gemm_q4k_few.hip fetch 1.38 times that), 16 columns of a super-block take 109 vector
+// instructions (two for a pair of codes) and nine products, and a CU's 16 to 20 waves keep 75 to 110 KB on the way.  Gate/up of that shape
+// 51 -> 48 us, of 512 experts of 2560 x 640 with 64 tokens 176 -> 167, with the loads alone 43 and 133, with the weights out of L2 45 and 139;
+// OLMoE, 20 tokens, 38.7 -> 37.2 + 23.5 -> 20.9.  Layers among others: 72.4 -> 67.6, 272 -> 262, 57.0 -> 52.1; 512 experts of 2048 x 768, 60
+// tokens 237 -> 206, 128 of 3072 x 768, 30 tokens 117 -> 103.
+#include "device_utils.h"
+#include "kernels.h"
+#include "q4k_half.h"
+#include "qact.h"
+
+namespace mummu {
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBlock = 144;
+constexpr int kUnits = 4;            // 16 columns of one matrix each: between two meetings of the sums
+constexpr int kRowC = 128 + 4;       // f32 row of the gate/up epilogue
+
+struct StreamArgs {
+    Q4kArgs q;
+    int cols;   // columns of a workgroup
+};
+
+template <bool R8>
+constexpr size_t stream_lds(int waves, bool gate_up) {
+    const int rows = R8 ? 8 : 16;
+    return (size_t)2 * kUnits * (size_t)waves * (size_t)rows * 64 + 64 + (gate_up ? (size_t)rows * kRowC * 4 : 0);
+}
+
+// Workgroup: one wave to a super-block of K, times n_groups of them side by side where a row has one or two; group g of a step has columns
+// 16 (step n_groups + g) .. + 15 of the workgroup's.
+template <bool GATE_UP, bool OUT_H, bool R8, int MAXW, int PER_SIMD, int DEPTH>
+__global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];
+    const Q4kArgs &p = a.q;
+    constexpr int kRows = R8 ? 8 : 16, kTile = kRows * 16, NB = GATE_UP ? 2 : 1, kSteps = kUnits / NB;
+    // As xcd_tile in gemm.hip: an XCD takes neighbouring tiles with the slab running fastest.
+    const int n_slabs = p.out_dim / a.cols;
+    const int total = *p.n_tiles, per_xcd = (total + 7) >> 3;
+    const int item = (int)(blockIdx.x >> 3);
+    const int within = item / n_slabs, slab = item - within * n_slabs;
+    const int tile = (int)(blockIdx.x & 7) * per_xcd + within;
+    if (within >= per_xcd || tile >= total) return;
+    const int e = uniform(p.tiles[3 * tile]), p0 = uniform(p.tiles[3 * tile + 1]), rows = uniform(p.tiles[3 * tile + 2]);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 15, kg = lane >> 4;
+    const int n_waves = (int)blockDim.x >> 6, n_sb = p.in_dim / 256, n_groups = n_waves / n_sb;
+    const int group = wave / n_sb, sb = wave - group * n_sb;
+    const uint32_t row_bytes = (uint32_t)n_sb * kBlock;
+    float *s_sum = (float *)s_lds;                                      // [2][unit][wave][kTile]
+    float *s_scale = s_sum + 2 * kUnits * n_waves * kTile;              // [16]
+    float *s_c = s_scale + 16;
+
+    // the row that this lane multiplies (rows past the last repeat it: multiplied, never stored)
+    const int my = R8 ? (c & 7) : c, my_row = my < rows ? my : rows - 1;
+    int source = p0 + my_row;
+    if (GATE_UP) source = p.sorted[p0 + my_row];
+
+    // weights: 64 neighbouring bytes of a super-block's codes by the four lanes of a row, twice, and its header
+    const size_t matrix = (size_t)e * (size_t)p.out_dim * row_bytes;
+    const int col0 = slab * a.cols + 16 * group, n_steps = a.cols / (16 * n_groups);
+    typedef __attribute__((address_space(1))) const uint8_t Global;   // (an address put together from scalars would be a flat one)
+    Global *base[NB];
+    base[0] = (Global *)uniform(p.w0 + matrix + (size_t)col0 * row_bytes);
+    if (GATE_UP) base[NB - 1] = (Global *)uniform(p.w1 + matrix + (size_t)col0 * row_bytes);
+    const uint32_t off_h = (uint32_t)c * row_bytes + (uint32_t)sb * kBlock, off_q = off_h + 16u + 16u * (uint32_t)kg;
+    const uint32_t step_bytes = 16u * (uint32_t)n_groups * row_bytes;
+    u32x4 hd[DEPTH], q0[DEPTH], q1[DEPTH];   // DEPTH - 1 of them on their way
+    auto load = [&](int step, int j, int to) {
+        Global *from = base[j] + (size_t)((uint32_t)step * step_bytes);
+        typedef __attribute__((address_space(1))) const u32x4 Words;
+        hd[to] = *(Words *)(from + off_h);
+        q0[to] = *(Words *)(from + off_q);
+        q1[to] = *(Words *)(from + off_q + 64);
+    };
+    MUMMU_CODE_FENCE();
+#pragma unroll
+    for (int u = 0; u < DEPTH - 1; u++) load(u / NB, u % NB, u);
+    MUMMU_CODE_FENCE();
+    if (GATE_UP) source /= p.k_slots;
+
+    // x: piece i of a plane = 8 elements; load l, half h, nibble n of the codes above meet piece 4 (4 l + 2 (kg / 2) + n) + 2 (kg % 2) + h
+    constexpr int kPlanes = R8 ? 1 : 2;
+    half8 x[kPlanes][2][2][2];
+    {
+        const uint32_t at = (uint32_t)(8 * (kg >> 1) + 2 * (kg & 1)) * 16u;
+        const size_t row_at = ((size_t)source * (size_t)p.in_dim + (size_t)sb * 256) * 2;
+#pragma unroll
+        for (int pl = 0; pl < kPlanes; pl++) {
+            const uint8_t *plane = (const uint8_t *)(R8 ? (c < 8 ? p.a.hi : p.a.lo) : (pl == 0 ? p.a.hi : p.a.lo)) + row_at;
+#pragma unroll
+            for (int l = 0; l < 2; l++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int n = 0; n < 2; n++) x[pl][l][h][n] = *(const half8 *)(plane + at + (uint32_t)((16 * l + 4 * n + h) * 16));
+        }
+    }
+    // sums of 32 elements as pairs of halfs: gate/up K = 16 (high of sub-blocks 0-3, 4-7, low of both), down K = 8 for either half
+    half4v am[GATE_UP ? 1 : 2];
+    float sr[GATE_UP ? 1 : 2][4];
+    {
+        const float *ss = p.a.ssum + (size_t)source * (size_t)(p.in_dim / 32) + (size_t)sb * 8;
+        const bool low = GATE_UP ? kg >= 2 : kg == 1, none = (R8 && c >= 8) || (!GATE_UP && kg >= 2);
+#pragma unroll
+        for (int l = 0; l < (GATE_UP ? 1 : 2); l++) {
+            const float4 v = *(const float4 *)(ss + (GATE_UP ? 4 * (kg & 1) : 4 * l));
+            const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const _Float16 hi = (_Float16)f[i], lo = (_Float16)__fsub_rn(f[i], (float)hi);
+                am[l][i] = none ? (_Float16)0.0f : low ? lo : hi;
+            }
+        }
+        if (GATE_UP) {
+            if (wave == 0 && lane < kRows) s_scale[lane] = p.a.scale[(size_t)source * (size_t)(p.in_dim / 128)];
+        } else {
+            // (element r of an accumulator: row 4 kg + r; of eight rows 4 (kg % 2) + r)
+#pragma unroll
+            for (int l = 0; l < 2; l++) {
+                const float s = p.a.scale[(size_t)source * (size_t)(p.in_dim / 128) + (size_t)sb * 2 + l];
+#pragma unroll
+                for (int r = 0; r < 4; r++) sr[l][r] = __shfl(s, 4 * (R8 ? kg & 1 : kg) + r, 64);
+            }
+        }
+    }
+
+    const f32x4 zero = {0, 0, 0, 0};
+    const uint32_t pick = kg >= 2 ? 0x04030402u : 0x04010400u;   // this lane's two sub-blocks of four
+    auto multiply = [&](int b, float *to) {
+        Q4kHeader head;
+        head.unpack(hd[b]);
+        f32x4 v = zero, c1 = zero;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const uint32_t t = __builtin_amdgcn_perm(0x64646464u, head.sc4[l], pick);
+            half2v m;
+            __builtin_memcpy(&m, &t, 4);
+            m = (m - half2v{(_Float16)1024.0f, (_Float16)1024.0f}) * half2v{(_Float16)1024.0f, (_Float16)64.0f};
+            const half2v ml = {m[0], m[0]}, mh = {m[1], m[1]};
+            const u32x4 q = l == 0 ? q0[b] : q1[b];
+            if (!GATE_UP) c1 = zero;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const half8 w[2] = {q4k_operand<false>(q[2 * h], q[2 * h + 1], ml), q4k_operand<true>(q[2 * h], q[2 * h + 1], mh)};
+#pragma unroll
+                for (int n = 0; n < 2; n++)
+#pragma unroll
+                    for (int pl = 0; pl < kPlanes; pl++) c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[pl][l][h][n], w[n], c1, 0, 0, 0);
+            }
+            if (!GATE_UP || l == 1) {
+                Q4kHeader h = head;
+                if (GATE_UP) h.mn4[0] = kg & 1 ? h.mn4[1] : h.mn4[0];
+                const f32x4 c2 = __builtin_amdgcn_mfma_f32_16x16x16f16(am[GATE_UP ? 0 : l], h.offsets(GATE_UP ? 0 : l), zero, 0, 0, 0);
+                const float fd = head.d(), fm = head.minus_dmin();
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float t = fmaf(fm, c2[r], __fmul_rn(fd, c1[r]));
+                    v[r] = GATE_UP ? t : l == 0 ? __fmul_rn(t, sr[0][r]) : fmaf(t, sr[GATE_UP ? 0 : 1][r], v[r]);
+                }
+            }
+        }
+        if constexpr (R8) {
+            // rows 4 (kg % 2) + (kg / 2), + 2: high + low
+            ((float2 *)to)[lane] = make_float2(swap32_add(v[0], v[1]), swap32_add(v[2], v[3]));
+        } else {
+            ((f32x4 *)to)[lane] = v;
+        }
+    };
+
+    const int n_phases = n_steps / kSteps;
+    auto phase = [&](int ph, auto last) {
+        float *sums = s_sum + (ph & 1) * kUnits * n_waves * kTile;
+#pragma unroll
+        for (int u = 0; u < kUnits; u++) {
+            const int ahead = u + DEPTH - 1;
+            if (!decltype(last)::value || ahead < kUnits) load(ph * kSteps + ahead / NB, ahead % NB, ahead % DEPTH);
+            MUMMU_CODE_FENCE();
+            multiply(u % DEPTH, sums + (u * n_waves + wave) * kTile);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int n_out = kSteps * n_groups * kTile;
+        // (the waves take turns where not all have some)
+        for (int i = (tid + (ph & 1) * 32 * n_waves) % (64 * n_waves); i < n_out; i += 64 * n_waves) {
+            const int block = i / kTile, d = i % kTile, ln = R8 ? d >> 1 : d >> 2, step = block / n_groups, g = block - step * n_groups;
+            const int row = R8 ? 4 * ((ln >> 4) & 1) + 2 * (d & 1) + (ln >> 5) : 4 * (ln >> 4) + (d & 3);
+            auto sum_of = [&](int u) {
+                const float *from = sums + (u * n_waves + g * n_sb) * kTile + d;
+                float s = 0.0f;
+                for (int k0 = 0; k0 < n_sb; k0 += 8) {
+                    float v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) v[k] = from[(k0 + k < n_sb ? k0 + k : 0) * kTile];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) s = k0 + k < n_sb ? __fadd_rn(s, v[k]) : s;
+                }
+                return s;
+            };
+            const int col = 16 * ((ph * kSteps + step) * n_groups + g) + (ln & 15);
+            if constexpr (GATE_UP) {
+                const float gate = __fmul_rn(s_scale[row], sum_of(2 * step)), up = __fmul_rn(s_scale[row], sum_of(2 * step + 1));
+                s_c[row * kRowC + col] = __fmul_rn(silu_of(gate), up);
+            } else {
+                const float v = sum_of(step);
+                if (row < rows) p.y[(size_t)(p0 + row) * (size_t)p.out_dim + (size_t)(slab * a.cols + col)] = v;
+            }
+        }
+    };
+    for (int ph = 0; ph < n_phases - 1; ph++) phase(ph, std::false_type());
+    phase(n_phases - 1, std::true_type());
+
+    if constexpr (GATE_UP) {
+        // silu(g) * u in the form the down product reads
+        __syncthreads();
+        for (int i = tid; i < kRows * 32; i += 64 * n_waves) {
+            if constexpr (OUT_H) {
+                const int row = i >> 5, c32 = i & 31;
+                const float4 v = *(const float4 *)&s_c[row * kRowC + 4 * c32];
+                const bool active = row < rows;
+                hact_store128(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, p.act_h, (size_t)(p0 + row), p.out_dim, slab * 128 + 4 * c32);
+            } else {
+                const int row = i >> 5, cb = (i >> 4) & 1;
+                const float4 v = *(const float4 *)&s_c[row * kRowC + cb * 64 + 4 * c];
+                const bool active = row < rows;
+                quantize_store64(active ? v : make_float4(0.f, 0.f, 0.f, 0.f), active, p.act_q, (size_t)(p0 + row), p.out_dim,
+                                 slab * 128 + cb * 64 + 4 * c);
+            }
+        }
+    }
+}
+
+template <bool GATE_UP, bool OUT_H, bool R8>
+hipError_t launch_stream(const Q4kArgs &q, int max_tiles, hipStream_t s) {
+    const int n_sb = q.in_dim / 256, groups = n_sb >= 3 ? 1 : n_sb == 2 ? 2 : 4, waves = n_sb * groups;
+    StreamArgs a{q, 128};   // (gate/up: what a scale of its output covers; down: the more, the less often rows are read into registers)
+    if (!GATE_UP) a.cols = q.out_dim % (256 * groups) == 0 ? 256 * groups : q.out_dim % (128 * groups) == 0 ? 128 * groups : 64 * groups;
+    if (n_sb < 1 || n_sb > kQ4kStreamBlocks || q.in_dim % 256 != 0 || q.out_dim % a.cols != 0) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)(q.out_dim / a.cols)), block(64 * waves);
+    const size_t lds = stream_lds<R8>(waves, GATE_UP);
+    if constexpr (R8) {
+        if (waves <= 6 || waves == 9 || waves == 10) {   // five waves a SIMD hold one workgroup more than four
+            launch_kernel(q4k_stream_kernel<GATE_UP, OUT_H, R8, 10, 5, 2>, grid, block, lds, s, a);
+            return hipGetLastError();
+        }
+    }
+    launch_kernel(q4k_stream_kernel<GATE_UP, OUT_H, R8, 16, 4, R8 ? 4 : 2>, grid, block, lds, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Tiles of 16 rows keep 64 registers of rows, four waves a SIMD: taken where workgroups of one wave to a super-block fill those.
+// us a layer among others, here / gemm_q4k_few.hip: OLMoE 24 / 64 tokens 57.7 / 58.8, 61.8 / 64.2, 512 experts of 2048 x 768, 40 / 128 tokens 177 / 189,
+// 302 / 316; hidden 2560 365 / 349, 4096 283 / 280, 1536 46.5 / 43.8, three super-blocks alike.
+bool q4k_stream_takes(int in_dim, int out_dim, int tile_rows) {
+    const int n_sb = in_dim / 256;
+    if (in_dim % 256 != 0 || out_dim % 128 != 0) return false;
+    return tile_rows <= 8 ? n_sb <= kQ4kStreamBlocks : n_sb == 4 || n_sb == 8;
+}
+
+hipError_t launch_q4k_stream_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
+                                     int max_tiles, int tile_rows, HAct act_h, QAct64 act_q, hipStream_t s) {
+    const Q4kArgs p{b.gate, b.up, x, sorted, tiles, n_tiles, k_slots, b.hidden, b.inter, act_h, act_q, nullptr};
+    if (tile_rows <= 8) return act_h.hi != nullptr ? launch_stream<true, true, true>(p, max_tiles, s) : launch_stream<true, false, true>(p, max_tiles, s);
+    return act_h.hi != nullptr ? launch_stream<true, true, false>(p, max_tiles, s) : launch_stream<true, false, false>(p, max_tiles, s);
+}
+
+hipError_t launch_q4k_stream_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows,
+                                  float *y, hipStream_t s) {
+    const Q4kArgs p{b.down, nullptr, act, nullptr, tiles, n_tiles, 1, b.inter, b.hidden, HAct(), QAct64(), y};
+    return tile_rows <= 8 ? launch_stream<false, true, true>(p, max_tiles, s) : launch_stream<false, true, false>(p, max_tiles, s);
+}
+
+}  // namespace mummu

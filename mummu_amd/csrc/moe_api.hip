@@ -311,7 +311,7 @@ int ensure_ws(mummu_moe *h, int64_t n, int64_t n_assign, int n_experts) {
     HIPCHK(h, hipMalloc(&h->actq.lo, ae));
     HIPCHK(h, hipMalloc(&h->actq.scale, sizeof(float) * (ae / 16)));
     HIPCHK(h, hipMalloc(&h->actq.sum, sizeof(int32_t) * (ae / 16)));
-    h->max_tiles = n_experts + (int)((na + 15) / 16) + 1;   // (the smallest tiles have 16 rows)
+    h->max_tiles = n_experts + (int)((na + 7) / 8) + 1;   // (the smallest tiles have 8 rows)
     HIPCHK(h, hipMalloc(&h->offsets, sizeof(int32_t) * (size_t)(n_experts + 1)));
     HIPCHK(h, hipMalloc(&h->sorted, sizeof(int32_t) * (size_t)na));
     HIPCHK(h, hipMalloc(&h->inv, sizeof(int32_t) * (size_t)na));
@@ -1129,10 +1129,10 @@ int mummu_moe_create(const mummu_moe_config *cfg, mummu_moe **out) {
     // 1.5e-3 by the reference's measure where that has 2e-4 and the pairs of halfs of gemm_q8.hip 1e-6 - which is why it is not the
     // default)
     if (const char *e = getenv("MUMMU_GEMM_Q8_F16")) h->gemm_q8_f16 = atoi(e) != 0;
-    // MUMMU_GEMM_TILE_ROWS=16 | 32 | 64: rows per tile of the f16-unit Q4_K kernels (default: by expected cost)
+    // MUMMU_GEMM_TILE_ROWS=8 | 16 | 32 | 64: rows per tile of the f16-unit Q4_K kernels (default: by expected cost)
     if (const char *e = getenv("MUMMU_GEMM_TILE_ROWS")) {
         const int v = atoi(e);
-        if (v == 16 || v == 32 || v == 64) h->gemm_tile_rows = v;
+        if (v == 8 || v == 16 || v == 32 || v == 64) h->gemm_tile_rows = v;
     }
     // MUMMU_GEMM_MIN_TOKENS: smallest batch that takes dispatch + grouped GEMM instead of the decode kernels
     if (const char *e = getenv("MUMMU_GEMM_MIN_TOKENS")) {

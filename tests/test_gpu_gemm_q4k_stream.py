@@ -1,0 +1,37 @@
+"""Grouped GEMM of Q4_K banks on tiles of up to 8 rows: every row count around a tile's end, one super-block to a row up to sixteen (each number of
+waves that a workgroup has its own share of columns for), in front of down banks of its own type, of Q6_K and of the int8 units' types; against
+the f64 product of the dequantized weights."""
+import numpy as np
+import pytest
+
+from mummu_amd import moe as M
+from mummu_amd import synth
+from oracle import binding as orc
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = [0, 1, 7, 8, 9, 0, 15, 16, 17, 2]
+
+
+@pytest.mark.parametrize("H,I,down", [(256, 256, "Q4_K"), (512, 768, "Q4_K"), (768, 512, "Q4_K"), (1024, 1280, "Q4_K"), (1280, 2560, "Q4_K"),
+                                      (1792, 2816, "Q4_K"), (2304, 256, "Q4_K"), (2048, 1024, "Q6_K"), (2560, 640, "Q5_1"), (4096, 1536, "Q4_K"),
+                                      (1536, 4096, "Q4_K")])
+def test_tiles_of_8_rows(monkeypatch, H, I, down):
+    if down != "Q5_1":
+        monkeypatch.setenv("MUMMU_GEMM_TILE_ROWS", "8")   # (in front of int8 downs: by the rows of an expert, below)
+    monkeypatch.setenv("MUMMU_GEMM_MIN_TOKENS", "1")
+    counts = COUNTS if down != "Q5_1" else [c % 8 for c in COUNTS]
+    E, n = len(counts), sum(counts)
+    rng = np.random.Generator(np.random.PCG64(H + I))
+    gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (61, 62))
+    downs = synth.random_bank_fast(getattr(M, down), [I, H, E], 63)
+    ids = np.repeat(np.arange(E), counts)[rng.permutation(n)].astype(np.int32)[:, None]
+    x = rng.standard_normal((n, H), dtype=np.float32) * np.exp2(rng.integers(-12, 1, (n, 1))).astype(np.float32)
+    w = rng.random((n, 1), dtype=np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q4_K, up, M.Q4_K, downs, getattr(M, down))
+        got, again = m.apply_routing(0, ids, w, x), m.apply_routing(0, ids, w, x)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, downs, orc.Q4_K, orc.Q4_K, getattr(orc, down)), ids, w, x)
+    # (as the other forms on these units; in front of an int8 down product 16 bits and a scale per 64, the bar of experts.rs:1264-1271)
+    assert orc.rel_err(got, want, mag).max() <= (2e-3 if down == "Q5_1" else 3e-5)
