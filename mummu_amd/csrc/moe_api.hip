@@ -93,23 +93,12 @@ struct mummu_moe {
     int32_t *offsets = nullptr, *sorted = nullptr, *inv = nullptr, *tiles = nullptr, *n_tiles = nullptr, *disp_scratch = nullptr;
     void *act16 = nullptr;       // f16 [pairs, inter]
     int max_tiles = 0;
-    // Batches at least this large take dispatch + grouped GEMM.  Crossovers of the OLMoE shape with the batched kernels of their time (16-bit
-    // float banks lose on the decode kernels from 7 tokens on, f32 from 10, Q8_0 from 13, Q4_K from 18, the others from 19); with the present ones
-    // the lines of the block types are late, but for 128 experts.  us of a block by the decode / batched kernels, a call and the wait for it
-    // (three streams of calls, a pass):
-    //   Q4_K        64 experts (2048 x 1024, top-8)    10 tokens 72 / 82 (47 / 47), 13: 84 / 83 (57 / 50), 17: 97 / 86 (72 / 56)
-    //               128 (2048 x 768, top-8)            13: 85 / 95 (55 / 56), 18: 100 / 112 (71 / 66), 24: 118 / 121 (90 / 73)
-    //               16 (4096 x 1792, top-2)            8: 88 / 90 (62 / 49), 12: 105 / 95 (75 / 52), 17: 131 / 97 (99 / 54)
-    //               512 (2560 x 768, top-10)           8: 170 / 118 (148 / 76), 17: 325 / 172 (297 / 125)
-    //   Q4_K + Q6_K 64                                 14: 98 / 103 (71 / 70), 16: 105 / 105 (78 / 74), 18: 113 / 105 (87 / 75)
-    //               128                                18: 115 / 132 (85 / 86), 24: 136 / 146 (106 / 96)
-    //   Q4_K + Q5_1 512 (2560 x 640, top-10)           8: 144 / 112 (123 / 69), 18: 285 / 170 (262 / 121)
-    //   Q8_0        64                                 8: 108 / 116 (84 / 69), 10: 129 / 116 (100 / 77), 12: 144 / 118 (114 / 80)
-    //               128                                8: 95 / 114 (71 / 70), 10: 122 / 119 (89 / 77), 12: 137 / 129 (104 / 86)
-    //               16                                 8: 125 / 112 (97 / 78), 12: 179 / 119 (143 / 83)
+    // Batches at least this large take dispatch + grouped GEMM: where the two met on the OLMoE shape (16-bit float banks lose on the decode kernels
+    // from 7 tokens on, f32 from 10, Q8_0 from 13, Q4_K from 18, the others from 19).  Banks on the f16 units go by what they read as well: batched_from.
     int gemm_min_f16 = 7, gemm_min_quant = 19, gemm_min_f32 = 10;
     int gemm_min_q8 = 13;
     int gemm_min_q4k = 18;
+    bool gemm_min_given = false;     // MUMMU_GEMM_MIN_TOKENS: the lines as they are
     int gemm_q4k_f16 = 1;        // Q4_K banks of the batched path on the f16 units (0: the int8 form)
     int gemm_q8_f16 = 0;         // 1: Q8_0 banks of the batched path through the f16 kernel (x and activations as halfs)
     int gemm_tile_rows = 0;          // 0: chosen per batch; else forced (f16-unit Q4_K kernels)
@@ -490,13 +479,31 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 // experts of an already-made routing: gate/up -> down -> combine.  x_quantized says h->xq
 // already holds the 16-bit form of x (the fused router produced it).
 // Smallest batch of this layer that takes the batched path (INT_MAX: never).
+//
+// gemm_min_*: where the two forms meet on the OLMoE shape with nothing else to go by.  Banks that take the f16 units (Q4_K gate and up, Q8_0)
+// meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and `from` tokens: below, they have fewer
+// launches) the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode against batched:
+//   Q4_K, OLMoE 11 tokens (311 MB) 80 / 48 against 80 / 44, 15: 94 / 62 against 82 / 47; 128 experts of 2048 x 768, 16 (339 MB): 96 / 63 against
+//   94 / 54; 512 of them top-10, 12 (318 MB): 133 / 104 against 123 / 72.
+//   Q4_K with other downs, OLMoE Q6_K, 14 / 16 tokens (456 / 522 MB): 100 / 70, 108 / 78 against 104 / 64, 104 / 73; Q5_1, 15 (472 MB): 98 / 64 against 93 / 57.
+//   Q8_0, OLMoE, 8 / 9 tokens (428 / 481 MB): 108 / 83, 124 / 90 against 118 / 70, 120 / 73; 128 experts of 2048 x 768, 12 (481 MB): 137 / 105 against 137 / 88.
+// Rows of more than 2048 elements are more than a wave's 64 blocks of 32, and the decode kernels take two a lane, some of them none:
+//   hidden 2560: 512 experts of 640 with Q5_1 downs, 4 / 9 tokens 86 / 60, 160 / 134 against 76 / 38, 112 / 69; 64 of them, 6: 75 / 50 against 69 / 33; 128 of
+//   768, 9: 111 / 70 against 114 / 54.  4096: 16 experts of 1792 top-4, 6: 102 / 73 against 82 / 49, Q6_K downs 111 / 83 against 99 / 65, Q8_0 140 / 110
+//   against 115 / 80; 128 of 1536, 6: 164 / 136 against 167 / 111.
 int batched_from(const mummu_moe *h, const Layer &L) {
     const ExpertBanks b = banks_of(h, L);
     if (!grouped_gemm_supported(b)) return 0x7fffffff;
     if (b.gate_type == T_F32) return h->gemm_min_f32;
-    if (h->gemm_q4k_f16 && grouped_gemm_q4k_f16_down(b)) return h->gemm_min_q4k;
-    if (q8_half_pairs(h, b)) return h->gemm_min_q8;
-    return grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
+    const bool q4k = h->gemm_q4k_f16 && grouped_gemm_q4k_f16(b), q4k_down = q4k && grouped_gemm_q4k_f16_down(b), q8 = q8_half_pairs(h, b);
+    const int line = q4k_down ? h->gemm_min_q4k : q8 ? h->gemm_min_q8 : grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
+    if (h->gemm_min_given || !(q4k || q8)) return line;
+    const bool wide = b.hidden > 2048;
+    const double bytes = 1e6 * (q8 ? (wide ? 300.0 : 450.0) : wide ? 180.0 : q4k_down ? 310.0 : 480.0);
+    auto row_bytes = [](int type, int d) { return (double)(d / block_elems(type)) * block_bytes(type); };
+    const double expert = 2.0 * b.inter * row_bytes(b.gate_type, b.hidden) + (double)b.hidden * row_bytes(b.down_type, b.inter);
+    const int from = wide ? 6 : 9, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));
+    return std::min(line, std::max(from, n));
 }
 
 // Q4_K and Q8_0 banks on the f16 units (batched path): whether gate/up (hf) and down (hf_down; q6: of Q6_K) take that form for this batch,
@@ -1137,7 +1144,7 @@ int mummu_moe_create(const mummu_moe_config *cfg, mummu_moe **out) {
     // MUMMU_GEMM_MIN_TOKENS: smallest batch that takes dispatch + grouped GEMM instead of the decode kernels
     if (const char *e = getenv("MUMMU_GEMM_MIN_TOKENS")) {
         const int v = atoi(e);
-        if (v >= 1) h->gemm_min_f16 = h->gemm_min_quant = h->gemm_min_f32 = h->gemm_min_q4k = h->gemm_min_q8 = v;
+        if (v >= 1) h->gemm_min_given = true, h->gemm_min_f16 = h->gemm_min_quant = h->gemm_min_f32 = h->gemm_min_q4k = h->gemm_min_q8 = v;
     }
     h->layers.resize((size_t)cfg->num_layers);
     auto bail = [&](int rc) {

@@ -1,0 +1,38 @@
+"""Where a batch leaves the decode kernels: by what its slots' experts would read, from six (rows of more than 2048 elements) or nine tokens on.
+On both sides of the line the block agrees with what the other form gives, the routing to the bit."""
+import numpy as np
+import pytest
+
+from mummu_amd import moe as M
+from mummu_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,I,E,k,bank,down,line", [(4096, 1792, 8, 4, "Q4_K", "Q4_K", 6), (2560, 640, 24, 10, "Q4_K", "Q5_1", 6), (2048, 1024, 16, 8, "Q8_0", "Q8_0", 9),
+                                                    (2048, 1024, 16, 8, "Q4_K", "Q4_K", 11), (2048, 1024, 16, 8, "Q4_K", "Q6_K", 15), (1024, 512, 8, 4, "Q4_K", "Q4_K", 18)])
+def test_both_sides_of_the_line(monkeypatch, H, I, E, k, bank, down, line):
+    rng = np.random.Generator(np.random.PCG64(H + E))
+    bt, dt = getattr(M, bank), getattr(M, down)
+    gate, up = (synth.random_bank_fast(bt, [H, I, E], seed) for seed in (71, 72))
+    downs = synth.random_bank_fast(dt, [I, H, E], 73)
+    router = (rng.standard_normal((E, H)) * 0.02).astype(np.float16)
+    x = rng.standard_normal((line, H), dtype=np.float32)
+
+    def run(lines):
+        if lines is not None:
+            monkeypatch.setenv("MUMMU_GEMM_MIN_TOKENS", str(lines))
+        with M.SparseMoe(M.SparseMoeConfig(H, I, E, k), max_tokens=line) as m:
+            m.load_layer(0, router, M.F16, gate, bt, up, bt, downs, dt)
+            out = [(np.asarray(m.forward(x[:n], k, True)), m.last_routing(n, k)) for n in (line - 1, line)]
+            return m.batched_from(0), out
+
+    at, by_rule = run(None)
+    assert at == line
+    forced = {lines: run(lines)[1] for lines in (1, 1 << 20)}
+    for i in range(2):
+        same, other = forced[1 if i else 1 << 20][i], forced[1 << 20 if i else 1][i]
+        assert np.array_equal(by_rule[i][0].view(np.uint32), same[0].view(np.uint32))
+        assert all(np.array_equal(np.asarray(a), np.asarray(b)) for a, b in zip(by_rule[i][1][:2], other[1][:2]))
+        # (16 bits and a scale per 16 elements in the decode kernels: 2^-17 of a block's largest element, twice and through three products)
+        assert np.linalg.norm(by_rule[i][0] - other[0]) <= 2e-4 * np.linalg.norm(other[0])
