@@ -25,9 +25,19 @@ constexpr int kBlock = 144;
 constexpr int kUnits = 4;            // 16 columns of one matrix each: between two meetings of the sums
 constexpr int kRowC = 128 + 4;       // f32 row of the gate/up epilogue
 
+// a / b for 0 <= a < 2^31, 1 <= b < 2^15 by the f32 quotient, one off at most up to 2^23 (else the integer one)
+__device__ inline int div_small(int a, int b) {
+    if (a >= (1 << 23)) return a / b;
+    int q = (int)__fmul_rn((float)a, __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    return r < 0 ? q - 1 : r >= b ? q + 1 : q;
+}
+
 struct StreamArgs {
     Q4kArgs q;
-    int cols;   // columns of a workgroup
+    int cols;        // columns of a workgroup
+    int n_sb;        // waves along K
+    int group_bits;  // 2^group_bits such rows of waves
 };
 
 template <bool R8>
@@ -53,7 +63,7 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
     const int e = uniform(p.tiles[3 * tile]), p0 = uniform(p.tiles[3 * tile + 1]), rows = uniform(p.tiles[3 * tile + 2]);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 15, kg = lane >> 4;
-    const int n_waves = (int)blockDim.x >> 6, n_sb = p.in_dim / 256, n_groups = n_waves / n_sb;
+    const int n_sb = a.n_sb, n_groups = 1 << a.group_bits, n_waves = n_sb << a.group_bits;
     const int group = wave / n_sb, sb = wave - group * n_sb;
     const uint32_t row_bytes = (uint32_t)n_sb * kBlock;
     float *s_sum = (float *)s_lds;                                      // [2][unit][wave][kTile]
@@ -86,7 +96,7 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
 #pragma unroll
     for (int u = 0; u < DEPTH - 1; u++) load(u / NB, u % NB, u);
     MUMMU_CODE_FENCE();
-    if (GATE_UP) source /= p.k_slots;
+    if (GATE_UP) source = div_small(source, p.k_slots);
 
     // x: piece i of a plane = 8 elements; load l, half h, nibble n of the codes above meet piece 4 (4 l + 2 (kg / 2) + n) + 2 (kg % 2) + h
     constexpr int kPlanes = R8 ? 1 : 2;
@@ -190,19 +200,26 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const int n_out = kSteps * n_groups * kTile;
         // (the waves take turns where not all have some)
-        for (int i = (tid + (ph & 1) * 32 * n_waves) % (64 * n_waves); i < n_out; i += 64 * n_waves) {
-            const int block = i / kTile, d = i % kTile, ln = R8 ? d >> 1 : d >> 2, step = block / n_groups, g = block - step * n_groups;
+        int first = tid + (ph & 1) * 32 * n_waves;
+        first -= first >= 64 * n_waves ? 64 * n_waves : 0;
+        for (int i = first; i < n_out; i += 64 * n_waves) {
+            const int block = i / kTile, d = i % kTile, ln = R8 ? d >> 1 : d >> 2, step = block >> a.group_bits, g = block & (n_groups - 1);
             const int row = R8 ? 4 * ((ln >> 4) & 1) + 2 * (d & 1) + (ln >> 5) : 4 * (ln >> 4) + (d & 3);
             auto sum_of = [&](int u) {
                 const float *from = sums + (u * n_waves + g * n_sb) * kTile + d;
                 float s = 0.0f;
-                for (int k0 = 0; k0 < n_sb; k0 += 8) {
-                    float v[8];
+                auto add = [&](auto count) {
+                    float v[decltype(count)::value];
 #pragma unroll
-                    for (int k = 0; k < 8; k++) v[k] = from[(k0 + k < n_sb ? k0 + k : 0) * kTile];
+                    for (int k = 0; k < decltype(count)::value; k++) v[k] = from[k * kTile];
 #pragma unroll
-                    for (int k = 0; k < 8; k++) s = k0 + k < n_sb ? __fadd_rn(s, v[k]) : s;
-                }
+                    for (int k = 0; k < decltype(count)::value; k++) s = __fadd_rn(s, v[k]);
+                    from += decltype(count)::value * kTile;
+                };
+                for (int k = 8; k <= n_sb; k += 8) add(std::integral_constant<int, 8>());
+                if (n_sb & 4) add(std::integral_constant<int, 4>());
+                if (n_sb & 2) add(std::integral_constant<int, 2>());
+                if (n_sb & 1) add(std::integral_constant<int, 1>());
                 return s;
             };
             const int col = 16 * ((ph * kSteps + step) * n_groups + g) + (ln & 15);
@@ -240,8 +257,8 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
 
 template <bool GATE_UP, bool OUT_H, bool R8>
 hipError_t launch_stream(const Q4kArgs &q, int max_tiles, hipStream_t s) {
-    const int n_sb = q.in_dim / 256, groups = n_sb >= 3 ? 1 : n_sb == 2 ? 2 : 4, waves = n_sb * groups;
-    StreamArgs a{q, 128};   // (gate/up: what a scale of its output covers; down: the more, the less often rows are read into registers)
+    const int n_sb = q.in_dim / 256, group_bits = n_sb >= 3 ? 0 : n_sb == 2 ? 1 : 2, groups = 1 << group_bits, waves = n_sb * groups;
+    StreamArgs a{q, 128, n_sb, group_bits};   // (gate/up: what a scale of its output covers; down: the more, the less often rows are read into registers)
     if (!GATE_UP) a.cols = q.out_dim % (256 * groups) == 0 ? 256 * groups : q.out_dim % (128 * groups) == 0 ? 128 * groups : 64 * groups;
     if (n_sb < 1 || n_sb > kQ4kStreamBlocks || q.in_dim % 256 != 0 || q.out_dim % a.cols != 0) return hipErrorInvalidValue;
     const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)(q.out_dim / a.cols)), block(64 * waves);
