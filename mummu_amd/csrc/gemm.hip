@@ -976,7 +976,7 @@ static double expected_tiles(double avg, double rows) {
     return t;
 }
 
-// Tiles of 8 instead of 16 rows (gemm_q4k_stream.hip) while next to no expert needs a second one: its first second tiles must not start a second
+// Tiles of 8 instead of 16 rows (gemm_stream.hip) while next to no expert needs a second one: its first second tiles must not start a second
 // round of workgroups, and beyond they read the weights again.  us a layer among others, tiles of 16 / 8: OLMoE 20 / 32 / 40 tokens 55.8 / 52.1,
 // 58.4 / 55.3, 60.0 / 60.0 (alone 95 / 105), 128 experts of 2048 x 768, 27 / 64 / 100 tokens 72.4 / 67.6, 88.5 / 86.3, 93.3 / 95.4, the 512-expert shape
 // with int8 downs, 64 / 200 / 300 tokens 272 / 262, 385 / 373, 407 / 423, 16 experts of 4096 x 1792, 18 tokens 55 / 61.
@@ -984,10 +984,10 @@ static int tiles_of_8_or_16(const ExpertBanks &b, int n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const double e8 = expected_tiles(avg, 8.0), e16 = expected_tiles(avg, 16.0), each = (double)b.n_experts * (double)((b.inter + 127) / 128);
     const bool second_round = each * e16 <= 512.0 && each * e8 > 1.03 * 512.0;
-    return q4k_stream_takes(b.hidden, b.inter, 8) && !second_round && e8 < 1.03 * e16 ? 8 : 16;
+    return gemm_stream_takes(b.hidden, b.inter, 8) && !second_round && e8 < 1.03 * e16 ? 8 : 16;
 }
 
-// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_q4k_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what they
+// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what they
 // have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
 // variance = mean).  Layers, 16 / 64 rows, us: in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it
 // weighs: 128 experts of 2048 x 768, 128 tokens 127 / 155, 160: 145 / 158, 208 (1.17 tiles an expert): 148 / 159, 240 (1.4): 162 / 161.  Where a
@@ -1165,8 +1165,8 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
         if (out_h && !grouped_gemm_q4k_f16_down(b) && !grouped_gemm_q6k_down(b)) return hipErrorInvalidValue;
         if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
         if (tile_rows > 16) return launch_q4k_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
-        if (q4k_stream_takes(b.hidden, b.inter, tile_rows))
-            return launch_q4k_stream_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, acth, actq, s);
+        if (gemm_stream_takes(b.hidden, b.inter, tile_rows))
+            return launch_gemm_stream_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, acth, actq, s);
         return launch_q4k_few_gate_up(b, xh, sorted, k_slots, tiles, n_tiles, max_tiles, acth, actq, s);
     }
     if (b.gate_type == T_F32)
@@ -1213,14 +1213,15 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
     }
     if (acth.hi != nullptr && b.down_type == T_Q6_K) {
         if (!grouped_gemm_q6k_down(b) || tile_rows > 64) return hipErrorInvalidValue;
+        if (tile_rows <= 8 && gemm_stream_takes(b.inter, b.hidden, tile_rows)) return launch_gemm_stream_down(b, acth, tiles, n_tiles, max_tiles, tile_rows, y, s);
         return launch_q6k_down(b, acth, tiles, n_tiles, max_tiles, tile_rows, y, s);
     }
     if (acth.hi != nullptr) {
         if (!grouped_gemm_q4k_f16_down(b)) return hipErrorInvalidValue;
         if (tile_rows > kQ4kRows) return hipErrorInvalidValue;
         if (tile_rows > 16) return launch_q4k_down(b, acth, tiles, n_tiles, max_tiles, y, s);
-        if (q4k_stream_takes(b.inter, b.hidden, tile_rows))
-            return launch_q4k_stream_down(b, acth, tiles, n_tiles, max_tiles, tile_rows, y, s);
+        if (gemm_stream_takes(b.inter, b.hidden, tile_rows))
+            return launch_gemm_stream_down(b, acth, tiles, n_tiles, max_tiles, tile_rows, y, s);
         return launch_q4k_few_down(b, acth, tiles, n_tiles, max_tiles, y, s);
     }
     if (b.down_type == T_F32)

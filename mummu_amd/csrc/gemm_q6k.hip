@@ -38,15 +38,6 @@ constexpr int at_scales(int mt) { return kAtA + 3 * slot_bytes(mt); }
 constexpr int lds_bytes(int mt) { return at_scales(mt) + 4 * 256; }
 static_assert(64 * kWLoads - 32 * kPieces == 32 && lds_bytes(2) <= 160 * 1024, "whole rows; fits");
 
-// Four codes as bytes (0..63) -> halfs of code - 32, two at a time in the element order of HAct: a byte under 0x64 is the half 1024 + byte.
-__device__ inline half2v code_pair(uint32_t codes, uint32_t pick) {
-    const half2v bias = {(_Float16)1056.0f, (_Float16)1056.0f};
-    const uint32_t u = __builtin_amdgcn_perm(0x64646464u, codes, pick);
-    half2v h;
-    __builtin_memcpy(&h, &u, 4);
-    return h - bias;
-}
-
 // a in sorted order, a scale per 128 elements; y[pos, n] = f32 sum.  Tiles of up to 32 MT rows, or (MT 1) of up to 16, which are the first eight
 // elements of an accumulator: the others are not folded (64 tokens, OLMoE shape: 44.0 -> 41.6 us).
 template <int MT, bool HALF = false>
@@ -219,8 +210,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void q6k_down_kernel(const uint8_t 
                     for (int p = 0; p < 2; p++) {
                         const uint32_t low = q[odd][2 * (j & 1) + i][p] >> (4 * (j >> 1)), high = q[odd][4 + i][p];
                         const uint32_t codes = (low & 0x0F0F0F0Fu) | ((j < 2 ? high << (4 - 2 * j) : high >> (2 * j - 4)) & 0x30303030u);
-                        f[2 * p] = code_pair(codes, 0x04020400u);
-                        f[2 * p + 1] = code_pair(codes, 0x04030401u);
+                        f[2 * p] = q6k_code_pair(codes, 0x04020400u);
+                        f[2 * p + 1] = q6k_code_pair(codes, 0x04030401u);
                     }
                     __builtin_memcpy(&op, f, 16);
                 }

@@ -1,5 +1,5 @@
-// Grouped GEMM of Q4_K banks on the f16 units for a few rows per expert: the operands and arithmetic of gemm_q4k.hip on tiles of up to 8 or
-// 16 rows (v_mfma_f32_16x16x32_f16).  A wave keeps ONE super-block of K of the tile's rows in registers and takes the weights of 16 columns
+// Grouped GEMM of Q4_K banks, and down products of Q6_K, on the f16 units for a few rows per expert: the operands and arithmetic of gemm_q4k.hip
+// and gemm_q6k.hip on tiles of up to 8 or 16 rows (v_mfma_f32_16x16x32_f16).  A wave keeps ONE super-block of K of the tile's rows in registers and takes the weights of 16 columns
 // after 16 of it from memory straight into the registers that multiply them; the waves of a workgroup have the super-blocks of a row side by
 // side, so that together they read whole rows front to back, and their sums meet in LDS in ascending order.  Tiles of 8 rows hold the high
 // halfs in the operand's first eight rows and the low ones in the others: one product where 16 rows take two.
@@ -10,6 +10,10 @@
 // 51 -> 48 us, of 512 experts of 2560 x 640 with 64 tokens 176 -> 167, with the loads alone 43 and 133, with the weights out of L2 45 and 139;
 // OLMoE, 20 tokens, 38.7 -> 37.2 + 23.5 -> 20.9.  Layers among others: 72.4 -> 67.6, 272 -> 262, 57.0 -> 52.1; 512 experts of 2048 x 768, 60
 // tokens 237 -> 206, 128 of 3072 x 768, 30 tokens 117 -> 103.
+//
+// Q6_K downs (tiles of 8 rows): a sub-block's 16 elements are an operand's K of 16 (v_mfma_f32_16x16x16_f16), four to a lane, so that its sum can
+// be folded with d * sc; a lane loads 16 neighbouring bytes and changes dwords with the three others of its row.  262 vector instructions a unit, 53 % of
+// the cycles, and 8 % products.  OLMoE, 24 tokens 42 -> 35 us (106 MB fetched, the weights' bytes), layers at 16 / 24 / 32 tokens 73 / 74 / 76 -> 62 / 65 / 67.
 #include "device_utils.h"
 #include "kernels.h"
 #include "q4k_half.h"
@@ -21,7 +25,6 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBlock = 144;
 constexpr int kUnits = 4;            // 16 columns of one matrix each: between two meetings of the sums
 constexpr int kRowC = 128 + 4;       // f32 row of the gate/up epilogue
 
@@ -48,10 +51,13 @@ constexpr size_t stream_lds(int waves, bool gate_up) {
 
 // Workgroup: one wave to a super-block of K, times n_groups of them side by side where a row has one or two; group g of a step has columns
 // 16 (step n_groups + g) .. + 15 of the workgroup's.
-template <bool GATE_UP, bool OUT_H, bool R8, int MAXW, int PER_SIMD, int DEPTH>
-__global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamArgs a) {
+template <int WT, bool GATE_UP, bool OUT_H, bool R8, int MAXW, int PER_SIMD, int DEPTH>
+__global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_lds[];
     const Q4kArgs &p = a.q;
+    constexpr bool Q6 = WT == T_Q6_K;
+    static_assert(WT == T_Q4_K || (Q6 && !GATE_UP), "banks this kernel reads");
+    constexpr int kBlock = block_bytes(WT);
     constexpr int kRows = R8 ? 8 : 16, kTile = kRows * 16, NB = GATE_UP ? 2 : 1, kSteps = kUnits / NB;
     // As xcd_tile in gemm.hip: an XCD takes neighbouring tiles with the slab running fastest.
     const int n_slabs = p.out_dim / a.cols;
@@ -82,15 +88,27 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
     Global *base[NB];
     base[0] = (Global *)uniform(p.w0 + matrix + (size_t)col0 * row_bytes);
     if (GATE_UP) base[NB - 1] = (Global *)uniform(p.w1 + matrix + (size_t)col0 * row_bytes);
-    const uint32_t off_h = (uint32_t)c * row_bytes + (uint32_t)sb * kBlock, off_q = off_h + 16u + 16u * (uint32_t)kg;
+    const uint32_t off_h = (uint32_t)c * row_bytes + (uint32_t)sb * kBlock, off_q = off_h + (Q6 ? 0u : 16u) + 16u * (uint32_t)kg;
     const uint32_t step_bytes = 16u * (uint32_t)n_groups * row_bytes;
-    u32x4 hd[DEPTH], q0[DEPTH], q1[DEPTH];   // DEPTH - 1 of them on their way
+    // (DEPTH - 1 units on their way.  Q4_K: header, codes; Q6_K: scales, ql, ql, qh, d)
+    u32x4 hd[DEPTH], q0[DEPTH], q1[DEPTH], qh[Q6 ? DEPTH : 1];
+    uint32_t dd[Q6 ? DEPTH : 1];
     auto load = [&](int step, int j, int to) {
         Global *from = base[j] + (size_t)((uint32_t)step * step_bytes);
         typedef __attribute__((address_space(1))) const u32x4 Words;
-        hd[to] = *(Words *)(from + off_h);
-        q0[to] = *(Words *)(from + off_q);
-        q1[to] = *(Words *)(from + off_q + 64);
+        if constexpr (Q6) {   // (a super-block begins at an even byte)
+            typedef u32x4 Loose __attribute__((aligned(2)));
+            typedef __attribute__((address_space(1))) const Loose LooseWords;
+            q0[to] = *(LooseWords *)(from + off_q);
+            q1[to] = *(LooseWords *)(from + off_q + 64);
+            qh[to] = *(LooseWords *)(from + off_q + 128);
+            hd[to] = *(LooseWords *)(from + off_h + 192);
+            dd[to] = *(__attribute__((address_space(1))) const uint16_t *)(from + off_h + 208);
+        } else {
+            hd[to] = *(Words *)(from + off_h);
+            q0[to] = *(Words *)(from + off_q);
+            q1[to] = *(Words *)(from + off_q + 64);
+        }
     };
     MUMMU_CODE_FENCE();
 #pragma unroll
@@ -98,21 +116,28 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
     MUMMU_CODE_FENCE();
     if (GATE_UP) source = div_small(source, p.k_slots);
 
-    // x: piece i of a plane = 8 elements; load l, half h, nibble n of the codes above meet piece 4 (4 l + 2 (kg / 2) + n) + 2 (kg % 2) + h
+    // x.  Q4_K: piece i of a plane = 8 elements; load l, half h, nibble n of the codes above meet piece 4 (4 l + 2 (kg / 2) + n) + 2 (kg % 2) + h.
+    // Q6_K: elements 4 kg .. + 3 of each sub-block of 16.
     constexpr int kPlanes = R8 ? 1 : 2;
-    half8 x[kPlanes][2][2][2];
+    half8 x[kPlanes][Q6 ? 1 : 2][2][2];
+    half4v x6[kPlanes][Q6 ? 16 : 1];
     {
         const uint32_t at = (uint32_t)(8 * (kg >> 1) + 2 * (kg & 1)) * 16u;
         const size_t row_at = ((size_t)source * (size_t)p.in_dim + (size_t)sb * 256) * 2;
 #pragma unroll
         for (int pl = 0; pl < kPlanes; pl++) {
             const uint8_t *plane = (const uint8_t *)(R8 ? (c < 8 ? p.a.hi : p.a.lo) : (pl == 0 ? p.a.hi : p.a.lo)) + row_at;
+            if constexpr (Q6) {
 #pragma unroll
-            for (int l = 0; l < 2; l++)
+                for (int n = 0; n < 16; n++) x6[pl][n] = *(const half4v *)(plane + 32 * n + 8 * kg);
+            } else {
 #pragma unroll
-                for (int h = 0; h < 2; h++)
+                for (int l = 0; l < 2; l++)
 #pragma unroll
-                    for (int n = 0; n < 2; n++) x[pl][l][h][n] = *(const half8 *)(plane + at + (uint32_t)((16 * l + 4 * n + h) * 16));
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int n = 0; n < 2; n++) x[pl][l][h][n] = *(const half8 *)(plane + at + (uint32_t)((16 * l + 4 * n + h) * 16));
+            }
         }
     }
     // sums of 32 elements as pairs of halfs: gate/up K = 16 (high of sub-blocks 0-3, 4-7, low of both), down K = 8 for either half
@@ -122,7 +147,7 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
         const float *ss = p.a.ssum + (size_t)source * (size_t)(p.in_dim / 32) + (size_t)sb * 8;
         const bool low = GATE_UP ? kg >= 2 : kg == 1, none = (R8 && c >= 8) || (!GATE_UP && kg >= 2);
 #pragma unroll
-        for (int l = 0; l < (GATE_UP ? 1 : 2); l++) {
+        for (int l = 0; !Q6 && l < (GATE_UP ? 1 : 2); l++) {
             const float4 v = *(const float4 *)(ss + (GATE_UP ? 4 * (kg & 1) : 4 * l));
             const float f[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -146,7 +171,46 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
 
     const f32x4 zero = {0, 0, 0, 0};
     const uint32_t pick = kg >= 2 ? 0x04030402u : 0x04010400u;   // this lane's two sub-blocks of four
-    auto multiply = [&](int b, float *to) {
+    auto products_q6 = [&](int b) {
+        // dword kg of each 16 bytes: lane group i has loaded the 16 bytes i (and 4 + i) of ql, i of qh
+        auto turn = [&](u32x4 &t) {
+            auto swap = [](uint32_t &u, uint32_t &w, bool far) {
+                const auto o = far ? __builtin_amdgcn_permlane32_swap(u, w, false, false) : __builtin_amdgcn_permlane16_swap(u, w, false, false);
+                u = o[0], w = o[1];
+            };
+            uint32_t r[4] = {t[0], t[1], t[2], t[3]};
+            swap(r[0], r[2], true), swap(r[1], r[3], true), swap(r[0], r[1], false), swap(r[2], r[3], false);
+            t = u32x4{r[0], r[1], r[2], r[3]};
+        };
+        turn(q0[b]), turn(q1[b]), turn(qh[Q6 ? b : 0]);
+        const float d = half_bits_to_float((uint16_t)dd[Q6 ? b : 0]);
+        f32x4 v = zero;
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            f32x4 run = zero;
+#pragma unroll
+            for (int n = 0; n < 8; n++) {
+                const int j = n >> 1, i = n & 1;
+                const u32x4 ql = half == 0 ? q0[b] : q1[b];
+                const uint32_t low = ql[2 * (j & 1) + i] >> (4 * (j >> 1)), high = qh[Q6 ? b : 0][2 * half + i];
+                const uint32_t codes = (low & 0x0F0F0F0Fu) | ((j < 2 ? high << (4 - 2 * j) : high >> (2 * j - 4)) & 0x30303030u);
+                const half2v f[2] = {q6k_code_pair(codes, 0x04020400u), q6k_code_pair(codes, 0x04030401u)};
+                half4v w;
+                __builtin_memcpy(&w, f, 8);
+                f32x4 s = zero;
+#pragma unroll
+                for (int pl = 0; pl < kPlanes; pl++) s = __builtin_amdgcn_mfma_f32_16x16x16f16(x6[pl][Q6 ? 8 * half + n : 0], w, s, 0, 0, 0);
+                const float fd = __fmul_rn(d, (float)(int8_t)(hd[b][2 * half + (n >> 2)] >> (8 * (n & 3))));
+#pragma unroll
+                for (int r = 0; r < 4; r++) run[r] = n == 0 ? __fmul_rn(fd, s[r]) : fmaf(fd, s[r], run[r]);
+                if (n & 1) asm volatile("" : "+v"(run[0]), "+v"(run[1]), "+v"(run[2]), "+v"(run[3]));   // (summed here: the compiler would carry all sixteen sub-blocks' sums to the end)
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = half == 0 ? __fmul_rn(run[r], sr[0][r]) : fmaf(run[r], sr[GATE_UP ? 0 : 1][r], v[r]);
+        }
+        return v;
+    };
+    auto products_q4 = [&](int b) {
         Q4kHeader head;
         head.unpack(hd[b]);
         f32x4 v = zero, c1 = zero;
@@ -165,7 +229,7 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
 #pragma unroll
                 for (int n = 0; n < 2; n++)
 #pragma unroll
-                    for (int pl = 0; pl < kPlanes; pl++) c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[pl][l][h][n], w[n], c1, 0, 0, 0);
+                    for (int pl = 0; pl < kPlanes; pl++) c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[pl][Q6 ? 0 : l][h][n], w[n], c1, 0, 0, 0);
             }
             if (!GATE_UP || l == 1) {
                 Q4kHeader h = head;
@@ -179,6 +243,12 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
                 }
             }
         }
+        return v;
+    };
+    auto multiply = [&](int b, float *to) {
+        f32x4 v;
+        if constexpr (Q6) v = products_q6(b);
+        else v = products_q4(b);
         if constexpr (R8) {
             // rows 4 (kg % 2) + (kg / 2), + 2: high + low
             ((float2 *)to)[lane] = make_float2(swap32_add(v[0], v[1]), swap32_add(v[2], v[3]));
@@ -255,21 +325,21 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void q4k_stream_kernel(StreamA
     }
 }
 
-template <bool GATE_UP, bool OUT_H, bool R8>
+template <int WT, bool GATE_UP, bool OUT_H, bool R8>
 hipError_t launch_stream(const Q4kArgs &q, int max_tiles, hipStream_t s) {
     const int n_sb = q.in_dim / 256, group_bits = n_sb >= 3 ? 0 : n_sb == 2 ? 1 : 2, groups = 1 << group_bits, waves = n_sb * groups;
     StreamArgs a{q, 128, n_sb, group_bits};   // (gate/up: what a scale of its output covers; down: the more, the less often rows are read into registers)
-    if (!GATE_UP) a.cols = q.out_dim % (256 * groups) == 0 ? 256 * groups : q.out_dim % (128 * groups) == 0 ? 128 * groups : 64 * groups;
-    if (n_sb < 1 || n_sb > kQ4kStreamBlocks || q.in_dim % 256 != 0 || q.out_dim % a.cols != 0) return hipErrorInvalidValue;
+    // (Q6_K: a unit takes twice as long, and half the columns leave four workgroups to a CU: 16 / 24 tokens 63.7 / 65.6 -> 61.9 / 64.6 us a layer)
+    if (!GATE_UP) a.cols = WT != T_Q6_K && q.out_dim % (256 * groups) == 0 ? 256 * groups : q.out_dim % (128 * groups) == 0 ? 128 * groups : 64 * groups;
+    if (n_sb < 1 || n_sb > kStreamBlocks || q.in_dim % 256 != 0 || q.out_dim % a.cols != 0) return hipErrorInvalidValue;
     const dim3 grid((unsigned)(max_tiles + 7) / 8 * 8 * (unsigned)(q.out_dim / a.cols)), block(64 * waves);
     const size_t lds = stream_lds<R8>(waves, GATE_UP);
-    if constexpr (R8) {
-        if (waves <= 6 || waves == 9 || waves == 10) {   // five waves a SIMD hold one workgroup more than four
-            launch_kernel(q4k_stream_kernel<GATE_UP, OUT_H, R8, 10, 5, 2>, grid, block, lds, s, a);
-            return hipGetLastError();
-        }
-    }
-    launch_kernel(q4k_stream_kernel<GATE_UP, OUT_H, R8, 16, 4, R8 ? 4 : 2>, grid, block, lds, s, a);
+    // (five waves a SIMD hold one workgroup more than four)
+    const bool five = R8 && (waves <= 6 || waves == 9 || waves == 10);
+    if constexpr (WT == T_Q6_K) launch_kernel(stream_kernel<WT, GATE_UP, OUT_H, R8, 16, 4, 2>, grid, block, lds, s, a);
+    else if constexpr (!R8) launch_kernel(stream_kernel<WT, GATE_UP, OUT_H, R8, 16, 4, 2>, grid, block, lds, s, a);
+    else if (five) launch_kernel(stream_kernel<WT, GATE_UP, OUT_H, R8, 10, 5, 2>, grid, block, lds, s, a);
+    else launch_kernel(stream_kernel<WT, GATE_UP, OUT_H, R8, 16, 4, 4>, grid, block, lds, s, a);
     return hipGetLastError();
 }
 
@@ -278,23 +348,24 @@ hipError_t launch_stream(const Q4kArgs &q, int max_tiles, hipStream_t s) {
 // Tiles of 16 rows keep 64 registers of rows, four waves a SIMD: taken where workgroups of one wave to a super-block fill those.
 // us a layer among others, here / gemm_q4k_few.hip: OLMoE 24 / 64 tokens 57.7 / 58.8, 61.8 / 64.2, 512 experts of 2048 x 768, 40 / 128 tokens 177 / 189,
 // 302 / 316; hidden 2560 365 / 349, 4096 283 / 280, 1536 46.5 / 43.8, three super-blocks alike.
-bool q4k_stream_takes(int in_dim, int out_dim, int tile_rows) {
+bool gemm_stream_takes(int in_dim, int out_dim, int tile_rows) {
     const int n_sb = in_dim / 256;
     if (in_dim % 256 != 0 || out_dim % 128 != 0) return false;
-    return tile_rows <= 8 ? n_sb <= kQ4kStreamBlocks : n_sb == 4 || n_sb == 8;
+    return tile_rows <= 8 ? n_sb <= kStreamBlocks : n_sb == 4 || n_sb == 8;
 }
 
-hipError_t launch_q4k_stream_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
+hipError_t launch_gemm_stream_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
                                      int max_tiles, int tile_rows, HAct act_h, QAct64 act_q, hipStream_t s) {
     const Q4kArgs p{b.gate, b.up, x, sorted, tiles, n_tiles, k_slots, b.hidden, b.inter, act_h, act_q, nullptr};
-    if (tile_rows <= 8) return act_h.hi != nullptr ? launch_stream<true, true, true>(p, max_tiles, s) : launch_stream<true, false, true>(p, max_tiles, s);
-    return act_h.hi != nullptr ? launch_stream<true, true, false>(p, max_tiles, s) : launch_stream<true, false, false>(p, max_tiles, s);
+    if (tile_rows <= 8) return act_h.hi != nullptr ? launch_stream<T_Q4_K, true, true, true>(p, max_tiles, s) : launch_stream<T_Q4_K, true, false, true>(p, max_tiles, s);
+    return act_h.hi != nullptr ? launch_stream<T_Q4_K, true, true, false>(p, max_tiles, s) : launch_stream<T_Q4_K, true, false, false>(p, max_tiles, s);
 }
 
-hipError_t launch_q4k_stream_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows,
+hipError_t launch_gemm_stream_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows,
                                   float *y, hipStream_t s) {
     const Q4kArgs p{b.down, nullptr, act, nullptr, tiles, n_tiles, 1, b.inter, b.hidden, HAct(), QAct64(), y};
-    return tile_rows <= 8 ? launch_stream<false, true, true>(p, max_tiles, s) : launch_stream<false, true, false>(p, max_tiles, s);
+    if (b.down_type == T_Q6_K) return tile_rows <= 8 ? launch_stream<T_Q6_K, false, true, true>(p, max_tiles, s) : hipErrorInvalidValue;
+    return tile_rows <= 8 ? launch_stream<T_Q4_K, false, true, true>(p, max_tiles, s) : launch_stream<T_Q4_K, false, true, false>(p, max_tiles, s);
 }
 
 }  // namespace mummu

@@ -243,12 +243,12 @@ hipError_t launch_q4k_few_gate_up(const ExpertBanks &b, HAct x, const int32_t *s
                                   const int32_t *n_tiles, int max_tiles, HAct act_h, QAct64 act_q, hipStream_t s);
 hipError_t launch_q4k_few_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, float *y,
                                hipStream_t s);
-// gemm_q4k_stream.hip: rows of up to kQ4kStreamBlocks super-blocks, tiles of up to 8 or 16 rows.
-constexpr int kQ4kStreamBlocks = 16;
-bool q4k_stream_takes(int in_dim, int out_dim, int tile_rows);
-hipError_t launch_q4k_stream_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
+// gemm_stream.hip: rows of up to kStreamBlocks super-blocks, tiles of up to 8 or 16 rows.
+constexpr int kStreamBlocks = 16;
+bool gemm_stream_takes(int in_dim, int out_dim, int tile_rows);
+hipError_t launch_gemm_stream_gate_up(const ExpertBanks &b, HAct x, const int32_t *sorted, int k_slots, const int32_t *tiles, const int32_t *n_tiles,
                                      int max_tiles, int tile_rows, HAct act_h, QAct64 act_q, hipStream_t s);
-hipError_t launch_q4k_stream_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows,
+hipError_t launch_gemm_stream_down(const ExpertBanks &b, HAct act, const int32_t *tiles, const int32_t *n_tiles, int max_tiles, int tile_rows,
                                   float *y, hipStream_t s);
 // gemm_q4k_one.hip: one expert's two products on a few rows of f32, act [rows][inter].
 hipError_t launch_q4k_one_gate_up(const ExpertBanks &b, int expert, const float *x, int rows, float *act, hipStream_t s);

@@ -26,6 +26,14 @@ __device__ inline half2v code_pair(uint32_t t, half2v mul) {
     __builtin_memcpy(&h, &u, 4);
     return h * mul;
 }
+// Four Q6_K codes as bytes (0..63) -> halfs of code - 32, two at a time in the element order of HAct: a byte under 0x64 is the half 1024 + byte.
+__device__ inline half2v q6k_code_pair(uint32_t codes, uint32_t pick) {
+    const half2v bias = {(_Float16)1056.0f, (_Float16)1056.0f};
+    const uint32_t u = __builtin_amdgcn_perm(0x64646464u, codes, pick);
+    half2v h;
+    __builtin_memcpy(&h, &u, 4);
+    return h - bias;
+}
 // Eight Q4_K codes (the low or high nibbles of two words, in the element order of HAct) times their sub-block's scale, over
 // 2^14 (exact: up to 63 * 15 in units of 2^-14): two masks, a shift and four products a word.
 template <bool HIGH>

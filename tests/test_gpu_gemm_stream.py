@@ -14,7 +14,7 @@ COUNTS = [0, 1, 7, 8, 9, 0, 15, 16, 17, 2]
 
 
 @pytest.mark.parametrize("H,I,down", [(256, 256, "Q4_K"), (512, 768, "Q4_K"), (768, 512, "Q4_K"), (1024, 1280, "Q4_K"), (1280, 2560, "Q4_K"),
-                                      (1792, 2816, "Q4_K"), (2304, 256, "Q4_K"), (2048, 1024, "Q6_K"), (2560, 640, "Q5_1"), (4096, 1536, "Q4_K"),
+                                      (1792, 2816, "Q4_K"), (2304, 256, "Q4_K"), (256, 256, "Q6_K"), (512, 768, "Q6_K"), (2048, 1024, "Q6_K"), (768, 2816, "Q6_K"), (2560, 640, "Q5_1"), (4096, 1536, "Q4_K"),
                                       (1536, 4096, "Q4_K")])
 def test_tiles_of_8_rows(monkeypatch, H, I, down):
     if down != "Q5_1":
