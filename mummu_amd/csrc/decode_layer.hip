@@ -138,15 +138,16 @@ __global__ __launch_bounds__(64 * kDlWaves) void decode_layer_kernel(const uint8
     const uint32_t drow_bytes = (uint32_t)type_row_bytes(DT, inter);
     const uint8_t *de = down + (size_t)uniform_index(e) * (size_t)hidden * drow_bytes;
     RawRow<DT, 1> rd[NITD];
+    const RowPieces<DT, 1> pieces(unit0d, rsd.units);
     auto fetch_down = [&](float after) {
         // (an offset of zero that the compiler cannot see through: the loads below wait for the value it is made of)
         unsigned zero;
         asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"(after));
 #pragma unroll
         for (int i = 0; i < NITD; i++) {
-            const int row = drow0 + i * rsd.rows_per_it + subd;
-            const bool ok = row < hidden;
-            load_row<DT, 1>(de, (uint32_t)(ok ? row : 0) * drow_bytes + zero, unit0d, rsd.units, ok, rd[i]);
+            const int first = drow0 + i * rsd.rows_per_it;
+            const RowsAt rows(first, hidden, drow_bytes, (uint32_t)subd * drow_bytes);
+            load_row<DT, 1>(de + rows.base, rows.off + zero, pieces, unit0d, rsd.units, first + subd < hidden, rd[i]);
         }
     };
     // (asked for behind the dots of iteration 0 / 1 / 2 / 3, one token on the OLMoE shape: 15.5 / 14.8 / 14.9 / 15.3 us per layer;

@@ -45,12 +45,14 @@ __device__ __forceinline__ void gate_up_tile(const uint8_t *gate, const uint8_t 
     // instead of after it (the scheduling barriers keep the compiler from hoisting every load
     // to the top, where a wave would sit blocked on issue until most of its data had arrived).
     RawRow<WT, UPL> rg[NIT], ru[NIT];
+    const RowPieces<WT, UPL> pieces(unit0, rs.units);
+    const uint32_t sub_off = (uint32_t)sub * row_bytes;
     auto fetch = [&](int i) {
-        const int row = row0 + i * rs.rows_per_it + sub;
-        const bool ok = row < inter;
-        const uint32_t row_off = (uint32_t)(ok ? row : 0) * row_bytes;
-        load_row<WT, UPL>(ge, row_off, unit0, rs.units, ok, rg[i]);
-        load_row<WT, UPL>(ue, row_off, unit0, rs.units, ok, ru[i]);
+        const int first = row0 + i * rs.rows_per_it;
+        const bool ok = first + sub < inter;
+        const RowsAt rows(first, inter, row_bytes, sub_off);
+        load_row<WT, UPL>(ge + rows.base, rows.off, pieces, unit0, rs.units, ok, rg[i]);
+        load_row<WT, UPL>(ue + rows.base, rows.off, pieces, unit0, rs.units, ok, ru[i]);
     };
     constexpr int AHEAD = NIT < 2 ? NIT : 2;
 #pragma unroll

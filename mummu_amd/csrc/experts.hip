@@ -307,11 +307,12 @@ __global__ __launch_bounds__(64 * kGemvWaves) void down_q_kernel(const uint8_t *
     float *yrow = y + (size_t)a * (size_t)hidden;
 
     RawRow<WT, UPL> rd[NIT];
+    const RowPieces<WT, UPL> pieces(unit0, rs.units);
 #pragma unroll
     for (int i = 0; i < NIT; i++) {
-        const int row = row0 + i * rs.rows_per_it + sub;
-        const bool ok = row < hidden;
-        load_row<WT, UPL>(de, (uint32_t)(ok ? row : 0) * row_bytes, unit0, rs.units, ok, rd[i]);
+        const int first = row0 + i * rs.rows_per_it;
+        const RowsAt rows(first, hidden, row_bytes, (uint32_t)sub * row_bytes);
+        load_row<WT, UPL>(de + rows.base, rows.off, pieces, unit0, rs.units, first + sub < hidden, rd[i]);
     }
     LaneAct<UPL> la;
     load_lane_act<WT, UPL>(actq, (size_t)a, inter, unit0, rs.units, la);
@@ -432,12 +433,13 @@ __global__ __launch_bounds__(64 * kDcWaves) void down_combine_q_kernel(
     // same software pipeline as gate/up, over the wave's KPW*NIT (expert, row iteration) steps
     RawRow<WT, UPL> rd[KPW][NIT];
     LaneAct<UPL> la[KPW];
+    const RowPieces<WT, UPL> pieces(unit0, rs.units);
     auto fetch = [&](int step) {
         const int i = step / NIT, it = step % NIT;
         const uint8_t *de = down + (size_t)uniform_index(on_p[i] ? e_p[i] : 0) * (size_t)hidden * row_bytes;
-        const int row = row0 + it * rs.rows_per_it + sub;
-        const bool ok = on_p[i] && row < hidden;
-        load_row<WT, UPL>(de, (uint32_t)(ok ? row : 0) * (uint32_t)row_bytes, unit0, rs.units, ok, rd[i][it]);
+        const int first = row0 + it * rs.rows_per_it;
+        const RowsAt rows(first, hidden, (uint32_t)row_bytes, (uint32_t)sub * (uint32_t)row_bytes);
+        load_row<WT, UPL>(de + rows.base, rows.off, pieces, unit0, rs.units, on_p[i] && first + sub < hidden, rd[i][it]);
     };
     constexpr int STEPS = KPW * NIT;
     constexpr int AHEAD = STEPS < 2 ? STEPS : 2;
@@ -724,9 +726,11 @@ hipError_t launch_gate_up_routed(const ExpertBanks &b, QAct xq, const RouteInlin
     return with_bank_type(b.gate_type, [&](auto tag) {
         constexpr int WT = decltype(tag)::value;
         if constexpr (is_quant_type(WT)) {
-            // (eight row iterations per wave from eight tokens on: the same routing and activation loads serve twice the
-            // rows - 29.3 against 30.0 us at 8 tokens of the OLMoE shape, but 12.7 against 11.8 at 2)
-            if (!wide && n_tokens >= 8 && b.inter % 32 == 0) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
+            // (eight row iterations per wave from some tokens on: the same routing and activation loads serve twice the rows, and the vector
+            // ALUs, which bound several tokens' launches, have a tenth less to do.  Q4_K, a layer among others, us, four / eight iterations:
+            // OLMoE 3 / 4 / 5 / 7 tokens 17.1 / 17.0, 21.3 / 20.4, 25.3 / 24.4, 31.5 / 30.1, 128 experts of 2048 x 768, 3 / 6 tokens 16.0 / 15.0, 30.6 / 27.2;
+            // at 2 tokens one on its own is no faster.  Q8_0 at 4 tokens 45.8 / 46.9, the launch at 8 29.3 against 30.0)
+            if (!wide && n_tokens >= (WT == T_Q4_K ? 3 : 8) && b.inter % 32 == 0) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
             return wide ? launch_gate_up_routed_t<WT, 2, 2>(b, xq, route, n_tokens, k, actq, flags, s)
                         : launch_gate_up_routed_t<WT, 1, 4>(b, xq, route, n_tokens, k, actq, flags, s);
         } else {

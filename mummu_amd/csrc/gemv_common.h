@@ -135,48 +135,74 @@ constexpr bool is_legacy32(int t) { return t == T_Q4_0 || t == T_Q4_1 || t == T_
 // scalar registers.
 __device__ __forceinline__ int uniform_index(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// The lane's share of the weight row that starts row_off bytes into the matrix at `base` (the same pointer in every
-// lane - see uniform_index - so that a load is a scalar base plus a 32-bit lane offset: the matrix of one expert stays
-// below 4 GB).
+// Where a lane's pieces lie from the first row of an iteration on (rows side by side: lane row `sub`), as 32-bit offsets that are the
+// same for every iteration and matrix: a load is a scalar base (the iteration's first row) plus one of them.  (As 64-bit lane
+// addresses, put together for each row, they took 8 to 14 of a row dot's 66 to 109 instructions.)
+template <int WT>
+constexpr int row_pieces() { return WT == T_Q6_K ? 4 : WT == T_Q5_K ? 3 : WT == T_Q4_K ? 2 : 1; }
 template <int WT, int UPL>
-__device__ inline void load_row(const uint8_t *base, uint32_t row_off, int unit0, int units, bool ok, RawRow<WT, UPL> &r) {
-    // Every lane loads unconditionally (a lane without a unit re-reads the row's last unit, a
-    // lane of a row past the matrix reads the valid row the caller passes instead): straight-line
-    // loads keep the wait counts exact, so rows still in flight are not waited for early.  What
-    // must not count gets a zero block scale, which makes its contribution exactly 0.
+struct RowPieces {
+    uint32_t at[UPL][row_pieces<WT>()];
+    __device__ RowPieces(int unit0, int units) {
+#pragma unroll
+        for (int i = 0; i < UPL; i++) {
+            const int u = unit0 + 64 * i;
+            const uint32_t uc = (uint32_t)(u < units ? u : units - 1);   // a lane without a unit re-reads the row's last one
+            if constexpr (WT == T_Q4_K) {
+                at[i][0] = (uc >> 3) * 144u;
+                at[i][1] = at[i][0] + 16u + (uc & 7) * 16u;
+            } else if constexpr (WT == T_Q5_K) {
+                at[i][0] = (uc >> 3) * 176u;   // 176 = 11 * 16: every piece is 16-byte aligned
+                at[i][1] = at[i][0] + 16u + (uc & 1) * 16u;
+                at[i][2] = at[i][0] + 48u + (uc & 7) * 16u;
+            } else if constexpr (WT == T_Q6_K) {
+                const uint32_t blk = (uc >> 3) * 210u, up = uc & 7;   // 2-byte aligned only
+                at[i][0] = blk + 16u * up;
+                at[i][1] = blk + 128u + (up >> 2) * 32u + (up & 1) * 16u;
+                at[i][2] = blk + 192u + (up >> 2) * 8u + ((up >> 1) & 1) * 2u + (up & 1);
+                at[i][3] = blk + 208u;
+            } else {
+                at[i][0] = uc * (uint32_t)block_bytes(WT);
+            }
+        }
+    }
+};
+
+// The lane's share of row `row_off` bytes behind `base`, the same pointer in every lane (see uniform_index); row_off below 4 GB.
+template <int WT, int UPL>
+__device__ inline void load_row(const uint8_t *base, uint32_t row_off, const RowPieces<WT, UPL> &pieces, int unit0, int units, bool ok, RawRow<WT, UPL> &r) {
+    // Every lane loads unconditionally (a lane of a row past the matrix reads the valid row the
+    // caller passes instead): straight-line loads keep the wait counts exact, so rows still in flight
+    // are not waited for early.  What must not count gets a zero block scale, which makes its
+    // contribution exactly 0.
 #pragma unroll
     for (int i = 0; i < UPL; i++) {
-        const int u = unit0 + 64 * i;
-        const bool on = ok && u < units;
-        const int uc = u < units ? u : units - 1;
+        const bool on = ok && unit0 + 64 * i < units;
+        auto from = [&](int piece) { return base + (row_off + pieces.at[i][piece]); };
         if constexpr (WT == T_Q4_K) {
-            const uint8_t *blk = base + (row_off + (uint32_t)(uc >> 3) * 144u);
-            r.hdr[i] = *(const uint4 *)blk;
-            r.q[i] = *(const uint4 *)(blk + 16 + (uc & 7) * 16);
+            r.hdr[i] = *(const uint4 *)from(0);
+            r.q[i] = *(const uint4 *)from(1);
             r.hdr[i].x = on ? r.hdr[i].x : 0u;  // d = dmin = 0
         } else if constexpr (WT == T_Q5_K) {
-            const uint8_t *blk = base + (row_off + (uint32_t)(uc >> 3) * 176u);  // 176 = 11 * 16: every piece is 16-byte aligned
-            r.hdr[i] = *(const uint4 *)blk;
-            r.qh[i] = *(const uint4 *)(blk + 16 + (uc & 1) * 16);
-            r.q[i] = *(const uint4 *)(blk + 48 + (uc & 7) * 16);
+            r.hdr[i] = *(const uint4 *)from(0);
+            r.qh[i] = *(const uint4 *)from(1);
+            r.q[i] = *(const uint4 *)from(2);
             r.hdr[i].x = on ? r.hdr[i].x : 0u;
         } else if constexpr (WT == T_Q6_K) {
-            const uint8_t *blk = base + (row_off + (uint32_t)(uc >> 3) * 210u);  // 2-byte aligned only
-            const int up = uc & 7;
+            const uint8_t *ql = from(0), *qh = from(1), *sc = from(2);
 #pragma unroll
             for (int w = 0; w < 4; w++) {
-                __builtin_memcpy(&r.ql[i][w], blk + 16 * up + 4 * w, 4);
-                __builtin_memcpy(&r.qh[i][w], blk + 128 + (up >> 2) * 32 + (up & 1) * 16 + 4 * w, 4);
+                __builtin_memcpy(&r.ql[i][w], ql + 4 * w, 4);
+                __builtin_memcpy(&r.qh[i][w], qh + 4 * w, 4);
             }
-            const uint8_t *sc = blk + 192 + (up >> 2) * 8 + ((up >> 1) & 1) * 2 + (up & 1);
             r.sc[i] = (uint32_t)sc[0] | ((uint32_t)sc[4] << 8);
             uint16_t db;
-            __builtin_memcpy(&db, blk + 208, 2);
+            __builtin_memcpy(&db, from(3), 2);
             r.d[i] = on ? (uint32_t)db : 0u;
         } else if constexpr (is_legacy32(WT)) {
             constexpr bool has_m = WT == T_Q4_1 || WT == T_Q5_1;
             constexpr bool has_h = WT == T_Q5_0 || WT == T_Q5_1;
-            const uint8_t *blk = base + (row_off + (uint32_t)uc * (uint32_t)block_bytes(WT));
+            const uint8_t *blk = from(0);
             uint16_t db, mb = 0;
             __builtin_memcpy(&db, blk, 2);
             if constexpr (has_m) __builtin_memcpy(&mb, blk + 2, 2);
@@ -190,7 +216,7 @@ __device__ inline void load_row(const uint8_t *base, uint32_t row_off, int unit0
 #pragma unroll
             for (int w = 0; w < 4; w++) __builtin_memcpy(&r.q[i][w], p + 4 * w, 4);
         } else {
-            const uint8_t *blk = base + (row_off + (uint32_t)uc * 34u);
+            const uint8_t *blk = from(0);
             uint16_t db;
             __builtin_memcpy(&db, blk, 2);
             r.d[i] = on ? (uint32_t)db : 0u;
@@ -199,6 +225,19 @@ __device__ inline void load_row(const uint8_t *base, uint32_t row_off, int unit0
         }
     }
 }
+
+// The rows of an iteration, first .. first + rows_per_it - 1 of `total` (first the same in every lane): where its first one lies, and how far behind it
+// the lane's (row first + sub; past the last one, the last).
+struct RowsAt {
+    size_t base;
+    uint32_t off;
+    __device__ RowsAt(int first, int total, uint32_t row_bytes, uint32_t sub_off) {
+        const uint32_t f = (uint32_t)uniform_index(first < total ? first : 0);
+        base = (size_t)f * row_bytes;
+        const uint32_t last = ((uint32_t)total - 1u - f) * row_bytes;
+        off = sub_off < last ? sub_off : last;
+    }
+};
 
 // The 6-bit (scale, min) of sub-blocks 2c and 2c+1 of a Q4_K / Q5_K super-block (ggml
 // get_scale_min_k4), each pair packed as two bytes (sub-block 2c in byte 0), without a branch:
@@ -307,8 +346,8 @@ __device__ inline float dot_row(const RawRow<WT, UPL> &r, int unit0, const LaneA
                 const float d = half_bits_to_float((uint16_t)r.d[i]);
 #pragma unroll
                 for (int w = 0; w < 4; w++) {
-                    c0[w] = (r.ql[i][w] & 0x0F0F0F0Fu) | (((r.qh[i][w] >> (2 * jj)) & 0x03030303u) << 4);
-                    c1[w] = ((r.ql[i][w] >> 4) & 0x0F0F0F0Fu) | (((r.qh[i][w] >> (2 * jj + 4)) & 0x03030303u) << 4);
+                    c0[w] = (r.ql[i][w] & 0x0F0F0F0Fu) | ((r.qh[i][w] << (4 - 2 * jj)) & 0x30303030u);
+                    c1[w] = ((r.ql[i][w] >> 4) & 0x0F0F0F0Fu) | ((r.qh[i][w] >> (2 * jj)) & 0x30303030u);
                 }
                 A0 = __fmul_rn(d, (float)(int)(int8_t)(r.sc[i] & 0xFFu));
                 A1 = __fmul_rn(d, (float)(int)(int8_t)((r.sc[i] >> 8) & 0xFFu));
