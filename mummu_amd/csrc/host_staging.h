@@ -36,6 +36,11 @@ public:
     // Enqueues the copy of `bytes` bytes to dev; `host` may be reused when the call returns.
     hipError_t upload(void *dev, const void *host, size_t bytes, hipStream_t s);
 
+    // Where a last kernel can leave `bytes` bytes for the host by itself: given to download() as a piece's `dev`, they are not copied, only
+    // marked as there behind everything enqueued before.  Null where they take more than a slot (several are copied and read in
+    // turns).  The kernel writes every byte once and reads none of them.
+    void *out_direct(size_t bytes) const;
+
     // Up to kPieces device arrays read back together behind everything enqueued on s.  `early` (nullable) is read back
     // ahead of them: check(early copy) runs before anything is written to the caller's memory, and its non-zero status
     // ends the call (returned through *status).

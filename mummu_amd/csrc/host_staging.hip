@@ -142,6 +142,8 @@ hipError_t HostStaging::finish(hipStream_t s) {
     return e;
 }
 
+void *HostStaging::out_direct(size_t bytes) const { return slab_ && bytes <= kSlot ? slab_->out(0) : nullptr; }
+
 const void *HostStaging::early_host() const { return slab_->early(); }
 
 HostStaging::Chunk HostStaging::chunk_at(int i) const {
@@ -235,7 +237,7 @@ hipError_t HostStaging::begin_download(const Piece *pieces, int n, const void *e
         for (int i = 0; i < n; i++) {
             r.src[r.n] = (const uint8_t *)pieces[i].dev;
             r.dst[r.n] = slab_->out(0) + at;
-            r.bytes[r.n] = pieces[i].bytes;
+            r.bytes[r.n] = pieces[i].dev == slab_->out(0) ? 0 : pieces[i].bytes;   // (out_direct: the one piece)
             r.row[r.n++] = 1 + i;
             at += round16(pieces[i].bytes);
         }

@@ -1552,8 +1552,11 @@ int mummu_expert_run(mummu_moe *h, int layer, int expert, const float *x, int64_
     const size_t bytes = sizeof(float) * (size_t)rows * (size_t)hidden;
     HostStaging io;
     if ((rc = upload_rows(h, io, h->xin, x, bytes, s))) return rc;
-    if ((rc = run_one_expert(h, h->layers[layer], expert, h->xin, (int)rows, h->y, s))) return rc;
-    return download_rows(h, io, out, h->y, bytes, s, false);
+    // The down product leaves up to 512 KB where the host takes them: 48 rows of OLMoE 65.4 -> 62.5 us, 8: 32.9 -> 31.3, Q8_0 16 / 64: 49.0 -> 46.3, 101 ->
+    // 99.  (The block's last kernels from the host's rows, the same way: 1 / 12 / 48 tokens 31.5 / 90.5 / 124 -> 32.1 / 89.5 / 128.)
+    float *direct = (float *)io.out_direct(bytes), *result = direct ? direct : h->y;
+    if ((rc = run_one_expert(h, h->layers[layer], expert, h->xin, (int)rows, result, s))) return rc;
+    return download_rows(h, io, out, result, bytes, s, false);
 }
 
 int mummu_expert_gate_energy(mummu_moe *h, int layer, int expert, const float *x, int64_t rows, int hidden, float *energy) {
