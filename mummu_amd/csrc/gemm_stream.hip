@@ -12,8 +12,9 @@
 // tokens 237 -> 206, 128 of 3072 x 768, 30 tokens 117 -> 103.
 //
 // Q6_K downs (tiles of 8 rows): a sub-block's 16 elements are an operand's K of 16 (v_mfma_f32_16x16x16_f16), four to a lane, so that its sum can
-// be folded with d * sc; a lane loads 16 neighbouring bytes and changes dwords with the three others of its row.  262 vector instructions a unit, 53 % of
-// the cycles, and 8 % products.  OLMoE, 24 tokens 42 -> 35 us (106 MB fetched, the weights' bytes), layers at 16 / 24 / 32 tokens 73 / 74 / 76 -> 62 / 65 / 67.
+// be folded with d * sc; a lane loads 16 neighbouring bytes, in whole dwords, and changes dwords with the three others of its row.  Some 280 vector
+// instructions a unit.  OLMoE, 24 tokens 42 -> 32 us (106 MB fetched, the weights' bytes; 35 with loads at odd halves of a dword), layers at 16 / 24 /
+// 32 tokens 73 / 74 / 76 -> 61 / 64 / 65, 128 experts of 2048 x 768, 30 tokens 99 -> 81 (92).
 #include "device_utils.h"
 #include "kernels.h"
 #include "q4k_half.h"
@@ -88,22 +89,26 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
     Global *base[NB];
     base[0] = (Global *)uniform(p.w0 + matrix + (size_t)col0 * row_bytes);
     if (GATE_UP) base[NB - 1] = (Global *)uniform(p.w1 + matrix + (size_t)col0 * row_bytes);
-    const uint32_t off_h = (uint32_t)c * row_bytes + (uint32_t)sb * kBlock, off_q = off_h + (Q6 ? 0u : 16u) + 16u * (uint32_t)kg;
+    // (a Q6_K super-block begins at an even byte: it is read by whole dwords, from `skip` bytes in front of it on - 16 bytes at an odd half of
+    // a dword keep the address units busy for several times as long.  Steps are multiples of 4 bytes.)
+    const uint32_t low = Q6 ? (uint32_t)(uint64_t)base[0] & 2u : 0u, begin = (uint32_t)c * row_bytes + (uint32_t)sb * kBlock + low, skip = Q6 ? begin & 2u : 0u;
+    base[0] -= low;
+    const uint32_t off_h = begin - skip, off_q = off_h + (Q6 ? 0u : 16u) + 16u * (uint32_t)kg;
     const uint32_t step_bytes = 16u * (uint32_t)n_groups * row_bytes;
-    // (DEPTH - 1 units on their way.  Q4_K: header, codes; Q6_K: scales, ql, ql, qh, d)
+    // (DEPTH - 1 units on their way.  Q4_K: header, codes; Q6_K: scales and d, ql, ql, qh)
     u32x4 hd[DEPTH], q0[DEPTH], q1[DEPTH], qh[Q6 ? DEPTH : 1];
-    uint32_t dd[Q6 ? DEPTH : 1];
+    uint32_t more[Q6 ? DEPTH : 1][4];   // ... the dword behind each of the four
     auto load = [&](int step, int j, int to) {
         Global *from = base[j] + (size_t)((uint32_t)step * step_bytes);
         typedef __attribute__((address_space(1))) const u32x4 Words;
-        if constexpr (Q6) {   // (a super-block begins at an even byte)
-            typedef u32x4 Loose __attribute__((aligned(2)));
+        if constexpr (Q6) {
+            typedef u32x4 Loose __attribute__((aligned(4)));
             typedef __attribute__((address_space(1))) const Loose LooseWords;
-            q0[to] = *(LooseWords *)(from + off_q);
-            q1[to] = *(LooseWords *)(from + off_q + 64);
-            qh[to] = *(LooseWords *)(from + off_q + 128);
-            hd[to] = *(LooseWords *)(from + off_h + 192);
-            dd[to] = *(__attribute__((address_space(1))) const uint16_t *)(from + off_h + 208);
+            typedef __attribute__((address_space(1))) const uint32_t Word;
+            q0[to] = *(LooseWords *)(from + off_q), more[to][0] = *(Word *)(from + off_q + 16);
+            q1[to] = *(LooseWords *)(from + off_q + 64), more[to][1] = *(Word *)(from + off_q + 80);
+            qh[to] = *(LooseWords *)(from + off_q + 128), more[to][2] = *(Word *)(from + off_q + 144);
+            hd[to] = *(LooseWords *)(from + off_h + 192), more[to][3] = *(Word *)(from + off_h + 208);   // (up to two bytes behind it: kBankSlack)
         } else {
             hd[to] = *(Words *)(from + off_h);
             q0[to] = *(Words *)(from + off_q);
@@ -182,8 +187,15 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
             swap(r[0], r[2], true), swap(r[1], r[3], true), swap(r[0], r[1], false), swap(r[2], r[3], false);
             t = u32x4{r[0], r[1], r[2], r[3]};
         };
+        const uint32_t(&behind)[4] = more[Q6 ? b : 0];
+        auto align = [&](u32x4 &t, uint32_t next) {
+            const uint32_t r[5] = {t[0], t[1], t[2], t[3], next};
+#pragma unroll
+            for (int i = 0; i < 4; i++) t[i] = __builtin_amdgcn_alignbyte(r[i + 1], r[i], skip);
+        };
+        align(q0[b], behind[0]), align(q1[b], behind[1]), align(qh[Q6 ? b : 0], behind[2]), align(hd[b], behind[3]);
         turn(q0[b]), turn(q1[b]), turn(qh[Q6 ? b : 0]);
-        const float d = half_bits_to_float((uint16_t)dd[Q6 ? b : 0]);
+        const float d = half_bits_to_float((uint16_t)(behind[3] >> (8u * skip)));
         f32x4 v = zero;
 #pragma unroll
         for (int half = 0; half < 2; half++) {
