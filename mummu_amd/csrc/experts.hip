@@ -523,7 +523,12 @@ static hipError_t launch_gate_up_t(const ExpertBanks &b, const float *x, QAct xq
             launch_kernel(gate_up_q_kernel<WT, UPL, NIT, false>, grid, block, lds, s,                                      \
                 b.gate, b.up, xq, ids, k, fixed_expert, b.hidden, b.inter, b.n_experts, act, actq, flags, RouteInline());      \
     } while (0)
-        if (upl == 1 && n_assign / slots >= 8 && fixed_expert < 0 && b.inter % 32 == 0) MUMMU_GUQ(1, 8);  // (as launch_gate_up_routed)
+        bool eight = false;   // (row iterations: as launch_gate_up_routed)
+        if constexpr (WT != T_Q8_0) {
+            eight = upl == 1 && n_assign / slots >= 8 && fixed_expert < 0 && b.inter % 32 == 0;
+            if (eight) MUMMU_GUQ(1, 8);
+        }
+        if (eight) {}
         else if (upl == 1) MUMMU_GUQ(1, 4);
         else if (upl == 2) MUMMU_GUQ(2, 2);
         else if (upl <= 4) MUMMU_GUQ(4, 1);
@@ -729,8 +734,9 @@ hipError_t launch_gate_up_routed(const ExpertBanks &b, QAct xq, const RouteInlin
             // (eight row iterations per wave from some tokens on: the same routing and activation loads serve twice the rows, and the vector
             // ALUs, which bound several tokens' launches, have a tenth less to do.  Q4_K, a layer among others, us, four / eight iterations:
             // OLMoE 3 / 4 / 5 / 7 tokens 17.1 / 17.0, 21.3 / 20.4, 25.3 / 24.4, 31.5 / 30.1, 128 experts of 2048 x 768, 3 / 6 tokens 16.0 / 15.0, 30.6 / 27.2;
-            // at 2 tokens one on its own is no faster.  Q8_0 at 4 tokens 45.8 / 46.9, the launch at 8 29.3 against 30.0)
-            if (!wide && n_tokens >= (WT == T_Q4_K ? 3 : 8) && b.inter % 32 == 0) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
+            // at 2 tokens one on its own is no faster.  Others from eight on, but for Q8_0, whose rows take more registers: 83 / 209 at 8.)
+            if constexpr (WT != T_Q8_0)
+                if (!wide && n_tokens >= (WT == T_Q4_K ? 3 : 8) && b.inter % 32 == 0) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
             return wide ? launch_gate_up_routed_t<WT, 2, 2>(b, xq, route, n_tokens, k, actq, flags, s)
                         : launch_gate_up_routed_t<WT, 1, 4>(b, xq, route, n_tokens, k, actq, flags, s);
         } else {

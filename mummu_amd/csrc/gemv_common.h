@@ -98,8 +98,9 @@ struct RawRow<T_Q4_K, UPL> {
 };
 template <int UPL>
 struct RawRow<T_Q8_0, UPL> {
-    uint32_t d[UPL];     // f16 scale bits
-    uint32_t q[UPL][8];  // 32 int8 codes
+    uint32_t d[UPL];     // f16 scale bits, in the low half
+    uint32_t w[UPL][9];  // the nine dwords that hold the block
+    uint32_t pick[UPL];  // v_perm selector: dword j of the codes out of w[j], w[j + 1]
 };
 
 // Legacy 32-element blocks (Q4_0 18 B, Q4_1 20 B, Q5_0 22 B, Q5_1 24 B): f16 d (, f16 m)
@@ -189,6 +190,8 @@ __device__ inline void load_row(const uint8_t *base, uint32_t row_off, const Row
             r.q[i] = *(const uint4 *)from(2);
             r.hdr[i].x = on ? r.hdr[i].x : 0u;
         } else if constexpr (WT == T_Q6_K) {
+            // (as they lie, at even bytes: in whole dwords as Q8_0 below, the eight instructions that put them together cost more, six tokens of
+            // eight layers 284 -> 301 us)
             const uint8_t *ql = from(0), *qh = from(1), *sc = from(2);
 #pragma unroll
             for (int w = 0; w < 4; w++) {
@@ -216,12 +219,16 @@ __device__ inline void load_row(const uint8_t *base, uint32_t row_off, const Row
 #pragma unroll
             for (int w = 0; w < 4; w++) __builtin_memcpy(&r.q[i][w], p + 4 * w, 4);
         } else {
-            const uint8_t *blk = from(0);
-            uint16_t db;
-            __builtin_memcpy(&db, blk, 2);
-            r.d[i] = on ? (uint32_t)db : 0u;
+            // A block of 34 bytes begins at an even byte: whole dwords from the one it begins in (or in the middle of).  Loads at odd halves
+            // of a dword keep the address units busy: 267 clocks for a row of 2176 bytes, gate/up of 6 tokens 48.8 us with the ALUs
+            // 21 % busy.  (The last may end two bytes behind the block: banks have kBankSlack behind them.)
+            const uint64_t at = (uint64_t)base;   // (the same in every lane)
+            const uint32_t off = row_off + pieces.at[i][0] + ((uint32_t)at & 2u), skip = off & 2u;
+            const uint32_t *from4 = (const uint32_t *)((base - ((uint32_t)at & 2u)) + (off - skip));
 #pragma unroll
-            for (int w = 0; w < 8; w++) __builtin_memcpy(&r.q[i][w], blk + 2 + 4 * w, 4);  // 2-byte aligned
+            for (int w = 0; w < 9; w++) r.w[i][w] = from4[w];
+            r.d[i] = on ? r.w[i][0] >> (8u * skip) : 0u;
+            r.pick[i] = skip ? 0x07060504u : 0x05040302u;
         }
     }
 }
@@ -375,21 +382,24 @@ __device__ inline float dot_row(const RawRow<WT, UPL> &r, int unit0, const LaneA
             acc = __builtin_fmaf(a.fsx[i][0], B0, acc);
             acc = __builtin_fmaf(a.fsx[i][1], B1, acc);
         } else {  // Q8_0
-            const float d = half_bits_to_float((uint16_t)r.d[i]);
+            const float d = half_bits_to_float((uint16_t)(r.d[i] & 0xFFFFu));
+            uint32_t q[8];
+#pragma unroll
+            for (int w = 0; w < 8; w++) q[w] = __builtin_amdgcn_perm(r.w[i][w + 1], r.w[i][w], r.pick[i]);
             int h0 = 0, l0 = 0, h1 = 0, l1 = 0;
 #pragma unroll
             for (int w = 0; w < 4; w++) {
                 if (w == 0) {
-                    h0 = sdot4_first((int)r.q[i][0], a.xh[i][0]);
-                    l0 = sdot4_first((int)r.q[i][0], a.xl[i][0]);
-                    h1 = sdot4_first((int)r.q[i][4], a.xh[i][4]);
-                    l1 = sdot4_first((int)r.q[i][4], a.xl[i][4]);
+                    h0 = sdot4_first((int)q[0], a.xh[i][0]);
+                    l0 = sdot4_first((int)q[0], a.xl[i][0]);
+                    h1 = sdot4_first((int)q[4], a.xh[i][4]);
+                    l1 = sdot4_first((int)q[4], a.xl[i][4]);
                     continue;
                 }
-                h0 = __builtin_amdgcn_sdot4((int)r.q[i][w], a.xh[i][w], h0, false);
-                l0 = __builtin_amdgcn_sdot4((int)r.q[i][w], a.xl[i][w], l0, false);
-                h1 = __builtin_amdgcn_sdot4((int)r.q[i][4 + w], a.xh[i][4 + w], h1, false);
-                l1 = __builtin_amdgcn_sdot4((int)r.q[i][4 + w], a.xl[i][4 + w], l1, false);
+                h0 = __builtin_amdgcn_sdot4((int)q[w], a.xh[i][w], h0, false);
+                l0 = __builtin_amdgcn_sdot4((int)q[w], a.xl[i][w], l0, false);
+                h1 = __builtin_amdgcn_sdot4((int)q[4 + w], a.xh[i][4 + w], h1, false);
+                l1 = __builtin_amdgcn_sdot4((int)q[4 + w], a.xl[i][4 + w], l1, false);
             }
             const float t = __builtin_fmaf(a.s[i][0], (float)(h0 * 256 + l0), __fmul_rn(a.s[i][1], (float)(h1 * 256 + l1)));
             acc = __builtin_fmaf(d, t, acc);
