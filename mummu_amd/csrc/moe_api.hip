@@ -480,27 +480,29 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 // already holds the 16-bit form of x (the fused router produced it).
 // Smallest batch of this layer that takes the batched path (INT_MAX: never).
 //
-// gemm_min_*: where the two forms meet on the OLMoE shape with nothing else to go by.  Banks that take the f16 units (Q4_K gate and up, Q8_0)
-// meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and `from` tokens: below, they have fewer
-// launches) the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode against batched:
-//   Q4_K, OLMoE 11 tokens (311 MB) 80 / 48 against 80 / 44, 15: 94 / 62 against 82 / 47; 128 experts of 2048 x 768, 16 (339 MB): 96 / 63 against
-//   94 / 54; 512 of them top-10, 12 (318 MB): 133 / 104 against 123 / 72.
-//   Q4_K with Q6_K downs, OLMoE, 11 / 12 tokens (359 / 391 MB): 90 / 59, 92 / 63 against 92 / 54, 91 / 54; 128 of 2048 x 768, 16 (416 MB): 109 / 75 against 108 / 71.
-//   Q4_K with other downs, OLMoE Q5_1, 15 (472 MB): 98 / 64 against 93 / 57.
-//   Q8_0, OLMoE, 8 / 9 tokens (428 / 481 MB): 108 / 83, 124 / 90 against 118 / 70, 120 / 73; 128 experts of 2048 x 768, 12 (481 MB): 137 / 105 against 137 / 88.
+// gemm_min_*: where the two forms met on the OLMoE shape with the kernels of their time.  Banks that take the f16 units (Q4_K gate and up; Q8_0
+// of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and six or nine
+// tokens: below, they have fewer launches) the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode
+// against batched:
+//   Q4_K, OLMoE 11 / 13 tokens (311 / 368 MB) 83 / 50, 90 / 57 against 80 / 44, 83 / 47; 128 experts of 2048 x 768, 15 (318 MB): 97 / 61 against 94 / 52; 512
+//   of them top-10, 12 (318 MB): 133 / 104 against 123 / 72.
+//   Q4_K with Q6_K downs, OLMoE, 11 / 12 tokens (359 / 391 MB): 91 / 59, 93 / 63 against 93 / 53, 94 / 53; 128 of 2048 x 768, 15 (390 MB): 108 / 71 against 102 / 62.
+//   Q4_K with other downs, OLMoE Q5_1, 16 (504 MB): 102 / 68 against 92 / 58.
 // Rows of more than 2048 elements are more than a wave's 64 blocks of 32, and the decode kernels take two a lane, some of them none:
-//   hidden 2560: 512 experts of 640 with Q5_1 downs, 4 / 9 tokens 86 / 60, 160 / 134 against 76 / 38, 112 / 69; 64 of them, 6: 75 / 50 against 69 / 33; 128 of
-//   768, 9: 111 / 70 against 114 / 54.  4096: 16 experts of 1792 top-4, 6: 102 / 73 against 82 / 49, Q6_K downs 112 / 84 against 102 / 68, Q8_0 140 / 110
-//   against 115 / 80; 128 of 1536, 6: 164 / 136 against 167 / 111.
+//   hidden 2560: 512 experts of 640 with Q5_1 downs, 6 tokens 113 / 91 against 99 / 55; 64 of them, 7: 76 / 49 against 70 / 34; 128 of 768, 7: 95 / 69
+//   against 90 / 45; 512 of 640 in Q8_0, 8: 157 / 130 against 159 / 104.  4096: 16 experts of 1792 top-4, 6: 92 / 64 against 80 / 48, Q6_K downs 101 / 73
+//   against 93 / 59, Q8_0 116 / 88 against 117 / 80; 128 of 1536, 6: 163 / 135 against 163 / 106.
+// (Q8_0 of 2048: since its blocks are read by whole dwords the decode kernels are ahead beyond 13 tokens, OLMoE 15: 109 / 88 against 126 / 86, 17: 117 / 97
+// against 127 / 90; from 13 on the batched form's pairs of halfs stay, 2.5e-7 off the 64-bit result where 16 bits a block are 3.3e-5.)
 int batched_from(const mummu_moe *h, const Layer &L) {
     const ExpertBanks b = banks_of(h, L);
     if (!grouped_gemm_supported(b)) return 0x7fffffff;
     if (b.gate_type == T_F32) return h->gemm_min_f32;
     const bool q4k = h->gemm_q4k_f16 && grouped_gemm_q4k_f16(b), q4k_down = q4k && grouped_gemm_q4k_f16_down(b), q8 = q8_half_pairs(h, b);
     const int line = q4k_down ? h->gemm_min_q4k : q8 ? h->gemm_min_q8 : grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
-    if (h->gemm_min_given || !(q4k || q8)) return line;
     const bool wide = b.hidden > 2048;
-    const double bytes = 1e6 * (q8 ? (wide ? 300.0 : 450.0) : wide ? 180.0 : q4k_down ? 310.0 : grouped_gemm_q6k_down(b) ? 400.0 : 480.0);
+    if (h->gemm_min_given || !(q4k || (q8 && wide))) return line;
+    const double bytes = 1e6 * (q8 ? 450.0 : wide ? 180.0 : q4k_down ? 310.0 : grouped_gemm_q6k_down(b) ? 390.0 : 480.0);
     auto row_bytes = [](int type, int d) { return (double)(d / block_elems(type)) * block_bytes(type); };
     const double expert = 2.0 * b.inter * row_bytes(b.gate_type, b.hidden) + (double)b.hidden * row_bytes(b.down_type, b.inter);
     const int from = wide ? 6 : 9, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));

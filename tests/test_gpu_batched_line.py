@@ -9,8 +9,8 @@ from mummu_amd import synth
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("H,I,E,k,bank,down,line", [(4096, 1792, 8, 4, "Q4_K", "Q4_K", 6), (2560, 640, 24, 10, "Q4_K", "Q5_1", 6), (2048, 1024, 16, 8, "Q8_0", "Q8_0", 9),
-                                                    (2048, 1024, 16, 8, "Q4_K", "Q4_K", 11), (2048, 1024, 16, 8, "Q4_K", "Q6_K", 13), (2048, 1024, 16, 8, "Q4_K", "Q5_1", 16), (1024, 512, 8, 4, "Q4_K", "Q4_K", 18)])
+@pytest.mark.parametrize("H,I,E,k,bank,down,line", [(4096, 1792, 8, 4, "Q4_K", "Q4_K", 6), (2560, 640, 24, 10, "Q4_K", "Q5_1", 6), (2048, 1024, 16, 8, "Q8_0", "Q8_0", 13), (4096, 1792, 8, 4, "Q8_0", "Q8_0", 6),
+                                                    (2048, 1024, 16, 8, "Q4_K", "Q4_K", 11), (2048, 1024, 16, 8, "Q4_K", "Q6_K", 12), (2048, 1024, 16, 8, "Q4_K", "Q5_1", 16), (1024, 512, 8, 4, "Q4_K", "Q4_K", 18)])
 def test_both_sides_of_the_line(monkeypatch, H, I, E, k, bank, down, line):
     rng = np.random.Generator(np.random.PCG64(H + E))
     bt, dt = getattr(M, bank), getattr(M, down)
