@@ -217,7 +217,7 @@ MUMMU_API int mummu_moe_dequantize_expert(mummu_moe *h, int layer, int which, in
  * a Q4_K expert from some ten rows of a large one on (there with a power of two per row and 256 elements, and an absolute error of at most
  * 2^-39 of the largest of those, where the per-row kernels' is 2^-16 of the largest of 16).
  * The environment variable MUMMU_GEMM_Q4K_F16=0, read by mummu_moe_create, keeps Q4_K on the
- * integer form above; MUMMU_GEMM_TILE_ROWS=16, 32 or 64 fixes the rows per tile of these kernels (by default the
+ * integer form above; MUMMU_GEMM_TILE_ROWS=8, 16, 32 or 64 fixes the rows per tile of these kernels (by default the
  * library picks the form with the smallest expected cost for the batch: same results, different speed).
  * Q8_0 banks have an optional further form on the batched path, MUMMU_GEMM_Q8_F16=1 (read by mummu_moe_create):
  * the grouped GEMM of the F16 banks with every weight d * code held exactly as two halfs, x and the activations
