@@ -145,9 +145,9 @@ __global__ __launch_bounds__(64 * kDlWaves) void decode_layer_kernel(const uint8
         asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"(after));
 #pragma unroll
         for (int i = 0; i < NITD; i++) {
-            const int first = drow0 + i * rsd.rows_per_it;
-            const RowsAt rows(first, hidden, drow_bytes, (uint32_t)subd * drow_bytes);
-            load_row<DT, 1>(de + rows.base, rows.off + zero, pieces, unit0d, rsd.units, first + subd < hidden, rd[i]);
+            const int row = drow0 + i * rsd.rows_per_it + subd;
+            const bool ok = row < hidden;
+            load_row<DT, 1, true>(de, (uint32_t)(ok ? row : 0) * drow_bytes + zero, pieces, unit0d, rsd.units, ok, rd[i]);
         }
     };
     // (asked for behind the dots of iteration 0 / 1 / 2 / 3, one token on the OLMoE shape: 15.5 / 14.8 / 14.9 / 15.3 us per layer;

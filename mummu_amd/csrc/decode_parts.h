@@ -50,9 +50,17 @@ __device__ __forceinline__ void gate_up_tile(const uint8_t *gate, const uint8_t 
     auto fetch = [&](int i) {
         const int first = row0 + i * rs.rows_per_it;
         const bool ok = first + sub < inter;
-        const RowsAt rows(first, inter, row_bytes, sub_off);
-        load_row<WT, UPL>(ge + rows.base, rows.off, pieces, unit0, rs.units, ok, rg[i]);
-        load_row<WT, UPL>(ue + rows.base, rows.off, pieces, unit0, rs.units, ok, ru[i]);
+        // (one token's launches, which have more than rows to wait for: the offset from the matrix, in the lanes; scalar bases in front of the first
+        // loads cost the step of a layer 1.5 %)
+        if constexpr (!STORE || !std::is_same<First, NoHook>::value) {
+            const uint32_t row_off = (uint32_t)(ok ? first + sub : 0) * row_bytes;
+            load_row<WT, UPL, true>(ge, row_off, pieces, unit0, rs.units, ok, rg[i]);
+            load_row<WT, UPL, true>(ue, row_off, pieces, unit0, rs.units, ok, ru[i]);
+        } else {
+            const RowsAt rows(first, inter, row_bytes, sub_off);
+            load_row<WT, UPL>(ge + rows.base, rows.off, pieces, unit0, rs.units, ok, rg[i]);
+            load_row<WT, UPL>(ue + rows.base, rows.off, pieces, unit0, rs.units, ok, ru[i]);
+        }
     };
     constexpr int AHEAD = NIT < 2 ? NIT : 2;
 #pragma unroll

@@ -170,7 +170,8 @@ struct RowPieces {
 };
 
 // The lane's share of row `row_off` bytes behind `base`, the same pointer in every lane (see uniform_index); row_off below 4 GB.
-template <int WT, int UPL>
+// FEW: for launches that wait for their loads and not for the ALUs (one token): the codes of Q4_K behind the header's address.
+template <int WT, int UPL, bool FEW = false>
 __device__ inline void load_row(const uint8_t *base, uint32_t row_off, const RowPieces<WT, UPL> &pieces, int unit0, int units, bool ok, RawRow<WT, UPL> &r) {
     // Every lane loads unconditionally (a lane of a row past the matrix reads the valid row the
     // caller passes instead): straight-line loads keep the wait counts exact, so rows still in flight
@@ -181,8 +182,9 @@ __device__ inline void load_row(const uint8_t *base, uint32_t row_off, const Row
         const bool on = ok && unit0 + 64 * i < units;
         auto from = [&](int piece) { return base + (row_off + pieces.at[i][piece]); };
         if constexpr (WT == T_Q4_K) {
-            r.hdr[i] = *(const uint4 *)from(0);
-            r.q[i] = *(const uint4 *)from(1);
+            const uint8_t *blk = from(0);
+            r.hdr[i] = *(const uint4 *)blk;
+            r.q[i] = *(const uint4 *)(FEW ? blk + (pieces.at[i][1] - pieces.at[i][0]) : from(1));
             r.hdr[i].x = on ? r.hdr[i].x : 0u;  // d = dmin = 0
         } else if constexpr (WT == T_Q5_K) {
             r.hdr[i] = *(const uint4 *)from(0);
