@@ -481,14 +481,15 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 // Smallest batch of this layer that takes the batched path (INT_MAX: never).
 //
 // gemm_min_*: where the two forms met on the OLMoE shape with the kernels of their time.  Banks that take the f16 units (Q4_K gate and up; Q8_0
-// of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and six or nine
-// tokens: below, they have fewer launches) the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode
-// against batched:
+// of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and more than
+// MUMMU_NOALLOC_MAX_TOKENS tokens: up to those the call that allocates nothing serves every block-quantized bank, with the bits that the others give)
+// the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode against batched:
 //   Q4_K, OLMoE 11 / 13 tokens (311 / 368 MB) 83 / 50, 90 / 57 against 80 / 44, 83 / 47; 128 experts of 2048 x 768, 15 (318 MB): 97 / 61 against 94 / 52; 512
 //   of them top-10, 12 (318 MB): 133 / 104 against 123 / 72.
 //   Q4_K with Q6_K downs, OLMoE, 11 / 12 tokens (359 / 391 MB): 91 / 59, 93 / 63 against 93 / 53, 94 / 53; 128 of 2048 x 768, 15 (390 MB): 108 / 71 against 102 / 62.
 //   Q4_K with other downs, OLMoE Q5_1, 16 (504 MB): 102 / 68 against 92 / 58.
-// Rows of more than 2048 elements are more than a wave's 64 blocks of 32, and the decode kernels take two a lane, some of them none:
+// Rows of more than 2048 elements are more than a wave's 64 blocks of 32, and the decode kernels take two a lane, some of them none, so that they are
+// behind before nine tokens already:
 //   hidden 2560: 512 experts of 640 with Q5_1 downs, 6 tokens 113 / 91 against 99 / 55; 64 of them, 7: 76 / 49 against 70 / 34; 128 of 768, 7: 95 / 69
 //   against 90 / 45; 512 of 640 in Q8_0, 8: 157 / 130 against 159 / 104.  4096: 16 experts of 1792 top-4, 6: 92 / 64 against 80 / 48, Q6_K downs 101 / 73
 //   against 93 / 59, Q8_0 116 / 88 against 117 / 80; 128 of 1536, 6: 163 / 135 against 163 / 106.
@@ -505,7 +506,7 @@ int batched_from(const mummu_moe *h, const Layer &L) {
     const double bytes = 1e6 * (q8 ? 450.0 : wide ? 180.0 : q4k_down ? 310.0 : grouped_gemm_q6k_down(b) ? 390.0 : 480.0);
     auto row_bytes = [](int type, int d) { return (double)(d / block_elems(type)) * block_bytes(type); };
     const double expert = 2.0 * b.inter * row_bytes(b.gate_type, b.hidden) + (double)b.hidden * row_bytes(b.down_type, b.inter);
-    const int from = wide ? 6 : 9, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));
+    const int from = MUMMU_NOALLOC_MAX_TOKENS + 1, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));
     return std::min(line, std::max(from, n));
 }
 

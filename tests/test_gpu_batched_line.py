@@ -1,4 +1,4 @@
-"""Where a batch leaves the decode kernels: by what its slots' experts would read, from six (rows of more than 2048 elements) or nine tokens on.
+"""Where a batch leaves the decode kernels: by what its slots' experts would read, from nine tokens on.
 On both sides of the line the block agrees with what the other form gives, the routing to the bit."""
 import numpy as np
 import pytest
@@ -9,7 +9,7 @@ from mummu_amd import synth
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("H,I,E,k,bank,down,line", [(4096, 1792, 8, 4, "Q4_K", "Q4_K", 6), (2560, 640, 24, 10, "Q4_K", "Q5_1", 6), (2048, 1024, 16, 8, "Q8_0", "Q8_0", 13), (4096, 1792, 8, 4, "Q8_0", "Q8_0", 6),
+@pytest.mark.parametrize("H,I,E,k,bank,down,line", [(4096, 1792, 8, 4, "Q4_K", "Q4_K", 9), (2560, 640, 24, 10, "Q4_K", "Q5_1", 9), (2048, 1024, 16, 8, "Q8_0", "Q8_0", 13), (4096, 1792, 8, 4, "Q8_0", "Q8_0", 9),
                                                     (2048, 1024, 16, 8, "Q4_K", "Q4_K", 11), (2048, 1024, 16, 8, "Q4_K", "Q6_K", 12), (2048, 1024, 16, 8, "Q4_K", "Q5_1", 16), (1024, 512, 8, 4, "Q4_K", "Q4_K", 18)])
 def test_both_sides_of_the_line(monkeypatch, H, I, E, k, bank, down, line):
     rng = np.random.Generator(np.random.PCG64(H + E))

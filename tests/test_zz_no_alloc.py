@@ -43,6 +43,25 @@ def test_noalloc_forward_gives_the_bits_of_forward_device_on_two_calls_in_a_row(
             assert np.array_equal(bits(want), bits(m.forward(x, k, False)))
 
 
+@pytest.mark.parametrize("H,I,E,k,gt,dt", [(4096, 1792, 5, 4, M.Q4_K, M.Q4_K), (2560, 640, 12, 10, M.Q4_K, M.Q5_1), (2560, 768, 12, 8, M.Q4_K, M.Q6_K),
+                                           (4096, 1792, 5, 4, M.Q8_0, M.Q8_0)], ids=["q4k", "q4k-q5_1", "q4k-q6k", "q8_0"])
+def test_noalloc_forward_serves_long_rows_up_to_its_most_tokens(H, I, E, k, gt, dt):
+    # rows of more than 2048 elements leave the decode kernels early in forward_device: never below what this call promises
+    gate, up = (synth.random_bank_fast(gt, [H, I, E], seed) for seed in (931, 932))
+    down = synth.random_bank_fast(dt, [I, H, E], 933)
+    g = np.random.Generator(np.random.PCG64(934))
+    router = (g.standard_normal((E, H), dtype=np.float32) * np.float32(0.02)).astype(np.float16)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, k), max_tokens=8) as m:
+        m.load_layer(0, router, M.F16, gate, gt, up, gt, down, dt)
+        assert m.batched_from(0) > 8
+        for n in (6, 7, 8, 1):
+            x = g.standard_normal((n, H), dtype=np.float32)
+            xd, od = M.DeviceBuffer.from_array(x), M.DeviceBuffer(x.nbytes)
+            m.forward_device_noalloc(0, xd, n, k, False, od)
+            m.check()
+            assert np.array_equal(bits(od.download(np.float32, (n, H))), bits(m.forward(x, k, False))), f"{n} tokens"
+
+
 def test_noalloc_forward_with_the_logit_table_at_every_offset_under_graph_capture_and_on_two_handles():
     # The static array is carved per call: with the two-launch form forced at every size, the router's logit table lands
     # behind buffers whose size follows the token count and top_k, on bytes that earlier calls used for activations.
