@@ -480,21 +480,22 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 // already holds the 16-bit form of x (the fused router produced it).
 // Smallest batch of this layer that takes the batched path (INT_MAX: never).
 //
-// gemm_min_*: where the two forms met on the OLMoE shape with the kernels of their time.  Banks that take the f16 units (Q4_K gate and up; Q8_0
-// of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and more than
+// gemm_min_*: where the two forms met on the OLMoE shape with the kernels of their time.  Banks that take the f16 units throughout (Q4_K gate and up with
+// Q4_K or Q6_K downs; Q8_0 of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and more than
 // MUMMU_NOALLOC_MAX_TOKENS tokens: up to those the call that allocates nothing serves every block-quantized bank, with the bits that the others give)
 // the batched path is ahead, whose launches read an expert once.  us a layer, alone / among others, decode against batched:
 //   Q4_K, OLMoE 11 / 13 tokens (311 / 368 MB) 83 / 50, 90 / 57 against 80 / 44, 83 / 47; 128 experts of 2048 x 768, 15 (318 MB): 97 / 61 against 94 / 52; 512
 //   of them top-10, 12 (318 MB): 133 / 104 against 123 / 72.
 //   Q4_K with Q6_K downs, OLMoE, 11 / 12 tokens (359 / 391 MB): 91 / 59, 93 / 63 against 93 / 53, 94 / 53; 128 of 2048 x 768, 15 (390 MB): 108 / 71 against 102 / 62.
-//   Q4_K with other downs, OLMoE Q5_1, 16 (504 MB): 102 / 68 against 92 / 58.
 // Rows of more than 2048 elements are more than a wave's 64 blocks of 32, and the decode kernels take two a lane, some of them none, so that they are
 // behind before nine tokens already:
-//   hidden 2560: 512 experts of 640 with Q5_1 downs, 6 tokens 113 / 91 against 99 / 55; 64 of them, 7: 76 / 49 against 70 / 34; 128 of 768, 7: 95 / 69
-//   against 90 / 45; 512 of 640 in Q8_0, 8: 157 / 130 against 159 / 104.  4096: 16 experts of 1792 top-4, 6: 92 / 64 against 80 / 48, Q6_K downs 101 / 73
+//   hidden 2560: 128 experts of 768, 7 tokens 95 / 69 against 90 / 45; 512 of 640 in Q8_0, 8: 157 / 130 against 159 / 104.  4096: 16 experts of 1792 top-4, 6: 92 / 64 against 80 / 48, Q6_K downs 101 / 73
 //   against 93 / 59, Q8_0 116 / 88 against 117 / 80; 128 of 1536, 6: 163 / 135 against 163 / 106.
 // (Q8_0 of 2048: since its blocks are read by whole dwords the decode kernels are ahead beyond 13 tokens, OLMoE 15: 109 / 88 against 126 / 86, 17: 117 / 97
 // against 127 / 90; from 13 on the batched form's pairs of halfs stay, 2.5e-7 off the 64-bit result where 16 bits a block are 3.3e-5.)
+// Q4_K gate and up in front of downs of the int8 units stay on the decode kernels to their line, although the batched ones are ahead earlier (Q5_1: OLMoE, 16
+// tokens 102 / 68 against 92 / 58; 512 experts of 2560 x 640, 16: 234 against 106): their hidden rows have a scale per 16 elements in the former and per 64
+// in the latter.  With hidden rows of which 16 in 64 stand out by 2^8 and meet weights of 0 the block is 2.9e-5 off the 64-bit result in the former, 5.2e-3 in the latter.
 int batched_from(const mummu_moe *h, const Layer &L) {
     const ExpertBanks b = banks_of(h, L);
     if (!grouped_gemm_supported(b)) return 0x7fffffff;
@@ -502,8 +503,8 @@ int batched_from(const mummu_moe *h, const Layer &L) {
     const bool q4k = h->gemm_q4k_f16 && grouped_gemm_q4k_f16(b), q4k_down = q4k && grouped_gemm_q4k_f16_down(b), q8 = q8_half_pairs(h, b);
     const int line = q4k_down ? h->gemm_min_q4k : q8 ? h->gemm_min_q8 : grouped_gemm_quantized(b) ? h->gemm_min_quant : h->gemm_min_f16;
     const bool wide = b.hidden > 2048;
-    if (h->gemm_min_given || !(q4k || (q8 && wide))) return line;
-    const double bytes = 1e6 * (q8 ? 450.0 : wide ? 180.0 : q4k_down ? 310.0 : grouped_gemm_q6k_down(b) ? 390.0 : 480.0);
+    if (h->gemm_min_given || !(q4k_down || (q4k && grouped_gemm_q6k_down(b)) || (q8 && wide))) return line;
+    const double bytes = 1e6 * (q8 ? 450.0 : wide ? 180.0 : q4k_down ? 310.0 : 390.0);
     auto row_bytes = [](int type, int d) { return (double)(d / block_elems(type)) * block_bytes(type); };
     const double expert = 2.0 * b.inter * row_bytes(b.gate_type, b.hidden) + (double)b.hidden * row_bytes(b.down_type, b.inter);
     const int from = MUMMU_NOALLOC_MAX_TOKENS + 1, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));
