@@ -122,7 +122,8 @@ MUMMU_API int mummu_moe_load_shared_expert(mummu_moe *h, int layer, int inter, c
 
 /* The smallest token count at which a call on this layer sorts the assignments by expert and runs
  * one grouped GEMM per projection (the reference's per-expert batched form, nn/moe.rs:275-316)
- * instead of the per-token decode kernels; INT32_MAX when the layer's banks never do (or the layer is
+ * instead of the per-token decode kernels, for a call with the configured num_experts_per_tok (the line goes by what the
+ * slots of a call read: with another top_k it may lie elsewhere); INT32_MAX when the layer's banks never do (or the layer is
  * not loaded).  Below it a token's result does not depend on the tokens sharing the call.  The
  * environment variable MUMMU_GEMM_MIN_TOKENS overrides the built-in crossover. */
 MUMMU_API int mummu_moe_batched_from(const mummu_moe *h, int layer);

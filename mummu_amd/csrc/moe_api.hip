@@ -478,7 +478,7 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 
 // experts of an already-made routing: gate/up -> down -> combine.  x_quantized says h->xq
 // already holds the 16-bit form of x (the fused router produced it).
-// Smallest batch of this layer that takes the batched path (INT_MAX: never).
+// Smallest batch of this layer, with k experts to a token, that takes the batched path (INT_MAX: never).
 //
 // gemm_min_*: where the two forms met on the OLMoE shape with the kernels of their time.  Banks that take the f16 units throughout (Q4_K gate and up with
 // Q4_K or Q6_K downs; Q8_0 of rows above 2048) meet by what the decode kernels read, every slot's expert for itself; from `bytes` of that on (and more than
@@ -493,10 +493,11 @@ bool q8_half_pairs(const mummu_moe *h, const ExpertBanks &b) { return q8_gemm_ta
 //   against 93 / 59, Q8_0 116 / 88 against 117 / 80; 128 of 1536, 6: 163 / 135 against 163 / 106.
 // (Q8_0 of 2048: since its blocks are read by whole dwords the decode kernels are ahead beyond 13 tokens, OLMoE 15: 109 / 88 against 126 / 86, 17: 117 / 97
 // against 127 / 90; from 13 on the batched form's pairs of halfs stay, 2.5e-7 off the 64-bit result where 16 bits a block are 3.3e-5.)
+// (The call's own k: OLMoE Q4_K with one expert to a token instead of eight, 11 / 17 tokens of one layer 26 / 32 us on the decode kernels, 38 / 39 batched.)
 // Q4_K gate and up in front of downs of the int8 units stay on the decode kernels to their line, although the batched ones are ahead earlier (Q5_1: OLMoE, 16
 // tokens 102 / 68 against 92 / 58; 512 experts of 2560 x 640, 16: 234 against 106): their hidden rows have a scale per 16 elements in the former and per 64
 // in the latter.  With hidden rows of which 16 in 64 stand out by 2^8 and meet weights of 0 the block is 2.9e-5 off the 64-bit result in the former, 5.2e-3 in the latter.
-int batched_from(const mummu_moe *h, const Layer &L) {
+int batched_from(const mummu_moe *h, const Layer &L, int k) {
     const ExpertBanks b = banks_of(h, L);
     if (!grouped_gemm_supported(b)) return 0x7fffffff;
     if (b.gate_type == T_F32) return h->gemm_min_f32;
@@ -507,7 +508,7 @@ int batched_from(const mummu_moe *h, const Layer &L) {
     const double bytes = 1e6 * (q8 ? 450.0 : wide ? 180.0 : q4k_down ? 310.0 : 390.0);
     auto row_bytes = [](int type, int d) { return (double)(d / block_elems(type)) * block_bytes(type); };
     const double expert = 2.0 * b.inter * row_bytes(b.gate_type, b.hidden) + (double)b.hidden * row_bytes(b.down_type, b.inter);
-    const int from = MUMMU_NOALLOC_MAX_TOKENS + 1, n = (int)__builtin_ceil(bytes / (expert * h->cfg.num_experts_per_tok));
+    const int from = MUMMU_NOALLOC_MAX_TOKENS + 1, n = (int)__builtin_ceil(bytes / (expert * k));
     return std::min(line, std::max(from, n));
 }
 
@@ -556,7 +557,7 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
                 float *out, hipStream_t s, bool count_hits = false, bool xh_done = false) {
     ExpertBanks b = banks_of(h, L);
     const int na = (int)(n * k);
-    if (n >= batched_from(h, L)) {
+    if (n >= batched_from(h, L, k)) {
         // batched: sort the assignments by expert, then one grouped GEMM per projection
         // the 16-bit activation buffers, viewed in the batched path's 64-element-block layout
         const QAct64 xq64{h->xq.hi, h->xq.lo, h->xq.scale, (float *)h->xq.sum};
@@ -679,7 +680,7 @@ int run_one_expert(mummu_moe *h, const Layer &L, int expert, const float *x, int
 bool decode_three_launches(const mummu_moe *h, const Layer &L, int64_t n, int k) {
     const int E = h->cfg.num_experts, H = h->cfg.hidden_size;
     const ExpertBanks b = banks_of(h, L);
-    const bool batched = n >= batched_from(h, L);
+    const bool batched = n >= batched_from(h, L, k);
     const bool want_xq = is_quant_type(L.gate_type) && H % 64 == 0 && !batched;
     return !(n > 8 && router_fused_supported(E)) && want_xq && gate_up_routes_inline(b, k) && down_combine_supported(b, k);
 }
@@ -878,7 +879,7 @@ int routed_impl(mummu_moe *h, int layer, const float *x, int64_t n, int k, int n
         if (rc) return rc;
     }
     // the fused router also quantizes x when the gate/up banks want it (whole 64-element slices)
-    const bool batched = n >= batched_from(h, L);
+    const bool batched = n >= batched_from(h, L, k);
     const bool want_xq = is_quant_type(L.gate_type) && H % 64 == 0 && !batched;
     const QAct xq = want_xq ? h->xq : QAct();
     if (norm_gamma && !decode_three_launches(h, L, n, k)) return fail(h, MUMMU_ERR_ARG, "fused RmsNorm outside the decode form");
@@ -990,7 +991,7 @@ int forward_impl(mummu_moe *h, int layer, const float *x, int64_t n, int k, int 
     } else {
         // the routed decode kernels leave x in the 16-bit decode layout when their own banks are quantized;
         // otherwise (float routed banks, or the batched path's layout) it is made here
-        const bool have_xq = is_quant_type(L.gate_type) && H % 64 == 0 && n < batched_from(h, L);
+        const bool have_xq = is_quant_type(L.gate_type) && H % 64 == 0 && n < batched_from(h, L, k);
         if (is_quant_type(b.gate_type) && !have_xq) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows(x, (int)n, H, h->xq, s));
         LAUNCH(h, K_SHARED, s, launch_gate_up(b, x, h->xq, nullptr, (int)n, 1, 0, h->sh_act, h->sh_actq, h->flags, s));
         LAUNCH(h, K_SHARED, s, launch_down(b, h->sh_act, h->sh_actq, nullptr, (int)n, 1, 0, h->sh_y, s));
@@ -1351,7 +1352,7 @@ int mummu_moe_load_shared_expert(mummu_moe *h, int layer, int inter, const void 
 
 int mummu_moe_batched_from(const mummu_moe *h, int layer) {
     if (!h || layer < 0 || layer >= (int)h->layers.size() || !h->layers[layer].loaded) return 0x7fffffff;
-    return batched_from(h, h->layers[layer]);
+    return batched_from(h, h->layers[layer], h->cfg.num_experts_per_tok);
 }
 
 int mummu_moe_get_config(const mummu_moe *h, mummu_moe_config *out) {
@@ -1517,7 +1518,7 @@ int mummu_moe_routed(mummu_moe *h, int layer, const float *router_logits, const 
     if ((rc = upload_rows(h, io, h->logits, router_logits, lbytes, s))) return rc;
     if ((rc = upload_rows(h, io, h->xin, xs, xbytes, s))) return rc;
     const ExpertBanks b = banks_of(h, L);
-    if (n <= 8 && n < batched_from(h, L) && is_quant_type(L.gate_type) && H % 64 == 0 && gate_up_routes_inline(b, top_k) &&
+    if (n <= 8 && n < batched_from(h, L, top_k) && is_quant_type(L.gate_type) && H % 64 == 0 && gate_up_routes_inline(b, top_k) &&
         down_combine_supported(b, top_k)) {
         // few tokens: the decode pair, gate/up routing by itself from the uploaded logits
         RouteInline route;

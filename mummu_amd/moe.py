@@ -181,7 +181,7 @@ class SparseMoe:
         return int(self._lib.mummu_moe_resident_bytes(self._h))
 
     def batched_from(self, layer: int = 0) -> int:
-        """Smallest token count that takes dispatch + grouped GEMM on this layer (2**31 - 1: never)."""
+        """Smallest token count that takes dispatch + grouped GEMM on this layer with the configured top_k (2**31 - 1: never)."""
         return int(self._lib.mummu_moe_batched_from(self._h, layer))
 
     # -- the block -------------------------------------------------------------------------

@@ -60,3 +60,34 @@ def test_few_rows_in_front_of_int8_downs_keep_a_scale_per_16(H, I, E, k):
     off = np.linalg.norm(got - want) / np.linalg.norm(want)
     print(f"off by {off:.2e}")
     assert off <= 1e-4
+
+
+def _top_k_handle(monkeypatch, k_handle, lines=None):
+    if lines is None:
+        monkeypatch.delenv("MUMMU_GEMM_MIN_TOKENS", raising=False)
+    else:
+        monkeypatch.setenv("MUMMU_GEMM_MIN_TOKENS", str(lines))
+    H, I, E = 2048, 1024, 16
+    m = M.SparseMoe(M.SparseMoeConfig(H, I, E, k_handle), max_tokens=18)
+    rng = np.random.Generator(np.random.PCG64(5))
+    banks = [synth.random_bank_fast(M.Q4_K, dims, seed) for dims, seed in (([H, I, E], 74), ([H, I, E], 75), ([I, H, E], 76))]
+    m.load_layer(0, (rng.standard_normal((E, H)) * 0.02).astype(np.float16), M.F16, banks[0], M.Q4_K, banks[1], M.Q4_K, banks[2], M.Q4_K)
+    return m, rng.standard_normal((18, H), dtype=np.float32)
+
+
+@pytest.mark.parametrize("k_handle,k,line", [(8, 1, 18), (8, 2, 18), (8, 8, 11), (1, 8, 11)])
+def test_the_line_is_that_of_the_calls_top_k(monkeypatch, k_handle, k, line):
+    """What the slots of a call read goes by its own top_k; batched_from() answers for the configured one."""
+    outs = {}
+    for lines in (None, 1, 1 << 20):
+        m, x = _top_k_handle(monkeypatch, k_handle, lines)
+        with m:
+            if lines is None:
+                assert m.batched_from(0) == {8: 11, 1: 18}[k_handle]
+            outs[lines] = {n: np.asarray(m.forward(x[:n], k, True)) for n in (10, 11, 17, 18)}
+            ids, w = m.last_routing(18, k)[:2]
+            outs[lines]["routed"] = {n: np.asarray(m.apply_routing(0, ids[:n], w[:n], x[:n])) for n in (10, 11, 17, 18)}
+    for n in (10, 11, 17, 18):
+        same = outs[1 if n >= line else 1 << 20]
+        assert np.array_equal(outs[None][n].view(np.uint32), same[n].view(np.uint32)), n
+        assert np.array_equal(outs[None]["routed"][n].view(np.uint32), same["routed"][n].view(np.uint32)), n
