@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * kDlWaves) void decode_layer_kernel(const uint8
         auto route_rest = [&]() {
             if (wave == 0) decode_route_finish<RJN, true>(carry.l, k, n_experts, flags, route, rx, sh);
         };
-        gate_up_tile<WT, 1, NIT, true, false, decltype(fetch_down), 1, decltype(route_rest)>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(),
+        gate_up_tile<WT, 1, NIT, true, true, false, decltype(fetch_down), 1, decltype(route_rest)>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(),
                                                                                              s_act, tile, fetch_down, route_rest);
         __syncthreads();
         if (sh.ids[slot] != e) {
@@ -169,11 +169,11 @@ __global__ __launch_bounds__(64 * kDlWaves) void decode_layer_kernel(const uint8
                 return;
             }
             de = down + (size_t)uniform_index(e) * (size_t)hidden * drow_bytes;
-            gate_up_tile<WT, 1, NIT, true, false, decltype(fetch_down), 1>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tile, fetch_down);
+            gate_up_tile<WT, 1, NIT, true, true, false, decltype(fetch_down), 1>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tile, fetch_down);
             __syncthreads();
         }
     } else {
-        gate_up_tile<WT, 1, NIT, true, false, decltype(fetch_down), 1>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tile, fetch_down);
+        gate_up_tile<WT, 1, NIT, true, true, false, decltype(fetch_down), 1>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tile, fetch_down);
         __syncthreads();
     }
     MUMMU_PHASE(4);
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(64 * kDlWaves) void decode_layer_kernel(const uint8
             const int first = tb * blocks_per_tile * 4;  // the tile's pieces: 4 * blocks_per_tile <= 32 of one wave's 64
             const unsigned long long bits = ((1ull << (4 * blocks_per_tile)) - 1ull) << (first & 63);
             if ((s_missing[first >> 6] & bits) == 0ull) continue;  // (uniform over the workgroup)
-            gate_up_tile<WT, 1, NIT, true, false>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tb);
+            gate_up_tile<WT, 1, NIT, true, true, false>(gate, up, e, a, la, rs, hidden, inter, nullptr, QAct(), s_act, tb);
             __syncthreads();
             quantize_tile_to_lds(s_act, rows_per_block, tb, inter, s_ahi, s_alo, s_ascale, s_asum);
             __syncthreads();

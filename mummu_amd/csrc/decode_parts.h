@@ -25,7 +25,9 @@ struct NoHook {
 // results: loads whose address it makes depend on that value cannot be asked for before the rows of that iteration have
 // arrived (the compiler hoists every independent load to the top of the function, whatever fences lie between).
 // `first` runs once the rows of the first iterations have been asked for, in front of every dot.
-template <int WT, int UPL, int NIT, bool ACTQ, bool STORE = true, typename Hook = NoHook, int HOOK_AT = NIT - 1, typename First = NoHook>
+// LANES: rows by an offset from the matrix, in the lanes, instead of one from the iteration's first row (scalar bases in front of the first loads cost one token's
+// step of a layer 1.5 %, where more than rows are waited for).
+template <int WT, int UPL, int NIT, bool ACTQ, bool LANES, bool STORE = true, typename Hook = NoHook, int HOOK_AT = NIT - 1, typename First = NoHook>
 __device__ __forceinline__ void gate_up_tile(const uint8_t *gate, const uint8_t *up /* (restrict or not is the kernel's choice) */, int e, int a,
                                              const LaneAct<UPL> &la, const RowSplit &rs, int hidden, int inter,
                                              float *__restrict__ act, const QAct &actq, float *s_act, int tile,
@@ -50,9 +52,7 @@ __device__ __forceinline__ void gate_up_tile(const uint8_t *gate, const uint8_t 
     auto fetch = [&](int i) {
         const int first = row0 + i * rs.rows_per_it;
         const bool ok = first + sub < inter;
-        // (one token's launches, which have more than rows to wait for: the offset from the matrix, in the lanes; scalar bases in front of the first
-        // loads cost the step of a layer 1.5 %)
-        if constexpr (!STORE || !std::is_same<First, NoHook>::value) {
+        if constexpr (LANES) {
             const uint32_t row_off = (uint32_t)(ok ? first + sub : 0) * row_bytes;
             load_row<WT, UPL, true>(ge, row_off, pieces, unit0, rs.units, ok, rg[i]);
             load_row<WT, UPL, true>(ue, row_off, pieces, unit0, rs.units, ok, ru[i]);

@@ -61,6 +61,16 @@ static hipError_t with_bank_type(int type, F &&f) {
 #undef MUMMU_TYPE_CASE
 }
 
+// Whether a wave's rows lie at an offset from the matrix, in the lanes (load_row's FEW), or behind a scalar base of each iteration (RowsAt).  The latter
+// has fewer vector instructions, but puts scalar work in front of the first loads: it is for the launches that the vector ALUs bound, from three tokens
+// on, which take eight row iterations where they can.  With four (one and two tokens) by type, us of eight layers of two tokens, scalar bases / lanes: Q4_K 128.3 /
+// 121.2, Q4_K with Q6_K downs 146.3 / 139.6, Q5_1 downs (four layers) 61.2 / 59.4; Q6_K downs, four layers of one token 54.5 / 53.4.  Q6_K gate and up and
+// the other types are ahead with scalar bases at two tokens already (Q6_K throughout, four layers 85.4 / 92.4, Q5_K 75.8 / 76.5).
+template <int WT, int UPL, int NIT>
+constexpr bool gate_up_rows_by_lanes() { return WT == T_Q4_K && UPL == 1 && NIT == 4; }
+template <int WT, int UPL, int NIT>
+constexpr bool down_rows_by_lanes() { return WT == T_Q6_K && UPL == 1 && NIT == 4; }
+
 // Several tokens per step (ExpertBanks::tile_order_from and up): tokens that routed to the same expert read the same
 // weight rows, and the eight XCDs each have an L2 of their own, so the second read only hits if both workgroups sit
 // on one XCD at about the same time.  Workgroups go to the XCDs round-robin by linear index; with grid = (kXcds,
@@ -141,7 +151,7 @@ __global__ __launch_bounds__(1024) void gate_up_q_kernel(const uint8_t *__restri
         if (threadIdx.x == 0) atomicAdd(&flags[FLAG_BAD_ID], 1);
         return;
     }
-    gate_up_tile<WT, UPL, NIT, ACTQ>(gate, up, e, a, la, rs, hidden, inter, act, actq, s_act, tile);
+    gate_up_tile<WT, UPL, NIT, ACTQ, gate_up_rows_by_lanes<WT, UPL, NIT>()>(gate, up, e, a, la, rs, hidden, inter, act, actq, s_act, tile);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -187,7 +197,7 @@ __global__ __launch_bounds__(256) void gate_up_fused_kernel(const uint8_t *__res
         auto route_rest = [&]() {
             if (wave == 0) decode_route_finish<RJN, true>(carry.l, k, n_experts, flags, route, rx, sh);
         };
-        gate_up_tile<WT, 1, NIT, true, true, NoHook, NIT - 1, decltype(route_rest)>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act,
+        gate_up_tile<WT, 1, NIT, true, true, true, NoHook, NIT - 1, decltype(route_rest)>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act,
                                                                                     blockIdx.y, NoHook(), route_rest);
         __syncthreads();
         if (sh.ids[blockIdx.x] != e) {  // (the same finding in every workgroup of the slot: its rows again, for the expert the routing names)
@@ -196,10 +206,11 @@ __global__ __launch_bounds__(256) void gate_up_fused_kernel(const uint8_t *__res
                 if (threadIdx.x == 0) atomicAdd(&flags[FLAG_BAD_ID], 1);
                 return;
             }
-            gate_up_tile<WT, 1, NIT, true>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act, blockIdx.y);
+            // (scalar bases: with this second copy by lanes too, four layers of one token in Q5_K 46 -> 54 us)
+            gate_up_tile<WT, 1, NIT, true, false>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act, blockIdx.y);
         }
     } else {
-        gate_up_tile<WT, 1, NIT, true>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act, blockIdx.y);
+        gate_up_tile<WT, 1, NIT, true, false>(gate, up, e, a, la, rs, hidden, inter, nullptr, actq, s_act, blockIdx.y);
     }
 }
 
@@ -438,8 +449,13 @@ __global__ __launch_bounds__(64 * kDcWaves) void down_combine_q_kernel(
         const int i = step / NIT, it = step % NIT;
         const uint8_t *de = down + (size_t)uniform_index(on_p[i] ? e_p[i] : 0) * (size_t)hidden * row_bytes;
         const int first = row0 + it * rs.rows_per_it;
-        const RowsAt rows(first, hidden, (uint32_t)row_bytes, (uint32_t)sub * (uint32_t)row_bytes);
-        load_row<WT, UPL>(de + rows.base, rows.off, pieces, unit0, rs.units, on_p[i] && first + sub < hidden, rd[i][it]);
+        const bool ok = on_p[i] && first + sub < hidden;
+        if constexpr (down_rows_by_lanes<WT, UPL, NIT>()) {
+            load_row<WT, UPL, true>(de, (uint32_t)(ok ? first + sub : 0) * (uint32_t)row_bytes, pieces, unit0, rs.units, ok, rd[i][it]);
+        } else {
+            const RowsAt rows(first, hidden, (uint32_t)row_bytes, (uint32_t)sub * (uint32_t)row_bytes);
+            load_row<WT, UPL>(de + rows.base, rows.off, pieces, unit0, rs.units, ok, rd[i][it]);
+        }
     };
     constexpr int STEPS = KPW * NIT;
     constexpr int AHEAD = STEPS < 2 ? STEPS : 2;
