@@ -147,10 +147,13 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
     }
     // sums of 32 elements as pairs of halfs: gate/up K = 16 (high of sub-blocks 0-3, 4-7, low of both), down K = 8 for either half
     half4v am[GATE_UP ? 1 : 2];
+    constexpr int kOut = R8 && !Q6 ? 2 : 4;   // sums of a lane that are multiplied by the weights' scales
     float sr[GATE_UP ? 1 : 2][4];
     {
-        const float *ss = p.a.ssum + (size_t)source * (size_t)(p.in_dim / 32) + (size_t)sb * 8;
-        const bool low = GATE_UP ? kg >= 2 : kg == 1, none = (R8 && c >= 8) || (!GATE_UP && kg >= 2);
+        // (of eight rows, those that the lane groups' first two sums are of once high and low halfs have met)
+        const int of_row = R8 && !Q6 ? __shfl(source, 4 * ((c >> 2) & 1) + (c >> 3) + 2 * (c & 1), 64) : source;
+        const float *ss = p.a.ssum + (size_t)of_row * (size_t)(p.in_dim / 32) + (size_t)sb * 8;
+        const bool low = GATE_UP ? kg >= 2 : kg == 1, none = !GATE_UP && kg >= 2;
 #pragma unroll
         for (int l = 0; !Q6 && l < (GATE_UP ? 1 : 2); l++) {
             const float4 v = *(const float4 *)(ss + (GATE_UP ? 4 * (kg & 1) : 4 * l));
@@ -164,12 +167,12 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
         if (GATE_UP) {
             if (wave == 0 && lane < kRows) s_scale[lane] = p.a.scale[(size_t)source * (size_t)(p.in_dim / 128)];
         } else {
-            // (element r of an accumulator: row 4 kg + r; of eight rows 4 (kg % 2) + r)
+            // (element r of an accumulator: row 4 kg + r; of eight rows 4 (kg % 2) + r, or with high and low halfs summed 4 (kg % 2) + (kg / 2) + 2 r)
 #pragma unroll
             for (int l = 0; l < 2; l++) {
                 const float s = p.a.scale[(size_t)source * (size_t)(p.in_dim / 128) + (size_t)sb * 2 + l];
 #pragma unroll
-                for (int r = 0; r < 4; r++) sr[l][r] = __shfl(s, 4 * (R8 ? kg & 1 : kg) + r, 64);
+                for (int r = 0; r < kOut; r++) sr[l][r] = __shfl(s, !R8 ? 4 * kg + r : Q6 ? 4 * (kg & 1) + r : 4 * (kg & 1) + (kg >> 1) + 2 * r, 64);
             }
         }
     }
@@ -248,8 +251,12 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
                 if (GATE_UP) h.mn4[0] = kg & 1 ? h.mn4[1] : h.mn4[0];
                 const f32x4 c2 = __builtin_amdgcn_mfma_f32_16x16x16f16(am[GATE_UP ? 0 : l], h.offsets(GATE_UP ? 0 : l), zero, 0, 0, 0);
                 const float fd = head.d(), fm = head.minus_dmin();
+                if constexpr (R8) {
+                    // high + low in front of the scales, as on 16 rows: an infinite one (a damaged block) times either would make a NaN of them
+                    c1[0] = swap32_add(c1[0], c1[1]), c1[1] = swap32_add(c1[2], c1[3]);
+                }
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
+                for (int r = 0; r < kOut; r++) {
                     const float t = fmaf(fm, c2[r], __fmul_rn(fd, c1[r]));
                     v[r] = GATE_UP ? t : l == 0 ? __fmul_rn(t, sr[0][r]) : fmaf(t, sr[GATE_UP ? 0 : 1][r], v[r]);
                 }
@@ -262,8 +269,8 @@ __global__ __launch_bounds__(64 * MAXW, PER_SIMD) void stream_kernel(StreamArgs 
         if constexpr (Q6) v = products_q6(b);
         else v = products_q4(b);
         if constexpr (R8) {
-            // rows 4 (kg % 2) + (kg / 2), + 2: high + low
-            ((float2 *)to)[lane] = make_float2(swap32_add(v[0], v[1]), swap32_add(v[2], v[3]));
+            // rows 4 (kg % 2) + (kg / 2), + 2 (Q6_K: high + low here, behind the scales: an infinite one times sixteen sums of either sign is a NaN anyhow)
+            ((float2 *)to)[lane] = Q6 ? make_float2(swap32_add(v[0], v[1]), swap32_add(v[2], v[3])) : make_float2(v[0], v[1]);
         } else {
             ((f32x4 *)to)[lane] = v;
         }

@@ -35,3 +35,27 @@ def test_tiles_of_8_rows(monkeypatch, H, I, down):
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, downs, orc.Q4_K, orc.Q4_K, getattr(orc, down)), ids, w, x)
     # (as the other forms on these units; in front of an int8 down product 16 bits and a scale per 64, the bar of experts.rs:1264-1271)
     assert orc.rel_err(got, want, mag).max() <= (2e-3 if down == "Q5_1" else 3e-5)
+
+
+@pytest.mark.parametrize("H,I", [(1024, 1024), (2048, 512)])
+@pytest.mark.parametrize("field,at", [("d", 0), ("dmin", 2)])
+def test_an_infinite_scale_is_what_it_is_on_tiles_of_16_rows(monkeypatch, H, I, field, at):
+    """A damaged block of the down bank: both halfs of a row's elements are summed before they meet it."""
+    monkeypatch.setenv("MUMMU_GEMM_MIN_TOKENS", "1")
+    E, n = 2, 13
+    rng = np.random.Generator(np.random.PCG64(H))
+    gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (64, 65))
+    downs = synth.random_bank_fast(M.Q4_K, [I, H, E], 66)
+    blocks = downs.reshape(E, H, I // 256, 144)
+    blocks[:, ::3, I // 512, at:at + 2] = np.full(1, np.inf, np.float16).view(np.uint8)
+    ids = (np.arange(n) % 5 == 0).astype(np.int32)[:, None]
+    x = rng.standard_normal((n, H), dtype=np.float32)
+    outs = []
+    for rows in ("8", "16"):
+        monkeypatch.setenv("MUMMU_GEMM_TILE_ROWS", rows)
+        with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+            m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q4_K, up, M.Q4_K, downs, M.Q4_K)
+            outs.append(np.asarray(m.apply_routing(0, ids, np.ones((n, 1), np.float32), x)))
+    assert np.isinf(outs[1][:, ::3]).any()
+    assert np.array_equal(np.isnan(outs[0]), np.isnan(outs[1])) and np.array_equal(np.sign(outs[0][np.isinf(outs[1])]), np.sign(outs[1][np.isinf(outs[1])]))
+    assert np.isfinite(outs[0][:, 1::3]).all()
