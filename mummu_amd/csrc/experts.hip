@@ -511,6 +511,15 @@ static int pick_rows_per_wave(int out_dim, int n_assign) {
     return rpw < 4 ? 4 : rpw;
 }
 
+// Eight row iterations per wave from some tokens on: the same routing and activation loads serve twice the rows, and the vector
+// ALUs, which bound several tokens' launches, have a tenth less to do.  Q4_K, a layer among others, us, four / eight iterations:
+// OLMoE 3 / 4 / 5 / 7 tokens 17.1 / 17.0, 21.3 / 20.4, 25.3 / 24.4, 31.5 / 30.1, 128 experts of 2048 x 768, 3 / 6 tokens 16.0 / 15.0, 30.6 / 27.2;
+// at 2 tokens one on its own is no faster.  Others from eight on, but for Q8_0, whose rows take more registers: 83 / 209 at 8.
+template <int WT>
+static bool eight_row_iterations(int tokens, int inter) {
+    return WT != T_Q8_0 && tokens >= (WT == T_Q4_K ? 3 : 8) && inter % 32 == 0;
+}
+
 template <int WT>
 static hipError_t launch_gate_up_t(const ExpertBanks &b, const float *x, QAct xq, const int32_t *ids, int n_assign,
                                    int k, int fixed_expert, float *act, QAct actq, int32_t *flags, hipStream_t s) {
@@ -539,9 +548,9 @@ static hipError_t launch_gate_up_t(const ExpertBanks &b, const float *x, QAct xq
             launch_kernel(gate_up_q_kernel<WT, UPL, NIT, false>, grid, block, lds, s,                                      \
                 b.gate, b.up, xq, ids, k, fixed_expert, b.hidden, b.inter, b.n_experts, act, actq, flags, RouteInline());      \
     } while (0)
-        bool eight = false;   // (row iterations: as launch_gate_up_routed)
+        bool eight = false;
         if constexpr (WT != T_Q8_0) {
-            eight = upl == 1 && n_assign / slots >= 8 && fixed_expert < 0 && b.inter % 32 == 0;
+            eight = upl == 1 && fixed_expert < 0 && eight_row_iterations<WT>(n_assign / slots, b.inter);
             if (eight) MUMMU_GUQ(1, 8);
         }
         if (eight) {}
@@ -747,12 +756,8 @@ hipError_t launch_gate_up_routed(const ExpertBanks &b, QAct xq, const RouteInlin
     return with_bank_type(b.gate_type, [&](auto tag) {
         constexpr int WT = decltype(tag)::value;
         if constexpr (is_quant_type(WT)) {
-            // (eight row iterations per wave from some tokens on: the same routing and activation loads serve twice the rows, and the vector
-            // ALUs, which bound several tokens' launches, have a tenth less to do.  Q4_K, a layer among others, us, four / eight iterations:
-            // OLMoE 3 / 4 / 5 / 7 tokens 17.1 / 17.0, 21.3 / 20.4, 25.3 / 24.4, 31.5 / 30.1, 128 experts of 2048 x 768, 3 / 6 tokens 16.0 / 15.0, 30.6 / 27.2;
-            // at 2 tokens one on its own is no faster.  Others from eight on, but for Q8_0, whose rows take more registers: 83 / 209 at 8.)
             if constexpr (WT != T_Q8_0)
-                if (!wide && n_tokens >= (WT == T_Q4_K ? 3 : 8) && b.inter % 32 == 0) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
+                if (!wide && eight_row_iterations<WT>(n_tokens, b.inter)) return launch_gate_up_routed_t<WT, 1, 8>(b, xq, route, n_tokens, k, actq, flags, s);
             return wide ? launch_gate_up_routed_t<WT, 2, 2>(b, xq, route, n_tokens, k, actq, flags, s)
                         : launch_gate_up_routed_t<WT, 1, 4>(b, xq, route, n_tokens, k, actq, flags, s);
         } else {
