@@ -572,7 +572,7 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         // (gate/up alone on the f16 units: the int8 down product takes a tile of 16 rows like one of 32)
         if (hf && !hf_down) tile_rows = grouped_gemm_tile_rows_q4k_f16(b, na, true);
         if (hp.q6) tile_rows = grouped_gemm_tile_rows_q6k_down(b, na);
-        if ((hf_down || hp.q6) && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
+        if (hf && h->gemm_tile_rows != 0) tile_rows = h->gemm_tile_rows;
         if (hp.q8) tile_rows = 32;
         const bool wide = wide_gemm_takes(b, (int)n, na);
         if (wide) tile_rows = kWideRows;
