@@ -977,9 +977,10 @@ static double expected_tiles(double avg, double rows) {
 }
 
 // Tiles of 8 instead of 16 rows (gemm_stream.hip) while next to no expert needs a second one: its first second tiles must not start a second
-// round of workgroups, and beyond they read the weights again.  us a layer among others, tiles of 16 / 8: OLMoE 20 / 32 / 40 tokens 55.8 / 52.1,
-// 58.4 / 55.3, 60.0 / 60.0 (alone 95 / 105), 128 experts of 2048 x 768, 27 / 64 / 100 tokens 72.4 / 67.6, 88.5 / 86.3, 93.3 / 95.4, the 512-expert shape
-// with int8 downs, 64 / 200 / 300 tokens 272 / 262, 385 / 373, 407 / 423, 16 experts of 4096 x 1792, 18 tokens 55 / 61.
+// round of workgroups, and beyond they read the weights again.  us a layer among others, tiles of 16 / 8 (alone): OLMoE 20 / 32 / 40 tokens 56.6 / 54.4,
+// 58.7 / 56.0, 60.0 / 63.9 (90 / 100), 128 experts of 2048 x 768, 27 / 64 / 100 tokens 73.3 / 69.1, 89.6 / 89.7 (127 / 132), 95.5 / 96.3, the 512-expert shape
+// with int8 downs, 64 / 200 / 300 tokens 286 / 263, 395 / 367, 414 / 418.  (16 experts of 4096 x 1792, 18 tokens: 16 rows by the second round, 62 / 58 (99 / 90)
+// with the present kernels, 55 / 61 with those that the rule was made by.)
 static int tiles_of_8_or_16(const ExpertBanks &b, int n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const double e8 = expected_tiles(avg, 8.0), e16 = expected_tiles(avg, 16.0), each = (double)b.n_experts * (double)((b.inter + 127) / 128);

@@ -5,16 +5,16 @@
 // halfs in the operand's first eight rows and the low ones in the others: one product where 16 rows take two.
 //
 // What bounds it: the vector ALUs and the stream, neither wholly beside the other.  Every line of the weights is fetched once (128 experts of 2048 x 768, 27
-// tokens: 177 MB where the 144-byte pieces of gemm_q4k_few.hip fetch 1.38 times that), 16 columns of a super-block take 109 vector
-// instructions (two for a pair of codes) and nine products, and a CU's 16 to 20 waves keep 75 to 110 KB on the way.  Gate/up of that shape
-// 51 -> 48 us, of 512 experts of 2560 x 640 with 64 tokens 176 -> 167, with the loads alone 43 and 133, with the weights out of L2 45 and 139;
-// OLMoE, 20 tokens, 38.7 -> 37.2 + 23.5 -> 20.9.  Layers among others: 72.4 -> 67.6, 272 -> 262, 57.0 -> 52.1; 512 experts of 2048 x 768, 60
-// tokens 237 -> 206, 128 of 3072 x 768, 30 tokens 117 -> 103.
+// tokens: 177 MB where the 144-byte pieces of gemm_q4k_few.hip fetch 1.38 times that), 16 columns of a super-block take 108 vector
+// instructions (two for a pair of codes; down 122) and nine products, and a CU's 16 to 20 waves keep 75 to 110 KB on the way.  Gate/up of that shape, here and
+// in gemm_q4k_few.hip, 48 and 51 us, of 512 experts of 2560 x 640 with 64 tokens 152 and 176, with the loads alone 43 and 133, with the weights out of L2
+// 45 and 139; OLMoE, 20 tokens, 37.2 + 20.9 and 38.7 + 23.5.  Layers among others, tiles of 8 rows here and of 16: 128 experts 27 tokens 69 and 73, 512 experts
+// 64 tokens 263 and 286, OLMoE 54 and 57; 512 experts of 2048 x 768, 60 tokens 209 and 230, 128 of 3072 x 768, 30 tokens 110 and 123.
 //
 // Q6_K downs (tiles of 8 rows): a sub-block's 16 elements are an operand's K of 16 (v_mfma_f32_16x16x16_f16), four to a lane, so that its sum can
 // be folded with d * sc; a lane loads 16 neighbouring bytes, in whole dwords, and changes dwords with the three others of its row.  Some 280 vector
 // instructions a unit.  OLMoE, 24 tokens 42 -> 32 us (106 MB fetched, the weights' bytes; 35 with loads at odd halves of a dword), layers at 16 / 24 /
-// 32 tokens 73 / 74 / 76 -> 61 / 64 / 65, 128 experts of 2048 x 768, 30 tokens 99 -> 81 (92).
+// 32 tokens 76 / 77 / 78 (tiles of 16 rows, q6k_down_kernel) and 62 / 64 / 65, 128 experts of 2048 x 768, 30 tokens 100 and 83.
 #include "device_utils.h"
 #include "kernels.h"
 #include "q4k_half.h"
@@ -364,9 +364,11 @@ hipError_t launch_stream(const Q4kArgs &q, int max_tiles, hipStream_t s) {
 
 }  // namespace
 
-// Tiles of 16 rows keep 64 registers of rows, four waves a SIMD: taken where workgroups of one wave to a super-block fill those.
-// us a layer among others, here / gemm_q4k_few.hip: OLMoE 24 / 64 tokens 57.7 / 58.8, 61.8 / 64.2, 512 experts of 2048 x 768, 40 / 128 tokens 177 / 189,
-// 302 / 316; hidden 2560 365 / 349, 4096 283 / 280, 1536 46.5 / 43.8, three super-blocks alike.
+// Tiles of 16 rows keep 64 registers of rows, four waves a SIMD.  us a layer among others, here / gemm_q4k_few.hip: OLMoE (eight and four super-blocks) 24 / 64
+// tokens 57.7 / 58.8, 61.8 / 64.2, 512 experts of 2048 x 768, 40 / 128 tokens 177 / 189, 302 / 316.  Ten super-blocks (hidden 2560) 365 / 349, sixteen (4096) 283 /
+// 280, with downs of 1024 elements, 24 / 60 tokens 64.1 / 63.9, 70.8 / 68.9, six 46.5 / 43.8, three alike.  One and two, whose workgroups have several rows of waves:
+// behind for gate/up (hidden 512, inter 512, 32 / 100 tokens 21.6 / 18.4, 25.0 / 21.7; hidden 256, 100 tokens 34.5 / 31.6), ahead for downs behind long rows (512 experts of
+// 2048 x 512, 64 tokens 155 / 166, of 2048 x 256 91 / 94), which the rule, the same for both products, leaves to gemm_q4k_few.hip.
 bool gemm_stream_takes(int in_dim, int out_dim, int tile_rows) {
     const int n_sb = in_dim / 256;
     if (in_dim % 256 != 0 || out_dim % 128 != 0) return false;
