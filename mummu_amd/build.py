@@ -19,7 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(HERE, "lib", "libmummu_moe.so")
 
-SOURCES = ["dequant.hip", "router.hip", "experts.hip", "decode_layer.hip", "dispatch.hip", "gemm.hip", "gemm_wide.hip", "gemm_q4k.hip", "gemm_q4k_few.hip", "gemm_q4k_one.hip", "gemm_stream.hip", "gemm_q8.hip", "gemm_q6k.hip", "moe_api.hip", "host_staging.hip", "packed_gemv.hip", "gguf_reader.cpp", "safetensors_loader.cpp"]
+SOURCES = ["dequant.hip", "router.hip", "router_matrix.hip", "experts.hip", "decode_layer.hip", "dispatch.hip", "gemm.hip", "gemm_wide.hip", "gemm_q4k.hip", "gemm_q4k_few.hip", "gemm_q4k_one.hip", "gemm_stream.hip", "gemm_q8.hip", "gemm_q6k.hip", "moe_api.hip", "host_staging.hip", "packed_gemv.hip", "gguf_reader.cpp", "safetensors_loader.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]

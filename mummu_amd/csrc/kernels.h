@@ -27,6 +27,10 @@ bool router_logits_can_norm(const float *x, const void *w, const float *gamma, i
 hipError_t launch_router_logits(const float *x, const void *w, int wtype, float *logits, int n, int hidden,
                                 int n_experts, QAct xq, hipStream_t s, const float *norm_gamma = nullptr,
                                 float norm_eps = 0.0f, float *xnorm_out = nullptr);
+// router_matrix.hip: the same logits on the f32 matrix units, bit for bit; with `route` (up to 64 experts) the routing in the same launch.
+bool router_matrix_takes(const float *x, const void *w, int hidden);
+hipError_t launch_router_matrix(const float *x, const void *w, int wtype, int n, int hidden, int n_experts, int k, int flavour, int norm, float *logits,
+                                int32_t *ids, float *weights, unsigned long long *hits, int32_t *flags, bool route, hipStream_t s);
 // softmax -> top-k -> (re)normalise per token; one wave per token.
 //   ids/weights [n, k] in slot order; hits (nullable) [E] += rows routed; flags see above.
 hipError_t launch_route_topk(const float *logits, int n, int n_experts, int k, int flavour, int norm,

@@ -272,6 +272,11 @@ hipError_t launch_router_logits(const float *x, const void *w, int wtype, float 
     if (norm_gamma && !router_logits_can_norm(x, w, norm_gamma, n, hidden)) return hipErrorInvalidValue;
     if (xnorm_out && (!norm_gamma || ((uintptr_t)xnorm_out & 15))) return hipErrorInvalidValue;
     const bool vec = (hidden % 8 == 0) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)w & 15) == 0);
+    // The matrix units from 128 workgroups of 16 tokens by 64 experts on, whose one round takes 19 us whatever their number (2048 elements, more in
+    // proportion), and half of that again what the tiles below take for as many: us of those / of the matrix units, 128 experts of 2048, 600 tokens 14 / 19
+    // (76 workgroups), 2000: 40 / 21, 4096: 78 / 41; 512 experts of 2560, 150 tokens 16 / 23 (80), 300: 29 / 24 (152), 1024: 75 / 45.
+    if (n > 8 && xq.hi == nullptr && !norm_gamma && router_matrix_takes(x, w, hidden) && (long long)((n + 15) / 16) * ((n_experts + 63) / 64) > 128)
+        return launch_router_matrix(x, w, wtype, n, hidden, n_experts, 1, 0, 0, logits, nullptr, nullptr, nullptr, nullptr, false, s);
     if (n > 8 && vec && xq.hi == nullptr && !norm_gamma && hidden % 512 == 0 && hidden <= kTileMaxHidden) {
         // (Also a dozen workgroups are no slower than a launch of router_logits_kernel: us of that / of the tiles, 2048 elements, 8 experts, 9 / 32 / 300
         // tokens 5.0 / 5.0, 6.1 / 5.0, 5.5 / 5.3, 64 experts 6.1 / 5.4, 6.4 / 5.5, 9.4 / 7.8, 128 6.0 / 5.6, 6.4 / 5.4, 15.3 / 10.8, 512 6.6 / 5.6, 8.0 / 6.5, 47.8 /
@@ -647,6 +652,11 @@ hipError_t launch_router_fused(const float *x, const void *w, int wtype, int n, 
     if (n_experts > 128 || k > n_experts || k < 1) return hipErrorInvalidValue;
     if (xq.hi != nullptr && hidden % 64 != 0) return hipErrorInvalidValue;
     const bool vec = (hidden % 8 == 0) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)w & 15) == 0);
+    // The matrix units (router_matrix.hip), 16 tokens to a workgroup, where those come near filling the chip: 64 experts of 2048, 1000 / 1500 / 2100 / 4096
+    // tokens 17 / 25 / 42 / 48 us in the streaming form, 22 / 23 / 24 / 25 there, but layers among others at 1700 459 / 461, at 2100 367 / 345.  (A tile's 64
+    // columns want more than 32 experts.)
+    if (xh.hi == nullptr && xq.hi == nullptr && n > 2048 && n_experts > 32 && n_experts <= 64 && router_matrix_takes(x, w, hidden))
+        return launch_router_matrix(x, w, wtype, n, hidden, n_experts, k, flavour, norm, logits, ids, weights, hits, flags, true, s);
     // enough tokens to fill the chip with independent waves: activations in registers, weight
     // rows streamed (on this path the caller quantizes x separately)
     if (n > 8 && vec && (xq.hi == nullptr || xq_beside) && hidden % 512 == 0 && hidden <= 512 * kRouterMaxChunks) {

@@ -1,5 +1,5 @@
-"""Router logits of many tokens, four by four experts to a wave: bit for bit the oracle's fixed summation order, at token and expert counts
-that end inside a tile, on one to four passes over the experts, for every router type."""
+"""Router logits of many tokens, four by four experts to a wave or sixteen by sixteen on the matrix units: bit for bit the oracle's fixed
+summation order, at token and expert counts that end inside a tile, on one to four passes over the experts, for every router type."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,9 @@ from oracle import binding as orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("H,E,n", [(512, 3, 9), (512, 130, 12), (2560, 512, 67), (1024, 129, 33), (512, 512, 600), (512, 501, 1101), (8192, 17, 10)])
+@pytest.mark.parametrize("H,E,n", [(512, 3, 9), (512, 130, 12), (2560, 512, 67), (1024, 129, 33), (512, 512, 600), (512, 501, 1101), (8192, 17, 10), (4608, 512, 600),
+                                   # (the matrix units: more than 128 workgroups of 16 by 64; one, two, five and eight chunks of 512, the last workgroup one token)
+                                   (1024, 130, 689), (2560, 512, 257), (4096, 65, 1041)])
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
     rng = np.random.Generator(np.random.PCG64(H + E + n))
@@ -23,6 +25,7 @@ def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
     else:
         t, ot = M.F32, orc.F32
     x = rng.standard_normal((n, H), dtype=np.float32)
+    x[1, ::3] *= 1e-30   # (subnormal products and sums)
     bank = synth.random_bank_fast(M.Q8_0, [H, 32, E], 1)
     with M.SparseMoe(M.SparseMoeConfig(H, 32, E, 2), max_tokens=n) as m:
         m.load_layer(0, w, t, bank, M.Q8_0, bank, M.Q8_0, synth.random_bank_fast(M.Q8_0, [32, H, E], 2), M.Q8_0)
@@ -33,7 +36,8 @@ def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
 
 # Batches of up to 128 experts on either side of the line from which they take these tiles and a launch for the routing: the oracle's routing
 # bit for bit, every row served counted once.
-@pytest.mark.parametrize("E,n", [(128, 256), (128, 257), (65, 300), (64, 300), (128, 2100)])
+@pytest.mark.parametrize("E,n", [(128, 256), (128, 257), (65, 300), (64, 300), (128, 2100),
+                                 (64, 2048), (64, 2049), (33, 2065), (32, 2100), (50, 4096)])   # (on the matrix units with the routing behind)
 def test_routing_and_hits_of_a_batch(E, n):
     H, I, k = 512, 64, 2
     rng = np.random.Generator(np.random.PCG64(E + n))
@@ -50,3 +54,20 @@ def test_routing_and_hits_of_a_batch(E, n):
     assert np.array_equal(ids, oids.astype(np.int32).reshape(n, k))
     assert np.array_equal(w.view(np.uint32), ow.reshape(n, k).view(np.uint32))
     assert np.array_equal(hits, np.bincount(ids.ravel(), minlength=E))
+
+
+# A token whose row holds an infinity or a NaN is refused, on either side of the line to the matrix units.
+@pytest.mark.parametrize("E,n", [(64, 40), (64, 2049), (130, 40), (130, 700)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_rows_that_are_not_finite_are_refused(E, n, value):
+    H = 1024
+    rng = np.random.Generator(np.random.PCG64(E + n))
+    router = (rng.standard_normal((E, H), dtype=np.float32) * np.float32(0.05)).astype(np.float16)
+    x = rng.standard_normal((n, H), dtype=np.float32)
+    x[n - 1, H - 1] = value
+    bank = synth.random_bank_fast(M.Q8_0, [H, 32, E], 1)
+    with M.SparseMoe(M.SparseMoeConfig(H, 32, E, 2), max_tokens=n) as m:
+        m.load_layer(0, router, M.F16, bank, M.Q8_0, bank, M.Q8_0, synth.random_bank_fast(M.Q8_0, [32, H, E], 2), M.Q8_0)
+        for call in (m.route, m.forward):
+            with pytest.raises(M.MoeError, match=f"token {n - 1} "):
+                call(x, 2, True)
