@@ -25,7 +25,7 @@
 //   offsets[E+1]      expert e owns sorted positions [offsets[e], offsets[e+1])
 //   sorted[A]         sorted position -> assignment index a
 //   inv[A]            assignment index a -> sorted position
-//   tiles, n_tiles    the work list and its length
+//   tiles, n_tiles    the work list, its length and the zeroed counters behind that
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -144,7 +144,10 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scan_place_kernel(
             if (e == n_experts - 1) offsets[n_experts] = begin + total;
             if (tiles != nullptr) {
                 write_tiles(tiles, base_t + incl_t - my_tiles, my_tiles, e, begin, total, unit);
-                if (e == n_experts - 1) *n_tiles = base_t + incl_t;
+                if (e == n_experts - 1) {
+                    *n_tiles = base_t + incl_t;
+                    for (int i = 1; i < WORK_INTS; i++) n_tiles[i] = 0;
+                }
             }
         }
     }
@@ -243,7 +246,10 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
         if (e == n_experts - 1) offsets[n_experts] = begin + total;
         if (tiles != nullptr) {
             write_tiles(tiles, base_t + incl_t - my_tiles, my_tiles, e, begin, total, unit);
-            if (e == n_experts - 1) *n_tiles = base_t + incl_t;
+            if (e == n_experts - 1) {
+                *n_tiles = base_t + incl_t;
+                for (int i = 1; i < WORK_INTS; i++) n_tiles[i] = 0;
+            }
         }
     }
     __syncthreads();

@@ -176,6 +176,9 @@ hipError_t launch_gate_energy(const float *w, const float *x, int rows, int hidd
 // triples.  scratch: dispatch_scratch_ints(A, E) ints.  hits (optional): per-expert row counters to
 // add this batch to.
 size_t dispatch_scratch_ints(int n_assign, int n_experts);
+// n_tiles: WORK_INTS ints, the number of tiles and the counters of the kernels whose workgroups take items as they come to them (one to
+// an XCD and product), zero.
+enum { WORK_GATE_UP = 1, WORK_DOWN = WORK_GATE_UP + 8, WORK_INTS = WORK_DOWN + 8 };
 // unit: an expert's tiles, as few as tile_rows allows, share its rows evenly in multiples of this many (tile_rows: all
 // but the last are full).
 hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *offsets,
@@ -229,8 +232,8 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
 constexpr int kWideRows = 320, kWideUnit = 64;
 bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign);   // can and should
 hipError_t launch_wide_gate_up(const ExpertBanks &b, const _Float16 *x16, const int32_t *sorted, int k_slots, const int32_t *tiles,
-                               const int32_t *n_tiles, int max_tiles, _Float16 *act16, hipStream_t s);
-hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, const int32_t *n_tiles, int max_tiles,
+                               int32_t *n_tiles, int max_tiles, _Float16 *act16, hipStream_t s);
+hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, int32_t *n_tiles, int max_tiles,
                             float *y, hipStream_t s);
 
 // gemm_q4k.hip ------------------------------------------------------------------------

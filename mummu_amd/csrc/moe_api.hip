@@ -305,7 +305,7 @@ int ensure_ws(mummu_moe *h, int64_t n, int64_t n_assign, int n_experts) {
     HIPCHK(h, hipMalloc(&h->sorted, sizeof(int32_t) * (size_t)na));
     HIPCHK(h, hipMalloc(&h->inv, sizeof(int32_t) * (size_t)na));
     HIPCHK(h, hipMalloc(&h->tiles, sizeof(int32_t) * 3 * (size_t)h->max_tiles));
-    HIPCHK(h, hipMalloc(&h->n_tiles, sizeof(int32_t)));
+    HIPCHK(h, hipMalloc(&h->n_tiles, sizeof(int32_t) * WORK_INTS));
     HIPCHK(h, hipMalloc(&h->disp_scratch, sizeof(int32_t) * dispatch_scratch_ints((int)na, n_experts)));
     HIPCHK(h, hipMalloc(&h->act16, 2 * (size_t)na * I));
     {

@@ -78,3 +78,26 @@ def test_infinite_gates_come_out_as_in_the_narrow_kernel():
         assert np.isnan(got[5]).all()
         assert np.array_equal(got[6], np.full(H, np.inf, np.float32))
         assert np.isfinite(np.delete(got, (5, 6), 0)).all()
+
+
+@pytest.mark.parametrize("H, I", [(256, 128), (320, 192)], ids=["4 and 2 steps of K", "5 and 3"])
+def test_several_items_to_a_workgroup_of_few_steps(H, I):
+    """More items than CUs, each height of a tile behind each other, with as few steps of K as the kernel takes and one more: what an
+    item's first stages and the stores before them find in LDS and in the counters.  Bounds as above."""
+    E = 480
+    counts = np.random.default_rng(11).permutation(np.resize([1, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321, 0, 0, 0, 3, 2], E))
+    ids = np.random.default_rng(5).permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    n = len(ids)
+    assert n >= 72 * E
+    g = torch.Generator().manual_seed(9)
+    bank = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(torch.float16).view(torch.int16).numpy().view(np.uint16)
+    gate, up, down = bank(E, I, H), bank(E, I, H), bank(E, H, I)
+    x, w = torch.randn(n, H, generator=g).numpy(), torch.rand(n, 1, generator=g).numpy()
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, bank(E, H), M.F16, gate, M.F16, up, M.F16, down, M.F16)
+        got = m.apply_routing(0, ids, w, x)
+        for _ in range(5):
+            assert np.array_equal(got.view(np.uint32), m.apply_routing(0, ids, w, x).view(np.uint32))
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.F16), ids, w, x)
+    assert orc.rel_err(got, want, mag).max() <= 4e-3
+    assert (np.linalg.norm(got - want, axis=1) <= 2e-3 * np.linalg.norm(want, axis=1)).all()
