@@ -119,6 +119,14 @@ __host__ __device__ constexpr int block_bytes(int t) {
 // The block-quantized types (everything but the plain float types).
 __host__ __device__ constexpr bool is_quant_type(int t) { return block_elems(t) > 1; }
 
+// Two halfs in a word, the first below.
+__device__ inline uint32_t pack_half2(float a, float b) {
+    _Float16 h[2] = {(_Float16)a, (_Float16)b};
+    uint32_t u;
+    __builtin_memcpy(&u, h, 4);
+    return u;
+}
+
 // IEEE half bits -> f32, exact (subnormals included: gfx9 keeps f16 denormals).
 __device__ inline float half_bits_to_float(uint16_t bits) {
     _Float16 h;

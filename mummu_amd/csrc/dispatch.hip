@@ -28,12 +28,51 @@
 //   tiles, n_tiles    the work list, its length and the zeroed counters behind that
 #include "device_utils.h"
 #include "kernels.h"
+#include "qact.h"
 
 namespace mummu {
 
 constexpr int kDispatchThreads = 1024;
 constexpr int kDispatchWaves = kDispatchThreads / 64;
 constexpr int kDispatchMaxExperts = 512;
+
+// Workgroup b of n_b of a launch makes its share of the rows that the products read.  Nothing of the sort waits for it, and the launch of its own that
+// it had took as long as the sort's first one (layers among others, us: 512 f16 tokens 178 -> 171, 300 of 512 experts with int8 downs 415 -> 402, 320 of
+// Q8_0 189 -> 184, 300 of Q4_K 127 -> 125, 1000: 268 / 269).
+__device__ inline void rows_part(const RowsJob &job, int b, int n_b) {
+    __shared__ float s_max[kDispatchWaves];
+    const int tid = threadIdx.x;
+    if (job.h.hi != nullptr && job.h.lo == nullptr) {
+        const size_t n4 = (size_t)job.n * (size_t)job.d / 4;
+        for (size_t i = (size_t)b * kDispatchThreads + tid; i < n4; i += (size_t)n_b * kDispatchThreads) {
+            const float4 v = ((const float4 *)job.x)[i];
+            ((uint2 *)job.h.hi)[i] = make_uint2(pack_half2(v.x, v.y), pack_half2(v.z, v.w));
+        }
+        return;
+    }
+    // a row to four waves
+    constexpr int NT = 256, kAtOnce = kDispatchThreads / NT;
+    const int part = tid / NT, t = tid % NT;
+    for (int row0 = b * kAtOnce; row0 < job.n; row0 += n_b * kAtOnce) {
+        const int row = row0 + part;
+        if (job.h.lo != nullptr) {
+            hact_quantize_row<NT>(job.x, job.d, job.h, row, s_max + part * (NT / 64), t, row < job.n);
+            __syncthreads();   // (s_max is free again)
+        } else {
+            for (int e0 = t * 4; e0 - t * 4 < job.d; e0 += NT * 4) {   // (whole groups of 16 lanes run together)
+                const bool active = e0 < job.d && row < job.n;
+                const float4 v = active ? *(const float4 *)(job.x + (size_t)row * (size_t)job.d + e0) : make_float4(0.f, 0.f, 0.f, 0.f);
+                quantize_store64(v, active, job.q, (size_t)row, job.d, e0);
+            }
+        }
+    }
+}
+unsigned rows_workgroups(const RowsJob &job) {
+    if (job.x == nullptr) return 0;
+    const size_t all = job.h.hi != nullptr && job.h.lo == nullptr ? ((size_t)job.n * (size_t)job.d / 4 + kDispatchThreads - 1) / kDispatchThreads
+                                                                  : ((size_t)job.n + 3) / 4;
+    return (unsigned)(all < 2048 ? all : 2048);
+}
 
 // Expert e's n tiles over its `rows` sorted rows from `begin`: whole units of rows dealt evenly, the first tiles one more.
 __device__ inline void write_tiles(int32_t *__restrict__ tiles, int at, int n, int e, int begin, int rows, int unit) {
@@ -66,8 +105,12 @@ __device__ inline int rank_in_wave(int e, int n_experts, int lane, int *counts) 
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_count_kernel(const int32_t *__restrict__ ids, int n_assign,
                                                                           int n_experts, int32_t *__restrict__ rank_out,
                                                                           int32_t *__restrict__ counts,
-                                                                          int32_t *__restrict__ flags) {
+                                                                          int32_t *__restrict__ flags, int n_chunks, RowsJob job) {
     __shared__ __attribute__((aligned(16))) int s_wave[kDispatchWaves][kDispatchMaxExperts];  // per-wave counts of this chunk
+    if ((int)blockIdx.x >= n_chunks) {
+        rows_part(job, (int)blockIdx.x - n_chunks, (int)gridDim.x - n_chunks);
+        return;
+    }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int chunk = blockIdx.x;
     for (int i = tid; i < kDispatchWaves * kDispatchMaxExperts / 4; i += kDispatchThreads) ((int4 *)s_wave)[i] = make_int4(0, 0, 0, 0);
@@ -171,7 +214,11 @@ constexpr int kFusedChunks = 3;
 __global__ __launch_bounds__(kDispatchThreads) void dispatch_fused_kernel(
     const int32_t *__restrict__ ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *__restrict__ offsets,
     int32_t *__restrict__ sorted, int32_t *__restrict__ inv, int32_t *__restrict__ tiles, int32_t *__restrict__ n_tiles,
-    unsigned long long *__restrict__ hits, int32_t *__restrict__ flags) {
+    unsigned long long *__restrict__ hits, int32_t *__restrict__ flags, RowsJob job) {
+    if (blockIdx.x > 0) {
+        rows_part(job, (int)blockIdx.x - 1, (int)gridDim.x - 1);
+        return;
+    }
     __shared__ __attribute__((aligned(16))) int s_wave[kDispatchWaves][kDispatchMaxExperts];   // per-wave counts of the current chunk
     __shared__ int s_chunk[kFusedChunks][kDispatchMaxExperts];    // per-chunk counts, then exclusive running counts
     __shared__ int s_off[kDispatchMaxExperts];
@@ -291,21 +338,23 @@ size_t dispatch_scratch_ints(int n_assign, int n_experts) {
 
 hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *offsets,
                            int32_t *sorted, int32_t *inv, int32_t *tiles, int32_t *n_tiles, int32_t *scratch,
-                           unsigned long long *hits, int32_t *flags, hipStream_t s) {
+                           unsigned long long *hits, int32_t *flags, const RowsJob &rows, hipStream_t s) {
     if (n_assign <= 0) return hipSuccess;
+    if (rows.x != nullptr && rows.d % (rows.h.lo != nullptr ? 128 : (rows.h.hi != nullptr ? 4 : 64)) != 0) return hipErrorInvalidValue;
+    const unsigned beside = rows_workgroups(rows);
     if (n_experts > kDispatchMaxExperts || tile_rows < 1 || unit < 1 || tile_rows % unit != 0) return hipErrorInvalidValue;
     const int chunks = (n_assign + kDispatchThreads - 1) / kDispatchThreads;
     if (chunks <= kFusedChunks) {
-        launch_kernel(dispatch_fused_kernel, dim3(1), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, tile_rows, unit, offsets,
-                      sorted, inv, tiles, n_tiles, hits, flags);
+        launch_kernel(dispatch_fused_kernel, dim3(1 + beside), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, tile_rows, unit, offsets,
+                      sorted, inv, tiles, n_tiles, hits, flags, rows);
         return hipGetLastError();
     }
     int32_t *rank = scratch, *counts = scratch + n_assign;
     // per-kernel timing brackets the two launches as one: start from the first, stop from the last
     const LaunchTiming timing = g_launch_timing;
     g_launch_timing.stop = nullptr;
-    launch_kernel(dispatch_count_kernel, dim3(chunks), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, rank, counts,
-                  flags);
+    launch_kernel(dispatch_count_kernel, dim3((unsigned)chunks + beside), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, rank, counts,
+                  flags, chunks, rows);
     g_launch_timing.start = nullptr;
     g_launch_timing.stop = timing.stop;
     launch_kernel(dispatch_scan_place_kernel, dim3(chunks), dim3(kDispatchThreads), 0, s, ids, n_assign, n_experts, chunks,

@@ -40,13 +40,6 @@ constexpr int kBK = 64;             // K step
 constexpr int kLds = kBK + 8;       // f16 LDS row (halfs): 144 B keeps 16-byte reads conflict-free
 constexpr int kLdsC = kBN + 4;      // f32 staging row of the gate/up epilogue
 
-__device__ inline uint32_t pack_half2(float a, float b) {
-    _Float16 h[2] = {(_Float16)a, (_Float16)b};
-    uint32_t u;
-    __builtin_memcpy(&u, h, 4);
-    return u;
-}
-
 __host__ __device__ inline size_t gemm_row_bytes(int type, int in_dim) {
     return (size_t)(in_dim / block_elems(type)) * (size_t)block_bytes(type);
 }
@@ -910,7 +903,7 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_q_kernel(
 // stores the row 1024 elements at a time.
 __global__ __launch_bounds__(256) void quantize_rows_h_kernel(const float *__restrict__ x, int d, HAct q) {
     __shared__ float s_max[4];
-    hact_quantize_row<256>(x, d, q, (int)blockIdx.x, s_max);
+    hact_quantize_row<256>(x, d, q, (int)blockIdx.x, s_max, (int)threadIdx.x);
 }
 
 // x [n, d] f32 -> f16, round to nearest.

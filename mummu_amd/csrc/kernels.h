@@ -181,9 +181,17 @@ size_t dispatch_scratch_ints(int n_assign, int n_experts);
 enum { WORK_GATE_UP = 1, WORK_DOWN = WORK_GATE_UP + 8, WORK_INTS = WORK_DOWN + 8 };
 // unit: an expert's tiles, as few as tile_rows allows, share its rows evenly in multiples of this many (tile_rows: all
 // but the last are full).
+// rows: x in the form the products read, made beside the sort by workgroups of their own (x null: nothing).  Where h.lo is set rows as pairs of halfs
+// (launch_quantize_rows_h), else with h.hi as halfs (launch_convert_rows_f16), else as QAct64 (launch_quantize_rows64); d as there.
+struct RowsJob {
+    const float *x = nullptr;
+    int n = 0, d = 0;
+    HAct h;
+    QAct64 q;
+};
 hipError_t launch_dispatch(const int32_t *ids, int n_assign, int n_experts, int tile_rows, int unit, int32_t *offsets,
                            int32_t *sorted, int32_t *inv, int32_t *tiles, int32_t *n_tiles, int32_t *scratch,
-                           unsigned long long *hits, int32_t *flags, hipStream_t s);
+                           unsigned long long *hits, int32_t *flags, const RowsJob &rows, hipStream_t s);
 
 // One expert serving rows 0..n-1 in order: sorted[i] = i and the tile list of expert 0 (tiles: 3 ints
 // per tile, at least ceil(n / tile_rows) tiles).

@@ -582,13 +582,12 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
         const bool half_banks = b.gate_type == T_F16 || b.gate_type == T_BF16 || q8h;
         const HAct xh = hf ? hp.xh : (half_banks ? HAct{(_Float16 *)h->y, nullptr, nullptr, nullptr} : HAct());
         const HAct acth = hf_down || hp.q6 ? HAct{(_Float16 *)h->act16, (_Float16 *)h->act, h->actq.scale, (float *)h->actq.sum} : HAct();
-        if (hf && !xh_done) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows_h(x, (int)n, b.hidden, xh, s));
-        else if (hf) {}   // (the router launch wrote them)
-        else if (half_banks) LAUNCH(h, K_QUANTIZE, s, launch_convert_rows_f16(x, (int)n, b.hidden, xh.hi, s));
-        else if (grouped_gemm_quantized(b)) LAUNCH(h, K_QUANTIZE, s, launch_quantize_rows64(x, (int)n, b.hidden, xq64, s));
+        // (Q4_K and Q8_0 as pairs of halfs: where the router launch has not written them; f32 banks read x itself)
+        RowsJob rows;
+        if (hf ? !xh_done : (half_banks || grouped_gemm_quantized(b))) rows = RowsJob{x, (int)n, b.hidden, xh, xq64};
         LAUNCH(h, K_DISPATCH, s,
                launch_dispatch(h->ids, na, b.n_experts, tile_rows, wide ? kWideUnit : tile_rows, h->offsets, h->sorted, h->inv, h->tiles,
-                               h->n_tiles, h->disp_scratch, count_hits ? L.hits : nullptr, h->flags, s));
+                               h->n_tiles, h->disp_scratch, count_hits ? L.hits : nullptr, h->flags, rows, s));
         if (wide) {
             LAUNCH(h, K_GEMM_GATE_UP, s,
                    launch_wide_gate_up(b, xh.hi, h->sorted, k, h->tiles, h->n_tiles, tiles_bound, (_Float16 *)h->act16, s));

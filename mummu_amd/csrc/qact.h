@@ -173,11 +173,12 @@ __device__ inline void hact_store128(float4 v, bool active, const HAct &q, size_
     }
 }
 
-// One workgroup of NT threads turns row `row` of x [n, d] into HAct with one scale for the whole row (d % 128 == 0):
-// the row's largest magnitude first, then the row NT * 4 elements at a time.  s_max: NT / 64 floats of LDS.
+// NT threads (whole waves; tid: of them) turn row `row` of x [n, d] into HAct with one scale for the whole row (d % 128 == 0):
+// the row's largest magnitude first, then the row NT * 4 elements at a time.  s_max: NT / 64 floats of LDS.  Every thread of the
+// workgroup comes here (a barrier); those of a row that is not there do nothing else.
 template <int NT>
-__device__ inline void hact_quantize_row(const float *__restrict__ x, int d, const HAct &q, int row, float *s_max) {
-    const int tid = threadIdx.x;
+__device__ inline void hact_quantize_row(const float *__restrict__ x, int d, const HAct &q, int row, float *s_max, int tid, bool there = true) {
+    if (!there) d = 0;
     const float *xr = x + (size_t)row * (size_t)d;
     float m = 0.0f;
     for (int e0 = tid * 4; e0 < d; e0 += NT * 4) {

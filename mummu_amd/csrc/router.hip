@@ -483,7 +483,7 @@ __global__ __launch_bounds__(64 * (SPLIT > 1 ? SPLIT : kStreamWaves)) void route
             __shared__ float s_max[SPLIT];
             const int row = (int)blockIdx.x - n;
             if (xh.hi != nullptr) {
-                hact_quantize_row<64 * SPLIT>(x, hidden, xh, row, s_max);
+                hact_quantize_row<64 * SPLIT>(x, hidden, xh, row, s_max, (int)threadIdx.x);
             } else {
                 // ... or into the 16-bit blocks of 16 the decode kernels read (hidden % 16 == 0: whole 16-lane rows)
                 for (int e0 = threadIdx.x; e0 < hidden; e0 += 64 * SPLIT)
