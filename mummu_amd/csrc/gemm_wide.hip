@@ -112,7 +112,7 @@ __device__ inline Item item_of(const WideArgs &p, int i) {
 }
 
 // What a wave moves of a stage: rows 8 mw wave .. of the activation tile (8 to a load: a lane per 16-byte piece) and
-// rows 32 wave .. of the weight tile.  Row r of a tile holds its eight pieces in the order q ^ (r % 8): eight lanes that
+// rows 32 wave .. of the weight tile.  Row r of a tile holds its eight pieces in the order q ^ (r / 2 % 8): sixteen lanes that
 // read the same piece of neighbouring rows then meet all 64 banks.
 struct Loader {
     uint32_t a_off[5], b_off[4];
@@ -129,13 +129,13 @@ struct Loader {
     template <bool GATE_UP>
     __device__ void rows_of(const WideArgs &p, const Item &t, int mw) {
         const int tid = thread_id(), lane = tid & 63, wave = uniform(tid >> 6), lrow = lane >> 3;
-        const uint32_t row_bytes = (uint32_t)p.in_dim * 2u, piece = (uint32_t)((lane & 7) ^ lrow) * 16u;
+        const uint32_t row_bytes = (uint32_t)p.in_dim * 2u, piece = (uint32_t)((lane & 7) ^ (lrow >> 1)) * 16u;   // (of an even eight of rows)
         a_base = (const uint8_t *)p.a;
 #pragma unroll
         for (int i = 0; i < 5; i++) {
             const int r = 8 * mw * wave + 8 * i + lrow;
             const int rr = r < t.rows ? r : t.rows - 1;   // (rows past the tile's end repeat its last: multiplied, never stored)
-            a_off[i] = (uint32_t)(GATE_UP ? p.sorted[t.p0 + rr] / p.k_slots : t.p0 + rr) * row_bytes + piece;
+            a_off[i] = (uint32_t)(GATE_UP ? p.sorted[t.p0 + rr] / p.k_slots : t.p0 + rr) * row_bytes + (piece ^ (uint32_t)(((mw * wave + i) & 1) * 64));
         }
         // weight rows: gate/up: 32 rows of gate, then 32 of up for each pair of waves; down: 64 rows for each pair
         const int col0 = GATE_UP ? t.slab * (kWCols / 2) + 32 * (wave >> 1) : t.slab * kWCols + 32 * wave;
@@ -143,7 +143,7 @@ struct Loader {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int col = col0 + 8 * i + lrow < p.out_dim ? col0 + 8 * i + lrow : p.out_dim - 1;
-            b_off[i] = (uint32_t)col * row_bytes + piece;
+            b_off[i] = (uint32_t)col * row_bytes + (piece ^ (uint32_t)((i & 1) * 64));
         }
     }
     // Its first two stages: for each of them four loads of weights and mw of rows.
@@ -182,7 +182,7 @@ __device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, Beh
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[b][m][r] = 0.0f;
     // piece 2 kk + g of the wave's rows: where group 0's is, and 2 kk more of a row's order
-    const uint32_t q = (uint32_t)(g ^ (lr & 7)) * 16u;
+    const uint32_t q = (uint32_t)(g ^ (lr >> 1 & 7)) * 16u;
     uint32_t a_rd = R::kAtA + (uint32_t)(32 * MW * wm + lr) * (kWK * 2) + q, b_rd = (uint32_t)(64 * wn + lr) * (kWK * 2) + q;
     // operands of 16 elements of K, read while the ones before are multiplied
     half8 ra[2][MW], rb[2][2];
