@@ -1,10 +1,14 @@
-// Grouped GEMM of F16 and BF16 banks with wide tiles, for many rows per expert: the operands and arithmetic of
-// grouped_gemm_f16_kernel (gemm.hip) - x and the activations between the two products as halfs, v_mfma_f32_32x32x16_f16,
-// f32 accumulators - on tiles of up to 320 rows by 256 weight rows (128 of gate and 128 of up, or 256 of down).
+// Grouped GEMM of F16 and BF16 banks with wide tiles, for many rows per expert: x and the activations between the two products as halfs and
+// f32 accumulators as in grouped_gemm_f16_kernel (gemm.hip), v_mfma_f32_16x16x32_f16, on tiles of up to 320 rows by 256 weight rows (128 of
+// gate and 128 of up, or 256 of down).
 //
 // What bounds it and why it looks the way it does (OLMoE shape, 4096 tokens = 512 rows per expert):
-//   - LDS reads.  A 64 x 128 tile reads one operand per matrix instruction, which keeps the LDS port (128 bytes a clock)
-//     busy all the time at half the matrix rate.  Eight waves of 32 MW x 64 outputs (MW up to 5) read 7 operands for 10.
+//   - Power.  The card lowers its clock as the matrix units are busy: with weights of zeros the same layer took 421 us instead of 540.  A product of 16 by
+//     16 and 32 of K passes through the accumulators half as often as one of 32 by 32 and 16 (on registers alone, normal data, 1950 against
+//     1697 TFLOP/s; 1726 / 1544 with four vector instructions to every 32 k operations): 1.79 -> 2.05 GHz, gate/up 277 -> 250 us; layers, us:
+//     4096 / 3000 bf16 tokens 517 -> 492, 413 -> 387, 4096 of f16 506 -> 483.  The same bits.
+//   - LDS reads.  A 64 x 128 tile reads one operand per 32 k operations, which keeps the LDS port (128 bytes a clock)
+//     busy all the time at half the matrix rate.  Eight waves of 32 MW x 64 outputs (MW up to 5) read 7 for 10.
 //   - The way into LDS.  Both tiles go from global memory straight into LDS, 64 elements of K (whole 128-byte lines: pieces
 //     of 64 bytes come out of the L2 at half the rate, 17 against 34 TB/s) at a time, without registers in between, the weights two
 //     stages ahead where the LDS holds them, and never a stage at once: 72 loads behind a barrier fill the address unit's queue, with
@@ -13,14 +17,13 @@
 //   - Whole rounds.  An expert's rows are split evenly, in steps of 64, over as few tiles as hold them, so that the
 //     workgroups of a launch are alike (full tiles and a remainder left a fifth of the launch to stragglers), and a wave
 //     multiplies only as many row blocks as the tile has.
-//   - Weights of bf16 become halfs beside the last products of the group before, not between their read and the next products.
-//   - One workgroup fills a CU, so that nothing hides what it does outside its loop over K.  It stays and takes items - from a counter
-//     of its XCD, since tiles are of unlike heights - and asks for the first stages of the next before it stores the results of the last.
-//     A workgroup an item, 4096 / 3000 bf16 tokens a layer 554 -> 519, 443 -> 416 us, 4096 / 2000 of f16 537 -> 514, 309 -> 304; where the
-//     stream of the weights bounds it the same (1000 tokens 235, 600: 203; with the next item looked up behind the last step, and both
-//     stages waited for, 600 tokens were 3 % slower).
-// What remains: the matrix units were busy for 52 / 38 % of the cycles at 4096 bf16 rows x 8 with a workgroup an item, and the card lowers its
-// clock as they are: 15 % fewer cycles were 7 % of the time (340 / 206 us -> 316 / 194, a trace of it on its own).
+//   - Weights of bf16 become halfs beside the last products of the half stage before, not between their read and the next products.
+//   - One workgroup fills a CU, so that nothing hides what it does outside its loop over K.  With many rows (items_in_turn) it stays and takes
+//     items - from a counter of its XCD, since tiles are of unlike heights - and asks for the first stages of the next before it stores
+//     the results of the last.
+//   - What a lane keeps from item to item - offsets of rows - has to stay in registers: reloaded ones are waited for in the loop, behind every load
+//     that is under way (bf16, 4096 tokens 492 -> 558).
+// What remains: the matrix units are busy for 60 / 46 % of the cycles at 4096 bf16 rows x 8.
 #include <type_traits>
 
 #include "device_utils.h"
@@ -31,7 +34,7 @@ namespace mummu {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWK = 64;                          // K elements of a stage: a line of 128 bytes per row, eight pieces of 16
@@ -79,10 +82,11 @@ __device__ inline float fast_silu(float x) {
 
 struct WideArgs {
     const uint8_t *w0, *w1;        // gate and up, or down [experts][out_dim][in_dim]
-    const _Float16 *a;             // rows of in_dim halfs: tokens (gate/up, through sorted / k_slots) or sorted positions
+    const _Float16 *a;             // rows of in_dim halfs: tokens (gate/up, through sorted / slots) or sorted positions
     const int32_t *sorted, *tiles;
     int32_t *n_tiles;              // the number of tiles, then the counters of items (WORK_GATE_UP, WORK_DOWN)
-    int k_slots, in_dim, out_dim;
+    uint32_t per_slot;             // 2^32 / k_slots, rounded up: an assignment's token is the upper half of their product (0: one slot)
+    int in_dim, out_dim;
     _Float16 *act;                 // gate/up: silu(g) * u, sorted positions
     float *y;                      // down
 };
@@ -115,14 +119,17 @@ __device__ inline Item item_of(const WideArgs &p, int i) {
 // rows 32 wave .. of the weight tile.  Row r of a tile holds its eight pieces in the order q ^ (r / 2 % 8): sixteen lanes that
 // read the same piece of neighbouring rows then meet all 64 banks.
 struct Loader {
-    uint32_t a_off[5], b_off[4];
+    uint32_t a_off[5], b_off;
     const uint8_t *a_base, *b_base;
 
     __device__ void load_a(uint32_t at, int step, int mw, int wave, int i) const {
         load_to_lds16(at + (uint32_t)(8 * mw * wave + 8 * i) * (kWK * 2), a_base + (size_t)step * (kWK * 2), a_off[i]);
     }
-    __device__ void load_b(uint32_t at, int step, int wave, int i) const {
-        load_to_lds16(at + (uint32_t)(32 * wave + 8 * i) * (kWK * 2), b_base + (size_t)step * (kWK * 2), b_off[i]);
+    // (eight rows of LDS: every second or fourth of the matrix from the (i % 2) * 16-th or * 32-nd, i / 2 on)
+    template <bool GATE_UP>
+    __device__ void load_b(uint32_t at, int step, uint32_t row_bytes, int wave, int i) const {
+        load_to_lds16(at + (uint32_t)(32 * wave + 8 * i) * (kWK * 2),
+                      b_base + (size_t)step * (kWK * 2) + (size_t)((i & 1) * (GATE_UP ? 16 : 32) + (i >> 1)) * row_bytes, b_off ^ (uint32_t)((i & 1) * 64));
     }
 
     // The rows of an item of 64 mw rows.
@@ -135,24 +142,30 @@ struct Loader {
         for (int i = 0; i < 5; i++) {
             const int r = 8 * mw * wave + 8 * i + lrow;
             const int rr = r < t.rows ? r : t.rows - 1;   // (rows past the tile's end repeat its last: multiplied, never stored)
-            a_off[i] = (uint32_t)(GATE_UP ? p.sorted[t.p0 + rr] / p.k_slots : t.p0 + rr) * row_bytes + (piece ^ (uint32_t)(((mw * wave + i) & 1) * 64));
+            uint32_t row = (uint32_t)(t.p0 + rr);
+            if (GATE_UP) {
+                row = (uint32_t)p.sorted[row];
+                row = p.per_slot != 0 ? __umulhi(row, p.per_slot) : row;
+            }
+            a_off[i] = row * row_bytes + (piece ^ (uint32_t)(((mw * wave + i) & 1) * 64));
         }
-        // weight rows: gate/up: 32 rows of gate, then 32 of up for each pair of waves; down: 64 rows for each pair
-        const int col0 = GATE_UP ? t.slab * (kWCols / 2) + 32 * (wave >> 1) : t.slab * kWCols + 32 * wave;
-        b_base = uniform((GATE_UP && (wave & 1) ? p.w1 : p.w0) + (size_t)t.e * (size_t)p.out_dim * row_bytes);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int col = col0 + 8 * i + lrow < p.out_dim ? col0 + 8 * i + lrow : p.out_dim - 1;
-            b_off[i] = (uint32_t)col * row_bytes + (piece ^ (uint32_t)((i & 1) * 64));
-        }
+        // weight rows: gate/up: 32 rows of gate, then 32 of up for each pair of waves; down: 64 rows for each pair (out_dim % 64 == 0: all of them there, or
+        // none, and the last ones instead).  Sixteen rows of LDS are an operand: those of operand j hold rows j, j + n, j + 2 n .. of the wave's 64
+        // (n: 4) or of the 32 of gate or up (2), so that a lane's results lie side by side.
+        constexpr int kRun = GATE_UP ? 32 : 64;
+        const int run0 = GATE_UP ? t.slab * (kWCols / 2) + 32 * (wave >> 1) : t.slab * kWCols + 64 * (wave >> 1);
+        const int first = (run0 < p.out_dim ? run0 : p.out_dim - kRun) + (GATE_UP ? 0 : 2 * (wave & 1));
+        b_base = uniform((GATE_UP && (wave & 1) ? p.w1 : p.w0) + ((size_t)t.e * (size_t)p.out_dim + (size_t)first) * row_bytes);
+        b_off = (uint32_t)((GATE_UP ? 2 : 4) * lrow) * row_bytes + piece;
     }
     // Its first two stages: for each of them four loads of weights and mw of rows.
-    __device__ void begin(int mw, uint32_t lds0, int wave) {
+    template <bool GATE_UP>
+    __device__ void begin(int mw, uint32_t lds0, uint32_t row_bytes, int wave) {
         const uint32_t lds_a = lds0 + (mw <= 4 ? Ring<4>::kAtA : Ring<5>::kAtA);
 #pragma unroll
         for (int step = 0; step < 2; step++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) load_b(lds0 + step * kWStageB, step, wave, i);
+            for (int i = 0; i < 4; i++) load_b<GATE_UP>(lds0 + step * kWStageB, step, row_bytes, wave, i);
 #pragma unroll
             for (int i = 0; i < 5; i++)
                 if (i < mw) load_a(lds_a + (uint32_t)(step * 64 * mw * (kWK * 2)), step, mw, wave, i);
@@ -160,133 +173,164 @@ struct Loader {
     }
 };
 
-// What is behind an item's first two stages when it begins: nothing, stores that may be left out of the wait for its second one, or so many
-// that this has landed too.
-enum Behind { NOTHING, SOME_STORES, MANY_STORES };
+// A step's wait: its loads but for so many have landed, and everybody has read what the next ones overwrite.
+template <int LOADS>
+__device__ inline void wait_and_meet() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+}
 
 // One item, of up to 64 MW rows; wave (wm, wn) multiplies rows 32 MW wm .. by its 64 weight rows.  Its first stage has landed as far as
 // this wave asked for it, the second is on its way.  Returns the workgroup's next item, of which the same is true then.
 template <bool GATE_UP, int WT, int MW>
-__device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, Behind &behind, uint8_t *s_lds) {
+__device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, int &behind, uint8_t *s_lds) {
     using R = Ring<MW>;
     const int tid = thread_id(), lane = tid & 63, wave = uniform(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3, g = lane >> 5, lr = lane & 31;
+    const int wm = wave >> 2, wn = wave & 3;
     const uint32_t lds0 = lds_offset(s_lds);
     const int n_steps = p.in_dim / kWK;
+    const uint32_t row_bytes = (uint32_t)p.in_dim * 2u;
 
-    float16v acc[2][MW];
+    // Products of 16 rows by 16 columns and 32 of K: two row blocks for a product of 32 by 32 and 16, as many clocks, but half the
+    // passes through the accumulators, and the card's power is what its clock goes by.  A unit: row block m of a half stage, by the wave's four operands
+    // of weights.  Lane (row or column lane % 16, K group lane / 16).
+    constexpr int kBlocks = 2 * MW, kUnits = 2 * kBlocks;
+    constexpr int kEnd = MW == 1 ? 2 : 3;   // units behind a step's barrier, and how far ahead the rows are read
+    const int kg = lane >> 4, lr = lane & 15;
+    f32x4 acc[kBlocks][4];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int m = 0; m < kBlocks; m++)
 #pragma unroll
-        for (int m = 0; m < MW; m++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[b][m][r] = 0.0f;
-    // piece 2 kk + g of the wave's rows: where group 0's is, and 2 kk more of a row's order
-    const uint32_t q = (uint32_t)(g ^ (lr >> 1 & 7)) * 16u;
+        for (int j = 0; j < 4; j++) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // (piece 4 half + kg of a row)
+    const uint32_t q = (uint32_t)(kg ^ (lr >> 1 & 7)) * 16u;
     uint32_t a_rd = R::kAtA + (uint32_t)(32 * MW * wm + lr) * (kWK * 2) + q, b_rd = (uint32_t)(64 * wn + lr) * (kWK * 2) + q;
-    // operands of 16 elements of K, read while the ones before are multiplied
-    half8 ra[2][MW], rb[2][2];
-    u32x4 raw[2];
-    auto read = [&](uint32_t at_a, uint32_t at_b, int kk) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) raw[j] = *(const u32x4 *)(s_lds + ((b_rd ^ (32u * kk)) + at_b) + 32 * (kWK * 2) * j);
-#pragma unroll
-        for (int m = 0; m < MW; m++) ra[kk & 1][m] = *(const half8 *)(s_lds + ((a_rd ^ (32u * kk)) + at_a) + 32 * (kWK * 2) * m);
+    half8 a_first[kEnd], b_now[4];   // of the step's first units
+    auto read_a = [&](uint32_t at, int u) {
+        return *(const half8 *)(s_lds + ((a_rd ^ (uint32_t)(u / kBlocks * 64)) + at) + 16 * (kWK * 2) * (u % kBlocks));
     };
-    auto convert = [&](int kk) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) rb[kk & 1][j] = weight_operand<WT>(raw[j]);
-    };
-    // row block m's two products of group kk
-    auto multiply = [&](int kk, int m) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[j][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ra[kk & 1][m], rb[kk & 1][j], acc[j][m], 0, 0, 0);
-    };
+    auto read_b = [&](uint32_t at, int half, int j) { return *(const u32x4 *)(s_lds + ((b_rd ^ (uint32_t)(half * 64)) + at) + 16 * (kWK * 2) * j); };
     // Behind the barrier of a step, beside its last products, the rows of the step after the next are asked for; beside the first
     // products after that the weights of one step more (tiles of more than 256 rows leave no room for that: of the same step).  All at once
     // they fill the address unit's queue, and every wave stands before it.
-    constexpr int kAhead = R::kB == 3 ? 2 : 1, kJ = GATE_UP ? 1 : 2;
+    constexpr int kAhead = R::kB == 3 ? 2 : 1;
     const uint32_t lds_a = lds0 + R::kAtA;
     asm volatile("s_barrier" ::: "memory");
-    read(0, 0, 0);
-    convert(0);
+#pragma unroll
+    for (int u = 0; u < kEnd; u++) a_first[u] = read_a(0, u);
+#pragma unroll
+    for (int j = 0; j < 4; j++) b_now[j] = weight_operand<WT>(read_b(0, 0, j));
     uint32_t at_b = 0, free_b = kAhead * kWStageB;   // of this step's weights; of those kAhead on
     int taken = 0;
     // The word that tells the other waves the next item, where no load is under way to: the weights' third stage, or behind the last
     int *const told = (int *)(s_lds + (R::kB == 3 ? n_steps % 3 * kWStageB : R::kAtA + 2 * R::kStageA));
     Item next{0, 0, 0, 0};
-    // LEFT: steps behind this one (2: or more)
-    auto multiply_step = [&](int step, auto left) {
+    // LEFT: steps behind this one (2: or more); FIRST: the first of three or more
+    auto multiply_step = [&](int step, auto left, auto first) {
         constexpr int LEFT = decltype(left)::value;
-        asm volatile("" : "+v"(a_rd), "+v"(b_rd));   // (no registers for their eight sums and differences over the steps)
+        constexpr bool FIRST = decltype(first)::value;
+        asm volatile("" : "+v"(a_rd), "+v"(b_rd));   // (no registers for their sums and differences over the steps)
         const uint32_t at_a = (uint32_t)(step & 1) * R::kStageA, next_a = R::kStageA - at_a;
         const uint32_t next_b = at_b == (R::kB - 1) * kWStageB ? 0u : at_b + kWStageB;
         // The next item is taken late, so that a workgroup with much to do takes fewer, and looked up in the last step.
         if (LEFT == 1 && tid == 0) taken = (int)(gridDim.x >> 3) + atomicAdd(p.n_tiles + (GATE_UP ? WORK_GATE_UP : WORK_DOWN) + (blockIdx.x & 7), 1);
         if (LEFT == 0) taken = *told;
+        half8 a[kUnits + kEnd], b[3][4];
+        u32x4 raw[4];
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            if (LEFT == 0 && kk == 1) next = item_of<GATE_UP>(p, uniform(taken));
-            if (LEFT == 0 && kk == 2 && next.rows > 0) l.rows_of<GATE_UP>(p, next, (next.rows + kWideUnit - 1) / kWideUnit);
-            if (LEFT == 1 && kk == 3 && tid == 0) *told = taken;
-            // The next stage has landed and this one has been read by everybody.  (In the first step the stores of the item before stand between the
-            // second stage and the third's weights.)
-            if (kk == 3) {
-                if ((LEFT == 0 && kAhead == 2) || (LEFT > 0 && step == 0 && behind == MANY_STORES)) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                else if (step == 0 && behind == SOME_STORES) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(16 * kJ) : "memory");
-                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kAhead == 2 && LEFT == 2 ? 4 : 0) : "memory");
+        for (int u = 0; u < kEnd; u++) a[u] = a_first[u];
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[0][j] = b_now[j];
+#pragma unroll
+        for (int u = 0; u < kUnits; u++) {
+            const int half = u / kBlocks, m = u % kBlocks, behind_barrier = u - (kUnits - kEnd), to_half_end = m - (kBlocks - kEnd);
+            if (LEFT == 0 && u == kUnits / 2) next = item_of<GATE_UP>(p, uniform(taken));
+            if (LEFT == 0 && u == kUnits - 2 && next.rows > 0) l.template rows_of<GATE_UP>(p, next, (next.rows + kWideUnit - 1) / kWideUnit);
+            if (behind_barrier == 0) {
+                if (LEFT == 1 && tid == 0) *told = taken;
+                // (In an item's first step the stores of the one before, eight to 64 of its rows, stand behind the stage that is waited for.)
+                if (LEFT == 0) wait_and_meet<kAhead == 2 ? 63 : 0>();
+                else if (FIRST && behind == 1) wait_and_meet<8>();
+                else if (FIRST && behind == 2) wait_and_meet<16>();
+                else if (FIRST && behind == 3) wait_and_meet<24>();
+                else if (FIRST && behind == 4) wait_and_meet<32>();
+                else if (FIRST && behind == 5) wait_and_meet<40>();
+                else wait_and_meet<kAhead == 2 && LEFT == 2 ? 4 : 0>();
             }
-            if (LEFT > 0 || kk < 3) read(kk == 3 ? next_a : at_a, kk == 3 ? next_b : at_b, (kk + 1) & 3);
+            // Rows kEnd units ahead; the stage's last two together, so that the barrier's wait for them is short
+            if (u < kUnits - kEnd - 1) a[u + kEnd] = read_a(at_a, u + kEnd);
+            if (u == kUnits - kEnd - 2) a[u + kEnd + 1] = read_a(at_a, u + kEnd + 1);
+            if (behind_barrier >= 0 && LEFT > 0) a[kUnits + behind_barrier] = read_a(next_a, behind_barrier);
+            // the next half stage's weights
+            if (half == 0 || LEFT > 0) {
+                const uint32_t from = half == 0 ? at_b : next_b;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (to_half_end == (kEnd == 2 ? 0 : j / 2)) raw[j] = read_b(from, half ^ 1, j);
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int m = 0; m < MW; m++) {
-                multiply(kk, m);
-                if (kk == 3 && LEFT == 2) l.load_a(lds_a + at_a, step + 2, MW, wave, m);
-                if (kk == 0 && LEFT >= kAhead) {
+            for (int j = 0; j < 4; j++) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u], b[half][j], acc[m][j], 0, 0, 0);
+            if (behind_barrier >= 0 && LEFT == 2) {
 #pragma unroll
-                    for (int i = m; i < 4; i += MW) l.load_b(lds0 + free_b, step + kAhead, wave, i);
-                }
-                if (m == MW - 1 && (LEFT > 0 || kk < 3)) convert((kk + 1) & 3);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int i = behind_barrier; i < MW; i += kEnd) l.load_a(lds_a + at_a, step + 2, MW, wave, i);
             }
+            if (half == 0 && LEFT >= kAhead) {
+#pragma unroll
+                for (int i = m; i < 4; i += kBlocks) l.template load_b<GATE_UP>(lds0 + free_b, step + kAhead, row_bytes, wave, i);
+            }
+            if ((half == 0 || LEFT > 0) && to_half_end >= 1) {
+                // (two of them in each of the last two units; one unit: all)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (kEnd == 2 || j / 2 == to_half_end - 1) b[half + 1][j] = weight_operand<WT>(raw[j]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (LEFT > 0) {
+#pragma unroll
+            for (int u = 0; u < kEnd; u++) a_first[u] = a[kUnits + u];
+#pragma unroll
+            for (int j = 0; j < 4; j++) b_now[j] = b[2][j];
         }
         free_b = at_b;
         at_b = next_b;
     };
-    for (int step = 0; step < n_steps - 2; step++) multiply_step(step, std::integral_constant<int, 2>());
-    multiply_step(n_steps - 2, std::integral_constant<int, 1>());
-    multiply_step(n_steps - 1, std::integral_constant<int, 0>());
+    if (n_steps > 2) multiply_step(0, std::integral_constant<int, 2>(), std::true_type());
+    for (int step = 1; step < n_steps - 2; step++) multiply_step(step, std::integral_constant<int, 2>(), std::false_type());
+    multiply_step(n_steps - 2, std::integral_constant<int, 1>(), std::false_type());
+    multiply_step(n_steps - 1, std::integral_constant<int, 0>(), std::false_type());
 
     // The next item's first stages are on their way while this one's results leave, and those have the next one's first step for it.
-    if (next.rows > 0) l.begin((next.rows + kWideUnit - 1) / kWideUnit, lds0, wave);
-    // Element r of an accumulator: row 8 (r / 4) + 4 g + r % 4, column lane % 32.  Stores by a resource that ends behind the tile's last
-    // row: what lies beyond is dropped, so that every tile makes the same number of them.
+    if (next.rows > 0) l.template begin<GATE_UP>((next.rows + kWideUnit - 1) / kWideUnit, lds0, row_bytes, wave);
+    // Element r of an accumulator: row 4 kg + r, column lane % 16, which is every second or fourth of the matrix's.  Stores by a resource that
+    // ends behind the tile's last row: what lies beyond is dropped, so that every tile makes the same number of them.
     const uint32_t ld = (uint32_t)p.out_dim * (GATE_UP ? 2u : 4u);
     uint8_t *const base = (GATE_UP ? (uint8_t *)p.act : (uint8_t *)p.y) + (size_t)t.p0 * ld;
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)((uint32_t)t.rows * ld), 0x20000);
+    const int n = GATE_UP ? t.slab * (kWCols / 2) + 32 * wn + 2 * lr : t.slab * kWCols + 64 * wn + 4 * lr;   // (whole: out_dim % 64 == 0)
+    const uint32_t at = n < p.out_dim ? (uint32_t)(32 * MW * wm + 4 * kg) * ld + (uint32_t)n * (GATE_UP ? 2u : 4u) : 1u << 31;
 #pragma unroll
-    for (int j = 0; j < kJ; j++) {
-        const int n = GATE_UP ? t.slab * (kWCols / 2) + 32 * wn + lr : t.slab * kWCols + 64 * wn + 32 * j + lr;
-        const uint32_t at = n < p.out_dim ? (uint32_t)(32 * MW * wm + 4 * g) * ld + (uint32_t)n * (GATE_UP ? 2u : 4u) : 1u << 31;
+    for (int m = 0; m < kBlocks; m++)
 #pragma unroll
-        for (int m = 0; m < MW; m++)
+        for (int r = 0; r < 4; r++) {
+            const uint32_t o = at + (uint32_t)(16 * m + r) * ld;
+            if constexpr (GATE_UP) {
+                _Float16 h[2];
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t o = at + (uint32_t)(32 * m + 8 * (r >> 2) + (r & 3)) * ld;
-                if constexpr (GATE_UP) {
-                    const _Float16 h = (_Float16)__fmul_rn(fast_silu(acc[0][m][r]), acc[1][m][r]);
-                    short v;
-                    __builtin_memcpy(&v, &h, 2);
-                    __builtin_amdgcn_raw_buffer_store_b16(v, rsrc, (int)o, 0, 0);
-                } else {
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[j][m][r]), rsrc, (int)o, 0, 0);
-                }
+                for (int j = 0; j < 2; j++) h[j] = (_Float16)__fmul_rn(fast_silu(acc[m][j][r]), acc[m][2 + j][r]);
+                uint32_t v;
+                __builtin_memcpy(&v, h, 4);
+                __builtin_amdgcn_raw_buffer_store_b32(v, rsrc, (int)o, 0, 0);
+            } else {
+                u32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = __float_as_uint(acc[m][j][r]);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, (int)o, 0, 0);
             }
-    }
+        }
     // The first stage, in front of the second's five loads or more and the stores.
-    constexpr int kStores = 16 * MW * kJ;
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kStores + 5 < 63 ? kStores + 5 : 63) : "memory");
-    behind = kStores >= 63 ? MANY_STORES : SOME_STORES;
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(8 * MW + 5) : "memory");
+    behind = MW;
     return next;
 }
 
@@ -297,10 +341,10 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(WideArgs p) {
     Item t = item_of<GATE_UP>(p, (int)(blockIdx.x >> 3));
     if (t.rows == 0) return;
     Loader l;
-    Behind behind = NOTHING;
+    int behind = 0;   // (the height of the item before)
     const int mw0 = (t.rows + kWideUnit - 1) / kWideUnit;
     l.rows_of<GATE_UP>(p, t, mw0);
-    l.begin(mw0, lds_offset(s_lds), uniform((int)threadIdx.x >> 6));
+    l.begin<GATE_UP>(mw0, lds_offset(s_lds), (uint32_t)p.in_dim * 2u, uniform((int)threadIdx.x >> 6));
     asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
     while (t.rows > 0) {
         switch ((t.rows + kWideUnit - 1) / kWideUnit) {
@@ -314,10 +358,10 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(WideArgs p) {
 }
 
 template <bool GATE_UP, int WT>
-hipError_t launch_wide(const WideArgs &p, int max_tiles, hipStream_t s) {
+hipError_t launch_wide(const WideArgs &p, int max_tiles, bool in_turn, hipStream_t s) {
     constexpr int kCols = GATE_UP ? kWCols / 2 : kWCols, kCusOfXcd = 32;
     const int per_xcd = (max_tiles + 7) / 8 * ((p.out_dim + kCols - 1) / kCols);
-    launch_kernel(wide_gemm_kernel<GATE_UP, WT>, dim3(8u * (unsigned)(per_xcd < kCusOfXcd ? per_xcd : kCusOfXcd)), dim3(512), (size_t)kWLds, s, p);
+    launch_kernel(wide_gemm_kernel<GATE_UP, WT>, dim3(8u * (unsigned)(per_xcd < kCusOfXcd || !in_turn ? per_xcd : kCusOfXcd)), dim3(512), (size_t)kWLds, s, p);
     return hipGetLastError();
 }
 
@@ -331,7 +375,9 @@ bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign) {
     };
     if (!((b.gate_type == T_F16 || b.gate_type == T_BF16) && b.up_type == b.gate_type && b.down_type == b.gate_type &&
           fits(b.hidden, b.inter) && fits(b.inter, b.hidden) && (size_t)n_tokens * (size_t)b.hidden * 2 < (1ull << 32) &&
-          (size_t)n_assign * (size_t)b.inter * 2 < (1ull << 32)))
+          (size_t)n_assign * (size_t)b.inter * 2 < (1ull << 32) &&
+          // (a - n_assign and less - over the slots of a token by way of 2^32 / slots: exact while a * slots < 2^32)
+          (size_t)n_assign * (size_t)(n_assign / n_tokens) < (1ull << 32)))
         return false;
     // Up to 64 rows per expert either kernel streams the weights once, and the smaller workgroups of grouped_gemm_f16_kernel,
     // several to a CU, do it better (this kernel with its loads still in one go; OLMoE layers, 64 rows: 207 us there, 237 us here; 72: 256 / 245, 80: 260 / 249, 128: 325 / 276; 512
@@ -344,16 +390,22 @@ bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign) {
     return (size_t)n_assign >= 72 * (size_t)b.n_experts && tiles * (out_dim / kWCols) >= 224;
 }
 
+// Whether the workgroups of a launch are a CU's each and take items in turn, or an item's: where the stream of the weights bounds it, other streams'
+// workgroups come in between as one ends, which is worth more.  Layers among others (three streams), us, an item / in turn: 600 tokens of f16 194 /
+// 204, 800 bf16 201 / 214, 1000: 209 / 213-220, 1200 f16 224 / 232, 1500 bf16 240 / 240-250, 2000: 294 / 290-293, 2800: 390 / 385, 4096: 518 / 503.
+static bool items_in_turn(const ExpertBanks &b, int n_assign) { return n_assign / 256 >= b.n_experts; }
+
 hipError_t launch_wide_gate_up(const ExpertBanks &b, const _Float16 *x16, const int32_t *sorted, int k_slots, const int32_t *tiles,
-                               int32_t *n_tiles, int max_tiles, _Float16 *act16, hipStream_t s) {
-    const WideArgs p{b.gate, b.up, x16, sorted, tiles, n_tiles, k_slots, b.hidden, b.inter, act16, nullptr};
-    return b.gate_type == T_F16 ? launch_wide<true, T_F16>(p, max_tiles, s) : launch_wide<true, T_BF16>(p, max_tiles, s);
+                               int32_t *n_tiles, int max_tiles, int n_assign, _Float16 *act16, hipStream_t s) {
+    const uint32_t per_slot = k_slots == 1 ? 0u : (uint32_t)(((1ull << 32) + (unsigned)k_slots - 1) / (unsigned)k_slots);
+    const WideArgs p{b.gate, b.up, x16, sorted, tiles, n_tiles, per_slot, b.hidden, b.inter, act16, nullptr};
+    return b.gate_type == T_F16 ? launch_wide<true, T_F16>(p, max_tiles, items_in_turn(b, n_assign), s) : launch_wide<true, T_BF16>(p, max_tiles, items_in_turn(b, n_assign), s);
 }
 
 hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, int32_t *n_tiles, int max_tiles,
-                            float *y, hipStream_t s) {
-    const WideArgs p{b.down, nullptr, act16, nullptr, tiles, n_tiles, 1, b.inter, b.hidden, nullptr, y};
-    return b.down_type == T_F16 ? launch_wide<false, T_F16>(p, max_tiles, s) : launch_wide<false, T_BF16>(p, max_tiles, s);
+                            int n_assign, float *y, hipStream_t s) {
+    const WideArgs p{b.down, nullptr, act16, nullptr, tiles, n_tiles, 0, b.inter, b.hidden, nullptr, y};
+    return b.down_type == T_F16 ? launch_wide<false, T_F16>(p, max_tiles, items_in_turn(b, n_assign), s) : launch_wide<false, T_BF16>(p, max_tiles, items_in_turn(b, n_assign), s);
 }
 
 }  // namespace mummu

@@ -240,9 +240,9 @@ hipError_t launch_gemm_down(const ExpertBanks &b, const void *act16, const float
 constexpr int kWideRows = 320, kWideUnit = 64;
 bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign);   // can and should
 hipError_t launch_wide_gate_up(const ExpertBanks &b, const _Float16 *x16, const int32_t *sorted, int k_slots, const int32_t *tiles,
-                               int32_t *n_tiles, int max_tiles, _Float16 *act16, hipStream_t s);
+                               int32_t *n_tiles, int max_tiles, int n_assign, _Float16 *act16, hipStream_t s);
 hipError_t launch_wide_down(const ExpertBanks &b, const _Float16 *act16, const int32_t *tiles, int32_t *n_tiles, int max_tiles,
-                            float *y, hipStream_t s);
+                            int n_assign, float *y, hipStream_t s);
 
 // gemm_q4k.hip ------------------------------------------------------------------------
 // Q4_K gate and up banks (and down banks) on the f16 units, tiles of up to kQ4kRows rows; the activations go to act_h, or to act_q

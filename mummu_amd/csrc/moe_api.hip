@@ -590,8 +590,8 @@ int run_experts(mummu_moe *h, const Layer &L, const float *x, bool x_quantized, 
                                h->n_tiles, h->disp_scratch, count_hits ? L.hits : nullptr, h->flags, rows, s));
         if (wide) {
             LAUNCH(h, K_GEMM_GATE_UP, s,
-                   launch_wide_gate_up(b, xh.hi, h->sorted, k, h->tiles, h->n_tiles, tiles_bound, (_Float16 *)h->act16, s));
-            LAUNCH(h, K_GEMM_DOWN, s, launch_wide_down(b, (const _Float16 *)h->act16, h->tiles, h->n_tiles, tiles_bound, h->y, s));
+                   launch_wide_gate_up(b, xh.hi, h->sorted, k, h->tiles, h->n_tiles, tiles_bound, na, (_Float16 *)h->act16, s));
+            LAUNCH(h, K_GEMM_DOWN, s, launch_wide_down(b, (const _Float16 *)h->act16, h->tiles, h->n_tiles, tiles_bound, na, h->y, s));
             LAUNCH(h, K_COMBINE, s, launch_combine(h->y, h->ids, h->weights, h->inv, (int)n, k, b.hidden, residual, out, s));
             return MUMMU_OK;
         }
