@@ -80,3 +80,22 @@ def test_gates_beyond_the_exponential():
     assert np.isfinite(got).all()
     # (a few roundings of f32; below -87 the product with 0 where the quotient is under 2e-36)
     assert (np.abs(got - want) <= 1e-6 * np.abs(want) + 2e-36).all()
+
+
+@pytest.mark.parametrize("down", [M.Q4_K, M.Q8_0])
+def test_last_tiles_of_every_number_of_sixteens(monkeypatch, down):
+    """Tiles of up to 64 rows cost what they have in steps of 16: the steps that the counts above leave out, as only tile and behind a full one."""
+    monkeypatch.setenv("MUMMU_GEMM_TILE_ROWS", "64")
+    counts, H, I = [47, 48, 49, 46, 79, 80, 81, 111, 112, 113, 50, 3], 512, 768
+    E, n = len(counts), sum(counts)
+    gate, up = (synth.random_bank_fast(M.Q4_K, [H, I, E], seed) for seed in (41, 42))
+    downs = synth.random_bank_fast(down, [I, H, E], 43)
+    rng = np.random.Generator(np.random.PCG64(3))
+    ids = np.repeat(np.arange(E), counts)[rng.permutation(n)].astype(np.int32)[:, None]
+    x, w = rng.standard_normal((n, H), dtype=np.float32), rng.random((n, 1), dtype=np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q4_K, up, M.Q4_K, downs, down)
+        got = m.apply_routing(0, ids, w, x)
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, downs, orc.Q4_K, orc.Q4_K, orc.Q4_K if down == M.Q4_K else orc.Q8_0), ids, w, x)
+    # (the bars of the test above)
+    assert orc.rel_err(got, want, mag).max() <= (2e-3 if down == M.Q8_0 else 3e-5)
