@@ -973,10 +973,15 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     }
 }
 
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
 // The same sums for hidden % 4 == 0 and k up to 64 slots, a lane a slot: a wave looks its token's slots up by itself - rows, weights and ids in one go,
 // sorted over the lanes - and asks for eight slots' columns at once.  What bounds it: the reads of y, which are all that is left behind the first wait.
 // (combine_kernel's row indexes follow its ids, with two barriers between: 512 / 1000 / 4096 tokens of 2048 elements, eight slots 8.8 / 14.8 / 55.1 us,
 // here 7.7 / 13.7 / 51.7, 5.8 TB/s; 64: 4.7 both.)
+// ONCE: y past the caches' order of use, for one that is about as large as the memory-side cache: 4096 tokens 57.7 -> 52.3 on the card that was measured
+// on, the layer of bf16 among others 509.5 -> 503.7; 512 / 1000 / 2000 tokens the same.
+template <bool ONCE>
 __global__ __launch_bounds__(256) void combine_slots_kernel(const float *__restrict__ y, const int32_t *__restrict__ ids, const float *__restrict__ weights,
                                                             const int32_t *__restrict__ inv, int k, int hidden, const float *__restrict__ residual,
                                                             float *__restrict__ out, unsigned long long *epoch_bump) {
@@ -1001,7 +1006,11 @@ __global__ __launch_bounds__(256) void combine_slots_kernel(const float *__restr
         sum.w = __fadd_rn(sum.w, __fmul_rn(wr, v.w));
     };
     for (int c = 4 * (blockIdx.y * blockDim.x + threadIdx.x); c < hidden; c += 4 * gridDim.y * blockDim.x) {
-        auto slot = [&](int r) { return *(const float4 *)(y + (size_t)__builtin_amdgcn_readlane(row, r) * (size_t)hidden + c); };
+        auto slot = [&](int r) {
+            const f32x4v *from = (const f32x4v *)(y + (size_t)__builtin_amdgcn_readlane(row, r) * (size_t)hidden + c);
+            const f32x4v v = ONCE ? __builtin_nontemporal_load(from) : *from;
+            return make_float4(v[0], v[1], v[2], v[3]);
+        };
         auto weight = [&](int r) { return __int_as_float(__builtin_amdgcn_readlane(w, r)); };
         float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         int r = 0;
@@ -1034,7 +1043,9 @@ hipError_t launch_combine(const float *y, const int32_t *ids, const float *weigh
     int ysplit = (1024 + n - 1) / n;
     ysplit = std::max(1, std::min(ysplit, (hidden + per_wg - 1) / per_wg));
     dim3 block(256), grid(n, ysplit);
-    if (vec4 && k <= kWave) launch_kernel(combine_slots_kernel, grid, block, 0, s, y, ids, weights, inv, k, hidden, residual, out, epoch_bump);
+    const bool once = (size_t)n * (size_t)k * (size_t)hidden * 4 >= 200000000;   // (the memory-side cache: 256 MiB)
+    if (vec4 && k <= kWave && once) launch_kernel(combine_slots_kernel<true>, grid, block, 0, s, y, ids, weights, inv, k, hidden, residual, out, epoch_bump);
+    else if (vec4 && k <= kWave) launch_kernel(combine_slots_kernel<false>, grid, block, 0, s, y, ids, weights, inv, k, hidden, residual, out, epoch_bump);
     else if (vec4) launch_kernel(combine_kernel<true>, grid, block, 0, s, y, ids, weights, inv, k, hidden, residual, out, epoch_bump);
     else launch_kernel(combine_kernel<false>, grid, block, 0, s, y, ids, weights, inv, k, hidden, residual, out, epoch_bump);
     return hipGetLastError();
