@@ -652,10 +652,11 @@ hipError_t launch_router_fused(const float *x, const void *w, int wtype, int n, 
     if (n_experts > 128 || k > n_experts || k < 1) return hipErrorInvalidValue;
     if (xq.hi != nullptr && hidden % 64 != 0) return hipErrorInvalidValue;
     const bool vec = (hidden % 8 == 0) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)w & 15) == 0);
-    // The matrix units (router_matrix.hip), 16 tokens to a workgroup, where those come near filling the chip: 64 experts of 2048, 1000 / 1500 / 2100 / 4096
-    // tokens 17 / 25 / 42 / 48 us in the streaming form, 22 / 23 / 24 / 25 there, but layers among others at 1700 459 / 461, at 2100 367 / 345.  (A tile's 64
-    // columns want more than 32 experts.)
-    if (xh.hi == nullptr && xq.hi == nullptr && n > 2048 && n_experts > 32 && n_experts <= 64 && router_matrix_takes(x, w, hidden))
+    // The matrix units (router_matrix.hip), 16 tokens to a workgroup, one round of which takes 22 to 25 us up to 4096 tokens: 64 experts of 2048, 1000 / 1500 /
+    // 2100 / 4096 tokens 17 / 25 / 42 / 48 us in the streaming form.  Beside other streams, which have the CUs that it leaves, they are ahead from some
+    // 400 tokens on (layers, streaming / here, f16 512 tokens 165.7 / 162.9, bf16 1000: 211 / 205, f16 1500: 244 / 233, bf16 2000: 293 / 280, Q4_K 1500: 371 /
+    // 368, 2000: 482 / 474), on their own from where a round is no longer, which is the line.  (A tile's 64 columns want more than 32 experts.)
+    if (xh.hi == nullptr && xq.hi == nullptr && n > 1024 && n_experts > 32 && n_experts <= 64 && router_matrix_takes(x, w, hidden))
         return launch_router_matrix(x, w, wtype, n, hidden, n_experts, k, flavour, norm, logits, ids, weights, hits, flags, true, s);
     // enough tokens to fill the chip with independent waves: activations in registers, weight
     // rows streamed (on this path the caller quantizes x separately)

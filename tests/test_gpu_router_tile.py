@@ -56,6 +56,13 @@ def test_routing_and_hits_of_a_batch(E, n):
     assert np.array_equal(hits, np.bincount(ids.ravel(), minlength=E))
 
 
+# The routing of 33 to 64 experts on either side of the line to the matrix units, and of few more tokens than a workgroup's: both forms sum a
+# logit in the same order, so no bit of the routing may differ.
+@pytest.mark.parametrize("E,n", [(64, 1024), (64, 1025), (33, 1030), (32, 1030), (50, 1537)])
+def test_routing_at_the_line_to_the_matrix_units(E, n):
+    test_routing_and_hits_of_a_batch(E, n)
+
+
 # A token whose row holds an infinity or a NaN is refused, on either side of the line to the matrix units.
 @pytest.mark.parametrize("E,n", [(64, 40), (64, 2049), (130, 40), (130, 700)])
 @pytest.mark.parametrize("value", [np.inf, np.nan])
