@@ -1166,7 +1166,7 @@ hipError_t launch_gemm_gate_up(const ExpertBanks &b, const float *x, QAct64 xq, 
     if (b.gate_type == T_F32)
         return launch_gemm_f32<true>(b.gate, b.up, x, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden, b.inter, act32,
                                      nullptr, s);
-    // (f16 and bf16 banks read x as halfs: xh.hi alone, from launch_convert_rows_f16)
+    // (f16 and bf16 banks read x as halfs: xh.hi alone, from launch_dispatch's rows or launch_convert_rows_f16)
     if ((b.gate_type == T_F16 || b.gate_type == T_BF16) && xh.hi == nullptr) return hipErrorInvalidValue;
     if (b.gate_type == T_F16)
         return launch_gemm_f16<true, T_F16>(b.gate, b.up, xh.hi, sorted, k_slots, tiles, n_tiles, max_tiles, tile_rows, b.hidden,
