@@ -1,5 +1,5 @@
 // Grouped GEMM of Q8_0 banks on the f16 units for few rows per expert (tiles of 32 rows).  Rows are pairs of halfs (HAct), a code
-// is a half as it is, and a block's 32 products are summed by v_mfma_f32_32x32x16_f16 into one f32 accumulator, hi and lo
+// is a half as it is, and a block's 32 products are summed by v_mfma_f32_16x16x32_f16 into one f32 accumulator, hi and lo
 // halfs alike; what is left for the vector ALUs is one multiply-add per output and block, with the block's scale.
 //
 // What bounds it: the stream of the weights and, not wholly beside it, the CU's own work (with every tile on one expert's weights, out
@@ -8,12 +8,16 @@
 // registers took 237.  Here a stage of a row (128 elements, 136 bytes) comes as the aligned pieces of 16 bytes that hold it, straight into LDS,
 // two stages ahead, the loads dealt over the products of a stage: a burst behind the barrier stalls all waves at the address units.
 // A workgroup fills a CU's LDS, so what it does outside the loop is not hidden by another: it takes several items, and loads for the
-// next while it stores the last.  A piece read by 16 lanes, 9 pieces a row, meets all banks of LDS; codes taken from there by dwords
-// met a quarter.  OLMoE layer, 150 tokens, gate/up + down, us: dwords loaded in a burst 86 + 47; pieces, dealt 80.5 + 45.5; several items 75.2 +
-// 42.5; whole pieces read 74 + 41 (the layer: 152, 147, 142, 139.5; 16 tokens 134 -> 117, 512: 296 -> 255, 1000: 491 -> 412).
+// next while it stores the last.  OLMoE layer, 150 tokens, gate/up + down, us: dwords loaded in a burst 86 + 47; pieces, dealt 80.5 + 45.5; several items 75.2 +
+// 42.5; codes read from LDS by whole pieces, 16 lanes of which meet all banks (so do the dwords of two K groups here), 74 + 41 (the layer: 152, 147, 142,
+// 139.5; 16 tokens 134 -> 117, 512: 296 -> 255, 1000: 491 -> 412).
 // Fetched once: 296 MB of 285.  Tried: half the rows of a stage and two workgroups a CU (84.7 + 60.2: more streams than L2 holds lines
 // for, 385 MB); a wave for one block of a stage and 128 columns, a quarter of the reads of rows (81.1 + 54.8: sums exchanged at the end).
-// Off the 64-bit result by 2.5e-7 where the int8 form is by 4.5e-5.
+// Products of 16 x 16 and 32 of K instead of 32 x 32 and 16, which pass through the accumulators half as often: less power, a higher clock, at four operands a
+// block instead of two.  Layers among others, us, 16 / 64 / 150 / 260 / 512 / 1000 / 2000 tokens 86.8 / 101.8 / 110.9 / 149.8 / 229.8 / 391.5 / 708 -> 85.8 / 100.2 / 108.3 / 146.4 /
+// 224.9 / 379.8 / 689.5.
+// Off the 64-bit result by 2.5e-7 where the int8 form is by 4.5e-5 (four shapes 2.51, 2.49, 2.42, 2.64 e-7 with the larger products, whose high halfs came first; 2.48, 2.47, 2.41,
+// 2.63 here).
 //
 // x has one scale for its whole row (HAct, the largest element lifted to 2^15): an element is off by at most 2^-39 of the row's largest, where
 // the int8 form's is off by 2^-16 of the largest of its block of 64.  That is less for every row but one whose large elements fill blocks of
@@ -23,8 +27,8 @@
 // and 4.8e-5.
 //
 // An item is a tile by 256 weight rows (128 of gate and 128 of up), a wave has 32 of them, which it loads for itself; the activation tile
-// is shared.  Lane (column c, K group g) reads 16 of a block's 32 codes, so element 16 g + 8 kk + i of the block is the K index
-// 8 g + i of its product kk, and the A operands are read from the tile to match.
+// is shared.  Lane (column c, K group g) reads 8 of the 32 codes of a block of columns c and c + 16 each: elements 8 g + i of the block are the K index
+// 8 g + i of its product, and the A operands, rows c and c + 16, are read from the tile to match.
 #include <type_traits>
 
 #include "device_utils.h"
@@ -38,7 +42,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 using namespace q8;
 
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     const int n_items = n_slabs * (total - tile0 < per_xcd ? total - tile0 : per_xcd), apart = (int)(gridDim.x >> 3);
     const int first_item = (int)(blockIdx.x >> 3);
     if (first_item >= n_items) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c = lane & 15, g = lane >> 4, row32 = lane & 31;
     const uint32_t row_bytes = (uint32_t)(in_dim / kStep) * kRowW;
     const uint32_t lds0 = lds_offset(s_lds);
     const uint32_t lds_as = lds_offset(s_as), lds_idx = lds_offset(s_idx);
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
         }
         if (GATE_UP) {
             const int rows = rows_of(w_item);
-            load_to_lds4(lds_idx + (uint32_t)w_flip * 256u, (const uint8_t *)(sorted + start_of(w_item)), (uint32_t)(c < rows ? c : rows - 1) * 4u);
+            load_to_lds4(lds_idx + (uint32_t)w_flip * 256u, (const uint8_t *)(sorted + start_of(w_item)), (uint32_t)(row32 < rows ? row32 : rows - 1) * 4u);
         }
     };
     // Activation pieces: load `wave` of each plane holds four rows.
@@ -117,8 +121,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
     // An item of up to 16 rows has its low halfs' rows behind its high halfs' in one A operand: half the products and row reads, a row's
     // two parts summed at the end.  OLMoE layer, three streams, 16 / 64 / 100 tokens 89.0 / 103.2 / 105.9 -> 86.3 / 100.8 / 104.1 us, 150 (a third of
     // the tiles) the same; off the 64-bit result by 2.43e-7 where one sum for both is by 2.52e-7.
-    const uint32_t a_full = row_read(c, false), a_half = row_read(c, true);
-    uint32_t a_rd = a_full, a_low = row_low(false);   // of the item whose rows are being loaded
+    const uint32_t a_rd0 = row_read(c, false), a_full = row_read(c + 16, false), a_half = row_read(c + 16, true);
+    uint32_t a_rd = a_full, a_low = row_low(false);   // of the item whose rows are being loaded (the first sixteen rows lie where they do either way)
     auto set_a = [&]() {
         const bool few = rows_of(a_item) <= 16;
         a_rd = few ? a_half : a_full, a_low = row_low(few);
@@ -128,7 +132,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
             return (uint32_t)(start_of(a_item) + (r < rows ? r : rows - 1));
         };
         a_off = source_row(a_row) * (uint32_t)in_dim * 2u + (uint32_t)((lane & 15) ^ (a_row & 15)) * 16u;
-        s_off = source_row(c) * (uint32_t)(in_dim / 128) * 4u;
+        s_off = source_row(row32) * (uint32_t)(in_dim / 128) * 4u;
         if (GATE_UP) load_to_lds4(lds_as + (uint32_t)a_flip * 256u, (const uint8_t *)a.scale, s_off);
     };
     auto next_w = [&]() {
@@ -172,59 +176,70 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
 #pragma unroll
     for (int j = 0; j < kWLoads; j++) load_w(kStageW, j);
 
-    const float16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // what a block's products take: 16 codes and the scale, the rows' pieces; of this block and of the next
-    uint32_t v[2][8];
-    float d[2];
+    const f32x4 zero = {0, 0, 0, 0};
+    // what a block's products take: 8 codes and the scale of either column, the rows' pieces; of this block and of the next
+    uint32_t v[2][2][3];
+    float d[2][2];
     half8 hi[2][2], lo[2][2];
-    const uint32_t w_rd = (uint32_t)wave * kWaveW + (uint32_t)c * (16 * PIECES) + (PIECES == 9 ? 0u : (uint32_t)c * row_bytes & 8u);
+    uint32_t w_rd[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) w_rd[j] = (uint32_t)wave * kWaveW + (uint32_t)(c + 16 * j) * (16 * PIECES) + (PIECES == 9 ? 0u : (uint32_t)c * row_bytes & 8u);
     auto read = [&](uint32_t slot, int odd, int which, int blk, uint32_t rd, uint32_t low, bool both) {   // (odd: of the stage, known where PIECES is 9)
-        const uint8_t *ds = s_lds + slot + w_rd + 8u * (uint32_t)odd;
         const int at = 34 * blk + 2, n = blk & 1;
-        if (PIECES == 9) {
-            // (sixteen lanes that read a piece each, rows of 9 pieces apart, meet all banks)
-            const uint8_t *from = s_lds + slot + w_rd + 16u * (uint32_t)g + (uint32_t)((at + 8 * odd) & ~15);
-            __builtin_memcpy(v[n], __builtin_assume_aligned(from, 16), 16);
-            if ((at + 8 * odd) & 15) __builtin_memcpy(v[n] + 4, __builtin_assume_aligned(from + 16, 16), 16);
-        } else {
 #pragma unroll
-            for (int i = 0; i < ((at & 2) ? 5 : 4); i++) v[n][i] = *(const uint32_t *)(ds + 16u * (uint32_t)g + (at & ~3) + 4 * i);
+        for (int j = 0; j < 2; j++) {
+            const uint8_t *ds = s_lds + slot + w_rd[j] + 8u * (uint32_t)odd;
+            // (the dwords of sixteen columns, 9 pieces apart, and two K groups lie in all banks)
+#pragma unroll
+            for (int i = 0; i < ((at & 2) ? 3 : 2); i++) v[n][j][i] = *(const uint32_t *)(ds + 8u * (uint32_t)g + (at & ~3) + 4 * i);
+            d[n][j] = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
         }
-        d[n] = half_bits_to_float(*(const uint16_t *)(ds + 34 * blk));
         const uint8_t *as = s_lds + rows_at(which);
+        const uint32_t piece = row_piece(c, g >> 1, blk, g & 1);
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
-            const uint32_t piece = row_piece(c, g, blk, kk);
-            hi[n][kk] = *(const half8 *)(as + rd + piece);
-            if (both) lo[n][kk] = *(const half8 *)(as + rd + piece + low);
+        for (int m = 0; m < 2; m++) {
+            const uint8_t *from = as + (m == 0 ? a_rd0 : rd) + piece;
+            hi[n][m] = *(const half8 *)from;
+            if (both) lo[n][m] = *(const half8 *)(from + low);
         }
     };
     // a block's sum -> acc, or (down) the 128 elements' sum
-    float16v acc = zero, run = zero, s[2] = {zero, zero};
-    float fd = 0.0f;
+    f32x4 acc[2][2], run[2][2], s[2][2][2];   // [16 rows][16 columns]; s of this block and of the one before
+    float fd[2] = {0.0f, 0.0f};
+    auto clear = [&]() {
+#pragma unroll
+        for (int m = 0; m < 4; m++) acc[m >> 1][m & 1] = run[m >> 1][m & 1] = s[1][m >> 1][m & 1] = zero;
+    };
+    clear();
     auto fold = [&](int n, int blk) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            if (GATE_UP) acc[r] = fmaf(fd, s[n][r], acc[r]);
-            else run[r] = blk == 0 ? __fmul_rn(fd, s[n][r]) : fmaf(fd, s[n][r], run[r]);
-        }
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (GATE_UP) acc[m][j][r] = fmaf(fd[j], s[n][m][j][r], acc[m][j][r]);
+                    else run[m][j][r] = blk == 0 ? __fmul_rn(fd[j], s[n][m][j][r]) : fmaf(fd[j], s[n][m][j][r], run[m][j][r]);
+                }
     };
     // the stage's row scales, read in front of its last barrier: the stage after the next lands in their place
-    float4 sr[4] = {};
+    float4 sr[2] = {};
     auto read_scales = [&](int which, bool half) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) sr[j] = *(const float4 *)&s_as[which][8 * (half ? j & 1 : j) + 4 * g];
+        for (int m = 0; m < 2; m++) sr[m] = *(const float4 *)&s_as[which][(half ? 0 : 16 * m) + 4 * g];
     };
     auto fold_run = [&]() {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float f[4] = {sr[j].x, sr[j].y, sr[j].z, sr[j].w};
+        for (int m = 0; m < 2; m++) {
+            const float f[4] = {sr[m].x, sr[m].y, sr[m].z, sr[m].w};
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[4 * j + i] = fmaf(run[4 * j + i], f[i], acc[4 * j + i]);
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[m][j][r] = fmaf(run[m][j][r], f[r], acc[m][j][r]);
         }
     };
-    // element r of an accumulator: row 8 (r / 4) + 4 g + r % 4, column lane % 32
-    auto acc_row = [&](int r) { return 8 * (r >> 2) + 4 * g + (r & 3); };
+    // element r of acc[m][j]: row 16 m + 4 g + r, column 16 j + c of the wave's
+    auto acc_row = [&](int m, int r) { return 16 * m + 4 * g + r; };
 
     // the first stage is there; its first block
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoads) : "memory");
@@ -251,28 +266,30 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
 #pragma unroll
                     for (int j = 3 * blk - 3; j < 3 * blk && j < kWLoads; j++) load_w(slot2, j);
                 }
-                const float now = d[n];
-                uint32_t q[4];
+                const float now[2] = {d[n][0], d[n][1]};
+                half8 w[2];
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
+                for (int j = 0; j < 2; j++) {
                     // (codes begin two bytes into a dword in every other block)
-                    const int at = 34 * blk + 2, j = i + (PIECES == 9 ? ((at + 8 * odd) & 15) >> 2 : 0);
-                    q[i] = (at & 2) ? __builtin_amdgcn_alignbyte(v[n][j + 1], v[n][j], 2) : v[n][j];
+                    const uint32_t *q = v[n][j];
+                    w[j] = ((34 * blk + 2) & 2) ? q8_codes(__builtin_amdgcn_alignbyte(q[1], q[0], 2), __builtin_amdgcn_alignbyte(q[2], q[1], 2))
+                                                : q8_codes(q[0], q[1]);
                 }
-                const half8 w[2] = {q8_codes(q[0], q[1]), q8_codes(q[2], q[3])};
                 const half8 h[2] = {hi[n][0], hi[n][1]}, l[2] = {lo[n][0], lo[n][1]};
                 if (blk < 3) read(slot, PIECES == 9 ? odd : step & 1, which, blk + 1, rd, row_low(half), !half);
                 else read(slot1, PIECES == 9 ? !odd : step + 1 < n_steps ? (step + 1) & 1 : 0, which ^ 1, 0, a_rd, a_low, true);
 #pragma unroll
-                for (int kk = 0; kk < 2; kk++) {
-                    s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[kk], w[kk], kk == 0 ? zero : s[n], 0, 0, 0);
-                    if (!half) s[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l[kk], w[kk], s[n], 0, 0, 0);
-                }
+                for (int part = half ? 1 : 0; part < 2; part++)   // (the low halfs first: the smaller sum is rounded less often at the size of the larger)
+#pragma unroll
+                    for (int m = 0; m < 2; m++)
+#pragma unroll
+                        for (int j = 0; j < 2; j++)
+                            s[n][m][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(part ? h[m] : l[m], w[j], part == (half ? 1 : 0) ? zero : s[n][m][j], 0, 0, 0);
                 // the block before this one, while these are multiplied
                 fold(n ^ 1, (blk + 3) & 3);
                 if (!GATE_UP && blk == 0) fold_run();
                 if (!GATE_UP && blk == 2) read_scales(which, half);
-                fd = now;
+                fd[0] = now[0], fd[1] = now[1];
             }
             slot = slot1;
             which ^= 1;
@@ -290,13 +307,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
         if (!GATE_UP) fold_run();
         if (rows <= 16) {
 #pragma unroll
-            for (int r = 0; r < 8; r++) acc[r] += acc[r + 8];
+            for (int j = 0; j < 2; j++) acc[0][j] += acc[1][j];
         }
         if (GATE_UP) {
             // (the last stage's weights are read: their place is free until the loads beside the next item's products)
             float *s_c = (float *)(s_lds + (slot == 0 ? (kRing - 1) * kStageW : slot - kStageW));   // [gate, up][row][kRowC]
 #pragma unroll
-            for (int r = 0; r < 16; r++) s_c[((wave >> 2) * kRows + acc_row(r)) * kRowC + 32 * (wave & 3) + c] = __fmul_rn(s_as[flip][acc_row(r)], acc[r]);
+            for (int i = 0; i < 16; i++) {
+                const int m = i >> 3, j = i >> 2 & 1, row = acc_row(m, i & 3);
+                s_c[((wave >> 2) * kRows + row) * kRowC + 32 * (wave & 3) + 16 * j + c] = __fmul_rn(s_as[flip][row], acc[m][j][i & 3]);
+            }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
             for (int pass = 0; pass < kRows / 16; pass++) {
@@ -310,15 +330,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void grouped_gemm_q8_kernel(const u
             }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         } else {
-            const int col = first_of(item) + c;
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (col < out_dim && acc_row(r) < rows) y[(size_t)(p0 + acc_row(r)) * (size_t)out_dim + (size_t)col] = acc[r];
+            for (int i = 0; i < 16; i++) {
+                const int m = i >> 3, j = i & 1, r = i >> 1 & 3, row = acc_row(m, r), col = first_of(item) + 16 * j + c;
+                if (col < out_dim && row < rows) y[(size_t)(p0 + row) * (size_t)out_dim + (size_t)col] = acc[m][j][r];
+            }
         }
-        acc = run = s[1] = zero;
-        fd = 0.0f;
+        clear();
+        fd[0] = fd[1] = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) sr[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int m = 0; m < 2; m++) sr[m] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load into LDS is under way when the workgroup ends)
 }
