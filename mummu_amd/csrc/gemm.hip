@@ -1019,6 +1019,10 @@ int grouped_gemm_tile_rows_q6k_down(const ExpertBanks &b, int n_assign) {
 // that streams its whole weight slab again, so the tile is sized to hold the average expert load
 // plus its spread (binomial: about +-sqrt(avg) per expert, 3.5 sigma here) when that fits; the f16
 // kernel goes up to 128 rows, the int8 kernel (more registers per row) to 64.
+// Banks of 16 bits keep 96 rows until one expert in eight needs a second tile, which costs them less than tiles of 128, whose workgroups hold a third more registers:
+// layers among others, us, 128 / 96 rows, OLMoE 69 / 74 rows an expert 199 / 165, - / 167, 128 experts of 2048 x 768, 71: 300 / 258, 16 of 4096 x 1792, 70: 294 / 284, 8 of 4096 x 1536,
+// 70: 150 / 142; from 79 rows on the wide GEMM takes what has workgroups enough for it (wide_gemm_takes).  Tiles of 32 and 64 rows kept as long (24 and 53 rows an expert): 139 / 140 and 161 / 160 for
+// OLMoE, 214 / 217 and 246 / 249 for the 128 experts, but 181 / 186 and 237 / 270 for the 16.
 int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bool q8_half) {
     const int max_rows = ((grouped_gemm_quantized(b) && !q8_half) || b.gate_type == T_F32) ? 64 : 128;
     const double avg = (double)n_assign / (double)n_experts;
@@ -1026,6 +1030,7 @@ int grouped_gemm_tile_rows(const ExpertBanks &b, int n_assign, int n_experts, bo
     if (want > max_rows) return 64;  // several full tiles per expert whatever the size: 64 rows measured best
     int rows = 32;
     while (rows < want) rows += 32;
+    if (rows == 128 && (b.gate_type == T_F16 || b.gate_type == T_BF16) && avg + 1.2 * __builtin_sqrt(avg) + 1.0 <= 96.0) return 96;
     return rows;
 }
 

@@ -379,15 +379,16 @@ bool wide_gemm_takes(const ExpertBanks &b, int n_tokens, int n_assign) {
           // (a - n_assign and less - over the slots of a token by way of 2^32 / slots: exact while a * slots < 2^32)
           (size_t)n_assign * (size_t)(n_assign / n_tokens) < (1ull << 32)))
         return false;
-    // Up to 64 rows per expert either kernel streams the weights once, and the smaller workgroups of grouped_gemm_f16_kernel,
-    // several to a CU, do it better (this kernel with its loads still in one go; OLMoE layers, 64 rows: 207 us there, 237 us here; 72: 256 / 245, 80: 260 / 249, 128: 325 / 276; 512
-    // experts of 2560 x 640, 64: 1852 / 1907, 72: 2195 / 2018; 128 of 2048 x 768, 64: 366 / 354, 72: 427 / 381; 16 of 4096 x 1792, 64: 411 /
-    // 402, 72: 428 / 417, 128: 568 / 490).
+    // Up to one tile per expert either kernel streams the weights once, and the smaller workgroups of grouped_gemm_f16_kernel, several to a CU, do it
+    // better, on tiles of 96 rows, until too many experts need a second one: at 79 rows one in 35, of evenly drawn ones (layers among others, us, there / here: OLMoE 64 rows 163 / 188, 69: 165 / 188, 74: 167 / 193, 80: 182 / 189, 83: 180 / 189, 86: 193 /
+    // 194, 95: 217 / 199; 128 experts of 2048 x 768, 78 rows 273 / 288, 88: 302 / 298; 16 of 4096 x 1792, 81: 331 / 329, 88: 368 / 343; 64 of 1024 x 512, 72 / 82:
+    // 56 / 62, 59 / 64; 128 of 512 x 512, 72 / 82: 64 / 71, 66 / 74).  Rows of a few steps of K are no stream: 224 experts of 256 x 128, 72 / 80 rows 73 / 71, 81 / 79.
+    const size_t from = b.hidden >= 512 && b.inter >= 512 ? 79 : 72;
     // One workgroup fills a CU here, so the line also asks for about as many of them as there are CUs.  The one smaller launch that
     // was measured on both sides is ahead all the same (8 experts of 4096 x 1536, 96 workgroups, 72 rows 311 / 275, 256: 491 / 484).
     const size_t tiles = (size_t)n_assign / kWideRows > (size_t)b.n_experts ? (size_t)n_assign / kWideRows : (size_t)b.n_experts;
     const size_t out_dim = (size_t)(b.inter * 2 < b.hidden ? b.inter * 2 : b.hidden);
-    return (size_t)n_assign >= 72 * (size_t)b.n_experts && tiles * (out_dim / kWCols) >= 224;
+    return (size_t)n_assign >= from * (size_t)b.n_experts && tiles * (out_dim / kWCols) >= 224;
 }
 
 // Whether the workgroups of a launch are a CU's each and take items in turn, or an item's: where the stream of the weights bounds it, other streams'

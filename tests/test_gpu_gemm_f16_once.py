@@ -41,3 +41,10 @@ def test_one_tile_and_several(kind, counts):
     # x and the activations between the products are halfs: 2^-12 of an element on average of each, twice
     err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert err.max() <= 1e-3
+
+
+# Tiles of 96 rows up to 83 rows an expert on average, experts just below, at and above one and two of them; 128 from there.
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("counts", [(67, 95, 96, 97, 0, 47), (83, 192, 193, 30, 0, 2), (84, 127, 128, 129, 0, 43)])
+def test_tiles_of_96_rows(kind, counts):
+    test_one_tile_and_several(kind, counts)

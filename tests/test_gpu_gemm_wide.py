@@ -101,3 +101,23 @@ def test_several_items_to_a_workgroup_of_few_steps(H, I):
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.F16), ids, w, x)
     assert orc.rel_err(got, want, mag).max() <= 4e-3
     assert (np.linalg.norm(got - want, axis=1) <= 2e-3 * np.linalg.norm(want, axis=1)).all()
+
+
+def test_either_side_of_the_line_from_the_narrow_tiles():
+    """78 rows an expert and 79, of rows of 512 elements: the same rows off the f64 reference by no more than x and the activations as halfs make, on either kernel."""
+    H = I = 512
+    E = 112
+    g = torch.Generator().manual_seed(4)
+    bank = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(torch.float16).view(torch.int16).numpy().view(np.uint16)
+    gate, up, down = bank(E, I, H), bank(E, I, H), bank(E, H, I)
+    n = 79 * E
+    x, ids = torch.randn(n, H, generator=g).numpy(), (np.arange(n, dtype=np.int32) % E)[:, None]
+    w = np.ones((n, 1), np.float32)
+    some = np.arange(0, 78 * E, 97)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, bank(E, H), M.F16, gate, M.F16, up, M.F16, down, M.F16)
+        both = [m.apply_routing(0, ids[:k * E], w[:k * E], x[:k * E])[some] for k in (78, 79)]
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.F16), ids[some], w[some], x[some])
+    for got in both:
+        assert orc.rel_err(got, want, mag).max() <= 4e-3
+        assert (np.linalg.norm(got - want, axis=1) <= 2e-3 * np.linalg.norm(want, axis=1)).all()
