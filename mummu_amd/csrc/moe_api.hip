@@ -522,9 +522,10 @@ struct HalfPlan {
 // Which Q8_0 batches take the 32-row tiles of gemm_q8.hip and which the int8 form's 64-row ones, by the rows of an expert.  Layers of
 // 64 / 128 experts (hidden x inter 2048 x 1024, 2048 x 768), 16 (4096 x 1792) and 512 (2560 x 640, whose rows come in ten pieces), us here / int8:
 //   up to 33 rows next to none needs a second tile: 16 rows 138 / 181, 201 / 273, 232 / 316, 844 / 985; 33: 201 / 218, 291 / 364, 301 / 379, 1279 / 1400.
-//   While a tile of 64 holds every expert the int8 form reads the weights once: 40 rows 207 / 225, 319 / 376, 329 / 419, 1496 / 1509.  A layer on
-//   its own is still faster here, by what the int8 form waits; where other streams fill that (three of them, 64 experts, 37 rows: 179 / 176 a
-//   layer) it is not, and the bytes decide.
+//   While a tile of 64 holds every expert the int8 form reads the weights once: 40 rows 207 / 225, 319 / 376, 329 / 419, 1496 / 1509 on its own, where it waits.
+//   Where other streams fill that (three of them) rows of up to 2048 elements in nine pieces are ahead here to 40 rows (64 experts, 34 / 39 / 43 rows 153 / 171, 171 /
+//   176, 179 / 180; 128 experts, 35 / 42 rows 241 / 258, 275 / 269; 256 of 2048 x 512, 40: 377 / 386; 32 of 1024 x 512, 40: 30 / 34), longer ones are not (16 experts, 35 rows
+//   239 / 233), and the bytes decide.
 //   Beyond, some need a second one: 54 rows 512 experts 1777 / 1841; 64: 257 / 353, 405 / -, 449 / 548, 2142 / 2250; 128: 424 / 512, 670 / -, 636 / 808.
 //   From 190 rows on: 192 rows 572 / 665, 934 / 1066, 951 / 1062; 512: 1361 / 1462, -, 2208 / 2331 (three streams 1400 / 1399), a hundred times nearer the
 //   64-bit result (but for rows with a block of 64 that is more than 2^24 above the rest and meets weights of 0, where one scale a row keeps less
@@ -533,7 +534,7 @@ bool q8_gemm_should(const ExpertBanks &b, size_t n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const size_t workgroups = (size_t)b.n_experts * (size_t)(b.inter / 128);   // of a gate/up launch with a tile per expert
     const bool nine_pieces = b.hidden % 256 == 0 && b.inter % 256 == 0;
-    return avg <= 33.0 || (avg + (workgroups <= 1024 ? 3.2 : 2.2) * __builtin_sqrt(avg) >= 64.0 && (avg <= 190.0 || nine_pieces));
+    return avg <= (nine_pieces && b.hidden <= 2048 ? 40.0 : 33.0) || (avg + (workgroups <= 1024 ? 3.2 : 2.2) * __builtin_sqrt(avg) >= 64.0 && (avg <= 190.0 || nine_pieces));
 }
 
 // (one_expert: all n rows go to the same one)

@@ -159,3 +159,19 @@ def test_tiles_of_up_to_16_rows_match_the_f64_reference(H, I):
     want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids, w, x)
     assert orc.rel_err(got, want, mag).max() <= 3e-5
     assert np.linalg.norm(got - want) <= 3e-6 * np.linalg.norm(want)
+
+
+# The same for rows whose pieces begin at multiples of 16 bytes, which take pairs of halfs to 40 rows an expert, and from where a tile of 64 is too small.
+@pytest.mark.parametrize("H,rows,pairs", [(256, 34, True), (256, 40, True), (256, 41, False), (256, 45, True), (2304, 33, True), (2304, 34, False)])
+def test_the_form_by_rows_per_expert_and_their_length(H, rows, pairs):
+    E, I, n = 8, 256, 8 * rows
+    gate, up = (synth.random_bank_fast(M.Q8_0, [H, I, E], seed) for seed in (1, 2))
+    down = synth.random_bank_fast(M.Q8_0, [I, H, E], 3)
+    x = np.random.default_rng(rows).standard_normal((n, H)).astype(np.float32)
+    ids, w = (np.arange(n, dtype=np.int32) % E)[:, None], np.ones((n, 1), np.float32)
+    with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
+        m.load_layer(0, np.zeros((E, H), np.float16), M.F16, gate, M.Q8_0, up, M.Q8_0, down, M.Q8_0)
+        got = m.apply_routing(0, ids, w, x)[:E]
+    want, _ = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.Q8_0), ids[:E], w[:E], x[:E])
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= 2e-3 and (err <= 3e-6) == pairs, err
