@@ -23,7 +23,7 @@
 //     the results of the last.
 //   - What a lane keeps from item to item - offsets of rows - has to stay in registers: reloaded ones are waited for in the loop, behind every load
 //     that is under way (bf16, 4096 tokens 492 -> 558).
-// What remains: the matrix units are busy for 60 / 46 % of the cycles at 4096 bf16 rows x 8.
+// What remains: the matrix units are busy for 53 / 37 % of the cycles at 4096 bf16 rows x 8.
 #include <type_traits>
 
 #include "device_utils.h"
