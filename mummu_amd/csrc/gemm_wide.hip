@@ -27,26 +27,19 @@
 #include <type_traits>
 
 #include "device_utils.h"
+#include "gemm_wide_ring.h"
 #include "kernels.h"
 
 namespace mummu {
 
 namespace {
 
+using namespace wide;
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kWK = 64;                          // K elements of a stage: a line of 128 bytes per row, eight pieces of 16
-constexpr int kWCols = 256;                      // weight rows of a tile
-constexpr int kWStageB = kWCols * kWK * 2;       // bytes of a stage of weights
-// Stages in LDS, for tiles of 64 MW rows: of the weights, then two of the activations.
-template <int MW>
-struct Ring {
-    static constexpr int kB = MW <= 4 ? 3 : 2, kStageA = 64 * MW * kWK * 2, kAtA = kB * kWStageB;
-    static_assert(kAtA + 2 * kStageA <= 160 * 1024, "the stages fit the LDS");
-};
-constexpr int kWLds = Ring<4>::kAtA + 2 * Ring<4>::kStageA;
 static_assert(kWideRows == 64 * 5 && Ring<5>::kAtA + 2 * Ring<5>::kStageA <= kWLds, "... all of them");
 
 template <int WT>
@@ -163,7 +156,7 @@ struct Loader {
     __device__ void begin(int mw, uint32_t lds0, uint32_t row_bytes, int wave) {
         const uint32_t lds_a = lds0 + (mw <= 4 ? Ring<4>::kAtA : Ring<5>::kAtA);
 #pragma unroll
-        for (int step = 0; step < 2; step++) {
+        for (int step = 0; step < kBegun; step++) {
 #pragma unroll
             for (int i = 0; i < 4; i++) load_b<GATE_UP>(lds0 + step * kWStageB, step, row_bytes, wave, i);
 #pragma unroll
@@ -212,7 +205,7 @@ __device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, int
     // Behind the barrier of a step, beside its last products, the rows of the step after the next are asked for; beside the first
     // products after that the weights of one step more (tiles of more than 256 rows leave no room for that: of the same step).  All at once
     // they fill the address unit's queue, and every wave stands before it.
-    constexpr int kAhead = R::kB == 3 ? 2 : 1;
+    constexpr int kAhead = R::kAhead;
     const uint32_t lds_a = lds0 + R::kAtA;
     asm volatile("s_barrier" ::: "memory");
 #pragma unroll
@@ -248,13 +241,12 @@ __device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, int
             if (behind_barrier == 0) {
                 if (LEFT == 1 && tid == 0) *told = taken;
                 // (In an item's first step the stores of the one before, eight to 64 of its rows, stand behind the stage that is waited for.)
-                if (LEFT == 0) wait_and_meet<kAhead == 2 ? 63 : 0>();
-                else if (FIRST && behind == 1) wait_and_meet<8>();
-                else if (FIRST && behind == 2) wait_and_meet<16>();
-                else if (FIRST && behind == 3) wait_and_meet<24>();
-                else if (FIRST && behind == 4) wait_and_meet<32>();
-                else if (FIRST && behind == 5) wait_and_meet<40>();
-                else wait_and_meet<kAhead == 2 && LEFT == 2 ? 4 : 0>();
+                if (FIRST && behind == 1) wait_and_meet<step_wait(kAhead, LEFT, 1)>();
+                else if (FIRST && behind == 2) wait_and_meet<step_wait(kAhead, LEFT, 2)>();
+                else if (FIRST && behind == 3) wait_and_meet<step_wait(kAhead, LEFT, 3)>();
+                else if (FIRST && behind == 4) wait_and_meet<step_wait(kAhead, LEFT, 4)>();
+                else if (FIRST && behind == 5) wait_and_meet<step_wait(kAhead, LEFT, 5)>();
+                else wait_and_meet<step_wait(kAhead, LEFT, 0)>();
             }
             // Rows kEnd units ahead; the stage's last two together, so that the barrier's wait for them is short
             if (u < kUnits - kEnd - 1) a[u + kEnd] = read_a(at_a, u + kEnd);
@@ -274,7 +266,7 @@ __device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, int
 #pragma unroll
                 for (int i = behind_barrier; i < MW; i += kEnd) l.load_a(lds_a + at_a, step + 2, MW, wave, i);
             }
-            if (half == 0 && LEFT >= kAhead) {
+            if (half == 0 && asks_weights(kAhead, LEFT, FIRST)) {
 #pragma unroll
                 for (int i = m; i < 4; i += kBlocks) l.template load_b<GATE_UP>(lds0 + free_b, step + kAhead, row_bytes, wave, i);
             }
@@ -329,7 +321,7 @@ __device__ inline Item wide_tile(const WideArgs &p, const Item t, Loader &l, int
             }
         }
     // The first stage, in front of the second's five loads or more and the stores.
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(8 * MW + 5) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(begin_wait(MW)) : "memory");
     behind = MW;
     return next;
 }
@@ -345,7 +337,7 @@ __global__ __launch_bounds__(512, 2) void wide_gemm_kernel(WideArgs p) {
     const int mw0 = (t.rows + kWideUnit - 1) / kWideUnit;
     l.rows_of<GATE_UP>(p, t, mw0);
     l.begin<GATE_UP>(mw0, lds_offset(s_lds), (uint32_t)p.in_dim * 2u, uniform((int)threadIdx.x >> 6));
-    asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(begin_wait(0)) : "memory");
     while (t.rows > 0) {
         switch ((t.rows + kWideUnit - 1) / kWideUnit) {
         case 1: t = wide_tile<GATE_UP, WT, 1>(p, t, l, behind, s_lds); break;
