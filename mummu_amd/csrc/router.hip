@@ -15,6 +15,7 @@
 #include "device_utils.h"
 #include "kernels.h"
 #include "route_common.h"
+#include "router_lines.h"
 
 MUMMU_TRACE_UNIT(router)
 
@@ -272,10 +273,7 @@ hipError_t launch_router_logits(const float *x, const void *w, int wtype, float 
     if (norm_gamma && !router_logits_can_norm(x, w, norm_gamma, n, hidden)) return hipErrorInvalidValue;
     if (xnorm_out && (!norm_gamma || ((uintptr_t)xnorm_out & 15))) return hipErrorInvalidValue;
     const bool vec = (hidden % 8 == 0) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)w & 15) == 0);
-    // The matrix units from 128 workgroups of 16 tokens by 64 experts on, whose one round takes 19 us whatever their number (2048 elements, more in
-    // proportion), and half of that again what the tiles below take for as many: us of those / of the matrix units, 128 experts of 2048, 600 tokens 14 / 19
-    // (76 workgroups), 2000: 40 / 21, 4096: 78 / 41; 512 experts of 2560, 150 tokens 16 / 23 (80), 300: 29 / 24 (152), 1024: 75 / 45.
-    if (n > 8 && xq.hi == nullptr && !norm_gamma && router_matrix_takes(x, w, hidden) && (long long)((n + 15) / 16) * ((n_experts + 63) / 64) > 128)
+    if (n > 8 && xq.hi == nullptr && !norm_gamma && router_matrix_takes(x, w, hidden) && router_matrix_should(n, n_experts))
         return launch_router_matrix(x, w, wtype, n, hidden, n_experts, 1, 0, 0, logits, nullptr, nullptr, nullptr, nullptr, false, s);
     if (n > 8 && vec && xq.hi == nullptr && !norm_gamma && hidden % 512 == 0 && hidden <= kTileMaxHidden) {
         // (Also a dozen workgroups are no slower than a launch of router_logits_kernel: us of that / of the tiles, 2048 elements, 8 experts, 9 / 32 / 300

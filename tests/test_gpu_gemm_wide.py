@@ -24,7 +24,7 @@ def test_every_tile_edge_matches_the_f64_reference(dtype):
     ids = np.repeat(np.arange(E), counts)
     ids = ids[np.random.default_rng(3).permutation(len(ids))].astype(np.int32)[:, None]
     n = len(ids)
-    assert n >= 72 * E, "the batch is too small to be served by the wide kernel"
+    assert n >= 79 * E, "the batch is too small to be served by the wide kernel"
     x = torch.randn(n, H, generator=g).numpy()
     w = torch.rand(n, 1, generator=g).numpy()
     with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
@@ -80,27 +80,46 @@ def test_infinite_gates_come_out_as_in_the_narrow_kernel():
         assert np.isfinite(np.delete(got, (5, 6), 0)).all()
 
 
-@pytest.mark.parametrize("H, I", [(256, 128), (320, 192)], ids=["4 and 2 steps of K", "5 and 3"])
-def test_several_items_to_a_workgroup_of_few_steps(H, I):
-    """More items than CUs, each height of a tile behind each other, with as few steps of K as the kernel takes and one more: what an
-    item's first stages and the stores before them find in LDS and in the counters.  Bounds as above."""
-    E = 480
-    counts = np.random.default_rng(11).permutation(np.resize([1, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321, 0, 0, 0, 3, 2], E))
+def few_steps(H, I, dtype, counts):
+    """A batch of `counts` rows per expert on banks of a few steps of K, the same bits six times over; bounds as above."""
+    E, n = len(counts), int(np.sum(counts))
     ids = np.random.default_rng(5).permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
-    n = len(ids)
-    assert n >= 72 * E
+    torch_t, t, ot = (torch.float16, M.F16, orc.F16) if dtype == "f16" else (torch.bfloat16, M.BF16, orc.BF16)
     g = torch.Generator().manual_seed(9)
-    bank = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(torch.float16).view(torch.int16).numpy().view(np.uint16)
+    bank = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(torch_t).view(torch.int16).numpy().view(np.uint16)
     gate, up, down = bank(E, I, H), bank(E, I, H), bank(E, H, I)
     x, w = torch.randn(n, H, generator=g).numpy(), torch.rand(n, 1, generator=g).numpy()
     with M.SparseMoe(M.SparseMoeConfig(H, I, E, 1), max_tokens=n) as m:
-        m.load_layer(0, bank(E, H), M.F16, gate, M.F16, up, M.F16, down, M.F16)
+        m.load_layer(0, bank(E, H), t, gate, t, up, t, down, t)
         got = m.apply_routing(0, ids, w, x)
         for _ in range(5):
             assert np.array_equal(got.view(np.uint32), m.apply_routing(0, ids, w, x).view(np.uint32))
-    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, orc.F16), ids, w, x)
+    want, mag = orc.moe_ref_f64(orc.LayerBanks(H, I, E, gate, up, down, ot), ids, w, x)
     assert orc.rel_err(got, want, mag).max() <= 4e-3
     assert (np.linalg.norm(got - want, axis=1) <= 2e-3 * np.linalg.norm(want, axis=1)).all()
+
+
+FEW_STEPS = pytest.mark.parametrize("H, I", [(256, 128), (320, 192)], ids=["4 and 2 steps of K", "5 and 3"])
+
+
+@FEW_STEPS
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_several_items_to_a_workgroup_of_few_steps(H, I, dtype):
+    """More items than CUs, each height of a tile behind each other, with as few steps of K as the kernel takes and one more: what an
+    item's first stages and the stores before them find in LDS and in the counters."""
+    counts = np.random.default_rng(11).permutation(np.resize([1, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321, 500, 640, 641, 900, 3, 0], 256))
+    tiles = int(((counts + 319) // 320).sum())
+    assert counts.sum() // 256 >= len(counts), "too few rows per expert for workgroups that take items in turn"
+    assert tiles > 8 * 32 + 64, "too few items for every XCD's workgroups to take a second one"
+    few_steps(H, I, dtype, counts)
+
+
+@FEW_STEPS
+def test_an_item_to_a_workgroup_of_few_steps(H, I):
+    """The same heights and steps with fewer rows per expert, where every workgroup has one item."""
+    counts = np.random.default_rng(11).permutation(np.resize([1, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321, 0, 0, 0, 3, 2], 480))
+    assert 72 * len(counts) <= counts.sum() < 256 * len(counts)
+    few_steps(H, I, "f16", counts)
 
 
 def test_either_side_of_the_line_from_the_narrow_tiles():
