@@ -43,8 +43,8 @@ def test_one_tile_and_several(kind, counts):
     assert err.max() <= 1e-3
 
 
-# Tiles of 96 rows up to 83 rows an expert on average, experts just below, at and above one and two of them; 128 from there.
+# Tiles of 96 rows up to 84 rows an expert on average (504 of six; 505 are past the line), experts just below, at and above one and two of them; 128 from there.
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
-@pytest.mark.parametrize("counts", [(67, 95, 96, 97, 0, 47), (83, 192, 193, 30, 0, 2), (84, 127, 128, 129, 0, 43)])
+@pytest.mark.parametrize("counts", [(67, 95, 96, 97, 0, 47), (83, 192, 193, 30, 0, 2), (84, 191, 96, 97, 0, 36), (84, 191, 96, 97, 0, 37), (84, 127, 128, 129, 0, 43)])
 def test_tiles_of_96_rows(kind, counts):
     test_one_tile_and_several(kind, counts)

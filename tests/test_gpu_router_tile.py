@@ -38,7 +38,8 @@ def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
 # Batches of up to 128 experts on either side of the line from which they take these tiles and a launch for the routing: the oracle's routing
 # bit for bit, every row served counted once.
 @pytest.mark.parametrize("E,n", [(128, 256), (128, 257), (65, 300), (64, 300), (128, 2100),
-                                 (64, 2048), (64, 2049), (33, 2065), (32, 2100), (50, 4096)])   # (on the matrix units with the routing behind)
+                                 # (33 to 64 experts from 1025 tokens: on the matrix units with the routing behind)
+                                 (64, 2048), (64, 2049), (33, 2065), (32, 2100), (50, 4096)])
 def test_routing_and_hits_of_a_batch(E, n):
     H, I, k = 512, 64, 2
     rng = np.random.Generator(np.random.PCG64(E + n))
@@ -62,6 +63,31 @@ def test_routing_and_hits_of_a_batch(E, n):
 @pytest.mark.parametrize("E,n", [(64, 1024), (64, 1025), (33, 1030), (32, 1030), (50, 1537)])
 def test_routing_at_the_line_to_the_matrix_units(E, n):
     test_routing_and_hits_of_a_batch(E, n)
+
+
+# The matrix units with the routing behind, of two to eight chunks of 512 elements (a quarter of 16 rows in LDS at a time), every router type, few slots and
+# more than the sixteen that the short ranking takes.
+@pytest.mark.parametrize("H,E,n,k", [(1024, 64, 1030, 33), (1536, 33, 1025, 8), (2048, 64, 1041, 8), (2560, 50, 1039, 50), (4096, 64, 1040, 17)])
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_routing_behind_several_chunks(H, E, n, k, kind):
+    rng = np.random.Generator(np.random.PCG64(H + E + n))
+    w32 = rng.standard_normal((E, H), dtype=np.float32) * np.float32(0.05)
+    if kind == "f16":
+        w, t, ot = w32.astype(np.float16), M.F16, orc.F16
+    elif kind == "bf16":
+        w = (w32.view(np.uint32) >> 16).astype(np.uint16)
+        t, ot = M.BF16, orc.BF16
+    else:
+        w, t, ot = w32, M.F32, orc.F32
+    x = rng.standard_normal((n, H), dtype=np.float32)
+    bank = synth.random_bank_fast(M.Q8_0, [H, 64, E], 1)
+    with M.SparseMoe(M.SparseMoeConfig(H, 64, E, k), max_tokens=n) as m:
+        m.load_layer(0, w, t, bank, M.Q8_0, bank, M.Q8_0, synth.random_bank_fast(M.Q8_0, [64, H, E], 2), M.Q8_0)
+        m.forward(x, k, True)
+        ids, weights = m.last_routing(n, k)
+    oids, ow = orc.route_olmoe(orc.router_logits(x, w, ot, E), n, E, k, True)
+    assert np.array_equal(ids, oids.astype(np.int32).reshape(n, k))
+    assert np.array_equal(weights.view(np.uint32), ow.reshape(n, k).view(np.uint32))
 
 
 # A token whose row holds an infinity or a NaN is refused, on either side of the line to the matrix units.
