@@ -37,8 +37,9 @@ constexpr int kDispatchWaves = kDispatchThreads / 64;
 constexpr int kDispatchMaxExperts = 512;
 
 // Workgroup b of n_b of a launch makes its share of the rows that the products read.  Nothing of the sort waits for it, and the launch of its own that
-// it had took as long as the sort's first one (layers among others, us: 512 f16 tokens 178 -> 171, 300 of 512 experts with int8 downs 415 -> 402, 320 of
-// Q8_0 189 -> 184, 300 of Q4_K 127 -> 125, 1000: 268 / 269).
+// it had took as long as the sort's first one: 2 to 6 us of a layer alone; among others, which fill the launch's gaps, up to 4 (a launch of its own / here, among others and
+// (alone), us: 320 tokens of Q8_0 180 / 176 (196 / 193), 512 of f16 163 / 163 (174 / 171), 300 of 512 experts with int8 downs 393 / 394 (438 / 432), 300 of Q4_K 104.6 / 103.7
+// (125.6 / 122.5), 1000: 260 / 261 (298 / 297), 4096 of bf16 500 / 499 (532 / 530)).
 __device__ inline void rows_part(const RowsJob &job, int b, int n_b) {
     __shared__ float s_max[kDispatchWaves];
     const int tid = threadIdx.x;

@@ -981,8 +981,8 @@ static int tiles_of_8_or_16(const ExpertBanks &b, int n_assign) {
     return gemm_stream_takes(b.hidden, b.inter, 8) && !second_round && e8 < 1.03 * e16 ? 8 : 16;
 }
 
-// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles of up to 32 rows cost what they
-// have).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
+// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles cost what they
+// have in steps of 16; the figures are those of its form in steps of 32, which the lines were drawn by).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
 // variance = mean).  Layers, 16 / 64 rows, us: in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it
 // weighs: 128 experts of 2048 x 768, 128 tokens 127 / 155, 160: 145 / 158, 208 (1.17 tiles an expert): 148 / 159, 240 (1.4): 162 / 161.  Where a
 // tile per expert fills the chip exactly once, the first second tiles start a second round: OLMoE, 24 tokens 76 / 92, 60: 77 / 93, 64: 96 / 93,

@@ -23,7 +23,9 @@
 //     the results of the last.
 //   - What a lane keeps from item to item - offsets of rows - has to stay in registers: reloaded ones are waited for in the loop, behind every load
 //     that is under way (bf16, 4096 tokens 492 -> 558).
-// What remains: the matrix units are busy for 53 / 37 % of the cycles at 4096 bf16 rows x 8.
+// What remains: the matrix units are busy for 54 / 37 % of the cycles at 4096 bf16 rows x 8, and an XCD's L2 fetches more than
+// the operands hold, 830 / 406 MB of 554 and 336 (the form on 32 x 32 x 16 products, with items of its own to each workgroup, 755 / 354; an item to a workgroup here 817 /
+// 412, so that it is not the order of the items; the cause is not known).
 #include <type_traits>
 
 #include "device_utils.h"

@@ -3,11 +3,11 @@
 
 namespace mummu {
 
-// The logits of n tokens: from 128 workgroups of 16 tokens by 64 experts on, whose one round takes 19 us whatever their number (2048 elements, more in
-// proportion), and half of that again what router_tile_kernel takes for as many: us of that / of the matrix units, 128 experts of 2048, 600 tokens 14 / 19
-// (76 workgroups), 2000: 40 / 21, 4096: 78 / 41; 512 experts of 2560, 150 tokens 16 / 23 (80), 300: 29 / 24 (152), 1024: 75 / 45.
+// The logits of n tokens: from 128 workgroups of 16 tokens by 64 experts on, whose one round takes 21 to 24 us whatever their number (2048 elements, more in
+// proportion), which is what router_tile_kernel takes for as many: us of that / of the matrix units, a launch among those of its layer, 128 experts of 2048, 600 tokens
+// 14 / 21 (76 workgroups), 1025: 23 / 21, 2000: 38 / 24, 4096: 61 / 44; 512 experts of 2560, 150 tokens 14 / 23 (80), 300: 26 / 25 (152), 1024: 65 / 48.
 // ... while experts fill two thirds of the tiles' columns: a round takes the same for a tile with one expert in it, router_tile_kernel what its experts are.
-// On their own, 2048 elements (by events, the matrix units' round 24 us): 8 experts 2049 / 4096 tokens 10 / 26, 16 / 28; 16: 11 / 26, 17 / 28; 32: 16 / 26, 27 / 30; 48: 22 / 25,
+// Calls of the routing alone, 2048 elements (between two copies, a tenth more than in a layer): 8 experts 2049 / 4096 tokens 10 / 26, 16 / 28; 16: 11 / 26, 17 / 28; 32: 16 / 26, 27 / 30; 48: 22 / 25,
 // 36 / 31; 65 at 1025 / 2049 / 4096 tokens 17 / 25, 29 / 46, 44 / 51; 80: 18 / 25, 30 / 46, 48 / 52; 96: 21 / 25, 35 / 46, 54 / 51.  Layers of 2048 x 768, among others and (alone),
 // where the matrix units leave other streams some of the chip: 72 experts, 2049 tokens 408 / 403 (438 / 451), 3000: 581 / 578 (609 / 617), 4096: 766 / 769 (790 / 796); 96
 // experts 2049: 422 / 410 (453 / 463), 3000: 594 / 588 (621 / 622), 4096: 781 / 783 (804 / 799).

@@ -7,10 +7,10 @@
 // bits of the fmaf chain, and adding up the partials is left to the vector ALUs.
 //
 // What bounds it: the instructions.  A product has 32 clocks for its 1024 multiply-adds (the vector ALUs need 64); the four sums
-// and the conversion that go with one follow it rather than run beside it, 53 clocks together.  4096 tokens, 64 experts of 2048:
-// 48 -> 25 us with the routing; 1024 tokens, 512 experts of 2560: 75 -> 45 us; a step's rows read from LDS a step ahead 5 % less (under a profiler 38.5 ->
-// 36.6).  With the tokens' rows read from the caches by every
-// wave instead of once into LDS 30 and 61.
+// and the conversion that go with one follow it rather than run beside it, 53 clocks together.  The streaming form or the
+// tiles (router.hip) -> here, a launch among those of its layer: 4096 tokens, 64 experts of 2048, with the routing 40 -> 26 us, 1024 tokens, 512 experts of 2560 65 -> 48
+// (a kernel trace has 53 -> 35 and 82 -> 60).  A step's rows read from LDS a step ahead 5 % less; with the tokens' rows read from the caches by every wave instead
+// of once into LDS a fifth and a third more.
 #include "device_utils.h"
 #include "kernels.h"
 #include "route_common.h"
