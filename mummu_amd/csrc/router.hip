@@ -650,12 +650,7 @@ hipError_t launch_router_fused(const float *x, const void *w, int wtype, int n, 
     if (n_experts > 128 || k > n_experts || k < 1) return hipErrorInvalidValue;
     if (xq.hi != nullptr && hidden % 64 != 0) return hipErrorInvalidValue;
     const bool vec = (hidden % 8 == 0) && (((uintptr_t)x & 15) == 0) && (((uintptr_t)w & 15) == 0);
-    // The matrix units (router_matrix.hip), 16 tokens to a workgroup, one round of which takes 23 to 26 us up to 4096 tokens: 64 experts of 2048, 1000 / 1025 / 1500 /
-    // 2000 / 2100 / 4096 tokens 15 / 19 / 24 / 26 / 38 / 40 us in the streaming form, fewer experts in proportion.  Beside other streams, which have the CUs that it
-    // leaves, they are ahead from some 400 tokens on; the line is where 64 experts lose little on their own.  Layers of f16 banks, streaming / here, among others and (alone),
-    // 1025 / 2048 / 4096 tokens: 64 experts 209 / 206 (246 / 249), 309 / 298 (339 / 336), 509 / 500 (551 / 536); 48: 172 / 169 (217 / 224), 295 / 290 (328 / 331), 501 /
-    // 497 (524 / 518); 33: 165 / 162 (241 / 253), 273 / 269 (338 / 346), 487 / 488 (552 / 551).  (A tile's 64 columns want more than 32 experts.)
-    if (xh.hi == nullptr && xq.hi == nullptr && n > 1024 && n_experts > 32 && n_experts <= 64 && router_matrix_takes(x, w, hidden))
+    if (xh.hi == nullptr && xq.hi == nullptr && router_matrix_routes(n, n_experts, hidden) && router_matrix_takes(x, w, hidden))
         return launch_router_matrix(x, w, wtype, n, hidden, n_experts, k, flavour, norm, logits, ids, weights, hits, flags, true, s);
     // enough tokens to fill the chip with independent waves: activations in registers, weight
     // rows streamed (on this path the caller quantizes x separately)

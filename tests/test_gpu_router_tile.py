@@ -38,7 +38,7 @@ def test_logits_match_the_oracle_bit_for_bit(H, E, n, kind):
 # Batches of up to 128 experts on either side of the line from which they take these tiles and a launch for the routing: the oracle's routing
 # bit for bit, every row served counted once.
 @pytest.mark.parametrize("E,n", [(128, 256), (128, 257), (65, 300), (64, 300), (128, 2100),
-                                 # (33 to 64 experts from 1025 tokens: on the matrix units with the routing behind)
+                                 # (57 to 64 experts from 1025 tokens, 33 to 56 from 2049: on the matrix units with the routing behind)
                                  (64, 2048), (64, 2049), (33, 2065), (32, 2100), (50, 4096)])
 def test_routing_and_hits_of_a_batch(E, n):
     H, I, k = 512, 64, 2
@@ -60,14 +60,14 @@ def test_routing_and_hits_of_a_batch(E, n):
 
 # The routing of 33 to 64 experts on either side of the line to the matrix units, and of few more tokens than a workgroup's: both forms sum a
 # logit in the same order, so no bit of the routing may differ.
-@pytest.mark.parametrize("E,n", [(64, 1024), (64, 1025), (33, 1030), (32, 1030), (50, 1537)])
+@pytest.mark.parametrize("E,n", [(64, 1024), (64, 1025), (33, 1030), (32, 1030), (50, 1537), (56, 1025), (57, 1025), (56, 2048), (56, 2049)])
 def test_routing_at_the_line_to_the_matrix_units(E, n):
     test_routing_and_hits_of_a_batch(E, n)
 
 
 # The matrix units with the routing behind, of two to eight chunks of 512 elements (a quarter of 16 rows in LDS at a time), every router type, few slots and
 # more than the sixteen that the short ranking takes.
-@pytest.mark.parametrize("H,E,n,k", [(1024, 64, 1030, 33), (1536, 33, 1025, 8), (2048, 64, 1041, 8), (2560, 50, 1039, 50), (4096, 64, 1040, 17)])
+@pytest.mark.parametrize("H,E,n,k", [(1024, 64, 1030, 33), (1536, 57, 1025, 8), (1536, 33, 2049, 8), (2048, 64, 1041, 8), (2560, 50, 1039, 50), (4096, 64, 1040, 17)])
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 def test_routing_behind_several_chunks(H, E, n, k, kind):
     rng = np.random.Generator(np.random.PCG64(H + E + n))
