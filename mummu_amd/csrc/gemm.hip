@@ -981,16 +981,16 @@ static int tiles_of_8_or_16(const ExpertBanks &b, int n_assign) {
     return gemm_stream_takes(b.hidden, b.inter, 8) && !second_round && e8 < 1.03 * e16 ? 8 : 16;
 }
 
-// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles cost what they
-// have in steps of 16; the figures are those of its form in steps of 32, which the lines were drawn by).  By the expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation,
-// variance = mean).  Layers, 16 / 64 rows, us: in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it
-// weighs: 128 experts of 2048 x 768, 128 tokens 127 / 155, 160: 145 / 158, 208 (1.17 tiles an expert): 148 / 159, 240 (1.4): 162 / 161.  Where a
-// tile per expert fills the chip exactly once, the first second tiles start a second round: OLMoE, 24 tokens 76 / 92, 60: 77 / 93, 64: 96 / 93,
-// 96: 97 / 95, 112 (1.27): 96 / 97.  Lists of 32 rows gained nothing between the two (96 tokens 94, 256: 132 against 129, 1000: 331 against
-// 302).
-// With the down product on the int8 units (int8_down) a launch of 32-row tiles costs 0.69 of one of 64-row tiles, both
-// products together: the 512-expert shape with Q5_1 downs, 1000 tokens: 788 / 1013 us.  One of 16-row tiles costs 0.7 of that, unless it is
-// the first second tiles that start a second round: 520 / 600 / 680 / 760 tokens, 16 / 32 rows 479 / 537, 489 / 546, 516 / 557, 547 / 570.
+// Tile rows for the f16-unit Q4_K kernels: 8, 16 (gemm_stream.hip, gemm_q4k_few.hip) or up to 64 (gemm_q4k.hip, whose tiles cost what they have in steps of 16).  By the
+// expected number of tiles when an expert's rows are spread like a binomial around the average (normal approximation, variance = mean).  Layers, 16 / 64 rows, us among
+// others and (alone): in a launch of several rounds of workgroups (two to a CU) a second tile for some costs what it weighs: 128 experts of 2048 x 768, 128 tokens 93 / 105
+// (126 / 146), 160: 99 / 108 (144 / 150), 208 (1.17 tiles an expert): 109 / 114 (146 / 159), 240 (1.35): 121 / 118 (163 / 163), 280: 129 / 119 (172 / 168).  Where a tile per
+// expert fills the chip exactly once, the first second tiles start a second round, which a layer alone waits for: OLMoE, 24 tokens 54 / 64 (76 / 82), 60: 62 / 68 (96 / 90), 64: 62 /
+// 68 (97 / 89), 96: 65 / 70 (103 / 91), 112 (1.25): 70 / 73 (102 / 94), 128: 79 / 75 (104 / 97).  Lists of 32 rows gain nothing between the two (96 tokens 71 (91), 256: 106 (138)
+// against 95 (120)).
+// With the down product on the int8 units (int8_down) tiles of 32 rows are ahead of those of 64, whose int8 form multiplies all of them: the 512-expert shape with Q5_1 downs, 1000
+// tokens: 561 / 655 (599 / 699).  Tiles of 16 rows are until a third of the experts need a second one (the line: 0.43 of them), unless it is the first second tiles that start a second round: 520 / 600 / 680 /
+// 760 / 840 tokens, 16 / 32 rows 429 / 471, 450 / 486, 474 / 498, 512 / 511, 552 / 526.  (0.69 and 0.7 were drawn by layers alone of the forms before, 788 / 1013 and 547 / 570 at 760.)
 int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8_down) {
     const int n_experts = b.n_experts;
     const double avg = (double)n_assign / (double)(n_experts > 0 ? n_experts : 1);
@@ -1001,10 +1001,11 @@ int grouped_gemm_tile_rows_q4k_f16(const ExpertBanks &b, int n_assign, bool int8
     return !second_round && e16 < 1.25 * e64 ? tiles_of_8_or_16(b, n_assign) : 64;
 }
 
-// With a Q6_K down product on the f16 units, whose 32-row form multiplies tiles of 16 as well.  us a layer by tiles of 16 / 32 / 64 rows, OLMoE
-// shape, 128 experts of 2048 x 768 and 16 of 4096 x 1792: 8 rows per expert 101 / 112 / 129, 159 / 175 / 196, 94 / 107 / 121; 16 rows - / 118 / 132,
-// - / 183 / 206, - / 202 / 218; 18: - / 149 / 139, - / 193 / 214, - / 204 / 219; 38 (the first alone): 227 / 197 / 168.  Tiles of 16 as long as next to no
-// expert needs two, and no launch a second round of workgroups for them (10 rows: 128 / 112, 180 / 178, 237 / 200).
+// With a Q6_K down product on the f16 units, whose 32-row form multiplies tiles of 16 as well.  us a layer among others by tiles of 16 / 32 / 64 rows and (alone), OLMoE
+// shape, 128 experts of 2048 x 768 and 16 of 4096 x 1792: 8 rows per expert 76 / 85 / 99 (100 / 105 / 122), 118 / 129 / 150 (151 / 173 / 195), 72 / 76 / 87 (95 / 111 / 117); 16 rows 106 / 91 /
+// 105 (132 / 112 / 130), 158 / 142 / 161, 92 / 80 / 91; 24: 138 / 105 / 113 (165 / 150 / 135), 209 / 155 / 173 (247 / 211 / 213), 168 / 153 / 139 (281 / 265 / 226); 38: 192 / 152 / 127 (222 / 188 / 155),
+// 289 / 231 / 195, 208 / 196 / 160.  Tiles of 16 as long as next to no expert needs two, and no launch a second round of workgroups for them.  (The line from 32 to 64 was drawn by the forms
+// before, OLMoE 18 rows 149 / 139; it is early by the present ones: 18 rows 94 / 109 (115 / 133), 141 / 163 (190 / 212), 118 / 127 (214 / 221).)
 int grouped_gemm_tile_rows_q6k_down(const ExpertBanks &b, int n_assign) {
     const double avg = (double)n_assign / (double)(b.n_experts > 0 ? b.n_experts : 1);
     const double e16 = expected_tiles(avg, 16.0), e32 = expected_tiles(avg, 32.0);
